@@ -317,6 +317,38 @@ __global__ __launch_bounds__(kBlock) void attention_context_kernel(const T *__re
 constexpr float kMaskedScore = -10000.0f;
 constexpr float kLog2e = 1.4426950408889634f;
 
+// Sequence lengths that are not a multiple of 32 run on the same kernels with the last key tile filled up: rows past
+// the end are read from the last valid row (finite values, no load under a branch), such a key's additive mask is
+// kNoKey -- its exp is exactly 0 whatever the other keys are, also in a sequence whose mask keeps none -- and such a
+// query row is computed and not stored.  (Before, such a length took 2 * min(batch, heads) library launches and a
+// softmax launch per layer: a BERT-base request of 20 x 100 tokens in fp32 6.20 -> 3.12 ms, 7 x 50 in fp16 2.38 -> 0.83 ms,
+// 5 x 24 in fp32 1.87 -> 0.84 ms.)
+constexpr float kNoKey = -1e30f;
+
+// Additive mask of key i in units of log 2; `row` is the sequence's mask row or null.
+__device__ __forceinline__ float additive_mask(const int8_t *row, int i, int seq) {
+    if (i >= seq) return kNoKey;
+    return row != nullptr && !row[i] ? kMaskedScore * kLog2e : 0.f;
+}
+
+// Bit kt of any: tile kt (32 keys) has a kept key; of all: its 32 keys exist and are all kept.  Read as bytes, 64 per
+// wavefront and load, so any alignment and length will do.  The same on every lane.
+__device__ __forceinline__ void key_tile_bits(const int8_t *row, int seq, int tiles, unsigned &any, unsigned &all) {
+    const int lane = threadIdx.x & (kWave - 1);
+    any = 0, all = 0;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+        if (2 * u < tiles) {
+            const int i = u * kWave + lane;
+            const int8_t m = row[i < seq ? i : seq - 1];
+            const unsigned long long kept = __ballot(i < seq && m != 0);
+            const unsigned lo = (unsigned) kept, hi = (unsigned) (kept >> 32);
+            any |= (lo != 0 ? 1u : 0u) << (2 * u) | (hi != 0 ? 2u : 0u) << (2 * u);
+            all |= (lo == ~0u ? 1u : 0u) << (2 * u) | (hi == ~0u ? 2u : 0u) << (2 * u);
+        }
+    }
+}
+
 // A probability from its exponential: times the reciprocal of the row's sum (one division per query instead of one
 // per score; at 128 sequences x 12 heads x 32 keys in fp32 the divisions were 0.7 us of a 12.4 us launch).  Within
 // 1.5 units in the last place of the quotient the reference forms (src/cuBERT/op/Softmax.cpp:32-35).
@@ -332,17 +364,19 @@ constexpr size_t fused_lds_bytes() {
     return (size_t) S * (D + V) * sizeof(T) + (size_t) D * (S + V) * sizeof(T) + S * sizeof(float);
 }
 
-// grid = batch * heads workgroups of KT wavefronts; seq = 32 * KT.
-template <typename T, int D, int KT, bool SPLIT>
+// grid = batch * heads workgroups of KT wavefronts; seq = 32 * KT, or with RAGGED 32 * (KT - 1) < seq_ragged < 32 * KT.
+template <typename T, int D, int KT, bool SPLIT, bool RAGGED>
 __global__ __launch_bounds__(KT * kWave) void attention_fused_kernel(const T *__restrict__ q, const T *__restrict__ k,
                                                                      const T *__restrict__ v, int ld,
                                                                      const int8_t *__restrict__ mask,
                                                                      T *__restrict__ ctx, int ld_ctx, float alpha,
-                                                                     int heads, SplitOut split) {
+                                                                     int heads, int seq_ragged, SplitOut split) {
     constexpr int V = Mma<T>::kVec;
     constexpr int kSteps = D / 2 / V;
     constexpr int kColTiles = D / 32;
     constexpr int S = KT * 32;
+    const int seq = RAGGED ? seq_ragged : S;
+    auto valid_row = [&](int row) { return RAGGED && row >= seq ? seq - 1 : row; };
     constexpr int kThreads = KT * kWave;
     constexpr int kPitchK = D + V;  // +16 bytes: conflict-free 16-byte reads down a column of rows
     constexpr int kPitchV = S + V;
@@ -356,11 +390,11 @@ __global__ __launch_bounds__(KT * kWave) void attention_fused_kernel(const T *__
     const int qt = wave_in_block();
     const int bh = blockIdx.x;
     const int b = bh / heads, h = bh - b * heads;
-    const T *k_head = k + (size_t) b * S * ld + (size_t) h * D;
-    const T *v_head = v + (size_t) b * S * ld + (size_t) h * D;
+    const T *k_head = k + (size_t) b * seq * ld + (size_t) h * D;
+    const T *v_head = v + (size_t) b * seq * ld + (size_t) h * D;
 
     // this wavefront's query operand, straight from memory: lane half hh takes head columns hh*D/2 .. +D/2
-    const T *q_row = q + ((size_t) b * S + qt * 32 + r) * ld + (size_t) h * D + hh * (D / 2);
+    const T *q_row = q + ((size_t) b * seq + valid_row(qt * 32 + r)) * ld + (size_t) h * D + hh * (D / 2);
     Vec<T, V> qv[kSteps];
 #pragma unroll
     for (int t = 0; t < kSteps; ++t) qv[t] = load_vec<T, V>(q_row + t * V);
@@ -376,7 +410,7 @@ __global__ __launch_bounds__(KT * kWave) void attention_fused_kernel(const T *__
     for (int u = 0; u < kLoadsK; ++u) {
         const int idx = threadIdx.x + u * kThreads;
         const int row = idx / kVecPerRow, c = idx - row * kVecPerRow;
-        kreg[u] = load_vec<T, V>(k_head + (size_t) row * ld + c * V);
+        kreg[u] = load_vec<T, V>(k_head + (size_t) valid_row(row) * ld + c * V);
     }
 #pragma unroll
     for (int u = 0; u < kLoadsV; ++u) {
@@ -386,11 +420,11 @@ __global__ __launch_bounds__(KT * kWave) void attention_fused_kernel(const T *__
         const int run = in_tile >> 1, half = in_tile & 1;
 #pragma unroll
         for (int e = 0; e < V; ++e) {
-            vreg[u].v[e] = v_head[(size_t) (kt * 32 + acc_row(run * V + e, half)) * ld + j];
+            vreg[u].v[e] = v_head[(size_t) valid_row(kt * 32 + acc_row(run * V + e, half)) * ld + j];
         }
     }
     for (int i = threadIdx.x; i < S; i += kThreads) {
-        s_mask[i] = (mask != nullptr && !mask[(size_t) b * S + i]) ? kMaskedScore * kLog2e : 0.f;
+        s_mask[i] = additive_mask(mask != nullptr ? mask + (size_t) b * seq : nullptr, i, seq);
     }
 #pragma unroll
     for (int u = 0; u < kLoadsK; ++u) {
@@ -470,11 +504,12 @@ __global__ __launch_bounds__(KT * kWave) void attention_fused_kernel(const T *__
         }
     }
     // lane holds output column jt*32 + r and 16 query rows
-    const size_t first_row = (size_t) b * S + qt * 32;
+    const size_t first_row = (size_t) b * seq + qt * 32;
 #pragma unroll
     for (int jt = 0; jt < kColTiles; ++jt) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
+            if (RAGGED && qt * 32 + acc_row(i, hh) >= seq) continue;
             store_context<T, SPLIT>(ctx, ld_ctx, first_row + acc_row(i, hh), h * D + jt * 32 + r, out[jt][i], split);
         }
     }
@@ -502,7 +537,8 @@ __global__ __launch_bounds__(KT * kWave) void attention_fused_kernel(const T *__
 //    different banks;
 //  * the context tile leaves through LDS as full 128-byte row segments (4 stores per lane instead of 32 two-byte
 //    ones).
-// Needs the mask (if any) readable as words and ctx rows 16-byte aligned; the launcher falls back otherwise.
+// Needs the mask (if any) readable as words (RAGGED: as bytes) and ctx rows 16-byte aligned; the launcher falls back
+// otherwise.
 typedef _Float16 v4f16 __attribute__((ext_vector_type(4)));
 
 // ds_read_b64_tr_b16: see the comment above for what arrives in which lane.
@@ -526,18 +562,20 @@ constexpr size_t fused_half_lds_bytes() {
     return (size_t) S * (D + 8) * 2 + (size_t) S * fused_half_v_pitch<D>() * 2 + S * sizeof(float);
 }
 
-template <int D, int KT>
+template <int D, int KT, bool RAGGED>
 __global__ __launch_bounds__(KT * kWave) void attention_fused_half_kernel(const half_t *__restrict__ q,
                                                                           const half_t *__restrict__ k,
                                                                           const half_t *__restrict__ v, int ld,
                                                                           const int8_t *__restrict__ mask,
                                                                           half_t *__restrict__ ctx, int ld_ctx,
-                                                                          float alpha, int heads) {
+                                                                          float alpha, int heads, int seq_ragged) {
     typedef half_t T;
     constexpr int V = 8;
     constexpr int kSteps = D / 2 / V;
     constexpr int kColTiles = D / 32;
     constexpr int S = KT * 32;
+    const int seq = RAGGED ? seq_ragged : S;
+    auto valid_row = [&](int row) { return RAGGED && row >= seq ? seq - 1 : row; };
     constexpr int kThreads = KT * kWave;
     constexpr int kPitchK = D + V;
     constexpr int kPitchV = fused_half_v_pitch<D>();  // halves per row of V
@@ -553,10 +591,10 @@ __global__ __launch_bounds__(KT * kWave) void attention_fused_half_kernel(const 
     const int qt = wave_in_block();
     const int bh = blockIdx.x;
     const int b = bh / heads, h = bh - b * heads;
-    const T *k_head = k + (size_t) b * S * ld + (size_t) h * D;
-    const T *v_head = v + (size_t) b * S * ld + (size_t) h * D;
+    const T *k_head = k + (size_t) b * seq * ld + (size_t) h * D;
+    const T *v_head = v + (size_t) b * seq * ld + (size_t) h * D;
 
-    const T *q_row = q + ((size_t) b * S + qt * 32 + r) * ld + (size_t) h * D + hh * (D / 2);
+    const T *q_row = q + ((size_t) b * seq + valid_row(qt * 32 + r)) * ld + (size_t) h * D + hh * (D / 2);
     Vec<T, V> qv[kSteps];
 #pragma unroll
     for (int t = 0; t < kSteps; ++t) qv[t] = load_vec<T, V>(q_row + t * V);
@@ -570,18 +608,22 @@ __global__ __launch_bounds__(KT * kWave) void attention_fused_half_kernel(const 
     for (int u = 0; u < kLoads; ++u) {
         const int idx = threadIdx.x + u * kThreads;
         const int row = idx / kVecPerRow, c = idx - row * kVecPerRow;
-        kreg[u] = load_vec<T, V>(k_head + row * ld + c * V);
+        kreg[u] = load_vec<T, V>(k_head + valid_row(row) * ld + c * V);
     }
 #pragma unroll
     for (int u = 0; u < kLoads; ++u) {
         const int idx = threadIdx.x + u * kThreads;
         const int row = idx / kVecPerRow, c = idx - row * kVecPerRow;
-        vreg[u] = load_vec<T, V>(v_head + row * ld + c * V);
+        vreg[u] = load_vec<T, V>(v_head + valid_row(row) * ld + c * V);
     }
 
     // bit kt of keep_any: tile kt has a kept key; of keep_all: all of its keys are kept (workgroup-uniform)
-    unsigned keep_any = kAllTiles, keep_all = kAllTiles;
-    if (mask != nullptr) {
+    unsigned keep_any = kAllTiles, keep_all = RAGGED ? kAllTiles >> 1 : kAllTiles;
+    if (RAGGED && mask != nullptr) {
+        key_tile_bits(mask + (size_t) b * seq, seq, KT, keep_any, keep_all);
+        if (keep_any == 0) keep_any = kAllTiles;
+    }
+    if (!RAGGED && mask != nullptr) {
         const uint32_t *words = reinterpret_cast<const uint32_t *>(mask + (size_t) b * S);
         keep_any = 0, keep_all = 0;
 #pragma unroll
@@ -605,7 +647,7 @@ __global__ __launch_bounds__(KT * kWave) void attention_fused_half_kernel(const 
     const bool general_tiles = (keep_any & ~keep_all) != 0;  // uniform
     if (general_tiles) {
         for (int i = threadIdx.x; i < S; i += kThreads) {
-            s_mask[i] = !mask[(size_t) b * S + i] ? kMaskedScore * kLog2e : 0.f;  // (mask is not null here)
+            s_mask[i] = additive_mask(mask != nullptr ? mask + (size_t) b * seq : nullptr, i, seq);
         }
     }
 #pragma unroll
@@ -727,10 +769,11 @@ __global__ __launch_bounds__(KT * kWave) void attention_fused_half_kernel(const 
     constexpr int kChunks = D / V;             // 16-byte chunks per row
     constexpr int kRowsPerPass = kWave / kChunks;
     const int chunk = lane % kChunks, row_in = lane / kChunks;
-    T *dst = ctx + ((size_t) b * S + qt * 32) * ld_ctx + (size_t) h * D + chunk * V;
+    T *dst = ctx + ((size_t) b * seq + qt * 32) * ld_ctx + (size_t) h * D + chunk * V;
 #pragma unroll
     for (int pass = 0; pass < 32 / kRowsPerPass; ++pass) {
         const int row = row_in + kRowsPerPass * pass;
+        if (RAGGED && qt * 32 + row >= seq) continue;
         store_vec<T, V>(dst + row * ld_ctx, load_vec<T, V>(stage + row * kPitchOut + chunk * V));
     }
 }
@@ -742,12 +785,12 @@ __global__ __launch_bounds__(KT * kWave) void attention_fused_half_kernel(const 
 // used by one lane only), the four partial score tiles are added in wavefront order through LDS, every
 // wavefront repeats the (cheap) softmax, and P V is split into (column tile, key half), the two key halves
 // meeting in LDS again.  Same arithmetic and rounding as attention_fused_kernel, other summation order.
-template <typename T, bool SPLIT>
+template <typename T, bool SPLIT, bool RAGGED>
 __global__ __launch_bounds__(4 * kWave) void attention_small_kernel(const T *__restrict__ q, const T *__restrict__ k,
                                                                     const T *__restrict__ v, int ld,
                                                                     const int8_t *__restrict__ mask,
                                                                     T *__restrict__ ctx, int ld_ctx, float alpha,
-                                                                    int heads, SplitOut split) {
+                                                                    int heads, int seq_ragged, SplitOut split) {
     constexpr int D = 64, S = 32;
     constexpr int V = Mma<T>::kVec;
     constexpr int kSteps = D / 8 / V;  // operand vectors per lane and contraction: a quarter of D over two lane halves
@@ -757,25 +800,36 @@ __global__ __launch_bounds__(4 * kWave) void attention_small_kernel(const T *__r
     const int w = wave_in_block();
     const int bh = blockIdx.x;
     const int b = bh / heads, h = bh - b * heads;
-    const size_t row0 = (size_t) b * S;
+    const int seq = RAGGED ? seq_ragged : S;
+    auto valid_row = [&](int row) { return RAGGED && row >= seq ? seq - 1 : row; };
+    const size_t row0 = (size_t) b * seq;
 
     // every load of the wavefront is requested here
     const size_t d0 = (size_t) h * D + w * (D / 4) + hh * (D / 8);
     Vec<T, V> qv[kSteps], kv[kSteps];
 #pragma unroll
     for (int t = 0; t < kSteps; ++t) {
-        qv[t] = load_vec<T, V>(q + (row0 + r) * ld + d0 + t * V);
-        kv[t] = load_vec<T, V>(k + (row0 + r) * ld + d0 + t * V);
+        qv[t] = load_vec<T, V>(q + (row0 + valid_row(r)) * ld + d0 + t * V);
+        kv[t] = load_vec<T, V>(k + (row0 + valid_row(r)) * ld + d0 + t * V);
     }
     const int jt = w & 1, kh = w >> 1;  // second contraction: output columns jt*32 .. +31, keys of registers kh*8 .. +7
     T vreg[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-        vreg[i] = v[(row0 + acc_row(kh * 8 + i, hh)) * ld + (size_t) h * D + jt * 32 + r];
+        vreg[i] = v[(row0 + valid_row(acc_row(kh * 8 + i, hh))) * ld + (size_t) h * D + jt * 32 + r];
     }
     float add[16];  // additive mask of this lane's 16 keys, in units of log 2
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
+        if (RAGGED) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int key = g * 8 + hh * 4 + e;
+                const int8_t kept = mask != nullptr ? mask[row0 + valid_row(key)] : (int8_t) 1;
+                add[g * 4 + e] = key >= seq ? kNoKey : (kept ? 0.f : kMaskedScore * kLog2e);
+            }
+            continue;
+        }
         uint32_t word = 0x01010101u;
         if (mask != nullptr) word = *reinterpret_cast<const uint32_t *>(mask + row0 + g * 8 + hh * 4);
 #pragma unroll
@@ -834,6 +888,7 @@ __global__ __launch_bounds__(4 * kWave) void attention_small_kernel(const T *__r
     if (kh == 0) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
+            if (RAGGED && acc_row(i, hh) >= seq) continue;
             store_context<T, SPLIT>(ctx, ld_ctx, (size_t) row0 + acc_row(i, hh), h * D + jt * 32 + r,
                              out[i] + s_part[jt][i * kWave + lane], split);
         }
@@ -853,8 +908,8 @@ __global__ __launch_bounds__(4 * kWave) void attention_small_kernel(const T *__r
 // masked key's score is 10000 below every unmasked one of its query, its exp is exactly 0 in fp32, so it adds
 // nothing to the sum or the context as long as the sequence has one unmasked key (a sequence without any keeps
 // all its tiles: there the shift cancels and the softmax runs over the raw scores, as in the reference).  Every
-// query row, padded or not, is still computed.  skip_masked_tiles = 0 (a mask that cannot be read as 32-bit
-// words) computes all tiles.
+// query row, padded or not, is still computed.  skip_masked_tiles = 0: the mask cannot be read as 32-bit words and is
+// read as bytes.
 template <typename T, int D, bool SPLIT>
 __global__ __launch_bounds__(1024) void attention_flash_kernel(const T *__restrict__ q, const T *__restrict__ k,
                                                                const T *__restrict__ v, int ld,
@@ -866,7 +921,8 @@ __global__ __launch_bounds__(1024) void attention_flash_kernel(const T *__restri
     constexpr int kColTiles = D / 32;
     constexpr int kChunk = 2;  // key tiles per step
     constexpr int kPitchK = D + V;
-    const int S = seq, KT = seq / 32;
+    const int KT = (seq + 31) / 32, S = KT * 32;  // (the last key tile may be filled up: kNoKey)
+    auto valid_row = [&](int row) { return row < seq ? row : seq - 1; };
     const int threads = blockDim.x;  // = KT * 64
     const int pitch_v = S + V;
     extern __shared__ __align__(16) unsigned char smem[];
@@ -881,24 +937,28 @@ __global__ __launch_bounds__(1024) void attention_flash_kernel(const T *__restri
     const int bh = blockIdx.x;
     const int rank = bh / heads, h = bh - rank * heads;
     const int b = order != nullptr ? order[rank] : rank;  // workgroup-uniform
-    const T *k_head = k + (size_t) b * S * ld + (size_t) h * D;
-    const T *v_head = v + (size_t) b * S * ld + (size_t) h * D;
+    const T *k_head = k + (size_t) b * seq * ld + (size_t) h * D;
+    const T *v_head = v + (size_t) b * seq * ld + (size_t) h * D;
 
-    const T *q_row = q + ((size_t) b * S + qt * 32 + r) * ld + (size_t) h * D + hh * (D / 2);
+    const T *q_row = q + ((size_t) b * seq + valid_row(qt * 32 + r)) * ld + (size_t) h * D + hh * (D / 2);
     Vec<T, V> qv[kSteps];
 #pragma unroll
     for (int t = 0; t < kSteps; ++t) qv[t] = load_vec<T, V>(q_row + t * V);
 
-    // bit kt: key tile kt has an unmasked key (workgroup-uniform: scalar loads of the mask row as words)
+    // bit kt: key tile kt has an unmasked key (workgroup-uniform: scalar loads of the mask row as words, or bytes and
+    // ballots where the row cannot be read as words)
     unsigned live = 0;
     if (mask != nullptr && skip_masked_tiles) {
-        const uint32_t *words = reinterpret_cast<const uint32_t *>(mask + (size_t) b * S);
+        const uint32_t *words = reinterpret_cast<const uint32_t *>(mask + (size_t) b * seq);
         for (int kt = 0; kt < KT; ++kt) {
             uint32_t any = 0;
 #pragma unroll
             for (int i = 0; i < 8; ++i) any |= words[kt * 8 + i];
             live |= (any != 0 ? 1u : 0u) << kt;
         }
+    } else if (mask != nullptr) {
+        unsigned all;
+        key_tile_bits(mask + (size_t) b * seq, seq, KT, live, all);
     }
     if (live == 0) live = KT >= 32 ? ~0u : (1u << KT) - 1u;
     live = __builtin_amdgcn_readfirstlane(live);
@@ -912,7 +972,7 @@ __global__ __launch_bounds__(1024) void attention_flash_kernel(const T *__restri
         const int idx = threadIdx.x + u * threads;
         const int row = idx / kVecPerRow, c = idx - row * kVecPerRow;
         kreg[u] = Vec<T, V>{};
-        if ((live >> (row >> 5)) & 1u) kreg[u] = load_vec<T, V>(k_head + (size_t) row * ld + c * V);
+        if ((live >> (row >> 5)) & 1u) kreg[u] = load_vec<T, V>(k_head + (size_t) valid_row(row) * ld + c * V);
     }
 #pragma unroll
     for (int u = 0; u < kLoads; ++u) {
@@ -924,12 +984,12 @@ __global__ __launch_bounds__(1024) void attention_flash_kernel(const T *__restri
         if ((live >> kt) & 1u) {
 #pragma unroll
             for (int e = 0; e < V; ++e) {
-                vreg[u].v[e] = v_head[(size_t) (kt * 32 + acc_row(run * V + e, half)) * ld + j];
+                vreg[u].v[e] = v_head[(size_t) valid_row(kt * 32 + acc_row(run * V + e, half)) * ld + j];
             }
         }
     }
     for (int i = threadIdx.x; i < S; i += threads) {
-        s_mask[i] = (mask != nullptr && !mask[(size_t) b * S + i]) ? kMaskedScore * kLog2e : 0.f;
+        s_mask[i] = additive_mask(mask != nullptr ? mask + (size_t) b * seq : nullptr, i, seq);
     }
 #pragma unroll
     for (int u = 0; u < kLoads; ++u) {
@@ -1048,7 +1108,7 @@ __global__ __launch_bounds__(1024) void attention_flash_kernel(const T *__restri
     if (hh == 0) factor[r] = 1.f / l;
     __builtin_amdgcn_s_waitcnt(0xc07f);
     __builtin_amdgcn_wave_barrier();
-    const size_t first_row = (size_t) b * S + qt * 32;
+    const size_t first_row = (size_t) b * seq + qt * 32;
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
         const Vec<float, 4> fr = load_vec<float, 4>(factor + g * 8 + hh * 4);
@@ -1056,6 +1116,7 @@ __global__ __launch_bounds__(1024) void attention_flash_kernel(const T *__restri
         for (int jt = 0; jt < kColTiles; ++jt) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
+                if (qt * 32 + acc_row(g * 4 + e, hh) >= seq) continue;
                 store_context<T, SPLIT>(ctx, ld_ctx, first_row + acc_row(g * 4 + e, hh), h * D + jt * 32 + r,
                                  out[jt][g * 4 + e] * fr.v[e], split);
             }
@@ -1072,10 +1133,10 @@ __global__ __launch_bounds__(1024) void attention_flash_kernel(const T *__restri
 // and, since the LDS no longer grows with the sequence, fp32 fits as well.  Measured at batch 64, 12 heads, ~4 live
 // tiles per sequence: 54.6 against 59.5 us; groups of 2 or 8 tiles are slower.  Arithmetic and rounding are those of
 // attention_flash_kernel.
-template <typename T, int D, bool SPLIT>
+template <typename T, int D, bool SPLIT, bool ANY_SEQ>
 __global__ __launch_bounds__(1024) void attention_flash_grouped_kernel(
     const T *__restrict__ q, const T *__restrict__ k, const T *__restrict__ v, int ld, const int8_t *__restrict__ mask,
-    T *__restrict__ ctx, int ld_ctx, float alpha, int heads, int skip_masked_tiles, SplitOut split,
+    T *__restrict__ ctx, int ld_ctx, float alpha, int heads, int any_seq, int skip_masked_tiles, SplitOut split,
     const int *__restrict__ order, int order_has_records) {
     constexpr int V = Mma<T>::kVec;
     constexpr int kSteps = D / 2 / V;
@@ -1089,7 +1150,9 @@ __global__ __launch_bounds__(1024) void attention_flash_grouped_kernel(
     constexpr int kVecPerRow = D / V;
     constexpr int kLoads = G * 32 * kVecPerRow / kThreads;  // = 1: vectors per thread for K, slot groups for V^T
     static_assert(kLoads == 1, "one K vector and one V^T slot group per thread");
-    constexpr int S = kSeq, KT = kSeq / 32;
+    const int seq = ANY_SEQ ? any_seq : kSeq;
+    const int KT = ANY_SEQ ? (seq + 31) / 32 : kSeq / 32, S = KT * 32;
+    auto valid_row = [&](int row) { return ANY_SEQ && row >= seq ? seq - 1 : row; };
     extern __shared__ __align__(16) unsigned char smem[];
     T *s_k = reinterpret_cast<T *>(smem);                                      // [G * 32][kPitchK]
     T *s_vt = s_k + G * 32 * kPitchK;                                          // [D][kPitchV], keys in slot order
@@ -1103,10 +1166,10 @@ __global__ __launch_bounds__(1024) void attention_flash_grouped_kernel(
     const int rank = bh / heads, h = bh - rank * heads;
     const int b = order != nullptr ? order[rank] : rank;  // workgroup-uniform
     const int qt = wave;
-    const T *k_head = k + (size_t) b * S * ld + (size_t) h * D;
-    const T *v_head = v + (size_t) b * S * ld + (size_t) h * D;
+    const T *k_head = k + (size_t) b * seq * ld + (size_t) h * D;
+    const T *v_head = v + (size_t) b * seq * ld + (size_t) h * D;
 
-    const T *q_row = q + ((size_t) b * S + qt * 32 + r) * ld + (size_t) h * D + hh * (D / 2);
+    const T *q_row = q + ((size_t) b * seq + valid_row(qt * 32 + r)) * ld + (size_t) h * D + hh * (D / 2);
     Vec<T, V> qv[kSteps];
 #pragma unroll
     for (int t = 0; t < kSteps; ++t) qv[t] = load_vec<T, V>(q_row + t * V);
@@ -1117,7 +1180,7 @@ __global__ __launch_bounds__(1024) void attention_flash_grouped_kernel(
     // (workgroup-uniform either way).
     int n_live = 0;
     unsigned long long tile_list = 0;
-    if (order != nullptr && order_has_records && mask != nullptr && skip_masked_tiles) {
+    if (order != nullptr && order_has_records && mask != nullptr && (skip_masked_tiles || seq % 32 != 0)) {
         const int batch = (int) gridDim.x / heads;
         const int *rec = order + 4 * (size_t) batch + 4 * (size_t) rank;
         n_live = rec[0];
@@ -1128,12 +1191,19 @@ __global__ __launch_bounds__(1024) void attention_flash_grouped_kernel(
         }
     } else {
         if (mask != nullptr && skip_masked_tiles) {
-            const uint32_t *words = reinterpret_cast<const uint32_t *>(mask + (size_t) b * S);
+            const uint32_t *words = reinterpret_cast<const uint32_t *>(mask + (size_t) b * seq);
             for (int kt = 0; kt < KT; ++kt) {
                 uint32_t any = 0;
 #pragma unroll
                 for (int i = 0; i < 8; ++i) any |= words[kt * 8 + i];
                 if (any != 0) tile_list |= (unsigned long long) kt << (4 * n_live++);
+            }
+        }
+        if (ANY_SEQ && mask != nullptr && !skip_masked_tiles) {  // (the row cannot be read as words)
+            unsigned any, all;
+            key_tile_bits(mask + (size_t) b * seq, seq, KT, any, all);
+            for (int kt = 0; kt < KT; ++kt) {
+                if ((any >> kt) & 1u) tile_list |= (unsigned long long) kt << (4 * n_live++);
             }
         }
         if (n_live == 0) {  // no mask, or no kept key at all: every tile
@@ -1146,7 +1216,7 @@ __global__ __launch_bounds__(1024) void attention_flash_grouped_kernel(
                 ((unsigned long long) (unsigned) __builtin_amdgcn_readfirstlane((int) (unsigned) (tile_list >> 32)) << 32);
 
     for (int i = threadIdx.x; i < S; i += kThreads) {
-        s_mask[i] = (mask != nullptr && !mask[(size_t) b * S + i]) ? kMaskedScore * kLog2e : 0.f;
+        s_mask[i] = additive_mask(mask != nullptr ? mask + (size_t) b * seq : nullptr, i, seq);
     }
 
     const float scale = alpha * kLog2e;
@@ -1169,7 +1239,7 @@ __global__ __launch_bounds__(1024) void attention_flash_grouped_kernel(
             const int slot = idx / (32 * kVecPerRow), within = idx - slot * (32 * kVecPerRow);
             const int row = within / kVecPerRow, c = within - row * kVecPerRow;
             kreg[u] = Vec<T, V>{};
-            if (slot < in_group) kreg[u] = load_vec<T, V>(k_head + (size_t) (tile_of(slot) * 32 + row) * ld + c * V);
+            if (slot < in_group) kreg[u] = load_vec<T, V>(k_head + (size_t) valid_row(tile_of(slot) * 32 + row) * ld + c * V);
         }
 #pragma unroll
         for (int u = 0; u < kLoads; ++u) {
@@ -1182,7 +1252,7 @@ __global__ __launch_bounds__(1024) void attention_flash_grouped_kernel(
                 const int kt = tile_of(slot);
 #pragma unroll
                 for (int e = 0; e < V; ++e) {
-                    vreg[u].v[e] = v_head[(size_t) (kt * 32 + acc_row(run * V + e, half)) * ld + j];
+                    vreg[u].v[e] = v_head[(size_t) valid_row(kt * 32 + acc_row(run * V + e, half)) * ld + j];
                 }
             }
         }
@@ -1200,6 +1270,7 @@ __global__ __launch_bounds__(1024) void attention_flash_grouped_kernel(
             store_vec<T, V>(s_vt + j * kPitchV + grp * V, vreg[u]);
         }
         __syncthreads();
+        if (ANY_SEQ && qt >= KT) continue;  // a wavefront without queries helps with the loads only
         for (int s0 = 0; s0 < in_group; s0 += kChunk) {  // the group's tiles in ascending order, kChunk per step
             int tiles[kChunk], slots[kChunk];
 #pragma unroll
@@ -1283,11 +1354,12 @@ __global__ __launch_bounds__(1024) void attention_flash_grouped_kernel(
             }
         }
     }
+    if (ANY_SEQ && qt >= KT) return;
     // divide row (query) i by its sum
     if (hh == 0) factor[r] = 1.f / l;
     __builtin_amdgcn_s_waitcnt(0xc07f);
     __builtin_amdgcn_wave_barrier();
-    const size_t first_row = (size_t) b * S + qt * 32;
+    const size_t first_row = (size_t) b * seq + qt * 32;
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
         const Vec<float, 4> fr = load_vec<float, 4>(factor + g * 8 + hh * 4);
@@ -1295,6 +1367,7 @@ __global__ __launch_bounds__(1024) void attention_flash_grouped_kernel(
         for (int jt = 0; jt < kColTiles; ++jt) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
+                if (ANY_SEQ && qt * 32 + acc_row(g * 4 + e, hh) >= seq) continue;
                 store_context<T, SPLIT>(ctx, ld_ctx, first_row + acc_row(g * 4 + e, hh), h * D + jt * 32 + r,
                                         out[jt][g * 4 + e] * fr.v[e], split);
             }
@@ -1315,32 +1388,45 @@ constexpr int kOrderMaxBatch = 4096;
 // sequence at position i -- {number of live tiles, their tile numbers in ascending order 4 bits each (low word, high
 // word), the live tiles as a bit mask} -- so that a long-sequence kernel gets its list of tiles with one scalar load
 // instead of reading the mask row again.  8 * batch ints in all.
-__global__ __launch_bounds__(kBlock) void attention_order_kernel(const int8_t *__restrict__ mask, int batch, int seq,
-                                                                 int *__restrict__ order) {
+// A wavefront reads four mask rows at a time, 64 bytes per load, all requested first: any length and alignment.
+constexpr int kOrderThreads = 1024;
+__global__ __launch_bounds__(kOrderThreads) void attention_order_kernel(const int8_t *__restrict__ mask, int batch, int seq,
+                                                                        int *__restrict__ order) {
     __shared__ unsigned char tiles_of[kOrderMaxBatch];
     __shared__ unsigned short bits_of[kOrderMaxBatch];
     __shared__ int bucket[20];  // [t]: sequences with t live tiles (t <= 16), then their first position
-    const int key_tiles = seq / 32;
+    constexpr int kRows = 4;
+    const int key_tiles = (seq + 31) / 32;
+    const int lane = threadIdx.x & (kWave - 1);
     if (threadIdx.x < 20) bucket[threadIdx.x] = 0;
     __syncthreads();
-    for (int b = threadIdx.x; b < batch; b += kBlock) {
-        const uint32_t *words = reinterpret_cast<const uint32_t *>(mask + (size_t) b * seq);
-        int live = 0;
-        unsigned bits = 0;
-        for (int kt = 0; kt < key_tiles; ++kt) {
-            uint32_t any = 0;
+    for (int b0 = wave_in_block() * kRows; b0 < batch; b0 += kOrderThreads / kWave * kRows) {
+        int8_t m[kRows][8];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) any |= words[kt * 8 + i];
-            live += any != 0;
-            bits |= (any != 0 ? 1u : 0u) << kt;
+        for (int t = 0; t < kRows; ++t) {
+            const int8_t *row = mask + (size_t) (b0 + t < batch ? b0 + t : batch - 1) * seq;
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const int i = u * kWave + lane;
+                m[t][u] = row[i < seq ? i : seq - 1];
+            }
         }
-        if (live == 0) {  // no kept key: the kernels compute every tile
-            live = key_tiles;
-            bits = (1u << key_tiles) - 1u;
+#pragma unroll
+        for (int t = 0; t < kRows; ++t) {
+            unsigned bits = 0;
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const unsigned long long kept = __ballot(u * kWave + lane < seq && m[t][u] != 0);
+                bits |= ((unsigned) kept != 0 ? 1u : 0u) << (2 * u) | (kept >> 32 != 0 ? 2u : 0u) << (2 * u);
+            }
+            if (bits == 0) bits = (1u << key_tiles) - 1u;  // no kept key: the kernels compute every tile
+            if (lane == 0 && b0 + t < batch) {
+                const int live = __popc(bits);
+                tiles_of[b0 + t] = (unsigned char) live;
+                bits_of[b0 + t] = (unsigned short) bits;
+                atomicAdd(&bucket[live], 1);
+            }
         }
-        tiles_of[b] = (unsigned char) live;
-        bits_of[b] = (unsigned short) bits;
-        atomicAdd(&bucket[live], 1);
     }
     __syncthreads();
     if (threadIdx.x == 0) {  // first position of each count, largest count first
@@ -1352,7 +1438,7 @@ __global__ __launch_bounds__(kBlock) void attention_order_kernel(const int8_t *_
         }
     }
     __syncthreads();
-    for (int b = threadIdx.x; b < batch; b += kBlock) {
+    for (int b = threadIdx.x; b < batch; b += kOrderThreads) {
         const int at = atomicAdd(&bucket[tiles_of[b]], 1);
         order[at] = b;
         const unsigned bits = bits_of[b];
@@ -1372,18 +1458,21 @@ __global__ __launch_bounds__(kBlock) void attention_order_kernel(const int8_t *_
 int attention_order(const int8_t *mask, int batch, int seq, int *order, void *stream) {
     if (!mask || !order || batch < 0 || seq <= 0) return CUBERT_BAD_ARGUMENT;
     if (batch == 0) return 0;
-    if (seq % 32 != 0 || seq > 512 || batch > kOrderMaxBatch || !is_aligned(mask, 4) || !is_aligned(order, 16)) {
+    // (up to 128 keys no kernel takes an order; rows of whole words have to be aligned as such, others need not be)
+    if ((seq % 32 != 0 && seq <= 128) || seq > 512 || batch > kOrderMaxBatch || (seq % 32 == 0 && !is_aligned(mask, 4)) ||
+        !is_aligned(order, 16)) {
         return CUBERT_UNSUPPORTED;
     }
-    return launch_untimed(attention_order_kernel, dim3(1), dim3(kBlock), 0u, (hipStream_t) stream, mask, batch, seq,
+    return launch_untimed(attention_order_kernel, dim3(1), dim3(kOrderThreads), 0u, (hipStream_t) stream, mask, batch, seq,
                           order);
 }
 
 template <typename T>
-bool shapes_ok(int batch, int heads, int seq, int head_size, int ld, std::initializer_list<const void *> ptrs) {
+bool shapes_ok(int batch, int heads, int seq, int head_size, int ld, std::initializer_list<const void *> ptrs,
+               bool any_seq = false) {
     constexpr int V = Mma<T>::kVec;
     if (batch <= 0 || heads <= 0 || seq <= 0) return false;
-    if (seq % 32 != 0 || (head_size != 32 && head_size != 64 && head_size != 128)) return false;
+    if ((seq % 32 != 0 && !any_seq) || (head_size != 32 && head_size != 64 && head_size != 128)) return false;
     if (ld % V != 0 || (long long) batch * heads > 65535) return false;
     for (const void *p : ptrs) {
         if (!is_aligned(p, 16)) return false;
@@ -1474,20 +1563,26 @@ int attention_context(const T *probs, const T *v, int ld, T *ctx, int ld_ctx, in
     }
 }
 
-template <typename T, int D, int KT>
-int launch_fused_kt(const T *q, const T *k, const T *v, int ld, const int8_t *mask, T *ctx, int ld_ctx, float alpha,
-                    int batch, int heads, SplitOut split, hipStream_t s) {
-    constexpr size_t lds = fused_lds_bytes<T, D, KT>();
+// One launch of a kernel with `lds` bytes of dynamic LDS, its limit raised first where that is needed.
+template <auto KERNEL, typename... Args>
+int launch_attention(dim3 grid, dim3 block, size_t lds, hipStream_t s, Args... args) {
     if (lds > 160 * 1024) return CUBERT_UNSUPPORTED;
+    if (lds > 48 * 1024) {
+        static std::atomic<unsigned long long> raised{0};  // per kernel
+        if (!allow_large_lds(KERNEL, raised)) return CUBERT_UNSUPPORTED;
+    }
+    return launch_lds(KERNEL, grid, block, (unsigned) lds, s, args...);
+}
+
+template <typename T, int D, int KT, bool RAGGED>
+int launch_fused_kt(const T *q, const T *k, const T *v, int ld, const int8_t *mask, T *ctx, int ld_ctx, float alpha,
+                    int batch, int heads, int seq, SplitOut split, hipStream_t s) {
+    constexpr size_t lds = fused_lds_bytes<T, D, KT>();
+    const dim3 grid(batch * heads), block(KT * kWave);
     if constexpr (sizeof(T) == 4) {
         if (split.width > 0) {
-            auto kernel = attention_fused_kernel<T, D, KT, true>;
-            if (lds > 48 * 1024) {
-                static std::atomic<unsigned long long> raised{0};  // per instantiation
-                if (!allow_large_lds(kernel, raised)) return CUBERT_UNSUPPORTED;
-            }
-            return launch_lds(kernel, dim3(batch * heads), dim3(KT * kWave), (unsigned) lds, s, q, k, v, ld, mask,
-                                  ctx, ld_ctx, alpha, heads, split);
+            return launch_attention<attention_fused_kernel<T, D, KT, true, RAGGED>>(
+                grid, block, lds, s, q, k, v, ld, mask, ctx, ld_ctx, alpha, heads, seq, split);
         }
     }
     if (split.width > 0) return CUBERT_UNSUPPORTED;
@@ -1501,67 +1596,61 @@ int launch_fused_kt(const T *q, const T *k, const T *v, int ld, const int8_t *ma
             return e == nullptr ? 0 : (std::string(e) == "general" ? 1 : (std::string(e) == "lean" ? 2 : 0));
         }();
         const bool lean = forced == 2 || (forced == 0 && batch * heads >= 1024);
-        if (lean && (mask == nullptr || is_aligned(mask, 4)) && is_aligned(ctx, 16) && ld_ctx % 8 == 0) {
-            auto kernel = attention_fused_half_kernel<D, KT>;
-            constexpr size_t half_lds = fused_half_lds_bytes<D, KT>();
-            if (half_lds > 48 * 1024) {
-                static std::atomic<unsigned long long> raised{0};  // per instantiation
-                if (!allow_large_lds(kernel, raised)) return CUBERT_UNSUPPORTED;
-            }
-            return launch_lds(kernel, dim3(batch * heads), dim3(KT * kWave), (unsigned) half_lds, s, q, k, v, ld,
-                                  mask, ctx, ld_ctx, alpha, heads);
+        if (lean && (RAGGED || mask == nullptr || is_aligned(mask, 4)) && is_aligned(ctx, 16) && ld_ctx % 8 == 0) {
+            return launch_attention<attention_fused_half_kernel<D, KT, RAGGED>>(
+                grid, block, fused_half_lds_bytes<D, KT>(), s, q, k, v, ld, mask, ctx, ld_ctx, alpha, heads, seq);
         }
     }
-    auto kernel = attention_fused_kernel<T, D, KT, false>;
-    if (lds > 48 * 1024) {
-        static std::atomic<unsigned long long> raised{0};  // per instantiation
-        if (!allow_large_lds(kernel, raised)) return CUBERT_UNSUPPORTED;
-    }
-    return launch_lds(kernel, dim3(batch * heads), dim3(KT * kWave), (unsigned) lds, s, q, k, v, ld, mask, ctx,
-                          ld_ctx, alpha, heads, split);
+    return launch_attention<attention_fused_kernel<T, D, KT, false, RAGGED>>(grid, block, lds, s, q, k, v, ld, mask, ctx,
+                                                                             ld_ctx, alpha, heads, seq, split);
 }
 
-template <typename T, int D>
+template <typename T, int D, bool RAGGED>
 int launch_fused(const T *q, const T *k, const T *v, int ld, const int8_t *mask, T *ctx, int ld_ctx, float alpha,
                  int batch, int heads, int seq, SplitOut split, hipStream_t s) {
     if constexpr (D == 64) {
         // split each problem over four wavefronts: a quarter of the dependent matrix instructions per wavefront
         // (12 problems 5.3 -> 4.7 us, 1536 problems 15.95 -> 15.0 us; not measured beyond)
-        if (seq == 32 && batch * heads <= 2048 && (mask == nullptr || is_aligned(mask, 4))) {
+        if (seq <= 32 && batch * heads <= 2048 && (RAGGED || mask == nullptr || is_aligned(mask, 4))) {
+            const dim3 grid(batch * heads), block(4 * kWave);
             if constexpr (sizeof(T) == 4) {
                 if (split.width > 0) {
-                    return launch_lds(attention_small_kernel<T, true>, dim3(batch * heads), dim3(4 * kWave), 0u, s, q,
-                                          k, v, ld, mask, ctx, ld_ctx, alpha, heads, split);
+                    return launch_attention<attention_small_kernel<T, true, RAGGED>>(grid, block, 0, s, q, k, v, ld, mask,
+                                                                                     ctx, ld_ctx, alpha, heads, seq, split);
                 }
             }
             if (split.width > 0) return CUBERT_UNSUPPORTED;
-            return launch_lds(attention_small_kernel<T, false>, dim3(batch * heads), dim3(4 * kWave), 0u, s, q, k, v,
-                                  ld, mask, ctx, ld_ctx, alpha, heads, split);
+            return launch_attention<attention_small_kernel<T, false, RAGGED>>(grid, block, 0, s, q, k, v, ld, mask, ctx,
+                                                                              ld_ctx, alpha, heads, seq, split);
         }
     }
-    switch (seq / 32) {
-        case 1:
-            return launch_fused_kt<T, D, 1>(q, k, v, ld, mask, ctx, ld_ctx, alpha, batch, heads, split, s);
-        case 2:
-            return launch_fused_kt<T, D, 2>(q, k, v, ld, mask, ctx, ld_ctx, alpha, batch, heads, split, s);
-        case 3:
-            return launch_fused_kt<T, D, 3>(q, k, v, ld, mask, ctx, ld_ctx, alpha, batch, heads, split, s);
-        case 4:
-            return launch_fused_kt<T, D, 4>(q, k, v, ld, mask, ctx, ld_ctx, alpha, batch, heads, split, s);
+#define CUBERT_FUSED_KT(KT) \
+    return launch_fused_kt<T, D, KT, RAGGED>(q, k, v, ld, mask, ctx, ld_ctx, alpha, batch, heads, seq, split, s)
+    switch ((seq + 31) / 32) {
+        case 1: CUBERT_FUSED_KT(1);
+        case 2: CUBERT_FUSED_KT(2);
+        case 3: CUBERT_FUSED_KT(3);
+        case 4: CUBERT_FUSED_KT(4);
         default: return CUBERT_UNSUPPORTED;
     }
+#undef CUBERT_FUSED_KT
 }
 
-template <typename T, int D>
+// 128 < seq <= 512.  seq 512 walks the keys in groups; other lengths hold K and V of the head in LDS where they fit
+// (fp16 always, fp32 up to 288 keys at head size 64) and walk them in groups where they do not.
+template <typename T, int D, bool SPLIT>
 int launch_flash(const T *q, const T *k, const T *v, int ld, const int8_t *mask, T *ctx, int ld_ctx, float alpha,
                  int batch, int heads, int seq, SplitOut split, const int *order, hipStream_t s) {
     constexpr int V = 16 / sizeof(T);
     if (seq > 512) return CUBERT_UNSUPPORTED;  // a workgroup has at most 16 wavefronts
-    const size_t lds = (size_t) seq * (D + V) * sizeof(T) + (size_t) D * (seq + V) * sizeof(T) +
-                       2 * (size_t) seq * sizeof(float);
-    const int skip_masked_tiles = mask != nullptr && is_aligned(mask, 4);  // seq is a multiple of 32
+    const int tiles = (seq + 31) / 32, padded = tiles * 32;
+    const size_t lds = (size_t) padded * (D + V) * sizeof(T) + (size_t) D * (padded + V) * sizeof(T) +
+                       2 * (size_t) padded * sizeof(float);
+    // the mask row can be read as 32-bit words (a whole number of them per tile, every row aligned)
+    const int skip_masked_tiles = mask != nullptr && is_aligned(mask, 4) && seq % 32 == 0;
     static const bool whole_head = getenv("CUBERT_FLASH_WHOLE") != nullptr;
-    if (seq == 512 && !whole_head) {
+    const dim3 grid(batch * heads);
+    if ((seq == 512 && !whole_head) || lds > 160 * 1024) {
         constexpr int G = 32 * V / D;
         // CUBERT_FLASH_RECORDS=0 in the environment: the kernel reads the mask row itself instead of the order array's
         // records (for comparison)
@@ -1570,35 +1659,18 @@ int launch_flash(const T *q, const T *k, const T *v, int ld, const int8_t *mask,
             return e != nullptr && std::string(e) == "0" ? 0 : 1;
         }();
         const size_t grouped_lds = ((size_t) G * 32 * (D + V) + (size_t) D * (G * 32 + V)) * sizeof(T) +
-                                   ((size_t) seq + 16 * 32) * sizeof(float);
-        if constexpr (sizeof(T) == 4) {
-            if (split.width > 0) {
-                return launch_lds(attention_flash_grouped_kernel<T, D, true>, dim3(batch * heads), dim3(1024),
-                                      (unsigned) grouped_lds, s, q, k, v, ld, mask, ctx, ld_ctx, alpha, heads,
-                                      skip_masked_tiles, split, order, use_records);
-            }
+                                   ((size_t) padded + 16 * 32) * sizeof(float);
+        if (seq == 512) {
+            return launch_attention<attention_flash_grouped_kernel<T, D, SPLIT, false>>(
+                grid, dim3(1024), grouped_lds, s, q, k, v, ld, mask, ctx, ld_ctx, alpha, heads, seq, skip_masked_tiles,
+                split, order, use_records);
         }
-        if (split.width > 0) return CUBERT_UNSUPPORTED;
-        return launch_lds(attention_flash_grouped_kernel<T, D, false>, dim3(batch * heads), dim3(1024),
-                              (unsigned) grouped_lds, s, q, k, v, ld, mask, ctx, ld_ctx, alpha, heads, skip_masked_tiles,
-                              split, order, use_records);
+        return launch_attention<attention_flash_grouped_kernel<T, D, SPLIT, true>>(
+            grid, dim3(1024), grouped_lds, s, q, k, v, ld, mask, ctx, ld_ctx, alpha, heads, seq, skip_masked_tiles, split,
+            order, use_records);
     }
-    if (lds > 160 * 1024) return CUBERT_UNSUPPORTED;
-    if constexpr (sizeof(T) == 4) {
-        if (split.width > 0) {
-            auto kernel = attention_flash_kernel<T, D, true>;
-            static std::atomic<unsigned long long> raised{0};  // per instantiation
-            if (!allow_large_lds(kernel, raised)) return CUBERT_UNSUPPORTED;
-            return launch_lds(kernel, dim3(batch * heads), dim3(seq / 32 * kWave), (unsigned) lds, s, q, k, v, ld,
-                                  mask, ctx, ld_ctx, alpha, heads, seq, skip_masked_tiles, split, order);
-        }
-    }
-    if (split.width > 0) return CUBERT_UNSUPPORTED;
-    auto kernel = attention_flash_kernel<T, D, false>;
-    static std::atomic<unsigned long long> raised{0};  // per instantiation
-    if (!allow_large_lds(kernel, raised)) return CUBERT_UNSUPPORTED;
-    return launch_lds(kernel, dim3(batch * heads), dim3(seq / 32 * kWave), (unsigned) lds, s, q, k, v, ld, mask,
-                          ctx, ld_ctx, alpha, heads, seq, skip_masked_tiles, split, order);
+    return launch_attention<attention_flash_kernel<T, D, SPLIT>>(grid, dim3(tiles * kWave), lds, s, q, k, v, ld, mask, ctx,
+                                                                 ld_ctx, alpha, heads, seq, skip_masked_tiles, split, order);
 }
 
 template <typename T>
@@ -1607,30 +1679,36 @@ int attention_fused(const T *q, const T *k, const T *v, int ld, const int8_t *ma
     if (batch == 0 || heads == 0 || seq == 0) return 0;
     if (!q || !k || !v || !ctx || batch < 0 || heads < 0 || seq < 0 || head_size <= 0) return CUBERT_BAD_ARGUMENT;
     if (ld < heads * head_size) return CUBERT_BAD_ARGUMENT;
-    if (!shapes_ok<T>(batch, heads, seq, head_size, ld, {q, k, v}) || ld_ctx < heads * head_size) {
+    if (!shapes_ok<T>(batch, heads, seq, head_size, ld, {q, k, v}, true) || ld_ctx < heads * head_size) {
         return CUBERT_UNSUPPORTED;
     }
     hipStream_t s = (hipStream_t) stream;
+#define CUBERT_ATTENTION_ARGS q, k, v, ld, mask, ctx, ld_ctx, alpha, batch, heads, seq, split
     if (seq > 128) {
-        switch (head_size) {
-            case 32:
-                return launch_flash<T, 32>(q, k, v, ld, mask, ctx, ld_ctx, alpha, batch, heads, seq, split, order, s);
-            case 64:
-                return launch_flash<T, 64>(q, k, v, ld, mask, ctx, ld_ctx, alpha, batch, heads, seq, split, order, s);
-            default: return CUBERT_UNSUPPORTED;  // head size 128 would spill the accumulators to scratch
+        if (head_size == 128) return CUBERT_UNSUPPORTED;  // would spill the accumulators to scratch
+        if constexpr (sizeof(T) == 4) {
+            if (split.width > 0) {
+                return head_size == 32 ? launch_flash<T, 32, true>(CUBERT_ATTENTION_ARGS, order, s)
+                                       : launch_flash<T, 64, true>(CUBERT_ATTENTION_ARGS, order, s);
+            }
         }
+        if (split.width > 0) return CUBERT_UNSUPPORTED;
+        return head_size == 32 ? launch_flash<T, 32, false>(CUBERT_ATTENTION_ARGS, order, s)
+                               : launch_flash<T, 64, false>(CUBERT_ATTENTION_ARGS, order, s);
     }
+    const bool ragged = seq % 32 != 0;
     switch (head_size) {
         case 32:
-            return launch_fused<T, 32>(q, k, v, ld, mask, ctx, ld_ctx, alpha, batch, heads, seq, split,
-                                       s);
+            return ragged ? launch_fused<T, 32, true>(CUBERT_ATTENTION_ARGS, s)
+                          : launch_fused<T, 32, false>(CUBERT_ATTENTION_ARGS, s);
         case 64:
-            return launch_fused<T, 64>(q, k, v, ld, mask, ctx, ld_ctx, alpha, batch, heads, seq, split,
-                                       s);
+            return ragged ? launch_fused<T, 64, true>(CUBERT_ATTENTION_ARGS, s)
+                          : launch_fused<T, 64, false>(CUBERT_ATTENTION_ARGS, s);
         default:
-            return launch_fused<T, 128>(q, k, v, ld, mask, ctx, ld_ctx, alpha, batch, heads, seq, split,
-                                        s);
+            return ragged ? launch_fused<T, 128, true>(CUBERT_ATTENTION_ARGS, s)
+                          : launch_fused<T, 128, false>(CUBERT_ATTENTION_ARGS, s);
     }
+#undef CUBERT_ATTENTION_ARGS
 }
 
 }  // namespace

@@ -133,9 +133,9 @@ int cubert_attention_context_f16(const cubert_half *probs, const cubert_half *v,
  * the storage type as the three-kernel sequence cubert_attention_scores, cubert_mask_scale_softmax,
  * cubert_attention_context does; fp32 storage gives the same result up to summation order, fp16 storage agrees
  * within its tolerance).  Up to seq_length 128 the softmax is the exact two-pass one; from 129 to 512 it runs
- * online over chunks of 64 keys and is normalised once at the end.  mask may be NULL.  Shape support as the two contractions, and seq_length <= 512
- * (<= 128 for head_size 128, and K, V of one head must fit 160 KB of LDS: fp32 up to seq_length 256 at head size
- * 64); anything else returns CUBERT_UNSUPPORTED and launches nothing.
+ * online over chunks of 64 keys and is normalised once at the end.  mask may be NULL.  head_size 32, 64 or 128, Q, K, V
+ * and their row stride 16-byte aligned, any seq_length up to 512 (up to 128 for head_size 128); anything else returns
+ * CUBERT_UNSUPPORTED and launches nothing.
  * replaces: AttentionSelf<T>::_in_compute's Att_Q_K -> Softmax -> Att_QK_V sequence and the mask tensor of
  * AttentionMask<T>::compute, reference src/cuBERT/op_att/AttentionSelf.cpp:96-111, AttentionMask.cpp:41-54. */
 int cubert_attention_fused_f32(const float *q, const float *k, const float *v, int ld, const int8_t *mask, float *ctx,
@@ -156,8 +156,9 @@ int cubert_attention_fused_f16(const cubert_half *q, const cubert_half *k, const
  * would take i, and the tiles to compute from that position's record (order may be NULL: batch order, tiles from
  * the mask; shapes of at most 128 keys ignore it).  Results are identical with any order, i.e. with any permutation
  * of the positions that moves the records along with the indices.
- * CUBERT_UNSUPPORTED from cubert_attention_order (seq_length not a multiple of 32 or above 512, more than 4096
- * sequences, a mask that is not 4-byte aligned, an order array that is not 16-byte aligned): pass NULL.
+ * CUBERT_UNSUPPORTED from cubert_attention_order (seq_length above 512, or not a multiple of 32 and at most 128, more
+ * than 4096 sequences, a mask that is not 4-byte aligned with seq_length a multiple of 32, an order array that is not
+ * 16-byte aligned): pass NULL.
  * No counterpart in the reference, which computes every key of every sequence (src/cuBERT/op_att/AttentionSelf.cpp:96-111). */
 int cubert_attention_order(const int8_t *mask, int batch, int seq_length, int *order, void *stream);
 int cubert_attention_fused_ordered_f32(const float *q, const float *k, const float *v, int ld, const int8_t *mask,

@@ -1083,3 +1083,47 @@ def test_unaligned_views_take_the_generic_path(K):
     K.bias_res_ln_(view, res, None, beta, gamma)
     want = oracle.layer_norm_(host(res), x, np.zeros(768), np.ones(768))
     assert_close(host(view), want, FP32_TOL)
+
+
+# ------------------------------------------------------------------ attention at any sequence length
+
+@pytest.mark.parametrize("name", ["f32", "f16"])
+@pytest.mark.parametrize("batch,heads,seq,d", [(2, 3, 1, 64), (5, 4, 8, 64), (3, 2, 31, 64), (200, 12, 24, 64), (2, 3, 33, 64),
+                                               (3, 2, 50, 32), (2, 2, 100, 64), (1, 2, 127, 128), (100, 12, 77, 64),
+                                               (90, 12, 40, 32), (2, 2, 129, 64), (3, 2, 200, 32), (2, 2, 333, 64),
+                                               (1, 2, 511, 64), (2, 2, 384, 64), (1, 1, 300, 64)])
+@pytest.mark.parametrize("kind", ["none", "prefix", "scattered"])
+def test_attention_fused_at_any_sequence_length(K, name, batch, heads, seq, d, kind):
+    """Lengths that are not a multiple of 32 (last key tile partly filled; one, two or three lanes short of a tile, and
+    one over), and fp32 heads whose K and V exceed the LDS, against float64.  A few rows of a large batch are compared.
+    The storage type's error: fp32 sums of 64 + 512 terms, 2e-5; fp16 one rounding of the probabilities and one of the
+    result, 2e-3.  Sequence 0 keeps no key (its scores sit at -10000, where fp32 resolves 1e-3): 2e-3."""
+    rng = np.random.default_rng(batch * 1000 + heads * 100 + seq + d)
+    H = heads * d
+    qkv = q(rng.normal(0, 1, (batch * seq, 3 * H)), name)
+    valid = rng.integers(1, seq + 1, batch)
+    mask = (np.arange(seq)[None, :] < valid[:, None]).astype(np.int8) if kind == "prefix" else \
+        (rng.random((batch, seq)) < 0.6).astype(np.int8)
+    mask[0, :] = 0
+    mask[1:, 0] = 1
+    order = None
+    if kind != "none" and seq > 128:
+        order = K.attention_order(dev(mask))
+        assert order is not None
+    ctx = K.attention_fused(dev(qkv, tdt(name)), None if kind == "none" else dev(mask), batch, heads, seq, d,
+                            1.0 / math.sqrt(d), order=order)
+    assert ctx is not None
+    got = host(ctx).reshape(batch, seq, heads, d)
+    x = qkv.astype(np.float64).reshape(batch, seq, 3, heads, d)
+    for b in sorted({0, 1 % batch, batch // 2, batch - 1}):
+        s = np.einsum("qhd,khd->hqk", x[b, :, 0], x[b, :, 1]) / math.sqrt(d)
+        if kind != "none":
+            s = s - 10000.0 * (mask[b] == 0)[None, None, :]
+        p = np.exp(s - s.max(-1, keepdims=True))
+        want = np.einsum("hqk,khd->qhd", p / p.sum(-1, keepdims=True), x[b, :, 2])
+        loose = name == "f16" or (b == 0 and kind != "none")
+        assert_close(got[b], want, 2e-3 if loose else 2e-5, "sequence %d" % b)
+    if name == "f32" and kind == "prefix" and seq <= 200:
+        got = K.attention_fused_split3(dev(qkv), dev(mask), batch, heads, seq, d, 1.0 / math.sqrt(d), scale=16.0)
+        plain = K.attention_fused(dev(qkv), dev(mask), batch, heads, seq, d, 1.0 / math.sqrt(d))
+        assert got is not None and torch.equal(got[:, :H], (plain * 16.0).half())
