@@ -39,7 +39,9 @@ Transformer<T>::Transformer(void *cublas, const std::string &var_prefix,
     const size_t H = hidden_size, I = intermediate_size;
     // The re-ordered copies pay off for 2-byte weights (the plain layout makes the few-token kernel read 64-byte
     // pieces): measured 2 us per GEMM at hidden 768; for 4-byte weights the gain is within 5 %, not worth the memory.
-    keep_packed = sizeof(T) == 2 && seq_length <= 64 && H % 16 == 0 && I % 16 == 0;
+    // (Only where the layer sizes are not whole steps of the library's own Dense kernel, which reads them as they are.)
+    own_dense = H % (128 / sizeof(T)) == 0 && I % (128 / sizeof(T)) == 0;
+    keep_packed = !own_dense && sizeof(T) == 2 && seq_length <= 64 && H % 16 == 0 && I % 16 == 0;
     // The library's fp16 GEMMs are 10-19 % faster with both operands contiguous along the reduction (measured at
     // 32768 tokens on every Dense shape of BERT-base and BERT-large, same bits out); its fp32 GEMMs do not care.
     // Half-precision models therefore keep their Dense kernels [out, in], transposed once here.
@@ -195,7 +197,7 @@ void Transformer<T>::layout_buffers() {
     layer_output[0] = buffers.take<T>(M * H);
     layer_output[1] = buffers.take<T>(M * H);
     if (split_dense) split_operand = buffers.take<half>(M * 3 * (H > intermediate_size ? H : intermediate_size));
-    if (seq_length <= 64) few_token_partials = buffers.take<float>(kFewTokenPartialFloats);
+    if (seq_length <= 64 || own_dense) few_token_partials = buffers.take<float>(kFewTokenPartialFloats);
 }
 
 template <typename T>
@@ -292,6 +294,18 @@ bool Transformer<T>::attention(size_t batch_size, const T *qkv, const int8_t *ma
     return false;
 }
 
+// Whether a Dense layer of this size runs on the library's own kernel (kernels/dense_mid.hip) instead of a library
+// GEMM.  Half precision: up to 1024 tokens and 2.3e9 multiply-adds, where the two cross (whole requests through compute + output,
+// seq 32, library against own, us: BERT-base 64 tokens 581 / 366, 128 603 / 415, 256 636 / 472, 512 691 / 573, 1024
+// 857 / 789, 1536 942 / 1085; BERT-large 32 1084 / 806, 256 1197 / 1063, 512 1415 / 1335, 768 1713 / 1761).  fp32, where
+// the kernel keeps the matrix cores less busy than the library does: up to 128 tokens (BERT-base 32 564 / 472, 64
+// 751 / 490, 128 784 / 622, 192 858 / 885, 256 940 / 829, 384 1089 / 1335).
+template <typename T>
+bool Transformer<T>::own_dense_takes(int tokens, int out_features, int in_features) const {
+    if (!own_dense) return false;
+    return sizeof(T) == 2 ? tokens <= 1024 && (double) tokens * out_features * in_features <= 2.3e9 : tokens <= 128;
+}
+
 // One Dense layer.  The bias goes into the GEMM only where the caller asks for it (bias_in_gemm: the Q/K/V
 // projection, whose consumer has no fused bias) or where the few-token kernel applies it together with the GELU;
 // otherwise it is left to the fused kernel that follows (which then reads the GEMM output once anyway).
@@ -301,8 +315,16 @@ bool Transformer<T>::dense(int out_features, int tokens, int in_features, const 
     void *stream = cuBERT::blas_get_stream(cublas);
     Timed t(profiler, profiler != nullptr ? profiler->dense_kind(kind) : Profiler::kDenseGemm, stream);
     if (ld_out == 0) ld_out = out_features;
+    if (own_dense_takes(tokens, out_features, in_features)) {
+        const bool with_bias = bias_in_gemm || gelu;
+        if (cuBERT::dense_mid(tokens, out_features, in_features, in, in_features, kernel,
+                              transposed_kernels ? in_features : out_features, with_bias ? bias : nullptr, gelu, out, ld_out,
+                              stream)) {
+            return with_bias;
+        }
+    }
     // (the few-token kernel reads [in, out] kernels or its own copy of them, not transposed ones)
-    if (tokens <= few_token_limit(kind) && (packed != nullptr || (!transposed_kernels && (gelu || tokens > 32) && dense_gelu_fits))) {
+    if (!own_dense && tokens <= few_token_limit(kind) && (packed != nullptr || (!transposed_kernels && (gelu || tokens > 32) && dense_gelu_fits))) {
         const bool with_bias = bias_in_gemm || gelu;
         if (cuBERT::dense_few_tokens(cublas, out_features, tokens, in_features, kernel, out_features, packed, in,
                                      in_features, out, ld_out, with_bias ? bias : nullptr, gelu)) {
@@ -367,7 +389,27 @@ void Transformer<T>::dense_norm(int tokens, int in_features, const T *kernel, co
                                 const T *residual, const T *beta, const T *gamma, T *out, Profiler::Kind kind) {
     void *stream = cuBERT::blas_get_stream(cublas);
     const int H = (int) hidden_size;
-    if (tokens <= few_token_limit(kind) && slices_to_norm && few_token_partials != nullptr && few_token_slices_enabled() &&
+    if (own_dense_takes(tokens, H, in_features) && own_slices_to_norm && few_token_slices_enabled()) {
+        int slices = 0;
+        bool done = false;
+        {
+            Timed t(profiler, profiler != nullptr ? profiler->dense_kind(kind) : Profiler::kDenseGemm, stream);
+            done = cuBERT::dense_mid_slices(tokens, H, in_features, in, in_features, kernel,
+                                            transposed_kernels ? in_features : H, few_token_partials,
+                                            kFewTokenPartialFloats, &slices, stream);
+            if (!done) t.cancel();
+        }
+        if (done) {
+            Timed t(profiler, Profiler::kBiasResLayerNorm, stream);
+            if (cuBERT::layer_norm_slices(out, few_token_partials, slices, residual, bias, beta, gamma, tokens, H, stream)) {
+                return;
+            }
+            t.cancel();
+            own_slices_to_norm = false;  // the hidden size is fixed per model: do not ask again
+        }
+    }
+    if (!own_dense && tokens <= few_token_limit(kind) && slices_to_norm && few_token_partials != nullptr &&
+        few_token_slices_enabled() &&
         (packed != nullptr || !transposed_kernels)) {
         int slices = 0, pitch = 0;
         bool done = false;

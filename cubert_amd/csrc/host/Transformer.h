@@ -113,11 +113,14 @@ private:
     // split_operand first, or, when null, split_operand already holds the [hi | hi | lo] rows.  `bias` may be null.
     void dense_split(int out_features, int tokens, int in_features, const SplitKernel &kernel, const T *in, T *out,
                      const T *bias, Profiler::Kind kind, int ld_out = 0);
-    // out = LayerNorm(in * kernel + bias + residual): dense(), then layer_norm_; for at most 32 tokens the few-token
-    // GEMM leaves its K slices in few_token_partials and the LayerNorm kernel adds them while it loads (same values,
-    // without the GEMM's 2 us hand-over between workgroups).
+    // out = LayerNorm(in * kernel + bias + residual): dense(), then layer_norm_; for a small request the Dense kernel
+    // leaves its K slices in few_token_partials and the LayerNorm kernel adds them while it loads (no hand-over between
+    // the GEMM's workgroups).
     void dense_norm(int tokens, int in_features, const T *kernel, const T *packed, const T *in, const T *bias,
                     const T *residual, const T *beta, const T *gamma, T *out, Profiler::Kind kind);
+
+    // whether a Dense layer of this size runs on the library's own kernel (reads the kernels as the model keeps them)
+    bool own_dense_takes(int tokens, int out_features, int in_features) const;
 
     // up to how many tokens the Dense layer of this kind runs on the few-token kernel (32 or 64)
     int few_token_limit(Profiler::Kind kind) const;
@@ -126,6 +129,8 @@ private:
     Profiler *profiler = nullptr;
     bool slices_to_norm = true;        // few-token Dense layers hand their K slices to the LayerNorm (cleared when declined)
     bool dense_gelu_fits = true;       // cleared when the few-token Dense + GELU kernel declines this model's shape
+    bool own_dense = false;            // layer sizes are whole steps of the library's own Dense kernel (any few tokens)
+    bool own_slices_to_norm = true;    // cleared when the LayerNorm over its slices declines the hidden size
     bool keep_packed = false;          // Dense kernels are also kept in the few-token kernel's order
     bool transposed_kernels = false;   // Dense kernels are stored [out, in] instead of [in, out] (half precision)
     bool split_dense = false;          // fp32 model with Dense layers in the two-term fp16 form (opt-in)
@@ -150,8 +155,8 @@ private:
     T *intermediate_output;  // [M, intermediate]
     T *layer_output[2];      // [M, hidden], alternating between layers
     half *split_operand = nullptr;  // [M, 3 * max(hidden, intermediate)] two-term rows of the current Dense input
-    static constexpr size_t kFewTokenPartialFloats = (size_t) 1 << 20;
-    float *few_token_partials = nullptr;  // K slices of the current few-token Dense layer (seq_length <= 64 only)
+    static constexpr size_t kFewTokenPartialFloats = (size_t) 1 << 21;
+    float *few_token_partials = nullptr;  // K slices of the current Dense layer of a small request
 };
 
 }  // namespace cuBERT

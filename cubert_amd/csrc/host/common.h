@@ -142,6 +142,54 @@ inline bool layer_norm_partials(half *out, const float *partials, int slices, in
     CUBERT_CHECK(rc);
     return true;
 }
+// One launch of the library's own Dense kernel, out = act(in W + bias) with W as the model keeps it; false when it does
+// not take the problem.  No counterpart in the reference.
+inline bool dense_mid(int tokens, int features, int in, const float *x, int ldx, const float *w, int ldw, const float *bias,
+                      bool gelu, float *out, int ldo, void *stream) {
+    const int rc = cubert_dense_f32(stream, tokens, features, in, x, ldx, w, ldw, bias, gelu, out, ldo);
+    if (rc == CUBERT_UNSUPPORTED) return false;
+    CUBERT_CHECK(rc);
+    return true;
+}
+inline bool dense_mid(int tokens, int features, int in, const half *x, int ldx, const half *w, int ldw, const half *bias,
+                      bool gelu, half *out, int ldo, void *stream) {
+    const int rc = cubert_dense_f16(stream, tokens, features, in, h(x), ldx, h(w), ldw, h(bias), gelu, h(out), ldo);
+    if (rc == CUBERT_UNSUPPORTED) return false;
+    CUBERT_CHECK(rc);
+    return true;
+}
+// The product left as K slices [slices][tokens][features] for layer_norm_slices.
+inline bool dense_mid_slices(int tokens, int features, int in, const float *x, int ldx, const float *w, int ldw,
+                             float *partials, size_t partial_floats, int *slices, void *stream) {
+    const int rc = cubert_dense_slices_f32(stream, tokens, features, in, x, ldx, w, ldw, partials, partial_floats, slices);
+    if (rc == CUBERT_UNSUPPORTED) return false;
+    CUBERT_CHECK(rc);
+    return true;
+}
+inline bool dense_mid_slices(int tokens, int features, int in, const half *x, int ldx, const half *w, int ldw,
+                             float *partials, size_t partial_floats, int *slices, void *stream) {
+    const int rc = cubert_dense_slices_f16(stream, tokens, features, in, h(x), ldx, h(w), ldw, partials, partial_floats,
+                                           slices);
+    if (rc == CUBERT_UNSUPPORTED) return false;
+    CUBERT_CHECK(rc);
+    return true;
+}
+inline bool layer_norm_slices(float *out, const float *partials, int slices, const float *residual, const float *bias,
+                              const float *beta, const float *gamma, int rows, int hidden, void *stream) {
+    const int rc = cubert_bias_res_ln_slices_f32(out, partials, slices, hidden, (long long) rows * hidden, residual, bias,
+                                                 beta, gamma, rows, hidden, stream);
+    if (rc == CUBERT_UNSUPPORTED) return false;
+    CUBERT_CHECK(rc);
+    return true;
+}
+inline bool layer_norm_slices(half *out, const float *partials, int slices, const half *residual, const half *bias,
+                              const half *beta, const half *gamma, int rows, int hidden, void *stream) {
+    const int rc = cubert_bias_res_ln_slices_f16(h(out), partials, slices, hidden, (long long) rows * hidden, h(residual),
+                                                 h(bias), h(beta), h(gamma), rows, hidden, stream);
+    if (rc == CUBERT_UNSUPPORTED) return false;
+    CUBERT_CHECK(rc);
+    return true;
+}
 inline void pack_few_token_weights(void *handle, const float *A, int lda, int M, int K, float *packed) {
     CUBERT_CHECK(cubert_gemm_skinny_pack_f32(handle, A, lda, M, K, packed));
 }

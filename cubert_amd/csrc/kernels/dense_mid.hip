@@ -1,0 +1,410 @@
+// Dense layer for some tens to some hundreds of tokens:  C[token, feature] = act(X[token, :] . W[:, feature] + bias).
+// X is [tokens, K] row-major; W is [features, K] for 2-byte weights and [K, features] for 4-byte weights (the layouts
+// the models keep, contiguous 128-byte pieces either way).
+//
+// What bounds it: a launch of this size moves a few MB and multiplies for 1-5 us, so its time is the chain dispatch ->
+// first operands from the Infinity Cache (about 2 us) -> the rest of a compute unit's operands -> hand-over, and what
+// shortens it is operands requested early, in whole cache lines, by every compute unit.  Hence:
+//   - a workgroup of four wavefronts owns a tile of TM tokens x TN features; the wavefronts share the K axis, not the
+//     tile: each walks every fourth 128-byte step of K through LDS of its own, so nothing in the main loop waits for
+//     another wavefront, and the four partial tiles meet in LDS once at the end (in wavefront order);
+//   - operands go from memory straight to LDS (16 bytes per lane, eight lanes per 128-byte row piece, DEPTH steps
+//     requested ahead), laid out so that the matrix-core operand reads hit all banks: the 16-byte unit u of row r
+//     sits at u ^ (r % 8), which the loads get by asking for permuted units within the row;
+//   - K can also be cut into slices over workgroups when the consumer adds them (LayerNorm over slices).
+#include <atomic>
+
+#include "activations.h"
+#include "cubert_kernels.h"
+#include "device_common.h"
+
+namespace cubert {
+namespace {
+
+typedef float v16f32 __attribute__((ext_vector_type(16)));
+typedef float v4f32 __attribute__((ext_vector_type(4)));
+typedef _Float16 v8f16 __attribute__((ext_vector_type(8)));
+
+constexpr int kMidWaves = 4;
+constexpr int kMidThreads = kMidWaves * kWave;
+constexpr int kStepBytes = 128;  // of a row of X that a wavefront consumes per step
+
+// 16 bytes per lane from memory to LDS at `base` + 16 * lane, without passing through registers
+__device__ __forceinline__ void load_to_lds(const void *src, void *base) {
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *) src,
+                                     (__attribute__((address_space(3))) void *) base, 16, 0, 0);
+}
+
+template <int N>
+__device__ __forceinline__ void wait_loads() {  // at most N vector-memory requests of this wavefront outstanding
+    __builtin_amdgcn_s_waitcnt(0x0f70 | (N & 15) | ((N >> 4) << 14));
+}
+
+template <typename T, int TM, int TN, int DEPTH>
+struct MidShape {
+    static constexpr int kStep = kStepBytes / sizeof(T);           // K values per step
+    static constexpr int kXBytes = TM * kStepBytes;                // of one step in LDS
+    static constexpr int kWBytes = TN * kStepBytes;                // the same size in either weight layout
+    static constexpr int kStageBytes = kXBytes + kWBytes;
+    static constexpr int kLoads = kStageBytes / 1024;              // requests per lane and step
+    static constexpr int kRedPitch = TN + 4;                       // floats between token rows of a partial tile
+    static constexpr int kWaveBytes = DEPTH * kStageBytes > TM * kRedPitch * 4 ? DEPTH * kStageBytes : TM * kRedPitch * 4;
+    static constexpr int kLdsBytes = kMidWaves * kWaveBytes;
+};
+
+enum MidOutput { kMidStore = 0, kMidGelu = 1, kMidSlices = 2 };
+
+template <typename T, int TM, int TN, int DEPTH, int OUT>
+__global__ __launch_bounds__(kMidThreads) void dense_mid_kernel(const T *__restrict__ W, int ldw,
+                                                                const T *__restrict__ X, int ldx,
+                                                                const T *__restrict__ bias, T *__restrict__ C, int ldc,
+                                                                int tokens, int features, int steps_total,
+                                                                int steps_per_slice, int token_tiles, int feature_tiles,
+                                                                float *__restrict__ partials, int pitch,
+                                                                long long slice_stride) {
+    typedef MidShape<T, TM, TN, DEPTH> S;
+    constexpr int FB = TN / 32, TB = TM / 32;  // 32 x 32 blocks of the tile
+    constexpr int U = 16 / sizeof(T);          // elements of a 16-byte unit
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int lane = threadIdx.x & (kWave - 1), wave = wave_in_block();
+    const int r = lane & 31, hh = lane >> 5;
+
+    // Workgroups are handed to the eight dies in turn: the token tiles of one feature tile go to the same die, so its
+    // weights come to that die's L2 once.
+    const int local = blockIdx.x / 8;
+    const int ft = (local / token_tiles) * 8 + blockIdx.x % 8, tt = local % token_tiles;
+    if (ft >= feature_tiles) return;
+    const int m0 = tt * TM, n0 = ft * TN;
+    const int s_begin = blockIdx.y * steps_per_slice;
+    const int s_end = s_begin + steps_per_slice < steps_total ? s_begin + steps_per_slice : steps_total;
+    const int steps = s_end - s_begin > wave ? (s_end - s_begin - wave + kMidWaves - 1) / kMidWaves : 0;
+
+    unsigned char *mine = smem + wave * S::kWaveBytes;
+
+    // lane l of a request brings the 16-byte unit l % 8 of the LDS row l / 8; rows past the end are read from the last
+    const int lrow = lane >> 3, lunit = (lane & 7) ^ lrow;
+    const T *xsrc[TM / 8], *wsrc[TN / 8];
+    const int k_first = (s_begin + wave) * S::kStep;
+#pragma unroll
+    for (int i = 0; i < TM / 8; ++i) {
+        const int row = m0 + i * 8 + lrow;
+        xsrc[i] = X + (size_t) (row < tokens ? row : tokens - 1) * ldx + k_first + lunit * U;
+    }
+    size_t w_advance;
+    if constexpr (sizeof(T) == 2) {
+        w_advance = kMidWaves * S::kStep;
+#pragma unroll
+        for (int i = 0; i < TN / 8; ++i) {
+            const int row = n0 + i * 8 + lrow;
+            wsrc[i] = W + (size_t) (row < features ? row : features - 1) * ldw + k_first + lunit * U;
+        }
+    } else {
+        // [K, features]: the 32 K values of a step are LDS rows of TN features; lane l brings 4 features
+        constexpr int kLanes = TN / 4, kRows = kWave / kLanes;
+        w_advance = (size_t) kMidWaves * S::kStep * ldw;
+        const int f = n0 + (lane % kLanes) * 4;
+#pragma unroll
+        for (int i = 0; i < TN / 8; ++i) {
+            wsrc[i] = W + (size_t) (k_first + i * kRows + lane / kLanes) * ldw + (f < features ? f : features - 4);
+        }
+    }
+
+    auto request = [&](int slot) {
+        unsigned char *stage = mine + slot * S::kStageBytes;
+#pragma unroll
+        for (int i = 0; i < TN / 8; ++i) {
+            load_to_lds(wsrc[i], stage + S::kXBytes + i * 1024);
+            wsrc[i] += w_advance;
+        }
+#pragma unroll
+        for (int i = 0; i < TM / 8; ++i) {
+            load_to_lds(xsrc[i], stage + i * 1024);
+            xsrc[i] += kMidWaves * S::kStep;
+        }
+    };
+
+    // the bias of the four features this thread stores, on its way together with the first operands
+    Vec<T, 4> b = {};
+    const bool has_bias = OUT != kMidSlices && bias != nullptr;
+    if (has_bias) {
+        const int f = n0 + (int) (threadIdx.x % (TN / 4)) * 4;
+        b = load_vec<T, 4>(bias + (f < features ? f : 0));
+    }
+
+    v16f32 acc[TB][FB];
+#pragma unroll
+    for (int t = 0; t < TB; ++t)
+#pragma unroll
+        for (int f = 0; f < FB; ++f) acc[t][f] = v16f32{};
+
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) {
+        if (d < steps) request(d);
+    }
+    int slot = 0;
+    for (int s = 0; s < steps; ++s) {
+        const int behind = steps - 1 - s;  // steps requested after this one (at most DEPTH - 1)
+        if (DEPTH >= 4 && behind >= 3) {
+            wait_loads<3 * S::kLoads>();
+        } else if (DEPTH >= 3 && behind >= 2) {
+            wait_loads<2 * S::kLoads>();
+        } else if (DEPTH >= 2 && behind >= 1) {
+            wait_loads<S::kLoads>();
+        } else {
+            wait_loads<0>();
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        const unsigned char *stage = mine + slot * S::kStageBytes;
+        auto refill = [&] {
+            __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this step has been read, its LDS may be written again
+            __builtin_amdgcn_sched_barrier(0);
+            if (s + DEPTH < steps) request(slot);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        if constexpr (sizeof(T) == 2) {
+            // every operand of the step is read before the first product, and the slot is asked for again right then
+            v8f16 x[4][TB], w[4][FB];  // 16 K values per q: 8 per lane half
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int unit = ((q * 2 + hh) ^ (r & 7)) * 16;
+#pragma unroll
+                for (int f = 0; f < FB; ++f)
+                    w[q][f] = *reinterpret_cast<const v8f16 *>(stage + S::kXBytes + (f * 32 + r) * kStepBytes + unit);
+#pragma unroll
+                for (int t = 0; t < TB; ++t)
+                    x[q][t] = *reinterpret_cast<const v8f16 *>(stage + (t * 32 + r) * kStepBytes + unit);
+            }
+            refill();
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int t = 0; t < TB; ++t)
+#pragma unroll
+                    for (int f = 0; f < FB; ++f)
+                        acc[t][f] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w[q][f], x[q][t], acc[t][f], 0, 0, 0);
+        } else {
+            // The fp32 products take sixteen times as long: they start with the first operands and the rest is read
+            // between them (all reads first: 1056 workgroups of 32 x 32 x 768 27.1 instead of 23.1 us).
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {  // 8 K values: 4 per lane half
+                v4f32 x[TB];
+                float w[FB][4];
+                const int unit = ((q * 2 + hh) ^ (r & 7)) * 16;
+#pragma unroll
+                for (int f = 0; f < FB; ++f)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        w[f][e] = *reinterpret_cast<const float *>(stage + S::kXBytes +
+                                                                   ((q * 8 + hh * 4 + e) * TN + f * 32 + r) * 4);
+#pragma unroll
+                for (int t = 0; t < TB; ++t)
+                    x[t] = *reinterpret_cast<const v4f32 *>(stage + (t * 32 + r) * kStepBytes + unit);
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int t = 0; t < TB; ++t)
+#pragma unroll
+                        for (int f = 0; f < FB; ++f)
+                            acc[t][f] = __builtin_amdgcn_mfma_f32_32x32x2f32(w[f][e], x[t][e], acc[t][f], 0, 0, 0);
+            }
+            refill();
+        }
+        slot = slot + 1 < DEPTH ? slot + 1 : 0;
+    }
+
+    // partial tiles to LDS (each wavefront over its own operands, which it has read): a lane owns one token and, per
+    // four accumulator registers, four consecutive features
+    __builtin_amdgcn_s_waitcnt(0xc07f);
+    __builtin_amdgcn_sched_barrier(0);
+    float *red = reinterpret_cast<float *>(mine);
+#pragma unroll
+    for (int t = 0; t < TB; ++t)
+#pragma unroll
+        for (int f = 0; f < FB; ++f)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                v4f32 v = {acc[t][f][g * 4], acc[t][f][g * 4 + 1], acc[t][f][g * 4 + 2], acc[t][f][g * 4 + 3]};
+                *reinterpret_cast<v4f32 *>(red + (t * 32 + r) * S::kRedPitch + f * 32 + g * 8 + hh * 4) = v;
+            }
+    __syncthreads();
+    constexpr int kQuads = TN / 4;
+#pragma unroll
+    for (int it = 0; it < TM * kQuads / kMidThreads; ++it) {
+        const int item = it * kMidThreads + threadIdx.x;
+        const int token = item / kQuads, q = item % kQuads;
+        v4f32 sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < kMidWaves; ++w) {
+            sum += *reinterpret_cast<const v4f32 *>(smem + w * S::kWaveBytes + (token * S::kRedPitch + q * 4) * 4);
+        }
+        const int row = m0 + token, col = n0 + q * 4;
+        if (row >= tokens || col >= features) continue;
+        if constexpr (OUT == kMidSlices) {
+            *reinterpret_cast<v4f32 *>(partials + blockIdx.y * slice_stride + (size_t) row * pitch + col) = sum;
+        } else {
+            Vec<T, 4> out;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                float v = sum[e] + to_f32(b.v[e]);
+                if (OUT == kMidGelu) v = GeluOp<T>()(v);
+                out.v[e] = from_f32<T>(v);
+            }
+            store_vec<T, 4>(C + (size_t) row * ldc + col, out);
+        }
+    }
+}
+
+// Raises the dynamic LDS limit of a kernel once per device (the attribute belongs to the function on the device).
+template <typename Kernel>
+bool raise_lds_limit(Kernel kernel, std::atomic<unsigned long long> &done) {
+    int device = 0;
+    if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= 64) return false;
+    const unsigned long long bit = 1ull << device;
+    if (done.load(std::memory_order_acquire) & bit) return true;
+    if (hipFuncSetAttribute((const void *) kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) !=
+        hipSuccess) {
+        (void) hipGetLastError();
+        return false;
+    }
+    done.fetch_or(bit, std::memory_order_release);
+    return true;
+}
+
+struct MidPlan {
+    int tile = 0;  // 0: 32 x 32, 1: 64 x 32, 2: 64 x 64
+    int depth = 2, slices = 1, steps_per_slice = 0;
+};
+
+// The tile and the number of K slices, by a model of the launch time that agrees with the measured ones within about
+// 10 % (in microseconds; 32 to 1000 tokens, the Dense shapes of BERT-base, every tile, depth and 1 to 8 slices):
+// 2.3 for dispatch, the first operands and the drain, then as many rounds as the fullest of the 256 compute units has
+// workgroups.  A workgroup takes its operands at 80 KB per microsecond in half precision (768 x 768 in 32 x 32 tiles:
+// 98 KB, 1.4 us with its epilogue); in fp32 a tile of 32 x 32 takes 4.1 us per 768 K values, 64 x 32 8.0, 64 x 64 14.5.
+// Workgroups that share a compute unit gain nothing over taking turns.  Slices cost their way through memory.
+// Depth: two steps ahead where one workgroup per compute unit is all there is (72 workgroups of 32 x 32 x 768, fp16: one
+// step ahead 4.2, two 3.7 us), one where more workgroups fit the LDS that way (504: 4.8 against 5.0 us); in fp32 two
+// pay off for every tile (504: 13.1 against 11.9 us).
+template <typename T>
+MidPlan plan_mid(int tokens, int features, int steps, bool sliced, size_t partial_floats) {
+    static const int kTile[3][2] = {{32, 32}, {64, 32}, {64, 64}};
+    static const float kEpilogue[3] = {0.15f, 0.5f, 1.3f};             // us, half precision
+    static const float kF32Step[3] = {4.1f / 24, 8.0f / 24, 14.5f / 24};  // us per step of a workgroup
+    MidPlan best;
+    float best_us = 0.f;
+    for (int t = 0; t < 3; ++t) {
+        const long long tiles = (long long) ((tokens + kTile[t][0] - 1) / kTile[t][0]) *
+                                ((features + kTile[t][1] - 1) / kTile[t][1]);
+        for (int want = 1; want <= (sliced ? 16 : 1); ++want) {
+            const int per = (steps + want - 1) / want, slices = (steps + per - 1) / per;
+            if (slices != want) continue;
+            if (slices > 1 && (per < kMidWaves || (size_t) slices * tokens * features > partial_floats)) break;
+            const float rounds = (float) ((tiles * slices + 255) / 256);
+            const float each = sizeof(T) == 2
+                                   ? per * (kTile[t][0] + kTile[t][1]) * (kStepBytes / 80e3f) + kEpilogue[t]
+                                   : per * kF32Step[t];
+            float us = 2.3f + rounds * each;
+            if (slices > 1) us += slices * (0.1f + (float) tokens * features * (8.f / 5e6f));
+            if (best_us == 0.f || us < best_us) {
+                best_us = us;
+                best.tile = t, best.slices = slices, best.steps_per_slice = per;
+                best.depth = sizeof(T) == 4 || tiles * slices <= 256 ? 2 : 1;
+            }
+        }
+    }
+    return best;
+}
+
+template <typename T, int TM, int TN, int DEPTH, int OUT>
+int launch_mid(const MidPlan &plan, const T *W, int ldw, const T *X, int ldx, const T *bias, T *C, int ldc, int tokens,
+               int features, int steps, float *partials, hipStream_t stream) {
+    typedef MidShape<T, TM, TN, DEPTH> S;
+    static_assert(S::kLdsBytes <= 160 * 1024, "LDS of a compute unit");
+    static std::atomic<unsigned long long> raised{0};  // per kernel
+    if (!raise_lds_limit(dense_mid_kernel<T, TM, TN, DEPTH, OUT>, raised)) return CUBERT_UNSUPPORTED;
+    const int token_tiles = (tokens + TM - 1) / TM, feature_tiles = (features + TN - 1) / TN;
+    const dim3 grid((unsigned) ((feature_tiles + 7) / 8 * 8 * token_tiles), plan.slices), block(kMidThreads);
+    return launch_lds(dense_mid_kernel<T, TM, TN, DEPTH, OUT>, grid, block, (unsigned) S::kLdsBytes, stream, W, ldw, X, ldx,
+                      bias, C, ldc, tokens, features, steps, plan.steps_per_slice, token_tiles, feature_tiles, partials,
+                      features, (long long) tokens * features);
+}
+
+template <typename T, int OUT, typename... Args>
+int launch_mid_tile(const MidPlan &plan, Args... args) {
+    if constexpr (sizeof(T) == 2) {
+        if (plan.depth == 1) {
+            switch (plan.tile) {
+                case 0: return launch_mid<T, 32, 32, 1, OUT>(plan, args...);
+                case 1: return launch_mid<T, 64, 32, 1, OUT>(plan, args...);
+                default: return launch_mid<T, 64, 64, 1, OUT>(plan, args...);
+            }
+        }
+    }
+    switch (plan.tile) {
+        case 0: return launch_mid<T, 32, 32, 2, OUT>(plan, args...);
+        case 1: return launch_mid<T, 64, 32, 2, OUT>(plan, args...);
+        default: return launch_mid<T, 64, 64, 2, OUT>(plan, args...);
+    }
+}
+
+// What the kernel assumes of its operands: whole steps of K, 16-byte pieces of X and W, four features per store.
+template <typename T>
+int check_mid(int tokens, int features, int in, const T *X, int ldx, const T *W, int ldw) {
+    if (!X || !W || tokens < 0 || features < 0 || in < 0) return CUBERT_BAD_ARGUMENT;
+    if (ldx < in || ldw < (sizeof(T) == 2 ? in : features)) return CUBERT_BAD_ARGUMENT;
+    constexpr int U = 16 / sizeof(T);
+    if (in == 0 || in % (int) (kStepBytes / sizeof(T)) != 0 || features % 4 != 0 || tokens > 65535 || features > (1 << 20) ||
+        !is_aligned(X, 16) || !is_aligned(W, 16) || ldx % U != 0 || ldw % U != 0) {
+        return CUBERT_UNSUPPORTED;
+    }
+    return 0;
+}
+
+}  // namespace
+
+// C[token, feature] = act(X W + bias) in one launch; CUBERT_UNSUPPORTED (and nothing launched) where it does not fit.
+template <typename T>
+int dense_mid(int tokens, int features, int in, const T *X, int ldx, const T *W, int ldw, const T *bias, int activation,
+              T *C, int ldc, hipStream_t stream) {
+    if (!C || ldc < features || (activation != 0 && activation != 1)) return CUBERT_BAD_ARGUMENT;
+    const int rc = check_mid(tokens, features, in, X, ldx, W, ldw);
+    if (rc) return rc;
+    if (ldc % 4 != 0 || !is_aligned(C, 4 * sizeof(T)) || !is_aligned(bias, 4 * sizeof(T))) return CUBERT_UNSUPPORTED;
+    if (tokens == 0 || features == 0) return 0;
+    const int steps = in / (int) (kStepBytes / sizeof(T));
+    const MidPlan plan = plan_mid<T>(tokens, features, steps, false, 0);
+    float *none = nullptr;
+    if (activation == 1) {
+        return launch_mid_tile<T, kMidGelu>(plan, W, ldw, X, ldx, bias, C, ldc, tokens, features, steps, none, stream);
+    }
+    return launch_mid_tile<T, kMidStore>(plan, W, ldw, X, ldx, bias, C, ldc, tokens, features, steps, none, stream);
+}
+
+// The product left as *slices slices partials[slice][token][feature] for a consumer that adds them; where one slice is
+// the best cut this declines (dense_mid stores the finished product).
+template <typename T>
+int dense_mid_slices(int tokens, int features, int in, const T *X, int ldx, const T *W, int ldw, float *partials,
+                     size_t partial_floats, int *slices, hipStream_t stream) {
+    if (!partials || !slices) return CUBERT_BAD_ARGUMENT;
+    const int rc = check_mid(tokens, features, in, X, ldx, W, ldw);
+    if (rc) return rc;
+    if (!is_aligned(partials, 16) || tokens == 0 || features == 0) return CUBERT_UNSUPPORTED;
+    const int steps = in / (int) (kStepBytes / sizeof(T));
+    const MidPlan plan = plan_mid<T>(tokens, features, steps, true, partial_floats);
+    if (plan.slices < 2) return CUBERT_UNSUPPORTED;
+    *slices = plan.slices;
+    const T *no_bias = nullptr;
+    T *no_output = nullptr;
+    return launch_mid_tile<T, kMidSlices>(plan, W, ldw, X, ldx, no_bias, no_output, features, tokens, features, steps,
+                                          partials, stream);
+}
+
+template int dense_mid<float>(int, int, int, const float *, int, const float *, int, const float *, int, float *, int,
+                              hipStream_t);
+template int dense_mid<half_t>(int, int, int, const half_t *, int, const half_t *, int, const half_t *, int, half_t *, int,
+                               hipStream_t);
+template int dense_mid_slices<float>(int, int, int, const float *, int, const float *, int, float *, size_t, int *,
+                                     hipStream_t);
+template int dense_mid_slices<half_t>(int, int, int, const half_t *, int, const half_t *, int, float *, size_t, int *,
+                                      hipStream_t);
+
+}  // namespace cubert

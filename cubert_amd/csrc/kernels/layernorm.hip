@@ -146,24 +146,24 @@ __device__ __forceinline__ void load_floats(const float *__restrict__ p, float (
 }
 
 // bias + residual + LayerNorm of a Dense layer that the few-token GEMM left as K slices
-// (partials[(slice * R + row) * pitch + col], fp32, R = rows rounded up to 32): the slices are added here, in slice
+// (partials[slice * slice_stride + row * pitch + col], fp32): the slices are added here, in slice
 // order from 0.f, and the
 // sum is rounded to the storage type before anything else happens to it -- the value the GEMM's own last workgroup
-// would have stored -- so the result has the bits of GEMM followed by bias_res_ln.  At most 64 rows.
+// would have stored -- so the result has the bits of GEMM followed by bias_res_ln.
 template <typename T, int VEC, int CHUNKS, bool HAS_BIAS>
 __global__ __launch_bounds__(kBlock) void bias_res_ln_partials_kernel(T *__restrict__ out,
                                                                       const float *__restrict__ partials, int slices,
                                                                       int pitch, const T *__restrict__ residual,
                                                                       const T *__restrict__ bias,
                                                                       const T *__restrict__ beta,
-                                                                      const T *__restrict__ gamma, int rows) {
+                                                                      const T *__restrict__ gamma, int rows,
+                                                                      long long slice_stride) {
     constexpr int H = kWave * VEC * CHUNKS;
     constexpr int kAhead = CHUNKS * VEC <= 12 ? 8 : 4;  // slices whose loads are in flight together
     const int row = blockIdx.x * (int) (blockDim.x / kWave) + wave_in_block();
     if (row >= rows) return;
     const int lane = threadIdx.x & (kWave - 1);
     const float *prow = partials + (size_t) row * pitch;
-    const size_t slice_stride = (size_t) ((rows + 31) / 32 * 32) * pitch;  // whole blocks of 32 token rows per slice
     const T *res = residual + (size_t) row * H;
 
     Vec<T, VEC> r[CHUNKS], bi[CHUNKS], g[CHUNKS], be[CHUNKS];
@@ -490,12 +490,12 @@ int bias_res_ln(T *inout, const T *residual, const T *bias, const T *beta, const
 // bias + residual + LayerNorm reading the Dense output as the few-token GEMM's K slices; only the register-resident
 // shapes of bias_res_ln, anything else is declined and nothing is launched.
 template <typename T>
-int bias_res_ln_partials(T *out, const float *partials, int slices, int pitch, const T *residual, const T *bias,
-                         const T *beta, const T *gamma, int rows, int hidden, void *stream) {
+int bias_res_ln_slices(T *out, const float *partials, int slices, int pitch, long long slice_stride, const T *residual,
+                       const T *bias, const T *beta, const T *gamma, int rows, int hidden, void *stream) {
     if (rows < 0 || hidden <= 0 || slices <= 0 || !out || !partials || !residual || !beta || !gamma) {
         return CUBERT_BAD_ARGUMENT;
     }
-    if (rows > 64 || pitch < hidden || pitch % 4 != 0 || !is_aligned(partials, 16)) return CUBERT_UNSUPPORTED;
+    if (pitch < hidden || pitch % 4 != 0 || slice_stride % 4 != 0 || !is_aligned(partials, 16)) return CUBERT_UNSUPPORTED;
     if (rows == 0) return 0;
     hipStream_t s = (hipStream_t) stream;
     // a wavefront per workgroup: what a row waits for is its slices arriving, and a compute unit pulls them at a
@@ -506,9 +506,9 @@ int bias_res_ln_partials(T *out, const float *partials, int slices, int pitch, c
     if (hidden == kWave * VEC * CHUNKS && vector_ok<T>(hidden, VEC, {out, residual, bias, beta, gamma})) {       \
         if (bias != nullptr)                                                                                     \
             return launch(bias_res_ln_partials_kernel<T, VEC, CHUNKS, true>, grid, block, s, out, partials, slices, \
-                          pitch, residual, bias, beta, gamma, rows);                                             \
+                          pitch, residual, bias, beta, gamma, rows, slice_stride);                                             \
         return launch(bias_res_ln_partials_kernel<T, VEC, CHUNKS, false>, grid, block, s, out, partials, slices, \
-                      pitch, residual, bias, beta, gamma, rows);                                                 \
+                      pitch, residual, bias, beta, gamma, rows, slice_stride);                                                 \
     }
     CUBERT_LN_CASE(V, 1)
     CUBERT_LN_CASE(V, 2)
@@ -519,6 +519,15 @@ int bias_res_ln_partials(T *out, const float *partials, int slices, int pitch, c
     CUBERT_LN_CASE(V / 2, 5)
 #undef CUBERT_LN_CASE
     return CUBERT_UNSUPPORTED;
+}
+
+// The slices of the few-token GEMM: whole blocks of 32 token rows each, at most 64 rows.
+template <typename T>
+int bias_res_ln_partials(T *out, const float *partials, int slices, int pitch, const T *residual, const T *bias,
+                         const T *beta, const T *gamma, int rows, int hidden, void *stream) {
+    if (rows > 64) return CUBERT_UNSUPPORTED;
+    return bias_res_ln_slices<T>(out, partials, slices, pitch, (long long) ((rows + 31) / 32 * 32) * pitch, residual, bias,
+                                 beta, gamma, rows, hidden, stream);
 }
 
 // bias + residual + LayerNorm of fp32 rows, in place, and the result again as two-term fp16 rows in split_out
@@ -626,6 +635,22 @@ extern "C" int cubert_bias_res_ln_partials_f16(cubert_half *out, const float *pa
     return cubert::bias_res_ln_partials<half_t>((half_t *) out, partials, slices, pitch, (const half_t *) residual,
                                                 (const half_t *) bias, (const half_t *) beta, (const half_t *) gamma,
                                                 rows, hidden, stream);
+}
+
+extern "C" int cubert_bias_res_ln_slices_f32(float *out, const float *partials, int slices, int pitch,
+                                             long long slice_stride, const float *residual, const float *bias,
+                                             const float *beta, const float *gamma, int rows, int hidden, void *stream) {
+    return cubert::bias_res_ln_slices<float>(out, partials, slices, pitch, slice_stride, residual, bias, beta, gamma, rows,
+                                             hidden, stream);
+}
+
+extern "C" int cubert_bias_res_ln_slices_f16(cubert_half *out, const float *partials, int slices, int pitch,
+                                             long long slice_stride, const cubert_half *residual,
+                                             const cubert_half *bias, const cubert_half *beta, const cubert_half *gamma,
+                                             int rows, int hidden, void *stream) {
+    return cubert::bias_res_ln_slices<half_t>((half_t *) out, partials, slices, pitch, slice_stride,
+                                              (const half_t *) residual, (const half_t *) bias, (const half_t *) beta,
+                                              (const half_t *) gamma, rows, hidden, stream);
 }
 
 extern "C" int cubert_embed_ln_f32(const int32_t *ids, const int8_t *segments, const float *word, const float *pos,

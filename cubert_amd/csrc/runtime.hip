@@ -35,6 +35,13 @@ int gemm_skinny_pack(const T *A, int lda, int M, int K, T *packed, hipStream_t s
 template <typename T>
 int gemm_skinny_partials(int M, int N, int K, const T *A, int lda, int packed, const T *B, int ldb, float *partials,
                          size_t partial_floats, int *slices, int *pitch, hipStream_t stream);
+// kernels/dense_mid.hip
+template <typename T>
+int dense_mid(int tokens, int features, int in, const T *X, int ldx, const T *W, int ldw, const T *bias, int activation,
+              T *C, int ldc, hipStream_t stream);
+template <typename T>
+int dense_mid_slices(int tokens, int features, int in, const T *X, int ldx, const T *W, int ldw, float *partials,
+                     size_t partial_floats, int *slices, hipStream_t stream);
 // kernels/gemm_batch.hip
 template <typename T>
 int gemm_batch(int transA, int transB, int M, int N, int K, float alpha, const T *const *A_array, int lda,
@@ -691,6 +698,35 @@ int cubert_gemm_skinny_partials_f16(void *handle, int M, int N, int K, const cub
     return cubert::gemm_skinny_partials<cubert::half_t>(M, N, K, (const cubert::half_t *) A, lda, packed,
                                                         (const cubert::half_t *) B, ldb, partials, partial_floats,
                                                         slices, pitch, ctx->stream);
+}
+
+int cubert_dense_f32(void *stream, int tokens, int features, int in, const float *x, int ldx, const float *w, int ldw,
+                     const float *bias, int activation, float *out, int ldo) {
+    if (library_gemm_only() || force_naive_gemm()) return CUBERT_UNSUPPORTED;
+    return cubert::dense_mid<float>(tokens, features, in, x, ldx, w, ldw, bias, activation, out, ldo, (hipStream_t) stream);
+}
+
+int cubert_dense_f16(void *stream, int tokens, int features, int in, const cubert_half *x, int ldx,
+                     const cubert_half *w, int ldw, const cubert_half *bias, int activation, cubert_half *out, int ldo) {
+    if (library_gemm_only() || force_naive_gemm()) return CUBERT_UNSUPPORTED;
+    return cubert::dense_mid<cubert::half_t>(tokens, features, in, (const cubert::half_t *) x, ldx,
+                                             (const cubert::half_t *) w, ldw, (const cubert::half_t *) bias, activation,
+                                             (cubert::half_t *) out, ldo, (hipStream_t) stream);
+}
+
+int cubert_dense_slices_f32(void *stream, int tokens, int features, int in, const float *x, int ldx, const float *w,
+                            int ldw, float *partials, size_t partial_floats, int *slices) {
+    if (library_gemm_only() || force_naive_gemm()) return CUBERT_UNSUPPORTED;
+    return cubert::dense_mid_slices<float>(tokens, features, in, x, ldx, w, ldw, partials, partial_floats, slices,
+                                           (hipStream_t) stream);
+}
+
+int cubert_dense_slices_f16(void *stream, int tokens, int features, int in, const cubert_half *x, int ldx,
+                            const cubert_half *w, int ldw, float *partials, size_t partial_floats, int *slices) {
+    if (library_gemm_only() || force_naive_gemm()) return CUBERT_UNSUPPORTED;
+    return cubert::dense_mid_slices<cubert::half_t>(tokens, features, in, (const cubert::half_t *) x, ldx,
+                                                    (const cubert::half_t *) w, ldw, partials, partial_floats, slices,
+                                                    (hipStream_t) stream);
 }
 
 int cubert_gemm_strided_batch_f32(void *handle, int transA, int transB, int M, int N, int K, float alpha,

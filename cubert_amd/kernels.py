@@ -244,6 +244,54 @@ def transpose(x):
     return out
 
 
+def _rows_ptr(t):
+    """Of a matrix whose rows are contiguous, at any pitch."""
+    if not t.is_cuda or t.dim() != 2 or t.stride(1) != 1:
+        raise ValueError("CUDA matrix with contiguous rows expected")
+    return t.data_ptr()
+
+
+def dense(x, w, bias=None, gelu=False, out=None):
+    """[gelu](x W + bias) with the library's own Dense kernel: w is [in, features] in fp32, [features, in] in half
+    precision; rows of x, w and out may be wider than they are long.  None when the problem does not fit."""
+    features = w.shape[1] if w.dtype == torch.float32 else w.shape[0]
+    if out is None:
+        out = torch.empty(x.shape[0], features, dtype=x.dtype, device=x.device)
+    fn = getattr(lib(), "cubert_dense_" + _suffix(x))
+    rc = fn(_stream(), x.shape[0], features, x.shape[1], _rows_ptr(x), x.stride(0), _rows_ptr(w), w.stride(0), _ptr(bias), int(gelu),
+            _rows_ptr(out), out.stride(0))
+    if rc == -2:
+        return None
+    _check(rc, fn.__name__)
+    return out
+
+
+def dense_slices(x, w, partial_floats=1 << 21):
+    """x W left as K slices [slices, tokens, features] fp32; None when the problem does not fit or one slice is best."""
+    features = w.shape[1] if w.dtype == torch.float32 else w.shape[0]
+    partials = torch.empty(partial_floats, dtype=torch.float32, device=x.device)
+    slices = ctypes.c_int(0)
+    fn = getattr(lib(), "cubert_dense_slices_" + _suffix(x))
+    rc = fn(_stream(), x.shape[0], features, x.shape[1], _rows_ptr(x), x.stride(0), _rows_ptr(w), w.stride(0), _ptr(partials),
+            partial_floats, ctypes.byref(slices))
+    if rc == -2:
+        return None
+    _check(rc, fn.__name__)
+    return partials[:slices.value * x.shape[0] * features].view(slices.value, x.shape[0], features)
+
+
+def bias_res_ln_slices(partials, residual, bias, beta, gamma):
+    """LayerNorm(storage type of (sum of the K slices partials[s]) + bias + residual); None when declined."""
+    out = torch.empty_like(residual)
+    fn = getattr(lib(), "cubert_bias_res_ln_slices_" + _suffix(residual))
+    rc = fn(_ptr(out), _ptr(partials), partials.shape[0], partials.shape[2], partials.stride(0), _ptr(residual), _ptr(bias),
+            _ptr(beta), _ptr(gamma), residual.shape[0], residual.shape[1], _stream())
+    if rc == -2:
+        return None
+    _check(rc, fn.__name__)
+    return out
+
+
 class Blas(object):
     """A BLAS context of the runtime bound to torch's current stream."""
 

@@ -89,6 +89,15 @@ int cubert_bias_res_ln_partials_f16(cubert_half *out, const float *partials, int
                                     const cubert_half *residual, const cubert_half *bias, const cubert_half *beta,
                                     const cubert_half *gamma, int rows, int hidden, void *stream);
 
+/* The same on slices[slice * slice_stride + r * pitch + c], any number of rows (what cubert_dense_slices_* leaves). */
+int cubert_bias_res_ln_slices_f32(float *out, const float *partials, int slices, int pitch, long long slice_stride,
+                                  const float *residual, const float *bias, const float *beta, const float *gamma,
+                                  int rows, int hidden, void *stream);
+int cubert_bias_res_ln_slices_f16(cubert_half *out, const float *partials, int slices, int pitch,
+                                  long long slice_stride, const cubert_half *residual, const cubert_half *bias,
+                                  const cubert_half *beta, const cubert_half *gamma, int rows, int hidden,
+                                  void *stream);
+
 /* bias + GELU (erf form), in place:  x = inout[r,c] + bias[c];  inout = x * 0.5 * (1 + erf(x / sqrt 2)).
  * `bias` may be NULL.
  * replaces: gelu<T>(N, inout, stream), reference src/cuBERT/op/GELU.h:6-7 (op/GELU.cu:14-26),
@@ -382,6 +391,26 @@ int cubert_gemm_skinny_partials_f32(void *handle, int M, int N, int K, const flo
 int cubert_gemm_skinny_partials_f16(void *handle, int M, int N, int K, const cubert_half *A, int lda, int packed,
                                     const cubert_half *B, int ldb, float *partials, size_t partial_floats, int *slices,
                                     int *pitch);
+
+/* A Dense layer for up to some hundreds of tokens in one launch of this library's own kernel:
+ *   out[t, f] = act(sum_k x[t, k] * w(k, f) + bias[f]),  act = identity (0) or the erf-form GELU (1), fp32 accumulation;
+ * x is [tokens, in] row-major with ldx elements per row, w the kernel in the layout the models keep: [in, features]
+ * (ldw >= features) in fp32, [features, in] (ldw >= in) in half precision; `bias` may be NULL.  in must be a multiple
+ * of 32 (fp32) or 64 (half), features of 4, x and w 16-byte aligned with rows of whole 16-byte pieces, out rows of
+ * four elements; anything else returns CUBERT_UNSUPPORTED and launches nothing.
+ * Asynchronous on `stream`; needs no handle and no workspace.
+ * replaces: Dense (src/cuBERT/op/Dense.cpp:47-57) and, with act = 1, the gelu<T> that follows it (op/GELU.h:6-7). */
+int cubert_dense_f32(void *stream, int tokens, int features, int in, const float *x, int ldx, const float *w, int ldw,
+                     const float *bias, int activation, float *out, int ldo);
+int cubert_dense_f16(void *stream, int tokens, int features, int in, const cubert_half *x, int ldx,
+                     const cubert_half *w, int ldw, const cubert_half *bias, int activation, cubert_half *out, int ldo);
+/* The product alone, left as *slices (>= 2) K slices partials[(slice * tokens + t) * features + f], fp32, for
+ * cubert_bias_res_ln_slices_*: a reduction cut over more workgroups, none of which waits for another.  At most
+ * partial_floats floats are written; CUBERT_UNSUPPORTED also where cutting K does not pay. */
+int cubert_dense_slices_f32(void *stream, int tokens, int features, int in, const float *x, int ldx, const float *w,
+                            int ldw, float *partials, size_t partial_floats, int *slices);
+int cubert_dense_slices_f16(void *stream, int tokens, int features, int in, const cubert_half *x, int ldx,
+                            const cubert_half *w, int ldw, float *partials, size_t partial_floats, int *slices);
 
 /* The same over `batch_count` problems at fixed strides (in elements).
  * replaces: blas_gemm_strided_batch<T>, reference src/cuBERT/common.h:82-92. */

@@ -1,0 +1,97 @@
+"""The library's own Dense kernels against float64 on the same (storage-rounded) operands."""
+import numpy as np
+import pytest
+from scipy.special import erf
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+
+@pytest.fixture(scope="module")
+def K():
+    if not torch.cuda.is_available():
+        pytest.fail("no GPU visible: the -m gpu tests must run on the MI355X box")
+    from cubert_amd import kernels
+    return kernels
+
+
+def operands(name, tokens, features, width, pad):
+    """x [tokens, width] in rows of width + pad, w as the models keep it, bias: device tensors and their float64 values."""
+    rng = np.random.default_rng(tokens + 3 * features + 7 * width)
+    dtype = torch.float32 if name == "f32" else torch.float16
+    x = torch.from_numpy(rng.normal(0, 1, (tokens, width + pad)).astype(np.float32)).to(dtype)
+    w = torch.from_numpy(rng.normal(0, 0.3, (width, features) if name == "f32" else (features, width)).astype(np.float32)).to(dtype)
+    bias = torch.from_numpy(rng.normal(0, 1, features).astype(np.float32)).to(dtype)
+    x64 = x[:, :width].double().numpy()
+    w64 = w.double().numpy() if name == "f32" else w.double().numpy().T
+    return x.cuda()[:, :width], w.cuda(), bias.cuda(), x64, w64, bias.double().numpy()
+
+
+def product_bound(x64, w64):
+    # fp32 additions: the longest chain holds a quarter of the products (four wavefronts share the reduction)
+    return (x64.shape[1] / 4 + 16) * 2.0 ** -24 * (np.abs(x64) @ np.abs(w64))
+
+
+def result_bound(name, want, product):
+    # the product's error (GELU's slope is below 1.13), its approximation (1e-6 |x|), and the rounding to the storage type
+    return 1.13 * product + 2e-6 * (1 + np.abs(want)) + (2.0 ** -24 if name == "f32" else 2.0 ** -11) * np.abs(want) + 6e-8
+
+
+# one step, fewer steps than wavefronts, remainders of token and feature tiles, every tile and depth of the plan
+SIZES = [(1, 4, 64), (33, 100, 128), (31, 36, 320), (32, 2304, 768), (64, 3072, 768), (65, 768, 3072), (120, 3072, 768),
+         (200, 2304, 768), (350, 2304, 768), (350, 3072, 768), (777, 1028, 192)]
+
+
+@pytest.mark.parametrize("name", ["f32", "f16"])
+@pytest.mark.parametrize("tokens,features,width", SIZES)
+def test_dense_against_float64(K, name, tokens, features, width):
+    x, w, bias, x64, w64, bias64 = operands(name, tokens, features, width, 16)
+    bound = product_bound(x64, w64)
+    for use_bias, gelu in ((True, False), (False, False), (True, True)):
+        out = torch.full((tokens + 1, features + 8), 7.0, dtype=x.dtype, device="cuda")
+        assert K.dense(x, w, bias if use_bias else None, gelu, out[:tokens, :features]) is not None
+        got = out.double().cpu().numpy()
+        want = x64 @ w64 + (bias64 if use_bias else 0.0)
+        if gelu:
+            want = 0.5 * want * (1 + erf(want / np.sqrt(2.0)))
+        assert (np.abs(got[:tokens, :features] - want) <= result_bound(name, want, bound)).all(), (use_bias, gelu)
+        assert (got[tokens:] == 7).all() and (got[:, features:] == 7).all()  # nothing beyond the result
+
+
+@pytest.mark.parametrize("name", ["f32", "f16"])
+@pytest.mark.parametrize("tokens,width", [(1, 768), (32, 3072), (65, 3072), (120, 768), (200, 3072), (350, 3072)])
+def test_dense_slices_add_up_and_reach_the_layer_norm(K, name, tokens, width):
+    H = 768
+    x, w, bias, x64, w64, _ = operands(name, tokens, H, width, 0)
+    slices = K.dense_slices(x, w)
+    assert slices is not None and slices.shape[0] >= 2
+    assert (np.abs(slices.double().sum(0).cpu().numpy() - x64 @ w64) <= product_bound(x64, w64)).all()
+    rng = np.random.default_rng(tokens)
+    residual, beta, gamma = (torch.from_numpy(rng.normal(0, 1, s).astype(np.float32)).to(x.dtype).cuda()
+                             for s in ((tokens, H), H, H))
+    got = K.bias_res_ln_slices(slices, residual, bias, beta, gamma)
+    added = torch.zeros_like(slices[0])
+    for s in slices:  # in slice order from 0.f, then rounded: what a finished product would be
+        added += s
+    plain = K.bias_res_ln_(added.to(x.dtype), residual, bias, beta, gamma)
+    # the same inputs through separately compiled kernels that add a row in another order: 1e-6 in fp32; in half
+    # precision a result may fall on the other side of a rounding, one unit in the last place of values up to 16
+    assert float((got.float() - plain.float()).abs().max()) <= (2e-5 if name == "f32" else 2.0 ** -7)
+
+
+@pytest.mark.parametrize("name", ["f32", "f16"])
+def test_dense_declines_what_it_cannot_do(K, name):
+    dtype = torch.float32 if name == "f32" else torch.float16
+    x = torch.zeros(64 * 1024, dtype=dtype, device="cuda")
+
+    def operands_of(width, features, shift=0, pad=0):
+        rows = x[shift:shift + 8 * (width + pad)].view(8, width + pad)[:, :width]
+        return rows, x[:width * features].view((width, features) if name == "f32" else (features, width))
+    assert K.dense(*operands_of(128, 64)) is not None
+    assert K.dense(*operands_of(48, 64)) is None            # not whole steps of the reduction
+    assert K.dense(*operands_of(128, 62)) is None           # features not a multiple of four
+    assert K.dense(*operands_of(128, 64, shift=1)) is None  # misaligned rows
+    assert K.dense(*operands_of(128, 64, pad=1)) is None    # rows of unaligned pitch
+    assert K.dense_slices(*operands_of(128, 64)) is None    # too short to cut
+    assert K.dense_slices(*operands_of(1024, 64), partial_floats=8 * 64) is None  # no room for two slices
