@@ -295,15 +295,16 @@ bool Transformer<T>::attention(size_t batch_size, const T *qkv, const int8_t *ma
 }
 
 // Whether a Dense layer of this size runs on the library's own kernel (kernels/dense_mid.hip) instead of a library
-// GEMM.  Half precision: up to 1024 tokens and 2.3e9 multiply-adds, where the two cross (whole requests through compute + output,
-// seq 32, library against own, us: BERT-base 64 tokens 581 / 366, 128 603 / 415, 256 636 / 472, 512 691 / 573, 1024
-// 857 / 789, 1536 942 / 1085; BERT-large 32 1084 / 806, 256 1197 / 1063, 512 1415 / 1335, 768 1713 / 1761).  fp32, where
-// the kernel keeps the matrix cores less busy than the library does: up to 128 tokens (BERT-base 32 564 / 472, 64
-// 751 / 490, 128 784 / 622, 192 858 / 885, 256 940 / 829, 384 1089 / 1335).
+// GEMM: up to where the two cross.  Whole requests through compute + output, seq 32, library against own, us --
+// half precision, BERT-base: 64 tokens 581 / 340, 128 603 / 400, 512 691 / 573, 768 821 / 705, 1024 859 / 768, 1152
+// 884 / 833, 1280 884 / 859, 1536 942 / 1085; BERT-large: 32 1084 / 774, 512 1497 / 1306, 640 1727 / 1610, 768 1753 /
+// 1740, 896 equal.  fp32, BERT-base: 64 751 / 473, 128 802 / 636, 192 868 / 754, 256 952 / 827, 320 961 / 902, 352
+// 1089 / 1128 (there the kernel keeps the matrix cores 60 % busy, the library 85 % from some thousand tokens on).
 template <typename T>
 bool Transformer<T>::own_dense_takes(int tokens, int out_features, int in_features) const {
     if (!own_dense) return false;
-    return sizeof(T) == 2 ? tokens <= 1024 && (double) tokens * out_features * in_features <= 2.3e9 : tokens <= 128;
+    const double products = (double) tokens * out_features * in_features;
+    return sizeof(T) == 2 ? tokens <= 1280 && products <= 3.05e9 : tokens <= 320 && products <= 7.6e8;
 }
 
 // One Dense layer.  The bias goes into the GEMM only where the caller asks for it (bias_in_gemm: the Q/K/V

@@ -10,7 +10,7 @@
 //     another wavefront, and the four partial tiles meet in LDS once at the end (in wavefront order);
 //   - operands go from memory straight to LDS (16 bytes per lane, eight lanes per 128-byte row piece, DEPTH steps
 //     requested ahead), laid out so that the matrix-core operand reads hit all banks: the 16-byte unit u of row r
-//     sits at u ^ (r % 8), which the loads get by asking for permuted units within the row;
+//     sits at u ^ (r / 2 % 8) (two rows span the 64 banks), which the loads get by asking for permuted units;
 //   - K can also be cut into slices over workgroups when the consumer adds them (LayerNorm over slices).
 #include <atomic>
 
@@ -69,26 +69,30 @@ __global__ __launch_bounds__(kMidThreads) void dense_mid_kernel(const T *__restr
     const int lane = threadIdx.x & (kWave - 1), wave = wave_in_block();
     const int r = lane & 31, hh = lane >> 5;
 
-    // Workgroups are handed to the eight dies in turn: the token tiles of one feature tile go to the same die, so its
-    // weights come to that die's L2 once.
-    const int local = blockIdx.x / 8;
-    const int ft = (local / token_tiles) * 8 + blockIdx.x % 8, tt = local % token_tiles;
-    if (ft >= feature_tiles) return;
+    // Workgroups are handed to the eight dies in turn.  Each die gets a contiguous run of the (slice, feature tile, token
+    // tile) triples, token tiles innermost: the token tiles of a feature tile mostly share a die, so its weights come to
+    // that die's L2 once, and no die gets more than one workgroup more than another.  (Feature tiles dealt out to the dies
+    // one by one: 12 of them over 8 dies, 7 slices, put 42 workgroups on the 32 compute units of four dies.)
+    const int die = blockIdx.x & 7, die_share = gridDim.x >> 3, extra = gridDim.x & 7;
+    const int index = die * die_share + (die < extra ? die : extra) + (int) (blockIdx.x >> 3);
+    const int pair = index / token_tiles, tt = index - pair * token_tiles;
+    const int slice = pair / feature_tiles, ft = pair - slice * feature_tiles;
     const int m0 = tt * TM, n0 = ft * TN;
-    const int s_begin = blockIdx.y * steps_per_slice;
+    const int s_begin = slice * steps_per_slice;
     const int s_end = s_begin + steps_per_slice < steps_total ? s_begin + steps_per_slice : steps_total;
     const int steps = s_end - s_begin > wave ? (s_end - s_begin - wave + kMidWaves - 1) / kMidWaves : 0;
 
     unsigned char *mine = smem + wave * S::kWaveBytes;
 
-    // lane l of a request brings the 16-byte unit l % 8 of the LDS row l / 8; rows past the end are read from the last
-    const int lrow = lane >> 3, lunit = (lane & 7) ^ lrow;
+    // lane l of request i brings the 16-byte unit l % 8 of the LDS row 8 i + l / 8; rows past the end are read from the last
+    const int lrow = lane >> 3;
+    auto unit_of = [&](int i) { return ((lane & 7) ^ (((i * 8 + lrow) >> 1) & 7)) * U; };
     const T *xsrc[TM / 8], *wsrc[TN / 8];
     const int k_first = (s_begin + wave) * S::kStep;
 #pragma unroll
     for (int i = 0; i < TM / 8; ++i) {
         const int row = m0 + i * 8 + lrow;
-        xsrc[i] = X + (size_t) (row < tokens ? row : tokens - 1) * ldx + k_first + lunit * U;
+        xsrc[i] = X + (size_t) (row < tokens ? row : tokens - 1) * ldx + k_first + unit_of(i);
     }
     size_t w_advance;
     if constexpr (sizeof(T) == 2) {
@@ -96,7 +100,7 @@ __global__ __launch_bounds__(kMidThreads) void dense_mid_kernel(const T *__restr
 #pragma unroll
         for (int i = 0; i < TN / 8; ++i) {
             const int row = n0 + i * 8 + lrow;
-            wsrc[i] = W + (size_t) (row < features ? row : features - 1) * ldw + k_first + lunit * U;
+            wsrc[i] = W + (size_t) (row < features ? row : features - 1) * ldw + k_first + unit_of(i);
         }
     } else {
         // [K, features]: the 32 K values of a step are LDS rows of TN features; lane l brings 4 features
@@ -166,7 +170,7 @@ __global__ __launch_bounds__(kMidThreads) void dense_mid_kernel(const T *__restr
             v8f16 x[4][TB], w[4][FB];  // 16 K values per q: 8 per lane half
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                const int unit = ((q * 2 + hh) ^ (r & 7)) * 16;
+                const int unit = ((q * 2 + hh) ^ ((r >> 1) & 7)) * 16;
 #pragma unroll
                 for (int f = 0; f < FB; ++f)
                     w[q][f] = *reinterpret_cast<const v8f16 *>(stage + S::kXBytes + (f * 32 + r) * kStepBytes + unit);
@@ -189,7 +193,7 @@ __global__ __launch_bounds__(kMidThreads) void dense_mid_kernel(const T *__restr
             for (int q = 0; q < 4; ++q) {  // 8 K values: 4 per lane half
                 v4f32 x[TB];
                 float w[FB][4];
-                const int unit = ((q * 2 + hh) ^ (r & 7)) * 16;
+                const int unit = ((q * 2 + hh) ^ ((r >> 1) & 7)) * 16;
 #pragma unroll
                 for (int f = 0; f < FB; ++f)
 #pragma unroll
@@ -240,7 +244,7 @@ __global__ __launch_bounds__(kMidThreads) void dense_mid_kernel(const T *__restr
         const int row = m0 + token, col = n0 + q * 4;
         if (row >= tokens || col >= features) continue;
         if constexpr (OUT == kMidSlices) {
-            *reinterpret_cast<v4f32 *>(partials + blockIdx.y * slice_stride + (size_t) row * pitch + col) = sum;
+            *reinterpret_cast<v4f32 *>(partials + slice * slice_stride + (size_t) row * pitch + col) = sum;
         } else {
             Vec<T, 4> out;
 #pragma unroll
@@ -275,15 +279,15 @@ struct MidPlan {
     int depth = 2, slices = 1, steps_per_slice = 0;
 };
 
-// The tile and the number of K slices, by a model of the launch time that agrees with the measured ones within about
-// 10 % (in microseconds; 32 to 1000 tokens, the Dense shapes of BERT-base, every tile, depth and 1 to 8 slices):
-// 2.3 for dispatch, the first operands and the drain, then as many rounds as the fullest of the 256 compute units has
-// workgroups.  A workgroup takes its operands at 80 KB per microsecond in half precision (768 x 768 in 32 x 32 tiles:
-// 98 KB, 1.4 us with its epilogue); in fp32 a tile of 32 x 32 takes 4.1 us per 768 K values, 64 x 32 8.0, 64 x 64 14.5.
-// Workgroups that share a compute unit gain nothing over taking turns.  Slices cost their way through memory.
-// Depth: two steps ahead where one workgroup per compute unit is all there is (72 workgroups of 32 x 32 x 768, fp16: one
-// step ahead 4.2, two 3.7 us), one where more workgroups fit the LDS that way (504: 4.8 against 5.0 us); in fp32 two
-// pay off for every tile (504: 13.1 against 11.9 us).
+// The tile and the number of K slices, by a model of the launch time (in microseconds) whose choice is within 12 % of the
+// best one measured for all but two of 112 shapes (32 to 1000 tokens, the Dense shapes of BERT-base, every tile, depth and
+// 1 to 8 slices): 2.3 for dispatch, the first operands and the drain, then as many rounds as the fullest of the 256
+// compute units has workgroups.  A workgroup takes its operands at 80 KB per microsecond in half precision (768 x 768 in
+// 32 x 32 tiles: 98 KB, 1.4 us with its epilogue); in fp32 a tile of 32 x 32 takes 4.1 us per 768 K values, 64 x 32 8.0,
+// 64 x 64 14.5.  Workgroups that share a compute unit gain nothing over taking turns.  Slices cost their way through memory.
+// Depth: two steps ahead where one workgroup per compute unit is all there is (96 workgroups of 32 x 32 x 768, fp16: one
+// step ahead 4.2, two 3.8 us), one where more workgroups fit the LDS that way (672: 6.1 against 6.9 us); in fp32 two pay
+// off for every tile (1056: 24.8 against 22.6 us).
 template <typename T>
 MidPlan plan_mid(int tokens, int features, int steps, bool sliced, size_t partial_floats) {
     static const int kTile[3][2] = {{32, 32}, {64, 32}, {64, 64}};
@@ -322,7 +326,7 @@ int launch_mid(const MidPlan &plan, const T *W, int ldw, const T *X, int ldx, co
     static std::atomic<unsigned long long> raised{0};  // per kernel
     if (!raise_lds_limit(dense_mid_kernel<T, TM, TN, DEPTH, OUT>, raised)) return CUBERT_UNSUPPORTED;
     const int token_tiles = (tokens + TM - 1) / TM, feature_tiles = (features + TN - 1) / TN;
-    const dim3 grid((unsigned) ((feature_tiles + 7) / 8 * 8 * token_tiles), plan.slices), block(kMidThreads);
+    const dim3 grid((unsigned) (feature_tiles * token_tiles * plan.slices)), block(kMidThreads);
     return launch_lds(dense_mid_kernel<T, TM, TN, DEPTH, OUT>, grid, block, (unsigned) S::kLdsBytes, stream, W, ldw, X, ldx,
                       bias, C, ldc, tokens, features, steps, plan.steps_per_slice, token_tiles, feature_tiles, partials,
                       features, (long long) tokens * features);
