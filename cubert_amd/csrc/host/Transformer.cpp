@@ -295,16 +295,44 @@ bool Transformer<T>::attention(size_t batch_size, const T *qkv, const int8_t *ma
 }
 
 // Whether a Dense layer of this size runs on the library's own kernel (kernels/dense_mid.hip) instead of a library
-// GEMM: up to where the two cross.  Whole requests through compute + output, seq 32, library against own, us --
-// half precision, BERT-base: 64 tokens 581 / 340, 128 603 / 400, 512 691 / 573, 768 821 / 705, 1024 859 / 768, 1152
-// 884 / 833, 1280 884 / 859, 1536 942 / 1085; BERT-large: 32 1084 / 774, 512 1497 / 1306, 640 1727 / 1610, 768 1753 /
+// GEMM or the few-token kernel: up to where they cross.  Whole requests through compute + output, seq 32, library against
+// own, us -- half precision, BERT-base: 64 tokens 581 / 340, 128 603 / 400, 512 691 / 573, 768 821 / 705, 1024 859 / 768,
+// 1152 884 / 833, 1280 884 / 859, 1536 942 / 1085; BERT-large: 32 1084 / 774, 512 1497 / 1306, 640 1727 / 1610, 768 1753 /
 // 1740, 896 equal.  fp32, BERT-base: 64 751 / 473, 128 802 / 636, 192 868 / 754, 256 952 / 827, 320 961 / 902, 352
 // 1089 / 1128 (there the kernel keeps the matrix cores 60 % busy, the library 85 % from some thousand tokens on).
-template <typename T>
-bool Transformer<T>::own_dense_takes(int tokens, int out_features, int in_features) const {
-    if (!own_dense) return false;
+//
+// fp32, more than 1024 inputs: only as K slices for the LayerNorm.  Otherwise a few workgroups walk all of K (32 tokens,
+// 6144 -> 1536 with its LayerNorm: 41.6 us, few-token kernel 23.5) in sums longer than the few-token kernel's (2.6e-7
+// against 1.4e-7 of float64; 1536 -> 4608: 1.43e-7 against 1.33e-7).
+// fp32, at most 32 tokens, 640 inputs or more and no more inputs than outputs: the few-token kernel, which cuts K for
+// these, is the faster one where no GELU follows (Q|K|V of 768 6.7 against 7.2 us, of 1024 8.6 / 8.8, of 512 6.1 / 5.7;
+// attention output with its LayerNorm 768 6.2 / 6.4, 1024 7.2 / 7.5, 512 5.3 / 5.2; the intermediate layer of 768 9.0 / 7.4,
+// of 1024 8.7 / 9.0; output 768 9.9 / 9.5, 1024 10.3 / 9.8).
+bool own_dense_is_best(bool half_precision, int tokens, int out_features, int in_features, DenseUse use, bool as_slices) {
     const double products = (double) tokens * out_features * in_features;
-    return sizeof(T) == 2 ? tokens <= 1280 && products <= 3.05e9 : tokens <= 320 && products <= 7.6e8;
+    if (half_precision) return tokens <= 1280 && products <= 3.05e9;
+    if (in_features > 1024 && !(use == DenseUse::kNorm && as_slices)) return false;
+    if (tokens <= 32 && in_features >= 640 && in_features <= out_features && use != DenseUse::kGelu) return false;
+    return tokens <= 320 && products <= 7.6e8;
+}
+
+// CUBERT_FEW_TOKEN_SLICES=0 in the environment keeps the Dense kernels of small requests adding their own K slices.
+static bool few_token_slices_enabled() {
+    static const bool on = [] {
+        const char *e = std::getenv("CUBERT_FEW_TOKEN_SLICES");
+        return e == nullptr || std::string(e) != "0";
+    }();
+    return on;
+}
+
+template <typename T>
+bool Transformer<T>::own_dense_takes(int tokens, int out_features, int in_features, Profiler::Kind kind) const {
+    if (!own_dense) return false;
+    const DenseUse use = kind == Profiler::kDenseQkv            ? DenseUse::kPlain
+                         : kind == Profiler::kDenseIntermediate ? DenseUse::kGelu
+                                                                : DenseUse::kNorm;
+    return own_dense_is_best(sizeof(T) == 2, tokens, out_features, in_features, use,
+                             own_slices_to_norm && few_token_slices_enabled());
 }
 
 // One Dense layer.  The bias goes into the GEMM only where the caller asks for it (bias_in_gemm: the Q/K/V
@@ -316,7 +344,7 @@ bool Transformer<T>::dense(int out_features, int tokens, int in_features, const 
     void *stream = cuBERT::blas_get_stream(cublas);
     Timed t(profiler, profiler != nullptr ? profiler->dense_kind(kind) : Profiler::kDenseGemm, stream);
     if (ld_out == 0) ld_out = out_features;
-    if (own_dense_takes(tokens, out_features, in_features)) {
+    if (own_dense_takes(tokens, out_features, in_features, kind)) {
         const bool with_bias = bias_in_gemm || gelu;
         if (cuBERT::dense_mid(tokens, out_features, in_features, in, in_features, kernel,
                               transposed_kernels ? in_features : out_features, with_bias ? bias : nullptr, gelu, out, ld_out,
@@ -325,7 +353,7 @@ bool Transformer<T>::dense(int out_features, int tokens, int in_features, const 
         }
     }
     // (the few-token kernel reads [in, out] kernels or its own copy of them, not transposed ones)
-    if (!own_dense && tokens <= few_token_limit(kind) && (packed != nullptr || (!transposed_kernels && (gelu || tokens > 32) && dense_gelu_fits))) {
+    if (tokens <= few_token_limit(kind) && (packed != nullptr || (!transposed_kernels && (gelu || tokens > 32) && dense_gelu_fits))) {
         const bool with_bias = bias_in_gemm || gelu;
         if (cuBERT::dense_few_tokens(cublas, out_features, tokens, in_features, kernel, out_features, packed, in,
                                      in_features, out, ld_out, with_bias ? bias : nullptr, gelu)) {
@@ -376,21 +404,12 @@ int Transformer<T>::few_token_limit(Profiler::Kind kind) const {
     }
 }
 
-// CUBERT_FEW_TOKEN_SLICES=0 in the environment keeps the few-token Dense kernels adding their own K slices.
-static bool few_token_slices_enabled() {
-    static const bool on = [] {
-        const char *e = std::getenv("CUBERT_FEW_TOKEN_SLICES");
-        return e == nullptr || std::string(e) != "0";
-    }();
-    return on;
-}
-
 template <typename T>
 void Transformer<T>::dense_norm(int tokens, int in_features, const T *kernel, const T *packed, const T *in, const T *bias,
                                 const T *residual, const T *beta, const T *gamma, T *out, Profiler::Kind kind) {
     void *stream = cuBERT::blas_get_stream(cublas);
     const int H = (int) hidden_size;
-    if (own_dense_takes(tokens, H, in_features) && own_slices_to_norm && few_token_slices_enabled()) {
+    if (own_dense_takes(tokens, H, in_features, kind) && own_slices_to_norm && few_token_slices_enabled()) {
         int slices = 0;
         bool done = false;
         {
@@ -409,8 +428,7 @@ void Transformer<T>::dense_norm(int tokens, int in_features, const T *kernel, co
             own_slices_to_norm = false;  // the hidden size is fixed per model: do not ask again
         }
     }
-    if (!own_dense && tokens <= few_token_limit(kind) && slices_to_norm && few_token_partials != nullptr &&
-        few_token_slices_enabled() &&
+    if (tokens <= few_token_limit(kind) && slices_to_norm && few_token_partials != nullptr && few_token_slices_enabled() &&
         (packed != nullptr || !transposed_kernels)) {
         int slices = 0, pitch = 0;
         bool done = false;

@@ -39,6 +39,13 @@
 
 namespace cuBERT {
 
+// What follows a Dense layer: nothing (its bias is added in the GEMM), bias + GELU, or bias + residual + LayerNorm.
+enum class DenseUse { kPlain, kGelu, kNorm };
+
+// Whether the library's own Dense kernel is the best one for a layer of this size whose sizes it takes; as_slices: the
+// LayerNorm that follows can add K slices.
+bool own_dense_is_best(bool half_precision, int tokens, int out_features, int in_features, DenseUse use, bool as_slices);
+
 template <typename T>
 class Transformer {
 public:
@@ -119,8 +126,8 @@ private:
     void dense_norm(int tokens, int in_features, const T *kernel, const T *packed, const T *in, const T *bias,
                     const T *residual, const T *beta, const T *gamma, T *out, Profiler::Kind kind);
 
-    // whether a Dense layer of this size runs on the library's own kernel (reads the kernels as the model keeps them)
-    bool own_dense_takes(int tokens, int out_features, int in_features) const;
+    // own_dense_is_best for a layer of this model
+    bool own_dense_takes(int tokens, int out_features, int in_features, Profiler::Kind kind) const;
 
     // up to how many tokens the Dense layer of this kind runs on the few-token kernel (32 or 64)
     int few_token_limit(Profiler::Kind kind) const;

@@ -54,7 +54,10 @@ struct MidShape {
 
 enum MidOutput { kMidStore = 0, kMidGelu = 1, kMidSlices = 2 };
 
-template <typename T, int TM, int TN, int DEPTH, int OUT>
+// CHAINS (a power of two) accumulators per block take turns over a wavefront's K values and are added at the end: a single fp32 chain over
+// 192 of 768 K values has 2.5e-7 relative error against float64 (the library's GEMM 2.5e-7 to 5.0e-7), eight 1.1e-7
+// (with K slices 0.9e-7; the few-token kernel, which adds runs of 16 values, 1.1e-7), for 0.2 to 0.5 us a launch.
+template <typename T, int TM, int TN, int DEPTH, int OUT, int CHAINS>
 __global__ __launch_bounds__(kMidThreads) void dense_mid_kernel(const T *__restrict__ W, int ldw,
                                                                 const T *__restrict__ X, int ldx,
                                                                 const T *__restrict__ bias, T *__restrict__ C, int ldc,
@@ -135,11 +138,14 @@ __global__ __launch_bounds__(kMidThreads) void dense_mid_kernel(const T *__restr
         b = load_vec<T, 4>(bias + (f < features ? f : 0));
     }
 
-    v16f32 acc[TB][FB];
+    v16f32 chains[CHAINS][TB][FB];
 #pragma unroll
-    for (int t = 0; t < TB; ++t)
+    for (int c = 0; c < CHAINS; ++c)
 #pragma unroll
-        for (int f = 0; f < FB; ++f) acc[t][f] = v16f32{};
+        for (int t = 0; t < TB; ++t)
+#pragma unroll
+            for (int f = 0; f < FB; ++f) chains[c][t][f] = v16f32{};
+    v16f32 (&acc)[TB][FB] = chains[0];
 
 #pragma unroll
     for (int d = 0; d < DEPTH; ++d) {
@@ -208,13 +214,24 @@ __global__ __launch_bounds__(kMidThreads) void dense_mid_kernel(const T *__restr
 #pragma unroll
                     for (int t = 0; t < TB; ++t)
 #pragma unroll
-                        for (int f = 0; f < FB; ++f)
-                            acc[t][f] = __builtin_amdgcn_mfma_f32_32x32x2f32(w[f][e], x[t][e], acc[t][f], 0, 0, 0);
+                        for (int f = 0; f < FB; ++f) {
+                            v16f32 &chain = chains[(q * 4 + e) * CHAINS / 16][t][f];
+                            chain = __builtin_amdgcn_mfma_f32_32x32x2f32(w[f][e], x[t][e], chain, 0, 0, 0);
+                        }
             }
             refill();
         }
         slot = slot + 1 < DEPTH ? slot + 1 : 0;
     }
+
+#pragma unroll
+    for (int half = CHAINS / 2; half >= 1; half /= 2)
+#pragma unroll
+        for (int c = 0; c < half; ++c)
+#pragma unroll
+            for (int t = 0; t < TB; ++t)
+#pragma unroll
+                for (int f = 0; f < FB; ++f) chains[c][t][f] += chains[c + half][t][f];
 
     // partial tiles to LDS (each wavefront over its own operands, which it has read): a lane owns one token and, per
     // four accumulator registers, four consecutive features
@@ -277,7 +294,10 @@ bool raise_lds_limit(Kernel kernel, std::atomic<unsigned long long> &done) {
 struct MidPlan {
     int tile = 0;  // 0: 32 x 32, 1: 64 x 32, 2: 64 x 64
     int depth = 2, slices = 1, steps_per_slice = 0;
+    int chains = 1;
 };
+
+constexpr int kShortSumTokens = 64, kShortSumChains = 8, kShortSumSteps = 32;
 
 // The tile and the number of K slices, by a model of the launch time (in microseconds) whose choice is within 12 % of the
 // best one measured for all but two of 112 shapes (32 to 1000 tokens, the Dense shapes of BERT-base, every tile, depth and
@@ -288,14 +308,18 @@ struct MidPlan {
 // Depth: two steps ahead where one workgroup per compute unit is all there is (96 workgroups of 32 x 32 x 768, fp16: one
 // step ahead 4.2, two 3.8 us), one where more workgroups fit the LDS that way (672: 6.1 against 6.9 us); in fp32 two pay
 // off for every tile (1056: 24.8 against 22.6 us).
+// fp32 up to 64 tokens, where a caller would otherwise have the few-token kernel's short sums: eight chains of at most 32
+// values each where K is cut (longer slices have 1.7e-7 instead of 1.3e-7, the few-token kernel 1.3e-7 to 1.5e-7), which
+// the registers hold for a tile of 32 x 32.
 template <typename T>
 MidPlan plan_mid(int tokens, int features, int steps, bool sliced, size_t partial_floats) {
     static const int kTile[3][2] = {{32, 32}, {64, 32}, {64, 64}};
     static const float kEpilogue[3] = {0.15f, 0.5f, 1.3f};             // us, half precision
     static const float kF32Step[3] = {4.1f / 24, 8.0f / 24, 14.5f / 24};  // us per step of a workgroup
+    const bool short_sums = sizeof(T) == 4 && tokens <= kShortSumTokens;
     MidPlan best;
     float best_us = 0.f;
-    for (int t = 0; t < 3; ++t) {
+    for (int t = 0; t < (short_sums ? 1 : 3); ++t) {
         const long long tiles = (long long) ((tokens + kTile[t][0] - 1) / kTile[t][0]) *
                                 ((features + kTile[t][1] - 1) / kTile[t][1]);
         for (int want = 1; want <= (sliced ? 16 : 1); ++want) {
@@ -308,6 +332,7 @@ MidPlan plan_mid(int tokens, int features, int steps, bool sliced, size_t partia
                                    : per * kF32Step[t];
             float us = 2.3f + rounds * each;
             if (slices > 1) us += slices * (0.1f + (float) tokens * features * (8.f / 5e6f));
+            if (short_sums && per > kShortSumSteps) us += 1e6f;  // taken only if no finer cut fits
             if (best_us == 0.f || us < best_us) {
                 best_us = us;
                 best.tile = t, best.slices = slices, best.steps_per_slice = per;
@@ -315,19 +340,20 @@ MidPlan plan_mid(int tokens, int features, int steps, bool sliced, size_t partia
             }
         }
     }
+    best.chains = short_sums ? kShortSumChains : 1;
     return best;
 }
 
-template <typename T, int TM, int TN, int DEPTH, int OUT>
+template <typename T, int TM, int TN, int DEPTH, int OUT, int CHAINS>
 int launch_mid(const MidPlan &plan, const T *W, int ldw, const T *X, int ldx, const T *bias, T *C, int ldc, int tokens,
                int features, int steps, float *partials, hipStream_t stream) {
     typedef MidShape<T, TM, TN, DEPTH> S;
     static_assert(S::kLdsBytes <= 160 * 1024, "LDS of a compute unit");
     static std::atomic<unsigned long long> raised{0};  // per kernel
-    if (!raise_lds_limit(dense_mid_kernel<T, TM, TN, DEPTH, OUT>, raised)) return CUBERT_UNSUPPORTED;
+    if (!raise_lds_limit(dense_mid_kernel<T, TM, TN, DEPTH, OUT, CHAINS>, raised)) return CUBERT_UNSUPPORTED;
     const int token_tiles = (tokens + TM - 1) / TM, feature_tiles = (features + TN - 1) / TN;
     const dim3 grid((unsigned) (feature_tiles * token_tiles * plan.slices)), block(kMidThreads);
-    return launch_lds(dense_mid_kernel<T, TM, TN, DEPTH, OUT>, grid, block, (unsigned) S::kLdsBytes, stream, W, ldw, X, ldx,
+    return launch_lds(dense_mid_kernel<T, TM, TN, DEPTH, OUT, CHAINS>, grid, block, (unsigned) S::kLdsBytes, stream, W, ldw, X, ldx,
                       bias, C, ldc, tokens, features, steps, plan.steps_per_slice, token_tiles, feature_tiles, partials,
                       features, (long long) tokens * features);
 }
@@ -337,16 +363,19 @@ int launch_mid_tile(const MidPlan &plan, Args... args) {
     if constexpr (sizeof(T) == 2) {
         if (plan.depth == 1) {
             switch (plan.tile) {
-                case 0: return launch_mid<T, 32, 32, 1, OUT>(plan, args...);
-                case 1: return launch_mid<T, 64, 32, 1, OUT>(plan, args...);
-                default: return launch_mid<T, 64, 64, 1, OUT>(plan, args...);
+                case 0: return launch_mid<T, 32, 32, 1, OUT, 1>(plan, args...);
+                case 1: return launch_mid<T, 64, 32, 1, OUT, 1>(plan, args...);
+                default: return launch_mid<T, 64, 64, 1, OUT, 1>(plan, args...);
             }
         }
     }
+    if constexpr (sizeof(T) == 4) {
+        if (plan.chains != 1) return launch_mid<T, 32, 32, 2, OUT, kShortSumChains>(plan, args...);
+    }
     switch (plan.tile) {
-        case 0: return launch_mid<T, 32, 32, 2, OUT>(plan, args...);
-        case 1: return launch_mid<T, 64, 32, 2, OUT>(plan, args...);
-        default: return launch_mid<T, 64, 64, 2, OUT>(plan, args...);
+        case 0: return launch_mid<T, 32, 32, 2, OUT, 1>(plan, args...);
+        case 1: return launch_mid<T, 64, 32, 2, OUT, 1>(plan, args...);
+        default: return launch_mid<T, 64, 64, 2, OUT, 1>(plan, args...);
     }
 }
 

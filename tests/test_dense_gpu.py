@@ -80,6 +80,27 @@ def test_dense_slices_add_up_and_reach_the_layer_norm(K, name, tokens, width):
     assert float((got.float() - plain.float()).abs().max()) <= (2e-5 if name == "f32" else 2.0 ** -7)
 
 
+@pytest.mark.parametrize("tokens", [1, 32, 33, 64])
+@pytest.mark.parametrize("features,width", [(3072, 768), (768, 768), (768, 3072), (1024, 1024), (1024, 4096), (256, 8192),
+                                            (9216, 512)])
+def test_fp32_sums_of_few_tokens_are_as_short_as_the_few_token_kernels(K, tokens, features, width):
+    """fp32 up to 64 tokens: the error against float64 is no larger than the few-token kernel's (K slices where the layer
+    stands in front of a LayerNorm).  The two have at least 768 errors each of the same size, so their root mean squares are
+    known to 1 / sqrt(2 * 768) = 2.6 % each; a single chain over a wavefront's K is 1.3 to 3.5 times as far off."""
+    x, w, _, x64, w64, _ = operands("f32", tokens, features, width, 0)
+    want = x64 @ w64
+
+    def error(y):
+        return np.sqrt(((y.double().cpu().numpy() - want) ** 2).mean())
+    blas = K.Blas()
+    few, _, _ = blas.gemm_skinny_partials(features, tokens, width, w, features, x, width)
+    slices = K.dense_slices(x, w) if width >= features else None
+    own = slices.sum(0) if slices is not None else K.dense(x, w)
+    few = few[:, :tokens, :features].sum(0)
+    blas.close()
+    assert error(own) <= (1 + 2 * 0.026) * error(few), (error(own), error(few))
+
+
 @pytest.mark.parametrize("name", ["f32", "f16"])
 def test_dense_declines_what_it_cannot_do(K, name):
     dtype = torch.float32 if name == "f32" else torch.float16

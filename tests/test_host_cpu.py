@@ -311,3 +311,18 @@ def test_bench_algorithmic_bytes_follow_the_published_formulas():
         del os.environ["CUBERT_FP32_DENSE"]
     assert two_term["bias_gelu"] == 4096 * 3072 * 10 + 3072 * 4 and two_term["dense_split"] == 4096 * 768 * 10
     assert half_model["bias_gelu"] == bench.algorithmic_bytes(CONFIGS["C3"])["bias_gelu"]  # fp16 models: unchanged
+
+
+def test_which_dense_layers_keep_to_short_sums():
+    """fp32 layers whose sums the own Dense kernel would make longer than the few-token kernel's (more than 1024 inputs
+    that nobody takes as K slices), and those of at most 32 tokens for which that kernel is the faster one."""
+    from cubert_amd._lib import lib
+    best = lib().cubert_dense_is_best
+    plain, gelu, norm = 0, 1, 2
+    for tokens in (1, 32, 33, 64, 128):
+        assert not best(0, tokens, 3 * 1280, 1280, plain, 0) and not best(0, tokens, 4 * 1280, 1280, gelu, 0)
+        assert not best(0, tokens, 1280, 5120, norm, 0) and not best(0, tokens, 896, 3584, norm, 0)
+        assert best(0, tokens, 768, 3072, norm, 1) and best(1, tokens, 896, 3584, norm, 0)
+        assert best(0, tokens, 1536, 512, plain, 0) and best(0, tokens, 3072, 768, gelu, 0)
+    for tokens, expected in ((1, 0), (32, 0), (33, 1), (64, 1)):
+        assert best(0, tokens, 2304, 768, plain, 0) == expected and best(0, tokens, 768, 768, norm, 1) == expected
