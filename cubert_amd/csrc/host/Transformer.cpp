@@ -295,12 +295,19 @@ bool Transformer<T>::attention(size_t batch_size, const T *qkv, const int8_t *ma
 }
 
 // Whether a Dense layer of this size runs on the library's own kernel (kernels/dense_mid.hip) instead of a library
-// GEMM or the few-token kernel: up to where they cross.  Whole requests through compute + output, seq 32, library against
-// own, us -- half precision, BERT-base: 64 tokens 581 / 340, 128 603 / 400, 512 691 / 573, 768 821 / 705, 1024 859 / 768,
-// 1152 884 / 833, 1280 884 / 859, 1536 942 / 1085; BERT-large: 32 1084 / 774, 512 1497 / 1306, 640 1727 / 1610, 768 1753 /
-// 1740, 896 equal.  fp32, BERT-base: 64 751 / 473, 128 802 / 636, 192 868 / 754, 256 952 / 827, 320 961 / 902, 352
-// 1089 / 1128 (there the kernel keeps the matrix cores 60 % busy, the library 85 % from some thousand tokens on).
-//
+// GEMM or the few-token kernel: up to where they cross, which depends on what follows.  A library GEMM adds the bias of
+// Q|K|V by itself, pays a launch for GELU, and leaves K uncut in front of a LayerNorm.  A layer with its GELU or
+// LayerNorm, weights from a model's worth of them, library against own, us:
+//   half Q|K|V      512 in: 1280 tokens 8.7 / 7.3; 640: 1024 8.2 / 8.4, 1152 9.0 / 11.0; 768: 384 7.6 / 6.1, 896
+//                   9.0 / 9.1, 1024 11.1 / 12.0, 1280 10.6 / 13.0; 1024: 512 10.2 / 9.6, 640 10.2 / 10.7, 896
+//                   11.8 / 13.7; 1536: 256 15.5 / 14.0, 320 12.4 / 13.9
+//   attention out   1024: 1280 13.2 / 12.8; 1536: 640 12.8 / 11.6, 768 15.4 / 16.9; 2048: 640 17.3 / 20.7
+//   intermediate    768 in: 1280 19.1 / 16.6; 1024 in: 896 20.7 / 19.5; 2048 in: 320 23.7 / 23.5
+//   output          3072 in: 1280 19.0 / 18.2; 4096 in: 896 20.8 / 18.5
+//   fp32 Q|K|V      768 in: 96 tokens 7.8 / 7.1, 128 9.7 / 10.8, 320 13.4 / 15.7; 1024 in: 64 9.9 / 9.2, 80 9.8 / 13.7
+//   attention out   768: 320 10.5 / 9.9; 1024: 256 12.1 / 11.5, 320 14.5 / 15.3
+//   intermediate    768 in: 320 20.0 / 18.2; 1024 in: 160 20.8 / 19.2, 224 23.7 / 23.1, 320 29.0 / 29.7
+//   output          3072 in: 256 21.6 / 19.5, 320 22.0 / 22.9; 4096 in: 160 26.0 / 20.4
 // fp32, more than 1024 inputs: only as K slices for the LayerNorm.  Otherwise a few workgroups walk all of K (32 tokens,
 // 6144 -> 1536 with its LayerNorm: 41.6 us, few-token kernel 23.5) in sums longer than the few-token kernel's (2.6e-7
 // against 1.4e-7 of float64; 1536 -> 4608: 1.43e-7 against 1.33e-7).
@@ -310,10 +317,17 @@ bool Transformer<T>::attention(size_t batch_size, const T *qkv, const int8_t *ma
 // of 1024 8.7 / 9.0; output 768 9.9 / 9.5, 1024 10.3 / 9.8).
 bool own_dense_is_best(bool half_precision, int tokens, int out_features, int in_features, DenseUse use, bool as_slices) {
     const double products = (double) tokens * out_features * in_features;
-    if (half_precision) return tokens <= 1280 && products <= 3.05e9;
+    const bool narrowing = in_features > out_features;
+    if (half_precision) {
+        if (tokens > 1280) return false;
+        if (use == DenseUse::kPlain) return products <= (tokens <= 1024 ? 1.65e9 : 1.3e9);
+        return products <= (use == DenseUse::kGelu || narrowing ? 3.05e9 : 1.7e9);
+    }
     if (in_features > 1024 && !(use == DenseUse::kNorm && as_slices)) return false;
-    if (tokens <= 32 && in_features >= 640 && in_features <= out_features && use != DenseUse::kGelu) return false;
-    return tokens <= 320 && products <= 7.6e8;
+    if (tokens <= 32 && in_features >= 640 && !narrowing && use != DenseUse::kGelu) return false;
+    if (tokens > 320) return false;
+    if (use == DenseUse::kPlain) return products <= 2.1e8;
+    return products <= (use == DenseUse::kGelu ? 7.6e8 : narrowing ? 7.0e8 : 3.0e8);
 }
 
 // CUBERT_FEW_TOKEN_SLICES=0 in the environment keeps the Dense kernels of small requests adding their own K slices.

@@ -326,3 +326,16 @@ def test_which_dense_layers_keep_to_short_sums():
         assert best(0, tokens, 1536, 512, plain, 0) and best(0, tokens, 3072, 768, gelu, 0)
     for tokens, expected in ((1, 0), (32, 0), (33, 1), (64, 1)):
         assert best(0, tokens, 2304, 768, plain, 0) == expected and best(0, tokens, 768, 768, norm, 1) == expected
+
+
+@pytest.mark.parametrize("dtype,use,layer,last,first", [
+    # the last token count measured ahead of the library's GEMM and the first one measured behind it
+    (1, 0, (768, 2304), 896, 1024), (1, 0, (1024, 3072), 512, 640), (1, 0, (1536, 4608), 128, 320), (1, 0, (512, 1536), 1280, 1281), (1, 0, (640, 1920), 1024, 1152),
+    (1, 2, (1024, 1024), 1280, 1281), (1, 2, (1536, 1536), 640, 768), (1, 2, (2048, 2048), 320, 640),
+    (1, 1, (768, 3072), 1280, 1281), (1, 1, (1024, 4096), 640, 1280), (1, 2, (3072, 768), 1280, 1281),
+    (0, 0, (768, 2304), 96, 128), (0, 0, (1024, 3072), 64, 80), (0, 2, (768, 768), 320, 321), (0, 2, (1024, 1024), 256, 320),
+    (0, 1, (768, 3072), 320, 321), (0, 1, (1024, 4096), 160, 320), (0, 2, (3072, 768), 256, 320)])
+def test_where_the_library_gemm_takes_over(dtype, use, layer, last, first):
+    from cubert_amd._lib import lib
+    best = lib().cubert_dense_is_best
+    assert best(dtype, last, layer[1], layer[0], use, 1) and not best(dtype, first, layer[1], layer[0], use, 1)
