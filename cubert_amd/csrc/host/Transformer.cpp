@@ -220,6 +220,22 @@ T *Transformer<T>::compute(size_t batch_size, T *input_gpu, int8_t *attention_ma
 template <typename T>
 void Transformer<T>::_pre_compute(size_t) {}
 
+// fp32 sequences of more than 288 keys, few (sequence, head) problems: the one-launch kernels give a problem to one
+// workgroup, which then walks all keys of all queries by itself, while the three steps spread over the chip.  Two layers of
+// BERT-base through compute + output, three steps against one launch, us (lengths drawn between a quarter and all of a
+// sequence): 1 x 333 196 / 259, 1 x 500 243 / 425, 2 x 450 334 / 433, 3 x 500 485 / 600, 4 x 450 571 / 616, 4 x 333 430 /
+// 426, 6 x 333 603 / 544; 16 heads: 3 x 480 688 / 725, 4 x 480 848 / 832.  Up to 288 keys one launch is level at worst (1 x
+// 250 213 / 214, 2 x 250 299 / 236), and at 512 the three steps lost before.  With a head size of 32 K and V stay in the
+// LDS, which 12 problems notice from 333 keys on (165 / 175, 1 x 500 185 / 261; 2 x 333 212 / 175) where the length is no
+// multiple of 32 and level otherwise.
+template <typename T>
+bool Transformer<T>::three_step_attention_is_faster(size_t batch_size) const {
+    if (sizeof(T) != 4 || seq_length <= 288 || seq_length >= 512) return false;
+    const size_t problems = batch_size * num_attention_heads, head_size = hidden_size / num_attention_heads;
+    if (head_size == 32) return problems <= 16 && seq_length > 320 && seq_length % 32 != 0;
+    return problems <= 48;
+}
+
 // scores[b, a, q, k] = (1/sqrt d) * sum_j Q[b, q, a, j] K[b, k, a, j];  softmax with mask;
 // ctx[b, q, a, :] = sum_k p[b, a, q, k] V[b, k, a, :].   Q, K, V are column blocks of qkv[M, 3H].
 // The contractions run as one matrix-core launch each where the shape allows.  Otherwise: the (b, a)
@@ -242,7 +258,7 @@ bool Transformer<T>::attention(size_t batch_size, const T *qkv, const int8_t *ma
         const char *e = std::getenv("CUBERT_ATTENTION");
         return e != nullptr && std::string(e) == "split";
     }();
-    if (!split_only && fused_attention_fits) {
+    if (!split_only && fused_attention_fits && !three_step_attention_is_faster(batch_size)) {
         Timed t(profiler, Profiler::kAttentionFused, stream);
         if constexpr (sizeof(T) == 4) {
             if (split_context != nullptr &&
@@ -481,6 +497,7 @@ T *Transformer<T>::_in_compute(size_t batch_size, T *input_gpu, int8_t *attentio
 
     // long sequences: the attention kernels take the sequences longest first (the mask is the same for every layer)
     order_ready = seq_length > 128 && attention_mask != nullptr && fused_attention_fits &&
+                  !three_step_attention_is_faster(batch_size) &&
                   cuBERT::attention_order(attention_mask, (int) batch_size, (int) seq_length, attention_order, stream);
 
     T *prev_output = input_gpu;

@@ -109,6 +109,8 @@ private:
     // one-launch kernel takes every BERT shape up to seq_length 512, so it is not part of `buffers` (it would be the
     // largest of them: 403 MB at batch 64 x 12 heads x seq 512 in fp16) but allocated on first use.
     T *scores();
+    // whether scores, softmax and context in three steps beat the one-launch attention kernel for this many sequences
+    bool three_step_attention_is_faster(size_t batch_size) const;
     // context_out = attention(qkv); with `split_context` (fp32 models in the two-term Dense form) the one-launch
     // kernel writes the context there as two-term rows instead and true is returned
     bool attention(size_t batch_size, const T *qkv, const int8_t *mask, half *split_context = nullptr);

@@ -165,6 +165,31 @@ def test_requests_of_33_to_64_tokens(cb, compute_type, seq_length, batches):
     bert.close()
 
 
+@pytest.mark.parametrize("seq_length,heads,hidden,three_steps,one_launch", [
+    (333, 2, 128, (1, 24), (25,)), (320, 3, 192, (16,), (17,)), (511, 2, 128, (2,), (25,)), (288, 2, 128, (), (1, 2)),
+    (333, 2, 64, (1, 8), (9,)), (352, 2, 64, (), (1,)), (512, 2, 128, (), (1,))])
+def test_long_fp32_sequences_by_number_of_problems(cb, seq_length, heads, hidden, three_steps, one_launch):
+    """fp32 sequences of more than 288 keys: few (sequence, head) problems run scores, softmax and context in three steps,
+    which use more of the chip than a workgroup per problem; more of them take the one-launch kernel.  Either way the
+    outputs are the oracle's."""
+    from cubert_amd.testing import random_bert_weights, random_inputs
+    m = dict(vocab=97, hidden=hidden, layers=1, heads=heads, intermediate=4 * hidden, max_position=512, type_vocab=2)
+    w = random_bert_weights(seed=31, labels=2, pooler=True, classifier=True, ln_random=True, **m)
+    largest = max(three_steps + one_launch)
+    ids, mask, seg = random_inputs(seed=32, batch=largest, seq_length=seq_length, vocab=97, min_valid=3, segment_split=9)
+    rows = 2  # rows of a batch are independent
+    want = oracle.bert_forward(w, ids[:rows], mask[:rows], seg[:rows], 1, heads)
+    bert = cb.Bert(w, largest, seq_length, 1, heads, 0)
+    bert.profile(["attention_fused", "attention_gemm", "mask_scale_softmax"])
+    for n in three_steps + one_launch:
+        got = bert.forward(ids[:n], mask[:n], seg[:n])
+        kinds = set(bert.profile_read())
+        assert kinds == ({"attention_gemm", "mask_scale_softmax"} if n in three_steps else {"attention_fused"}), (n, kinds)
+        for k in ("sequence_output", "pooled_output", "logits", "probs"):
+            assert_close(got[k][:rows], want[k][:n], FP32_TOL, "%s, %d sequences" % (k, n))
+    bert.close()
+
+
 def test_repeated_calls_and_smaller_batches_reuse_buffers(cb):
     """The reference's BertMTest calls one model four times; results must not depend on what ran before."""
     from cubert_amd.testing import random_bert_weights, random_inputs
