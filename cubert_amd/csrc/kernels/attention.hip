@@ -908,9 +908,11 @@ __global__ __launch_bounds__(4 * kWave) void attention_small_kernel(const T *__r
 // masked key's score is 10000 below every unmasked one of its query, its exp is exactly 0 in fp32, so it adds
 // nothing to the sum or the context as long as the sequence has one unmasked key (a sequence without any keeps
 // all its tiles: there the shift cancels and the softmax runs over the raw scores, as in the reference).  Every
-// query row, padded or not, is still computed.  skip_masked_tiles = 0: the mask cannot be read as 32-bit words and is
-// read as bytes.
-template <typename T, int D, bool SPLIT>
+// query row, padded or not, is still computed.  skip_masked_tiles = 0: the mask cannot be read as 32-bit words; with
+// RAGGED it is read as bytes, otherwise every tile is computed.
+// RAGGED: seq is not a multiple of 32 (with the clamped rows and guarded stores in every launch: 13 x 384, 12 heads, fp16
+// 20.3 instead of 19.5 us, 32 x 256 18.5 instead of 17.1).
+template <typename T, int D, bool SPLIT, bool RAGGED>
 __global__ __launch_bounds__(1024) void attention_flash_kernel(const T *__restrict__ q, const T *__restrict__ k,
                                                                const T *__restrict__ v, int ld,
                                                                const int8_t *__restrict__ mask, T *__restrict__ ctx,
@@ -921,8 +923,8 @@ __global__ __launch_bounds__(1024) void attention_flash_kernel(const T *__restri
     constexpr int kColTiles = D / 32;
     constexpr int kChunk = 2;  // key tiles per step
     constexpr int kPitchK = D + V;
-    const int KT = (seq + 31) / 32, S = KT * 32;  // (the last key tile may be filled up: kNoKey)
-    auto valid_row = [&](int row) { return row < seq ? row : seq - 1; };
+    const int KT = RAGGED ? (seq + 31) / 32 : seq / 32, S = RAGGED ? KT * 32 : seq;
+    auto valid_row = [&](int row) { return RAGGED && row >= seq ? seq - 1 : row; };
     const int threads = blockDim.x;  // = KT * 64
     const int pitch_v = S + V;
     extern __shared__ __align__(16) unsigned char smem[];
@@ -956,7 +958,7 @@ __global__ __launch_bounds__(1024) void attention_flash_kernel(const T *__restri
             for (int i = 0; i < 8; ++i) any |= words[kt * 8 + i];
             live |= (any != 0 ? 1u : 0u) << kt;
         }
-    } else if (mask != nullptr) {
+    } else if (RAGGED && mask != nullptr) {
         unsigned all;
         key_tile_bits(mask + (size_t) b * seq, seq, KT, live, all);
     }
@@ -989,7 +991,7 @@ __global__ __launch_bounds__(1024) void attention_flash_kernel(const T *__restri
         }
     }
     for (int i = threadIdx.x; i < S; i += threads) {
-        s_mask[i] = additive_mask(mask != nullptr ? mask + (size_t) b * seq : nullptr, i, seq);
+        s_mask[i] = additive_mask(mask != nullptr ? mask + (size_t) b * seq : nullptr, i, RAGGED ? seq : S);
     }
 #pragma unroll
     for (int u = 0; u < kLoads; ++u) {
@@ -1116,7 +1118,7 @@ __global__ __launch_bounds__(1024) void attention_flash_kernel(const T *__restri
         for (int jt = 0; jt < kColTiles; ++jt) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                if (qt * 32 + acc_row(g * 4 + e, hh) >= seq) continue;
+                if (RAGGED && qt * 32 + acc_row(g * 4 + e, hh) >= seq) continue;
                 store_context<T, SPLIT>(ctx, ld_ctx, first_row + acc_row(g * 4 + e, hh), h * D + jt * 32 + r,
                                  out[jt][g * 4 + e] * fr.v[e], split);
             }
@@ -1669,8 +1671,14 @@ int launch_flash(const T *q, const T *k, const T *v, int ld, const int8_t *mask,
             grid, dim3(1024), grouped_lds, s, q, k, v, ld, mask, ctx, ld_ctx, alpha, heads, seq, skip_masked_tiles, split,
             order, use_records);
     }
-    return launch_attention<attention_flash_kernel<T, D, SPLIT>>(grid, dim3(tiles * kWave), lds, s, q, k, v, ld, mask, ctx,
-                                                                 ld_ctx, alpha, heads, seq, skip_masked_tiles, split, order);
+    if (seq % 32 == 0) {
+        return launch_attention<attention_flash_kernel<T, D, SPLIT, false>>(grid, dim3(tiles * kWave), lds, s, q, k, v, ld, mask,
+                                                                            ctx, ld_ctx, alpha, heads, seq,
+                                                                            skip_masked_tiles, split, order);
+    }
+    return launch_attention<attention_flash_kernel<T, D, SPLIT, true>>(grid, dim3(tiles * kWave), lds, s, q, k, v, ld, mask, ctx,
+                                                                       ld_ctx, alpha, heads, seq, skip_masked_tiles, split,
+                                                                       order);
 }
 
 template <typename T>
