@@ -1390,10 +1390,12 @@ constexpr int kOrderMaxBatch = 4096;
 // sequence at position i -- {number of live tiles, their tile numbers in ascending order 4 bits each (low word, high
 // word), the live tiles as a bit mask} -- so that a long-sequence kernel gets its list of tiles with one scalar load
 // instead of reading the mask row again.  8 * batch ints in all.
-// A wavefront reads four mask rows at a time, 64 bytes per load, all requested first: any length and alignment.
-constexpr int kOrderThreads = 1024;
-__global__ __launch_bounds__(kOrderThreads) void attention_order_kernel(const int8_t *__restrict__ mask, int batch, int seq,
-                                                                        int *__restrict__ order) {
+// Rows of whole tiles are read as 32-bit words, a thread per row (64 x 256: 4.8 us, 4096 x 256 39).  RAGGED rows may start
+// at any address: a wavefront reads four of them at a time, 64 bytes per load, all requested first (7.3 and 200 us).
+template <bool RAGGED>
+__global__ __launch_bounds__(RAGGED ? 1024 : kBlock) void attention_order_kernel(const int8_t *__restrict__ mask, int batch,
+                                                                                 int seq, int *__restrict__ order) {
+    constexpr int kThreads = RAGGED ? 1024 : kBlock;
     __shared__ unsigned char tiles_of[kOrderMaxBatch];
     __shared__ unsigned short bits_of[kOrderMaxBatch];
     __shared__ int bucket[20];  // [t]: sequences with t live tiles (t <= 16), then their first position
@@ -1402,7 +1404,25 @@ __global__ __launch_bounds__(kOrderThreads) void attention_order_kernel(const in
     const int lane = threadIdx.x & (kWave - 1);
     if (threadIdx.x < 20) bucket[threadIdx.x] = 0;
     __syncthreads();
-    for (int b0 = wave_in_block() * kRows; b0 < batch; b0 += kOrderThreads / kWave * kRows) {
+    auto keep = [&](int b, unsigned bits) {
+        if (bits == 0) bits = (1u << key_tiles) - 1u;  // no kept key: the kernels compute every tile
+        const int live = __popc(bits);
+        tiles_of[b] = (unsigned char) live;
+        bits_of[b] = (unsigned short) bits;
+        atomicAdd(&bucket[live], 1);
+    };
+    for (int b = threadIdx.x; !RAGGED && b < batch; b += kThreads) {
+        const uint32_t *words = reinterpret_cast<const uint32_t *>(mask + (size_t) b * seq);
+        unsigned bits = 0;
+        for (int kt = 0; kt < key_tiles; ++kt) {
+            uint32_t any = 0;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) any |= words[kt * 8 + i];
+            bits |= (any != 0 ? 1u : 0u) << kt;
+        }
+        keep(b, bits);
+    }
+    for (int b0 = wave_in_block() * kRows; RAGGED && b0 < batch; b0 += kThreads / kWave * kRows) {
         int8_t m[kRows][8];
 #pragma unroll
         for (int t = 0; t < kRows; ++t) {
@@ -1421,13 +1441,7 @@ __global__ __launch_bounds__(kOrderThreads) void attention_order_kernel(const in
                 const unsigned long long kept = __ballot(u * kWave + lane < seq && m[t][u] != 0);
                 bits |= ((unsigned) kept != 0 ? 1u : 0u) << (2 * u) | (kept >> 32 != 0 ? 2u : 0u) << (2 * u);
             }
-            if (bits == 0) bits = (1u << key_tiles) - 1u;  // no kept key: the kernels compute every tile
-            if (lane == 0 && b0 + t < batch) {
-                const int live = __popc(bits);
-                tiles_of[b0 + t] = (unsigned char) live;
-                bits_of[b0 + t] = (unsigned short) bits;
-                atomicAdd(&bucket[live], 1);
-            }
+            if (lane == 0 && b0 + t < batch) keep(b0 + t, bits);
         }
     }
     __syncthreads();
@@ -1440,7 +1454,7 @@ __global__ __launch_bounds__(kOrderThreads) void attention_order_kernel(const in
         }
     }
     __syncthreads();
-    for (int b = threadIdx.x; b < batch; b += kOrderThreads) {
+    for (int b = threadIdx.x; b < batch; b += kThreads) {
         const int at = atomicAdd(&bucket[tiles_of[b]], 1);
         order[at] = b;
         const unsigned bits = bits_of[b];
@@ -1465,7 +1479,8 @@ int attention_order(const int8_t *mask, int batch, int seq, int *order, void *st
         !is_aligned(order, 16)) {
         return CUBERT_UNSUPPORTED;
     }
-    return launch_untimed(attention_order_kernel, dim3(1), dim3(kOrderThreads), 0u, (hipStream_t) stream, mask, batch, seq,
+    const auto kernel = seq % 32 == 0 ? attention_order_kernel<false> : attention_order_kernel<true>;
+    return launch_untimed(kernel, dim3(1), dim3(seq % 32 == 0 ? kBlock : 1024), 0u, (hipStream_t) stream, mask, batch, seq,
                           order);
 }
 

@@ -1085,6 +1085,24 @@ def test_unaligned_views_take_the_generic_path(K):
     assert_close(host(view), want, FP32_TOL)
 
 
+def test_order_of_whole_tiles_reads_words(K):
+    """Rows of whole tiles are read as words (39 to 72 us for 4096 rows of 256 to 512 keys), rows of any length as bytes
+    (200 us): less than seven tenths of it, best of several runs each."""
+    def best(seq):
+        mask = torch.ones((4096, seq), dtype=torch.int8, device="cuda")
+        times = []
+        for _ in range(8):
+            start, stop = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            for _ in range(10):
+                K.attention_order(mask)
+            stop.record()
+            torch.cuda.synchronize()
+            times.append(start.elapsed_time(stop))
+        return min(times)
+    assert best(256) < 0.7 * best(255)
+
+
 # ------------------------------------------------------------------ attention at any sequence length
 
 @pytest.mark.parametrize("name", ["f32", "f16"])
