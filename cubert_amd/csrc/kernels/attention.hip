@@ -318,17 +318,27 @@ constexpr float kMaskedScore = -10000.0f;
 constexpr float kLog2e = 1.4426950408889634f;
 
 // Sequence lengths that are not a multiple of 32 run on the same kernels with the last key tile filled up: rows past
-// the end are read from the last valid row (finite values, no load under a branch), such a key's additive mask is
-// kNoKey -- its exp is exactly 0 whatever the other keys are, also in a sequence whose mask keeps none -- and such a
-// query row is computed and not stored.  (Before, such a length took 2 * min(batch, heads) library launches and a
-// softmax launch per layer: a BERT-base request of 20 x 100 tokens in fp32 6.20 -> 3.12 ms, 7 x 50 in fp16 2.38 -> 0.83 ms,
-// 5 x 24 in fp32 1.87 -> 0.84 ms.)
-constexpr float kNoKey = -1e30f;
+// the end are read from the last valid row (no load under a branch), such a key's additive mask is kNoKey, so that its
+// exp is exactly 0 whatever the other keys are, also in a sequence whose mask keeps none; its row of V counts as zeros (a
+// probability of 0 times the infinity or NaN that the last valid row may hold would not be 0); and such a query row is
+// computed and not stored.  Against library GEMMs per sequence or head and a softmax launch: 20 x 100 tokens of BERT-base
+// in fp32 3.12 instead of 6.20 ms, 7 x 50 in half precision 0.83 instead of 2.38, 5 x 24 in fp32 0.84 instead of 1.87.
+constexpr float kNoKey = -__builtin_huge_valf();
 
 // Additive mask of key i in units of log 2; `row` is the sequence's mask row or null.
 __device__ __forceinline__ float additive_mask(const int8_t *row, int i, int seq) {
     if (i >= seq) return kNoKey;
     return row != nullptr && !row[i] ? kMaskedScore * kLog2e : 0.f;
+}
+
+// Zeros in place of the keys past the end among the V keys of slot group `grp` (of a tile's 32 / V), read from tile kt.
+template <typename T, int V>
+__device__ __forceinline__ void zero_missing_keys(Vec<T, V> &values, int grp, int kt, int seq) {
+    const int in_tile = grp % (32 / V), run = in_tile >> 1, half = in_tile & 1;
+#pragma unroll
+    for (int e = 0; e < V; ++e) {
+        values.v[e] = keep_or_zero(values.v[e], kt * 32 + acc_row(run * V + e, half) < seq);
+    }
 }
 
 // Bit kt of any: tile kt (32 keys) has a kept key; of all: its 32 keys exist and are all kept.  Read as bytes, 64 per
@@ -481,6 +491,7 @@ __global__ __launch_bounds__(KT * kWave) void attention_fused_kernel(const T *__
     for (int u = 0; u < kLoadsV; ++u) {
         const int idx = threadIdx.x + u * kThreads;
         const int j = idx % D, grp = idx / D;
+        if (RAGGED) zero_missing_keys<T, V>(vreg[u], grp, grp / (32 / V), seq);
         store_vec<T, V>(s_vt + j * kPitchV + grp * V, vreg[u]);
     }
     __syncthreads();
@@ -703,6 +714,10 @@ __global__ __launch_bounds__(KT * kWave) void attention_fused_half_kernel(const 
     for (int u = 0; u < kLoads; ++u) {
         const int idx = threadIdx.x + u * kThreads;
         const int row = idx / kVecPerRow, c = idx - row * kVecPerRow;
+        if (RAGGED) {
+#pragma unroll
+            for (int e = 0; e < V; ++e) vreg[u].v[e] = keep_or_zero(vreg[u].v[e], row < seq);
+        }
         store_vec<T, V>(s_v + row * kPitchV + c * V, vreg[u]);
     }
     __syncthreads();  // (also: every wavefront is done with K, whose space the context tiles use below)
@@ -875,7 +890,7 @@ __global__ __launch_bounds__(4 * kWave) void attention_small_kernel(const T *__r
 #pragma unroll
         for (int e = 0; e < V; ++e) {
             a.v[e] = from_f32<T>(normalise_prob<T>(p[kh * 8 + run * V + e], sum, inv));
-            bv.v[e] = vreg[run * V + e];
+            bv.v[e] = RAGGED ? keep_or_zero(vreg[run * V + e], acc_row(kh * 8 + run * V + e, hh) < seq) : vreg[run * V + e];
         }
         Mma<T>::run(out, a, bv);
     }
@@ -1003,6 +1018,7 @@ __global__ __launch_bounds__(1024) void attention_flash_kernel(const T *__restri
     for (int u = 0; u < kLoads; ++u) {
         const int idx = threadIdx.x + u * threads;
         const int j = idx % D, grp = idx / D;
+        if (RAGGED) zero_missing_keys<T, V>(vreg[u], grp, grp / (32 / V), seq);
         store_vec<T, V>(s_vt + j * pitch_v + grp * V, vreg[u]);
     }
     __syncthreads();
@@ -1269,6 +1285,7 @@ __global__ __launch_bounds__(1024) void attention_flash_grouped_kernel(
         for (int u = 0; u < kLoads; ++u) {
             const int idx = threadIdx.x + u * kThreads;
             const int j = idx % D, grp = idx / D;
+            if (ANY_SEQ && grp / (32 / V) < in_group) zero_missing_keys<T, V>(vreg[u], grp, tile_of(grp / (32 / V)), seq);
             store_vec<T, V>(s_vt + j * kPitchV + grp * V, vreg[u]);
         }
         __syncthreads();

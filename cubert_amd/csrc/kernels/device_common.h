@@ -56,6 +56,9 @@ __device__ __forceinline__ bool two_term_overflow(float x) { return !(fabsf(x) <
 __device__ __forceinline__ float keep_or_zero(float x, bool keep) {
     return __builtin_bit_cast(float, __builtin_bit_cast(unsigned, x) & (keep ? 0xffffffffu : 0u));
 }
+__device__ __forceinline__ half_t keep_or_zero(half_t x, bool keep) {
+    return __builtin_bit_cast(half_t, (uint16_t) (__builtin_bit_cast(uint16_t, x) & (keep ? 0xffffu : 0u)));
+}
 
 // An empty statement that counts as a use and a redefinition of x (whole 32-bit registers).  Such statements keep
 // their order among themselves, and a loaded value has to have arrived before one that names it: a way to make the

@@ -1145,3 +1145,30 @@ def test_attention_fused_at_any_sequence_length(K, name, batch, heads, seq, d, k
         got = K.attention_fused_split3(dev(qkv), dev(mask), batch, heads, seq, d, 1.0 / math.sqrt(d), scale=16.0)
         plain = K.attention_fused(dev(qkv), dev(mask), batch, heads, seq, d, 1.0 / math.sqrt(d))
         assert got is not None and torch.equal(got[:, :H], (plain * 16.0).half())
+
+
+@pytest.mark.parametrize("name", ["f32", "f16"])
+@pytest.mark.parametrize("batch,heads,seq,d", [(2, 3, 20, 64), (2, 2, 31, 32), (2, 2, 50, 64), (100, 12, 77, 64), (2, 2, 200, 64),
+                                               (2, 2, 333, 64)])
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+def test_attention_fused_last_row_not_finite(K, name, batch, heads, seq, d, value):
+    """The keys that fill up the last tile are read from the last valid row and must add nothing, not even 0 * infinity:
+    with one infinity in the last row of V only that column of that sequence is infinite.  And scores beyond 1e30 (fp32) in
+    that row do not bring the fill-up keys back."""
+    rng = np.random.default_rng(seq + d)
+    H = heads * d
+    qkv = q(rng.normal(0, 1, (batch * seq, 3 * H)), name)
+    qkv[seq - 1, 2 * H + 5] = value
+    ctx = K.attention_fused(dev(qkv, tdt(name)), dev(np.ones((batch, seq), np.int8)), batch, heads, seq, d, 1.0 / math.sqrt(d))
+    assert ctx is not None
+    got = host(ctx).reshape(batch, seq, H)
+    assert (np.isinf(got[0, :, 5]) if math.isinf(value) else np.isnan(got[0, :, 5])).all()
+    got[0, :, 5] = 0
+    assert np.isfinite(got).all()
+    if name == "f32":
+        qkv[:seq, :] = 0.0
+        qkv[:seq, 0], qkv[seq - 1, H] = 1e19, 1e19      # the last key's score: 1e38 / sqrt d, every other key's 0
+        qkv[:seq, 2 * H] = 3.0
+        qkv[seq - 1, 2 * H] = 2.0
+        ctx = host(K.attention_fused(dev(qkv), None, batch, heads, seq, d, 1.0 / math.sqrt(d))).reshape(batch, seq, H)
+        assert (ctx[0, :, 0] == 2.0).all()              # all weight on that key, none on its copies
