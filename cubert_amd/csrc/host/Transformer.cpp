@@ -320,10 +320,11 @@ bool Transformer<T>::attention(size_t batch_size, const T *qkv, const int8_t *ma
 //   attention out   1024: 1280 13.2 / 12.8; 1536: 640 12.8 / 11.6, 768 15.4 / 16.9; 2048: 640 17.3 / 20.7
 //   intermediate    768 in: 1280 19.1 / 16.6; 1024 in: 896 20.7 / 19.5; 2048 in: 320 23.7 / 23.5
 //   output          3072 in: 1280 19.0 / 18.2; 4096 in: 896 20.8 / 18.5
-//   fp32 Q|K|V      768 in: 96 tokens 7.8 / 7.1, 128 9.7 / 10.8, 320 13.4 / 15.7; 1024 in: 64 9.9 / 9.2, 80 9.8 / 13.7
-//   attention out   768: 320 10.5 / 9.9; 1024: 256 12.1 / 11.5, 320 14.5 / 15.3
+//   attention out   fp32, 768: 320 10.5 / 9.9; 1024: 256 12.1 / 11.5, 320 14.5 / 15.3
 //   intermediate    768 in: 320 20.0 / 18.2; 1024 in: 160 20.8 / 19.2, 224 23.7 / 23.1, 320 29.0 / 29.7
 //   output          3072 in: 256 21.6 / 19.5, 320 22.0 / 22.9; 4096 in: 160 26.0 / 20.4
+// fp32 Q|K|V by whole requests, whose weights come from memory rather than from a cache, library against own: BERT-base 120
+// tokens 652 / 644, 160 640 / 634, 264 955 / 935, 300 945 / 950, 320 888 / 901; BERT-large 96 1441 / 1449, 128 1447 / 1459.
 // fp32, more than 1024 inputs: only as K slices for the LayerNorm.  Otherwise a few workgroups walk all of K (32 tokens,
 // 6144 -> 1536 with its LayerNorm: 41.6 us, few-token kernel 23.5) in sums longer than the few-token kernel's (2.6e-7
 // against 1.4e-7 of float64; 1536 -> 4608: 1.43e-7 against 1.33e-7).
@@ -342,8 +343,7 @@ bool own_dense_is_best(bool half_precision, int tokens, int out_features, int in
     if (in_features > 1024 && !(use == DenseUse::kNorm && as_slices)) return false;
     if (tokens <= 32 && in_features >= 640 && !narrowing && use != DenseUse::kGelu) return false;
     if (tokens > 320) return false;
-    if (use == DenseUse::kPlain) return products <= 2.1e8;
-    return products <= (use == DenseUse::kGelu ? 7.6e8 : narrowing ? 7.0e8 : 3.0e8);
+    return products <= (use == DenseUse::kPlain ? 4.7e8 : use == DenseUse::kGelu ? 7.6e8 : 7.0e8);
 }
 
 // CUBERT_FEW_TOKEN_SLICES=0 in the environment keeps the Dense kernels of small requests adding their own K slices.

@@ -333,7 +333,7 @@ def test_which_dense_layers_keep_to_short_sums():
     (1, 0, (768, 2304), 896, 1024), (1, 0, (1024, 3072), 512, 640), (1, 0, (1536, 4608), 128, 320), (1, 0, (512, 1536), 1280, 1281), (1, 0, (640, 1920), 1024, 1152),
     (1, 2, (1024, 1024), 1280, 1281), (1, 2, (1536, 1536), 640, 768), (1, 2, (2048, 2048), 320, 640),
     (1, 1, (768, 3072), 1280, 1281), (1, 1, (1024, 4096), 640, 1280), (1, 2, (3072, 768), 1280, 1281),
-    (0, 0, (768, 2304), 96, 128), (0, 0, (1024, 3072), 64, 80), (0, 2, (768, 768), 320, 321), (0, 2, (1024, 1024), 256, 320),
+    (0, 0, (768, 2304), 264, 300), (0, 0, (1024, 3072), 128, 160), (0, 2, (768, 768), 320, 321),
     (0, 1, (768, 3072), 320, 321), (0, 1, (1024, 4096), 160, 320), (0, 2, (3072, 768), 256, 320)])
 def test_where_the_library_gemm_takes_over(dtype, use, layer, last, first):
     from cubert_amd._lib import lib
