@@ -102,6 +102,8 @@ SIGNATURES = {
     "cubert_gemm_skinny_noalloc_f32": (ci, [vp, ci, ci, ci, cf, vp, ci, vp, ci, vp, ci, vp, ci]),
     "cubert_gemm_skinny_packed_elements": (ctypes.c_size_t, [ci, ci]),
     "cubert_gemm_f16_f32": (ci, [vp, ci, ci, ci, ci, ci, cf, vp, ci, vp, ci, cf, vp, ci, vp]),
+    "cubert_dense_plan": (ci, [ci, ci, ci, ci, ci, ctypes.c_size_t, ctypes.POINTER(ci), ctypes.POINTER(ci),
+                               ctypes.POINTER(ci)]),
     "cubert_split3_f32": (ci, [vp, ci, ci, cf, ci, vp, vp, vp]),
     "cubert_bias_gelu_split3_f32": (ci, [vp, vp, ci, ci, cf, vp, vp, vp]),
     "cubert_attention_fused_split3_f32": (ci, [vp, vp, vp, ci, vp, cf, vp, cf, ci, ci, ci, ci, vp, vp]),

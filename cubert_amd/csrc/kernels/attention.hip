@@ -21,7 +21,6 @@
 //     transposed in LDS once per workgroup ([head_size][seq + pad]) because an MFMA B operand needs
 //     consecutive k for a fixed column and V is stored with consecutive columns.
 
-#include <atomic>
 #include <cstdlib>
 #include <initializer_list>
 #include <string>
@@ -1511,23 +1510,6 @@ bool shapes_ok(int batch, int heads, int seq, int head_size, int ld, std::initia
     for (const void *p : ptrs) {
         if (!is_aligned(p, 16)) return false;
     }
-    return true;
-}
-
-// Kernels that ask for more than 48 KB of dynamic LDS need their limit raised once per device (the attribute
-// belongs to the function on the current device).  One bit per device ordinal, set after a successful call.
-template <typename Kernel>
-bool allow_large_lds(Kernel kernel, std::atomic<unsigned long long> &done) {
-    int device = 0;
-    if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= 64) return false;
-    const unsigned long long bit = 1ull << device;
-    if (done.load(std::memory_order_acquire) & bit) return true;
-    if (hipFuncSetAttribute((const void *) kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) !=
-        hipSuccess) {
-        (void) hipGetLastError();
-        return false;
-    }
-    done.fetch_or(bit, std::memory_order_release);
     return true;
 }
 

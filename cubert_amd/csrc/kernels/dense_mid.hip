@@ -12,8 +12,6 @@
 //     requested ahead), laid out so that the matrix-core operand reads hit all banks: the 16-byte unit u of row r
 //     sits at u ^ (r / 2 % 8) (two rows span the 64 banks), which the loads get by asking for permuted units;
 //   - K can also be cut into slices over workgroups when the consumer adds them (LayerNorm over slices).
-#include <atomic>
-
 #include "activations.h"
 #include "cubert_kernels.h"
 #include "device_common.h"
@@ -54,9 +52,10 @@ struct MidShape {
 
 enum MidOutput { kMidStore = 0, kMidGelu = 1, kMidSlices = 2 };
 
-// CHAINS (a power of two) accumulators per block take turns over a wavefront's K values and are added at the end: a single fp32 chain over
-// 192 of 768 K values has 2.5e-7 relative error against float64 (the library's GEMM 2.5e-7 to 5.0e-7), eight 1.1e-7
-// (with K slices 0.9e-7; the few-token kernel, which adds runs of 16 values, 1.1e-7), for 0.2 to 0.5 us a launch.
+// CHAINS (a power of two) accumulators per block take turns over a wavefront's K values and are added at the end: a
+// single fp32 chain over 192 of 768 K values has 2.5e-7 relative error against float64 (the library's GEMM 2.5e-7 to
+// 5.0e-7), eight 1.1e-7 (with K slices 0.9e-7; the few-token kernel, which adds runs of 16 values, 1.1e-7), for 0.2 to
+// 0.5 us a launch.
 template <typename T, int TM, int TN, int DEPTH, int OUT, int CHAINS>
 __global__ __launch_bounds__(kMidThreads) void dense_mid_kernel(const T *__restrict__ W, int ldw,
                                                                 const T *__restrict__ X, int ldx,
@@ -65,6 +64,7 @@ __global__ __launch_bounds__(kMidThreads) void dense_mid_kernel(const T *__restr
                                                                 int steps_per_slice, int token_tiles, int feature_tiles,
                                                                 float *__restrict__ partials, int pitch,
                                                                 long long slice_stride) {
+    static_assert(DEPTH == 1 || DEPTH == 2, "steps requested ahead");
     typedef MidShape<T, TM, TN, DEPTH> S;
     constexpr int FB = TN / 32, TB = TM / 32;  // 32 x 32 blocks of the tile
     constexpr int U = 16 / sizeof(T);          // elements of a 16-byte unit
@@ -153,12 +153,7 @@ __global__ __launch_bounds__(kMidThreads) void dense_mid_kernel(const T *__restr
     }
     int slot = 0;
     for (int s = 0; s < steps; ++s) {
-        const int behind = steps - 1 - s;  // steps requested after this one (at most DEPTH - 1)
-        if (DEPTH >= 4 && behind >= 3) {
-            wait_loads<3 * S::kLoads>();
-        } else if (DEPTH >= 3 && behind >= 2) {
-            wait_loads<2 * S::kLoads>();
-        } else if (DEPTH >= 2 && behind >= 1) {
+        if (DEPTH == 2 && s + 1 < steps) {  // the step after this one has been requested too
             wait_loads<S::kLoads>();
         } else {
             wait_loads<0>();
@@ -275,22 +270,6 @@ __global__ __launch_bounds__(kMidThreads) void dense_mid_kernel(const T *__restr
     }
 }
 
-// Raises the dynamic LDS limit of a kernel once per device (the attribute belongs to the function on the device).
-template <typename Kernel>
-bool raise_lds_limit(Kernel kernel, std::atomic<unsigned long long> &done) {
-    int device = 0;
-    if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= 64) return false;
-    const unsigned long long bit = 1ull << device;
-    if (done.load(std::memory_order_acquire) & bit) return true;
-    if (hipFuncSetAttribute((const void *) kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) !=
-        hipSuccess) {
-        (void) hipGetLastError();
-        return false;
-    }
-    done.fetch_or(bit, std::memory_order_release);
-    return true;
-}
-
 struct MidPlan {
     int tile = 0;  // 0: 32 x 32, 1: 64 x 32, 2: 64 x 64
     int depth = 2, slices = 1, steps_per_slice = 0;
@@ -350,7 +329,7 @@ int launch_mid(const MidPlan &plan, const T *W, int ldw, const T *X, int ldx, co
     typedef MidShape<T, TM, TN, DEPTH> S;
     static_assert(S::kLdsBytes <= 160 * 1024, "LDS of a compute unit");
     static std::atomic<unsigned long long> raised{0};  // per kernel
-    if (!raise_lds_limit(dense_mid_kernel<T, TM, TN, DEPTH, OUT, CHAINS>, raised)) return CUBERT_UNSUPPORTED;
+    if (!allow_large_lds(dense_mid_kernel<T, TM, TN, DEPTH, OUT, CHAINS>, raised)) return CUBERT_UNSUPPORTED;
     const int token_tiles = (tokens + TM - 1) / TM, feature_tiles = (features + TN - 1) / TN;
     const dim3 grid((unsigned) (feature_tiles * token_tiles * plan.slices)), block(kMidThreads);
     return launch_lds(dense_mid_kernel<T, TM, TN, DEPTH, OUT, CHAINS>, grid, block, (unsigned) S::kLdsBytes, stream, W, ldw, X, ldx,
@@ -431,6 +410,19 @@ int dense_mid_slices(int tokens, int features, int in, const T *X, int ldx, cons
                                           partials, stream);
 }
 
+// What dense_mid (as_slices = 0) or dense_mid_slices would launch.
+template <typename T>
+int dense_mid_plan(int tokens, int features, int in, bool as_slices, size_t partial_floats, int *tile, int *depth, int *slices) {
+    if (tokens <= 0 || features <= 0 || in <= 0 || !tile || !depth || !slices) return CUBERT_BAD_ARGUMENT;
+    if (in % (int) (kStepBytes / sizeof(T)) != 0) return CUBERT_UNSUPPORTED;
+    const MidPlan plan = plan_mid<T>(tokens, features, in / (int) (kStepBytes / sizeof(T)), as_slices, partial_floats);
+    if (as_slices && plan.slices < 2) return CUBERT_UNSUPPORTED;
+    *tile = plan.tile, *depth = plan.depth, *slices = plan.slices;
+    return 0;
+}
+
+template int dense_mid_plan<float>(int, int, int, bool, size_t, int *, int *, int *);
+template int dense_mid_plan<half_t>(int, int, int, bool, size_t, int *, int *, int *);
 template int dense_mid<float>(int, int, int, const float *, int, const float *, int, const float *, int, float *, int,
                               hipStream_t);
 template int dense_mid<half_t>(int, int, int, const half_t *, int, const half_t *, int, const half_t *, int, half_t *, int,

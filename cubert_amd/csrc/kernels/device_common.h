@@ -6,6 +6,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
+
 namespace cubert {
 
 constexpr int kWave = 64;        // CDNA wavefront width
@@ -162,6 +164,23 @@ inline int launch_untimed(void (*kernel)(Params...), dim3 grid, dim3 block, unsi
     hipLaunchKernelGGL(kernel, grid, block, lds_bytes, stream, static_cast<Params>(args)...);
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? 0 : (int) e;
+}
+
+// Kernels that ask for more than 48 KB of dynamic LDS need their limit raised once per device (the attribute
+// belongs to the function on the current device).  One bit per device ordinal, set after a successful call.
+template <typename Kernel>
+bool allow_large_lds(Kernel kernel, std::atomic<unsigned long long> &done) {
+    int device = 0;
+    if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= 64) return false;
+    const unsigned long long bit = 1ull << device;
+    if (done.load(std::memory_order_acquire) & bit) return true;
+    if (hipFuncSetAttribute((const void *) kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) !=
+        hipSuccess) {
+        (void) hipGetLastError();
+        return false;
+    }
+    done.fetch_or(bit, std::memory_order_release);
+    return true;
 }
 
 template <typename... Params, typename... Args>

@@ -42,6 +42,8 @@ int dense_mid(int tokens, int features, int in, const T *X, int ldx, const T *W,
 template <typename T>
 int dense_mid_slices(int tokens, int features, int in, const T *X, int ldx, const T *W, int ldw, float *partials,
                      size_t partial_floats, int *slices, hipStream_t stream);
+template <typename T>
+int dense_mid_plan(int tokens, int features, int in, bool as_slices, size_t partial_floats, int *tile, int *depth, int *slices);
 // kernels/gemm_batch.hip
 template <typename T>
 int gemm_batch(int transA, int transB, int M, int N, int K, float alpha, const T *const *A_array, int lda,
@@ -727,6 +729,14 @@ int cubert_dense_slices_f16(void *stream, int tokens, int features, int in, cons
     return cubert::dense_mid_slices<cubert::half_t>(tokens, features, in, (const cubert::half_t *) x, ldx,
                                                     (const cubert::half_t *) w, ldw, partials, partial_floats, slices,
                                                     (hipStream_t) stream);
+}
+
+int cubert_dense_plan(int half_precision, int tokens, int features, int in, int as_slices, size_t partial_floats, int *tile,
+                      int *depth, int *slices) {
+    return half_precision ? cubert::dense_mid_plan<cubert::half_t>(tokens, features, in, as_slices != 0, partial_floats, tile,
+                                                                   depth, slices)
+                          : cubert::dense_mid_plan<float>(tokens, features, in, as_slices != 0, partial_floats, tile, depth,
+                                                          slices);
 }
 
 int cubert_gemm_strided_batch_f32(void *handle, int transA, int transB, int M, int N, int K, float alpha,

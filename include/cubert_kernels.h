@@ -411,6 +411,11 @@ int cubert_dense_slices_f32(void *stream, int tokens, int features, int in, cons
                             int ldw, float *partials, size_t partial_floats, int *slices);
 int cubert_dense_slices_f16(void *stream, int tokens, int features, int in, const cubert_half *x, int ldx,
                             const cubert_half *w, int ldw, float *partials, size_t partial_floats, int *slices);
+/* How cubert_dense_* (as_slices = 0) or cubert_dense_slices_* (partial_floats as there) would cut a problem: *tile 0 = 32 x 32,
+ * 1 = 64 x 32, 2 = 64 x 64 tokens x features to a workgroup, *depth steps of K requested ahead, *slices of K.
+ * CUBERT_UNSUPPORTED where K is not whole steps or slices would not be taken.  Launches nothing; no GPU needed. */
+int cubert_dense_plan(int half_precision, int tokens, int features, int in, int as_slices, size_t partial_floats, int *tile,
+                      int *depth, int *slices);
 
 /* The same over `batch_count` problems at fixed strides (in elements).
  * replaces: blas_gemm_strided_batch<T>, reference src/cuBERT/common.h:82-92. */
