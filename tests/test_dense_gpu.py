@@ -3,6 +3,8 @@ import numpy as np
 import pytest
 from scipy.special import erf
 
+from util import DENSE_SIZES, DENSE_SLICE_SIZES
+
 pytestmark = pytest.mark.gpu
 
 torch = pytest.importorskip("torch")
@@ -38,13 +40,8 @@ def result_bound(name, want, product):
     return 1.13 * product + 2e-6 * (1 + np.abs(want)) + (2.0 ** -24 if name == "f32" else 2.0 ** -11) * np.abs(want) + 6e-8
 
 
-# one step, fewer steps than wavefronts, remainders of token and feature tiles, every tile and depth of the plan
-SIZES = [(1, 4, 64), (33, 100, 128), (31, 36, 320), (32, 2304, 768), (64, 3072, 768), (65, 768, 3072), (120, 3072, 768),
-         (200, 2304, 768), (350, 2304, 768), (350, 3072, 768), (777, 1028, 192)]
-
-
 @pytest.mark.parametrize("name", ["f32", "f16"])
-@pytest.mark.parametrize("tokens,features,width", SIZES)
+@pytest.mark.parametrize("tokens,features,width", DENSE_SIZES)
 def test_dense_against_float64(K, name, tokens, features, width):
     x, w, bias, x64, w64, bias64 = operands(name, tokens, features, width, 16)
     bound = product_bound(x64, w64)
@@ -60,9 +57,8 @@ def test_dense_against_float64(K, name, tokens, features, width):
 
 
 @pytest.mark.parametrize("name", ["f32", "f16"])
-@pytest.mark.parametrize("tokens,width", [(1, 768), (32, 3072), (65, 3072), (120, 768), (200, 3072), (350, 3072)])
-def test_dense_slices_add_up_and_reach_the_layer_norm(K, name, tokens, width):
-    H = 768
+@pytest.mark.parametrize("tokens,H,width", DENSE_SLICE_SIZES)
+def test_dense_slices_add_up_and_reach_the_layer_norm(K, name, tokens, H, width):
     x, w, bias, x64, w64, _ = operands(name, tokens, H, width, 0)
     slices = K.dense_slices(x, w)
     assert slices is not None and slices.shape[0] >= 2
@@ -71,13 +67,20 @@ def test_dense_slices_add_up_and_reach_the_layer_norm(K, name, tokens, width):
     residual, beta, gamma = (torch.from_numpy(rng.normal(0, 1, s).astype(np.float32)).to(x.dtype).cuda()
                              for s in ((tokens, H), H, H))
     got = K.bias_res_ln_slices(slices, residual, bias, beta, gamma)
+    if name == "f32" and H > 1024:
+        assert got is None  # no fp32 row of this width in registers
+        return
     added = torch.zeros_like(slices[0])
     for s in slices:  # in slice order from 0.f, then rounded: what a finished product would be
         added += s
     plain = K.bias_res_ln_(added.to(x.dtype), residual, bias, beta, gamma)
-    # the same inputs through separately compiled kernels that add a row in another order: 1e-6 in fp32; in half
-    # precision a result may fall on the other side of a rounding, one unit in the last place of values up to 16
-    assert float((got.float() - plain.float()).abs().max()) <= (2e-5 if name == "f32" else 2.0 ** -7)
+    if name == "f32":
+        assert torch.equal(got, plain)
+    else:
+        # separately compiled kernels, at 768 halves one that adds a row in another order: the last bit of a few elements
+        diff = (got.float() - plain.float()).abs()
+        assert (diff <= plain.float().abs() * 2.0 ** -9 + 1e-6).all()
+        assert (diff > 0).float().mean().item() < 0.01
 
 
 @pytest.mark.parametrize("tokens", [1, 32, 33, 64])

@@ -1,6 +1,7 @@
 """CPU-side checks: the shared library loads and exports exactly what include/*.h declares, the
 GraphDef writer produces files its reader (and the wire format) agree on, and the synthetic
 weight/input generators are deterministic.  No device call is made here."""
+import ctypes
 import os
 import re
 import subprocess
@@ -339,3 +340,33 @@ def test_where_the_library_gemm_takes_over(dtype, use, layer, last, first):
     from cubert_amd._lib import lib
     best = lib().cubert_dense_is_best
     assert best(dtype, last, layer[1], layer[0], use, 1) and not best(dtype, first, layer[1], layer[0], use, 1)
+
+
+def test_the_dense_tests_run_every_tile_a_model_does():
+    """Every (type, tile, depth, output, short sums or not) that the Dense layers of models of hidden size 64 to 2048 reach at
+    any token count is among the sizes of test_dense_gpu.py."""
+    from cubert_amd._lib import lib
+    from util import DENSE_SIZES, DENSE_SLICE_SIZES
+    L = lib()
+
+    def plan(half, tokens, features, width, sliced):
+        tile, depth, slices = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
+        rc = L.cubert_dense_plan(half, tokens, features, width, sliced, 1 << 21, tile, depth, slices)
+        assert rc in (0, -2)
+        return None if rc else (half, tile.value, depth.value, not half and tokens <= 64)
+    run = set()
+    for half in (0, 1):
+        run |= {plan(half, *size, 0) + (output,) for size in DENSE_SIZES for output in ("store", "gelu")}
+        run |= {plan(half, *size, 1) + ("slices",) for size in DENSE_SLICE_SIZES}
+    reached = set()
+    for hidden, inner in ((64, 256), (128, 512), (256, 1024), (384, 1536), (512, 2048), (768, 3072), (768, 1024),
+                          (1024, 4096), (1024, 8192), (1536, 6144), (2048, 8192)):
+        for half in (0, 1):
+            for use, features, width in ((0, 3 * hidden, hidden), (2, hidden, hidden), (1, inner, hidden), (2, hidden, inner)):
+                for tokens in range(1, 1281):
+                    if not L.cubert_dense_is_best(half, tokens, features, width, use, 1):
+                        continue
+                    sliced = plan(half, tokens, features, width, 1) if use == 2 else None
+                    reached.add(sliced + ("slices",) if sliced else
+                                plan(half, tokens, features, width, 0) + ("gelu" if use == 1 else "store",))
+    assert len(reached) > 20 and not reached - run, sorted(reached - run)

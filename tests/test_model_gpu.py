@@ -62,6 +62,8 @@ def test_missing_weight_raises_like_unordered_map_at(cb, case):
 # ------------------------------------------------------------------ seeded models vs the oracle
 
 SMALL = dict(vocab=211, hidden=128, layers=3, heads=4, intermediate=512, max_position=64, type_vocab=2)
+# an intermediate size that is no whole number of steps of the own Dense kernel: few-token kernel and library
+ODD = dict(SMALL, intermediate=528)
 
 
 def run_both(cb, weights, ids, mask, seg, layers, heads, max_batch, compute_type=0, oracle_rows=None):
@@ -112,43 +114,51 @@ def test_small_model_fp16(cb):
         assert_close(got[k], want[k], FP16_TOL, k)
 
 
+@pytest.mark.parametrize("model", [SMALL, ODD], ids=["own_dense", "odd_intermediate"])
 @pytest.mark.parametrize("compute_type", [0, 1])
 @pytest.mark.parametrize("seq_length", [32, 16])
-def test_requests_of_at_most_32_tokens(cb, compute_type, seq_length):
-    """Batch 1 (and batch 2 at seq 16) run the Dense layers on the few-token kernel, the intermediate layer with
-    its GELU in the same launch, and a half-precision model on its re-ordered weight copies; a larger batch of the
-    same model takes the library GEMM.  Both must match the oracle, and the single request must match itself as a
+def test_requests_of_at_most_32_tokens(cb, compute_type, seq_length, model):
+    """Batch 1 (and batch 2 at seq 16) of a model whose layer sizes are whole steps of the own Dense kernel run on that one;
+    with an odd intermediate size the Dense layers run on the few-token kernel, the intermediate layer with its GELU in the
+    same launch, and a half-precision model on its re-ordered weight copies.  A larger batch of the same model (1312 tokens,
+    of the odd one 192) takes the library GEMM.  Both must match the oracle, and the single request must match itself as a
     row of the larger batch."""
     from cubert_amd.testing import random_bert_weights, random_inputs
-    w = random_bert_weights(seed=11, labels=2, pooler=True, classifier=True, ln_random=True, **SMALL)
-    ids, mask, seg = random_inputs(seed=12, batch=6, seq_length=seq_length, vocab=SMALL["vocab"], min_valid=3,
+    w = random_bert_weights(seed=11, labels=2, pooler=True, classifier=True, ln_random=True, **model)
+    total = (1312 if model is SMALL else 192) // seq_length
+    ids, mask, seg = random_inputs(seed=12, batch=total, seq_length=seq_length, vocab=SMALL["vocab"], min_valid=3,
                                    segment_split=7)
     tol = FP16_TOL if compute_type else FP32_TOL
     wo = {k: oracle.round_to_half(v) for k, v in w.items()} if compute_type else w
     want = oracle.bert_forward(wo, ids, mask, seg, 3, 4)
-    bert = cb.Bert(w, 6, seq_length, 3, 4, compute_type)
+    bert = cb.Bert(w, total, seq_length, 3, 4, compute_type)
+    bert.profile(["bias_gelu"])
     full = bert.forward(ids, mask, seg)
+    assert bert.profile_read()["bias_gelu"][1] == 3  # a GELU launch of its own per layer: the library's GEMM
     for n in (1, 2):
         if n * seq_length > 32:
             continue
         few = bert.forward(ids[:n], mask[:n], seg[:n])
+        assert "bias_gelu" not in bert.profile_read()
         for k in ("sequence_output", "pooled_output", "logits", "probs"):
             assert_close(few[k], want[k][:n], tol, "%s, %d request(s)" % (k, n))
-            assert_close(few[k], full[k][:n], tol, "%s vs the same rows of a batch of 6" % k)
+            assert_close(few[k], full[k][:n], tol, "%s vs the same rows of a batch of %d" % (k, total))
     bert.close()
     for k in ("sequence_output", "pooled_output", "logits"):
         assert_close(full[k], want[k], tol, k)
 
 
+@pytest.mark.parametrize("model", [SMALL, ODD], ids=["own_dense", "odd_intermediate"])
 @pytest.mark.parametrize("compute_type", [0, 1])
 @pytest.mark.parametrize("seq_length,batches", [(32, (2,)), (64, (1,)), (16, (3, 4)), (8, (5, 8))])
-def test_requests_of_33_to_64_tokens(cb, compute_type, seq_length, batches):
-    """From 33 to 64 tokens the Dense layers in front of a LayerNorm (and, in half precision, the intermediate layer
-    with its GELU) still run on the few-token kernel, two blocks of 32 tokens per wavefront, the others on the
-    library: the request must match the oracle and itself as rows of a larger batch."""
+def test_requests_of_33_to_64_tokens(cb, compute_type, seq_length, batches, model):
+    """From 33 to 64 tokens: the own Dense kernel, or with an odd intermediate size the few-token kernel with two blocks of
+    32 tokens per wavefront for the layers in front of a LayerNorm (and, in half precision, the intermediate layer with its
+    GELU) and the library for the others.  The request must match the oracle and itself as rows of a larger batch, which
+    runs on the library's GEMMs."""
     from cubert_amd.testing import random_bert_weights, random_inputs
-    w = random_bert_weights(seed=21, labels=2, pooler=True, classifier=True, ln_random=True, **SMALL)
-    total = 160 // seq_length
+    w = random_bert_weights(seed=21, labels=2, pooler=True, classifier=True, ln_random=True, **model)
+    total = (1312 if model is SMALL else 192) // seq_length
     ids, mask, seg = random_inputs(seed=22, batch=total, seq_length=seq_length, vocab=SMALL["vocab"], min_valid=3,
                                    segment_split=5)
     tol = FP16_TOL if compute_type else FP32_TOL
@@ -162,6 +172,29 @@ def test_requests_of_33_to_64_tokens(cb, compute_type, seq_length, batches):
         for k in ("sequence_output", "pooled_output", "logits", "probs"):
             assert_close(few[k], want[k][:n], tol, "%s, %d request(s) of %d tokens" % (k, n, seq_length))
             assert_close(few[k], full[k][:n], tol, "%s vs the same rows of a batch of %d" % (k, total))
+    bert.close()
+
+
+@pytest.mark.parametrize("compute_type,batches", [(0, ((8, True), (10, True), (11, False))),
+                                                  (1, ((17, True), (28, True), (37, True), (40, True), (41, False)))])
+def test_requests_around_the_switch_to_the_library(cb, compute_type, batches):
+    """Two layers of BERT-base's width, 32 tokens a sequence, on either side of the token counts where a Dense layer goes
+    over to the library's GEMM (whose GELU is a launch of its own); between them some layers run on one and some on the
+    other.  Against the oracle, the first and the last sequences of each batch."""
+    from cubert_amd.testing import random_bert_weights, random_inputs
+    m = dict(vocab=97, hidden=768, layers=2, heads=12, intermediate=3072, max_position=64, type_vocab=2)
+    w = random_bert_weights(seed=41, labels=2, pooler=True, classifier=True, ln_random=True, **m)
+    largest = batches[-1][0]
+    ids, mask, seg = random_inputs(seed=42, batch=largest, seq_length=32, vocab=97, min_valid=3, segment_split=9)
+    wo = {k: oracle.round_to_half(v) for k, v in w.items()} if compute_type else w
+    want = oracle.bert_forward(wo, ids, mask, seg, 2, 12)
+    bert = cb.Bert(w, largest, 32, 2, 12, compute_type)
+    bert.profile(["bias_gelu"])
+    for n, own in batches:
+        got = bert.forward(ids[:n], mask[:n], seg[:n])
+        assert ("bias_gelu" not in bert.profile_read()) == own, n
+        for k in ("sequence_output", "pooled_output", "logits", "probs"):
+            assert_close(got[k], want[k][:n], FP16_TOL if compute_type else FP32_TOL, "%s, %d sequences" % (k, n))
     bert.close()
 
 
