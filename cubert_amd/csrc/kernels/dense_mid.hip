@@ -278,12 +278,15 @@ struct MidPlan {
 
 constexpr int kShortSumTokens = 64, kShortSumChains = 8, kShortSumSteps = 32;
 
-// The tile and the number of K slices, by a model of the launch time (in microseconds) whose choice is within 12 % of the
-// best one measured for all but two of 112 shapes (32 to 1000 tokens, the Dense shapes of BERT-base, every tile, depth and
-// 1 to 8 slices): 2.3 for dispatch, the first operands and the drain, then as many rounds as the fullest of the 256
-// compute units has workgroups.  A workgroup takes its operands at 80 KB per microsecond in half precision (768 x 768 in
-// 32 x 32 tiles: 98 KB, 1.4 us with its epilogue); in fp32 a tile of 32 x 32 takes 4.1 us per 768 K values, 64 x 32 8.0,
-// 64 x 64 14.5.  Workgroups that share a compute unit gain nothing over taking turns.  Slices cost their way through memory.
+// The tile and the number of K slices, by a model of the launch time (in microseconds): 2.3 for dispatch, the first
+// operands and the drain, then as many rounds as the fullest of the 256 compute units has workgroups.  A workgroup takes its
+// operands at 80 KB per microsecond in half precision (768 x 768 in 32 x 32 tiles: 98 KB, 1.4 us with its epilogue); in fp32 a
+// tile of 32 x 32 takes 4.1 us per 768 K values, 64 x 32 8.0, 64 x 64 14.5.  Workgroups that share a compute unit gain
+// nothing over taking turns.  Slices cost their way through memory, and at most eight are worth it: the LayerNorm has eight
+// of a row on their way together (32 tokens, 3072 -> 768, fp32, with the LayerNorm: 8 slices 8.6 us, 10 9.6, 16 10.6).
+// Measured with the LayerNorm or GELU over every tile, depth and 1 to 16 slices at the four Dense shapes of BERT-base and
+// BERT-large, 8 to 320 fp32 and 8 to 1280 half-precision tokens as far as models take this kernel: the choice is within
+// 9 % of the best one at 151 of 152, within 17 % at the other.
 // Depth: two steps ahead where one workgroup per compute unit is all there is (96 workgroups of 32 x 32 x 768, fp16: one
 // step ahead 4.2, two 3.8 us), one where more workgroups fit the LDS that way (672: 6.1 against 6.9 us); in fp32 two pay
 // off for every tile (1056: 24.8 against 22.6 us).
@@ -296,12 +299,13 @@ MidPlan plan_mid(int tokens, int features, int steps, bool sliced, size_t partia
     static const float kEpilogue[3] = {0.15f, 0.5f, 1.3f};             // us, half precision
     static const float kF32Step[3] = {4.1f / 24, 8.0f / 24, 14.5f / 24};  // us per step of a workgroup
     const bool short_sums = sizeof(T) == 4 && tokens <= kShortSumTokens;
+    const int most_slices = !sliced ? 1 : short_sums && steps >= 8 * kShortSumSteps ? 16 : 8;
     MidPlan best;
     float best_us = 0.f;
     for (int t = 0; t < (short_sums ? 1 : 3); ++t) {
         const long long tiles = (long long) ((tokens + kTile[t][0] - 1) / kTile[t][0]) *
                                 ((features + kTile[t][1] - 1) / kTile[t][1]);
-        for (int want = 1; want <= (sliced ? 16 : 1); ++want) {
+        for (int want = 1; want <= most_slices; ++want) {
             const int per = (steps + want - 1) / want, slices = (steps + per - 1) / per;
             if (slices != want) continue;
             if (slices > 1 && (per < kMidWaves || (size_t) slices * tokens * features > partial_floats)) break;

@@ -370,3 +370,18 @@ def test_the_dense_tests_run_every_tile_a_model_does():
                     reached.add(sliced + ("slices",) if sliced else
                                 plan(half, tokens, features, width, 0) + ("gelu" if use == 1 else "store",))
     assert len(reached) > 20 and not reached - run, sorted(reached - run)
+
+
+def test_dense_slices_stay_within_the_measured_number():
+    """At most the eight slices that the LayerNorm has on their way together, unless K is so long that the short sums of fp32
+    requests of at most 64 tokens need more."""
+    from cubert_amd._lib import lib
+    tile, depth, slices = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
+    most = 0
+    for half in (0, 1):
+        for features, width in ((768, 768), (768, 3072), (640, 2560), (512, 2048), (1024, 4096), (256, 3072)):
+            for tokens in range(1, 321):
+                if lib().cubert_dense_plan(half, tokens, features, width, 1, 1 << 21, tile, depth, slices) == 0:
+                    most = max(most, slices.value)
+    assert most == 8
+    assert lib().cubert_dense_plan(0, 64, 256, 16384, 1, 1 << 21, tile, depth, slices) == 0 and slices.value == 16
