@@ -418,7 +418,8 @@ void Transformer<T>::dense_split(int out_features, int tokens, int in_features, 
     }
 }
 
-// Up to how many tokens a Dense layer runs on the few-token kernel.  32 for all of them; 64 where the kernel with two
+// Up to how many tokens a Dense layer that the own Dense kernel does not take runs on the few-token kernel.  32 for all of
+// them; 64 where the kernel with two
 // blocks of 32 tokens per wavefront is ahead of the library.  Measured at BERT-base, batch 2 x seq 32, a launch
 // event-timed inside the forward pass, library against kernel -- fp32: attention output 9.1 / 7.6 us, output
 // 20.4 / 15.1 us, but Q|K|V 11.7 / 12.5 and intermediate + GELU 16.4 / 18.7 (the fp32 MFMAs of a second token block
@@ -458,6 +459,7 @@ void Transformer<T>::dense_norm(int tokens, int in_features, const T *kernel, co
             own_slices_to_norm = false;  // the hidden size is fixed per model: do not ask again
         }
     }
+    // (also for an fp32 layer too short to be cut by the own kernel: 128 -> 128 at 32 tokens 4.4 against 5.0 us)
     if (tokens <= few_token_limit(kind) && slices_to_norm && few_token_partials != nullptr && few_token_slices_enabled() &&
         (packed != nullptr || !transposed_kernels)) {
         int slices = 0, pitch = 0;
@@ -565,7 +567,7 @@ T *Transformer<T>::_in_compute(size_t batch_size, T *input_gpu, int8_t *attentio
                    layer_input, w.attention_norm_beta, w.attention_norm_gamma, attention_output,
                    Profiler::kDenseAttentionOutput);
 
-        // intermediate: dense, then bias + GELU (one launch for all three at <= 32 tokens)
+        // intermediate: dense, then bias + GELU (one launch for all three in a small request)
         if (!dense(I, M, H, w.intermediate_kernel, w.intermediate_packed, attention_output, intermediate_output,
                    w.intermediate_bias, false, true, Profiler::kDenseIntermediate)) {
             Timed t(profiler, Profiler::kBiasGelu, stream);

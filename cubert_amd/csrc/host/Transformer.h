@@ -3,20 +3,21 @@
 // named-weight map under a variable prefix, then compute(batch, input, mask)
 // with device pointers, returning a device pointer to [batch, seq, hidden].
 //
-// Inside, a layer is 8 launches (7 for at most 32 tokens, where the two Dense kernels in front of a LayerNorm also
-// leave their K slices to it instead of adding them up themselves; up to 64 tokens those two, and in half precision
-// the intermediate one, still run on the few-token kernel):
+// Inside, a layer is 8 launches (7 for small requests, whose intermediate Dense applies its GELU and whose two Dense
+// layers in front of a LayerNorm may leave their K slices to it; which of the own Dense kernel, the few-token kernel and
+// the library's GEMM a layer runs on: own_dense_is_best, few_token_limit):
 //   qkv   = x * [Wq|Wk|Wv] + [bq|bk|bv]          one GEMM, bias in its epilogue
 //   ctx   = softmax((1/sqrt d) Q K^T + mask) V    one attention kernel (scores stay in registers); where its
 //                                                 shape limits do not hold: scores kernel or batched GEMM into
 //                                                 scores[B, A, S, S], mask_scale_softmax_, context kernel or GEMM
 //   a     = LN(ctx * Wo + bo + x)                 GEMM, then layer_norm_   (fused kernel)
-//   i     = GELU(a * Wi + bi)                     GEMM, then gelu          (fused kernel; one launch for both at
-//                                                 <= 32 tokens)
+//   i     = GELU(a * Wi + bi)                     GEMM, then gelu          (fused kernel; one launch for both in
+//                                                 small requests)
 //   out   = LN(i * Wout + bout + a)               GEMM, then layer_norm_   (fused kernel)
 // Activation buffers are shared by all layers (the reference keeps four private
-// buffers per layer); weights live in one device allocation.  A half-precision model whose seq_length allows
-// requests of at most 32 tokens also keeps its four Dense kernels in the few-token GEMM kernel's own order.
+// buffers per layer); weights live in one device allocation.  A half-precision model of seq_length
+// <= 64 whose layer sizes are not whole steps of the own Dense kernel also keeps its four Dense kernels in the few-token
+// GEMM kernel's own order.
 //
 // CUBERT_FP32_DENSE=f16x3 in the environment when an fp32 model is opened makes its Dense layers run on the fp16
 // matrix cores for requests of at least 384 tokens (measured break-even at BERT-base: below it the GEMMs are bound

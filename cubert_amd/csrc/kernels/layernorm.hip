@@ -145,11 +145,10 @@ __device__ __forceinline__ void load_floats(const float *__restrict__ p, float (
     }
 }
 
-// bias + residual + LayerNorm of a Dense layer that the few-token GEMM left as K slices
-// (partials[slice * slice_stride + row * pitch + col], fp32): the slices are added here, in slice
-// order from 0.f, and the
-// sum is rounded to the storage type before anything else happens to it -- the value the GEMM's own last workgroup
-// would have stored -- so the result has the bits of GEMM followed by bias_res_ln.
+// bias + residual + LayerNorm of a Dense layer that was left as K slices (partials[slice * slice_stride + row * pitch +
+// col], fp32): the slices are added here, in slice order from 0.f, and the sum is rounded to the storage type before
+// anything else happens to it.  In fp32 the result has the bits of bias_res_ln on that sum; in half precision a few results
+// differ in the last bit (separately compiled kernels, at 768 halves another order of a row's sums).
 template <typename T, int VEC, int CHUNKS, bool HAS_BIAS>
 __global__ __launch_bounds__(kBlock) void bias_res_ln_partials_kernel(T *__restrict__ out,
                                                                       const float *__restrict__ partials, int slices,

@@ -373,7 +373,7 @@ bool force_naive_gemm() {
     return forced;
 }
 
-// CUBERT_GEMM=library sends every GEMM to hipBLASLt, also those the few-token kernel would take.
+// CUBERT_GEMM=library sends every GEMM to hipBLASLt, also those the few-token or the own Dense kernel would take.
 bool library_gemm_only() {
     static const bool forced = gemm_mode_is("library");
     return forced;

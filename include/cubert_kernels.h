@@ -89,7 +89,8 @@ int cubert_bias_res_ln_partials_f16(cubert_half *out, const float *partials, int
                                     const cubert_half *residual, const cubert_half *bias, const cubert_half *beta,
                                     const cubert_half *gamma, int rows, int hidden, void *stream);
 
-/* The same on slices[slice * slice_stride + r * pitch + c], any number of rows (what cubert_dense_slices_* leaves). */
+/* The same on slices[slice * slice_stride + r * pitch + c], any number of rows (what cubert_dense_slices_* leaves); the
+ * statement about bits holds for any number of rows too. */
 int cubert_bias_res_ln_slices_f32(float *out, const float *partials, int slices, int pitch, long long slice_stride,
                                   const float *residual, const float *bias, const float *beta, const float *gamma,
                                   int rows, int hidden, void *stream);
