@@ -212,7 +212,7 @@ def standalone_kernel(kind, cfg, mask, alg_bytes, reps=20):
     return {"avg_us": round(us, 2), "launches": reps, "GB/s": round(alg_bytes / (us * 1e-6) / 1e9, 1),
             "frac_hbm_peak": round(alg_bytes / (us * 1e-6) / 1e9 / HBM_PEAK_GBS, 4),
             "note": "standalone back-to-back launches: the forward pass of this workload does this work inside "
-                    "another kernel (%s)" % ("attention_fused" if kind == "mask_scale_softmax" else "the few-token Dense")}
+                    "another kernel (%s)" % ("attention_fused" if kind == "mask_scale_softmax" else "the Dense kernel")}
 
 
 def dense_flops(cfg):
@@ -287,7 +287,7 @@ def kernel_table(bert, cfg, mask, alg, batch, passes):
             table[k]["frac_hbm_peak"] = round(alg[k] / (us * 1e-6) / 1e9 / HBM_PEAK_GBS, 4)
     bert.profile([])
     # the forward pass runs the attention core as one kernel where the shape allows and then never launches the
-    # mask + scale + softmax kernel, and at <= 32 tokens bias + GELU runs inside the few-token Dense kernel: those are
+    # mask + scale + softmax kernel, and in small requests bias + GELU runs inside the Dense kernel: those are
     # timed by themselves at the workload's shape
     for kind in ("mask_scale_softmax", "bias_gelu"):
         if kind not in table:
@@ -445,7 +445,7 @@ def main():
     if dominant in prof:
         total_ms, launches = prof[dominant]
         avg_us = total_ms * 1e3 / launches
-    else:  # at <= 32 tokens bias+GELU runs inside the few-token Dense kernel: time it by itself
+    else:  # in small requests bias+GELU runs inside the Dense kernel: time it by itself
         alone = standalone_kernel(dominant, cfg, mask, alg[dominant])
         avg_us, launches = alone["avg_us"], alone["launches"]
     achieved = alg[dominant] / (avg_us * 1e-6) / 1e9
