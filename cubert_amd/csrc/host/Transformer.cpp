@@ -201,14 +201,18 @@ void Transformer<T>::layout_buffers() {
 }
 
 template <typename T>
-T *Transformer<T>::scores() {
-    if (attention_scores == nullptr) {
-        const size_t count = max_batch_size * num_attention_heads * seq_length * seq_length;
-        score_memory.take<T>(count);
-        score_memory.allocate();
-        attention_scores = score_memory.take<T>(count);
+T *Transformer<T>::scores(bool few_problems) {
+    T *&tensor = few_problems ? few_scores : attention_scores;
+    if (tensor == nullptr) {
+        Arena &memory = few_problems ? few_score_memory : score_memory;
+        const size_t all = max_batch_size * num_attention_heads;
+        const size_t problems = few_problems && all > kThreeStepProblems ? kThreeStepProblems : all;
+        const size_t count = problems * seq_length * seq_length;
+        memory.take<T>(count);
+        memory.allocate();
+        tensor = memory.take<T>(count);
     }
-    return attention_scores;
+    return tensor;
 }
 
 template <typename T>
@@ -233,7 +237,7 @@ bool Transformer<T>::three_step_attention_is_faster(size_t batch_size) const {
     if (sizeof(T) != 4 || seq_length <= 288 || seq_length >= 512) return false;
     const size_t problems = batch_size * num_attention_heads, head_size = hidden_size / num_attention_heads;
     if (head_size == 32) return problems <= 16 && seq_length > 320 && seq_length % 32 != 0;
-    return problems <= 48;
+    return problems <= kThreeStepProblems;
 }
 
 // scores[b, a, q, k] = (1/sqrt d) * sum_j Q[b, q, a, j] K[b, k, a, j];  softmax with mask;
@@ -258,7 +262,8 @@ bool Transformer<T>::attention(size_t batch_size, const T *qkv, const int8_t *ma
         const char *e = std::getenv("CUBERT_ATTENTION");
         return e != nullptr && std::string(e) == "split";
     }();
-    if (!split_only && fused_attention_fits && !three_step_attention_is_faster(batch_size)) {
+    const bool few_problems = !split_only && fused_attention_fits && three_step_attention_is_faster(batch_size);
+    if (!split_only && fused_attention_fits && !few_problems) {
         Timed t(profiler, Profiler::kAttentionFused, stream);
         if constexpr (sizeof(T) == 4) {
             if (split_context != nullptr &&
@@ -275,7 +280,7 @@ bool Transformer<T>::attention(size_t batch_size, const T *qkv, const int8_t *ma
         t.cancel();
     }
 
-    T *score_tensor = scores();
+    T *score_tensor = scores(few_problems);
     const bool loop_heads = A <= B;
     const int outer = loop_heads ? A : B, inner = loop_heads ? B : A;
     const long long in_outer = loop_heads ? head_stride : seq_stride, in_inner = loop_heads ? seq_stride : head_stride;

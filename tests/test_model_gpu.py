@@ -223,6 +223,26 @@ def test_long_fp32_sequences_by_number_of_problems(cb, seq_length, heads, hidden
     bert.close()
 
 
+def test_score_tensor_of_few_long_sequences_is_small(cb):
+    """A model for 256 sequences of 511 tokens that is asked for one: the three attention steps hold the scores of at most
+    48 (sequence, head) problems (50 MB), not of its largest batch (535 MB)."""
+    import ctypes
+    from cubert_amd._lib import lib
+    from cubert_amd.testing import random_bert_weights, random_inputs
+    m = dict(vocab=97, hidden=128, layers=1, heads=2, intermediate=512, max_position=512, type_vocab=2)
+    w = random_bert_weights(seed=31, labels=2, pooler=True, classifier=True, ln_random=True, **m)
+    ids, mask, seg = random_inputs(seed=32, batch=1, seq_length=511, vocab=97, min_valid=3, segment_split=9)
+    bert = cb.Bert(w, 256, 511, 1, 2, 0)
+    free = [ctypes.c_size_t(), ctypes.c_size_t()]
+    assert lib().cubert_mem_info(ctypes.byref(free[0]), None) == 0
+    bert.profile(["mask_scale_softmax"])
+    bert.forward(ids, mask, seg)
+    assert "mask_scale_softmax" in bert.profile_read()
+    assert lib().cubert_mem_info(ctypes.byref(free[1]), None) == 0
+    bert.close()
+    assert free[0].value - free[1].value < 200e6
+
+
 def test_repeated_calls_and_smaller_batches_reuse_buffers(cb):
     """The reference's BertMTest calls one model four times; results must not depend on what ran before."""
     from cubert_amd.testing import random_bert_weights, random_inputs
