@@ -54,6 +54,11 @@ Transformer<T>::Transformer(void *cublas, const std::string &var_prefix,
     split_dense = sizeof(T) == 4 && dense_mode != nullptr && std::string(dense_mode) == "f16x3" &&
                   max_batch_size * seq_length >= kTwoTermMinTokens;
 
+    // (also where the library's own kernel is switched off by CUBERT_GEMM the rows are the ones of the library GEMM)
+    int tile_tokens = 0, tile_features = 0;
+    pair_dense = split_dense && H % 32 == 0 && I % 32 == 0 &&
+                 cubert_dense_pairs_plan(1, (int) H, (int) H, 0, &tile_tokens, &tile_features) == 0;
+
     if (split_dense) {
         split_overflow = static_cast<int *>(cubert_malloc_host(64));
         if (split_overflow == nullptr) throw std::runtime_error("no page-locked host memory for the two-term overflow flag");
@@ -92,8 +97,12 @@ Transformer<T>::Transformer(void *cublas, const std::string &var_prefix,
                 split.unscale = std::ldexp(1.f, -exponent);
                 cuBERT::transpose(dst, (int) in, (int) out, staging, stream);
                 // (weights are scaled into [512, 1024): no overflow flag needed on this side)
-                cuBERT::split3(staging, (int) out, (int) in, std::ldexp(1.f, exponent), true, split.weights, nullptr,
-                               stream);
+                if (pair_dense) {
+                    cuBERT::split_pairs(staging, (int) out, (int) in, std::ldexp(1.f, exponent), split.weights, nullptr, stream);
+                } else {
+                    cuBERT::split3(staging, (int) out, (int) in, std::ldexp(1.f, exponent), true, split.weights, nullptr,
+                                   stream);
+                }
                 cuBERT::cuda_stream_synchronize(stream);
             }
         }
@@ -172,10 +181,11 @@ void Transformer<T>::layout_weights() {
             w.output_packed = weights.take<T>(cubert_gemm_skinny_packed_elements((int) H, (int) I));
         }
         if (split_dense) {
-            w.qkv_split.weights = weights.take<half>(3 * H * 3 * H);
-            w.attention_output_split.weights = weights.take<half>(3 * H * H);
-            w.intermediate_split.weights = weights.take<half>(3 * H * I);
-            w.output_split.weights = weights.take<half>(3 * I * H);
+            const size_t terms = pair_dense ? 2 : 3;
+            w.qkv_split.weights = weights.take<half>(terms * H * 3 * H);
+            w.attention_output_split.weights = weights.take<half>(terms * H * H);
+            w.intermediate_split.weights = weights.take<half>(terms * H * I);
+            w.output_split.weights = weights.take<half>(terms * I * H);
         }
     }
 }
@@ -196,7 +206,12 @@ void Transformer<T>::layout_buffers() {
     intermediate_output = buffers.take<T>(M * intermediate_size);
     layer_output[0] = buffers.take<T>(M * H);
     layer_output[1] = buffers.take<T>(M * H);
-    if (split_dense) split_operand = buffers.take<half>(M * 3 * (H > intermediate_size ? H : intermediate_size));
+    if (split_dense && pair_dense) {
+        split_operand = buffers.take<half>(M * 2 * H);
+        split_intermediate = buffers.take<half>(M * 2 * intermediate_size);
+    } else if (split_dense) {
+        split_operand = buffers.take<half>(M * 3 * (H > intermediate_size ? H : intermediate_size));
+    }
     if (seq_length <= 64 || own_dense) few_token_partials = buffers.take<float>(kFewTokenPartialFloats);
 }
 
@@ -267,8 +282,10 @@ bool Transformer<T>::attention(size_t batch_size, const T *qkv, const int8_t *ma
         Timed t(profiler, Profiler::kAttentionFused, stream);
         if constexpr (sizeof(T) == 4) {
             if (split_context != nullptr &&
-                cuBERT::attention_fused_split3(Q, K, V, ld, mask, kTwoTermActivationScale, split_context, alpha, B, A, S,
-                                               d, split_overflow, stream)) {
+                (pair_dense ? cuBERT::attention_fused_split_pairs(Q, K, V, ld, mask, kTwoTermActivationScale, split_context,
+                                                                  alpha, B, A, S, d, split_overflow, stream)
+                            : cuBERT::attention_fused_split3(Q, K, V, ld, mask, kTwoTermActivationScale, split_context, alpha,
+                                                             B, A, S, d, split_overflow, stream))) {
                 return true;
             }
         }
@@ -410,14 +427,39 @@ void Transformer<T>::dense_split(int out_features, int tokens, int in_features, 
         void *stream = cuBERT::blas_get_stream(cublas);
         if (in != nullptr) {
             Timed t(profiler, Profiler::kDenseSplit, stream);
-            cuBERT::split3(in, tokens, in_features, kTwoTermActivationScale, false, split_operand, split_overflow,
-                           stream);
+            if (pair_dense) {
+                cuBERT::split_pairs(in, tokens, in_features, kTwoTermActivationScale, split_operand, split_overflow, stream);
+            } else {
+                cuBERT::split3(in, tokens, in_features, kTwoTermActivationScale, false, split_operand, split_overflow,
+                               stream);
+            }
         }
         Timed t(profiler, profiler != nullptr ? profiler->dense_kind(kind) : Profiler::kDenseGemm, stream);
+        if (pair_dense) {
+            const bool gelu = kind == Profiler::kDenseIntermediate;
+            cuBERT::dense_pairs(tokens, out_features, in_features, kind == Profiler::kDenseOutput ? split_intermediate : split_operand,
+                                kernel.weights, bias, gelu, kernel.unscale / kTwoTermActivationScale, kTwoTermActivationScale,
+                                gelu ? reinterpret_cast<float *>(split_intermediate) : out, ld_out, split_overflow, stream);
+            return;
+        }
         cuBERT::blas_gemm_f16_f32(cublas, true, false, out_features, tokens, 3 * in_features,
                                   kernel.unscale / kTwoTermActivationScale,
                                   kernel.weights, 3 * in_features, split_operand, 3 * in_features, 0.f, out,
                                   ld_out, bias);
+    } else {
+        throw std::logic_error("the two-term fp16 Dense form is for fp32 models");
+    }
+}
+
+template <typename T>
+bool Transformer<T>::norm_split(const T *residual, T *inout, int tokens, const T *bias, const T *beta, const T *gamma) {
+    if constexpr (sizeof(T) == 4) {
+        void *stream = cuBERT::blas_get_stream(cublas);
+        const int H = (int) hidden_size;
+        return pair_dense ? cuBERT::layer_norm_split_pairs(residual, inout, tokens, H, bias, beta, gamma, kTwoTermActivationScale,
+                                                           split_operand, split_overflow, stream)
+                          : cuBERT::layer_norm_split3(residual, inout, tokens, H, bias, beta, gamma, kTwoTermActivationScale,
+                                                      split_operand, split_overflow, stream);
     } else {
         throw std::logic_error("the two-term fp16 Dense form is for fp32 models");
     }
@@ -525,10 +567,8 @@ T *Transformer<T>::_in_compute(size_t batch_size, T *input_gpu, int8_t *attentio
                 {
                     Timed t(profiler, Profiler::kBiasResLayerNorm, stream);
                     operand_ready = norm_writes_operand &&
-                                    cuBERT::layer_norm_split3(layer_input, attention_output, M, H, w.attention_output_bias,
-                                                              w.attention_norm_beta, w.attention_norm_gamma,
-                                                              kTwoTermActivationScale, split_operand, split_overflow,
-                                                              stream);
+                                    norm_split(layer_input, attention_output, M, w.attention_output_bias,
+                                               w.attention_norm_beta, w.attention_norm_gamma);
                     if (!operand_ready) {
                         norm_writes_operand = false;  // the hidden size is fixed per model: do not ask again
                         cuBERT::layer_norm_(layer_input, attention_output, M, H, w.attention_output_bias,
@@ -536,8 +576,8 @@ T *Transformer<T>::_in_compute(size_t batch_size, T *input_gpu, int8_t *attentio
                     }
                 }
                 dense_split(I, M, H, w.intermediate_split, operand_ready ? nullptr : attention_output,
-                            intermediate_output, nullptr, Profiler::kDenseIntermediate);
-                {
+                            intermediate_output, pair_dense ? w.intermediate_bias : nullptr, Profiler::kDenseIntermediate);
+                if (!pair_dense) {
                     // bias + GELU straight into the two-term rows the output Dense reads
                     Timed t(profiler, Profiler::kBiasGelu, stream);
                     cuBERT::bias_gelu_split3(intermediate_output, w.intermediate_bias, M, I, kTwoTermActivationScale,
@@ -547,10 +587,8 @@ T *Transformer<T>::_in_compute(size_t batch_size, T *input_gpu, int8_t *attentio
                 {
                     Timed t(profiler, Profiler::kBiasResLayerNorm, stream);
                     operand_ready = norm_writes_operand &&
-                                    cuBERT::layer_norm_split3(attention_output, out, M, H, w.output_bias,
-                                                              w.output_norm_beta, w.output_norm_gamma,
-                                                              kTwoTermActivationScale, split_operand, split_overflow,
-                                                              stream);
+                                    norm_split(attention_output, out, M, w.output_bias, w.output_norm_beta,
+                                               w.output_norm_gamma);
                     if (!operand_ready) {
                         norm_writes_operand = false;
                         cuBERT::layer_norm_(attention_output, out, M, H, w.output_bias, w.output_norm_beta,

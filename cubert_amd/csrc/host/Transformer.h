@@ -80,7 +80,8 @@ public:
     void use_fp32_dense_once() { fp32_dense_once = true; }
 
 private:
-    // A Dense kernel for the two-term fp16 form: rows [hi | lo | hi] of scale * W^T, [out, 3 * in]; unscale = 1 / scale
+    // A Dense kernel for the two-term fp16 form: rows of pairs of scale * W^T, [out, 2 * in], or, for the library's GEMM, rows
+    // [hi | lo | hi], [out, 3 * in]; unscale = 1 / scale
     static constexpr size_t kTwoTermMinTokens = 384;
     // activations are multiplied by this before they are taken apart (undone by the GEMM's alpha): rows whose
     // entries are of order 2^-7 .. 2^12 keep full accuracy (fp16 subnormals below, clamping above)
@@ -122,9 +123,12 @@ private:
     bool dense(int out_features, int tokens, int in_features, const T *kernel, const T *packed, const T *in, T *out,
                const T *bias, bool bias_in_gemm, bool gelu, Profiler::Kind kind, int ld_out = 0);
     // The same on the fp16 matrix cores from two-term operands (fp32 models only): `in` is split into
-    // split_operand first, or, when null, split_operand already holds the [hi | hi | lo] rows.  `bias` may be null.
+    // split_operand first, or, when null, split_operand already holds its two-term rows.  `bias` may be null.  With pair_dense
+    // the intermediate layer applies GELU and leaves two-term rows in split_intermediate, where the output layer finds them.
     void dense_split(int out_features, int tokens, int in_features, const SplitKernel &kernel, const T *in, T *out,
                      const T *bias, Profiler::Kind kind, int ld_out = 0);
+    // inout = LayerNorm(inout + bias + residual), and its two-term rows in split_operand; false: the hidden size is declined
+    bool norm_split(const T *residual, T *inout, int tokens, const T *bias, const T *beta, const T *gamma);
     // out = LayerNorm(in * kernel + bias + residual): dense(), then layer_norm_; for a small request the Dense kernel
     // leaves its K slices in few_token_partials and the LayerNorm kernel adds them while it loads (no hand-over between
     // the GEMM's workgroups).
@@ -146,6 +150,7 @@ private:
     bool keep_packed = false;          // Dense kernels are also kept in the few-token kernel's order
     bool transposed_kernels = false;   // Dense kernels are stored [out, in] instead of [in, out] (half precision)
     bool split_dense = false;          // fp32 model with Dense layers in the two-term fp16 form (opt-in)
+    bool pair_dense = false;           // ... on the library's own kernel, whose operand rows hold every term once
     bool fp32_dense_once = false;      // the next request takes the fp32 GEMMs (set after a two-term overflow)
     int *split_overflow = nullptr;     // page-locked host word the two-term kernels set to 1 on overflow (split_dense)
     bool norm_writes_operand = true;   // cleared when the LayerNorm that also writes two-term rows declines the hidden size
@@ -168,7 +173,8 @@ private:
     T *attention_output;     // [M, hidden]
     T *intermediate_output;  // [M, intermediate]
     T *layer_output[2];      // [M, hidden], alternating between layers
-    half *split_operand = nullptr;  // [M, 3 * max(hidden, intermediate)] two-term rows of the current Dense input
+    half *split_operand = nullptr;  // [M, 3 * max(hidden, intermediate)] two-term rows of the current Dense input; with pair_dense
+    half *split_intermediate = nullptr;  // [M, 2 * hidden], and those of the output layer's input, [M, 2 * intermediate], here
     static constexpr size_t kFewTokenPartialFloats = (size_t) 1 << 21;
     float *few_token_partials = nullptr;  // K slices of the current Dense layer of a small request
 };

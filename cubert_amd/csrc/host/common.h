@@ -228,6 +228,32 @@ inline bool attention_fused_split3(const float *q, const float *k, const float *
     CUBERT_CHECK(rc);
     return true;
 }
+// the same operands in rows of pairs (the library's own Dense kernel, kernels/dense_pairs.hip)
+inline void split_pairs(const float *in, int rows, int width, float scale, half *out, int *overflow, void *stream) {
+    CUBERT_CHECK(cubert_split_pairs_f32(in, rows, width, scale, h(out), overflow, stream));
+}
+inline bool layer_norm_split_pairs(const float *in, float *inout, int rows, int channels, const float *bias,
+                                   const float *beta, const float *gamma, float scale, half *split_out, int *overflow,
+                                   void *stream) {
+    const int rc = cubert_bias_res_ln_split_pairs_f32(inout, in, bias, beta, gamma, rows, channels, scale, h(split_out),
+                                                      overflow, stream);
+    if (rc == CUBERT_UNSUPPORTED) return false;
+    CUBERT_CHECK(rc);
+    return true;
+}
+inline bool attention_fused_split_pairs(const float *q, const float *k, const float *v, int ld, const int8_t *mask,
+                                        float scale, half *split_ctx, float alpha, int batch, int heads, int seq,
+                                        int head_size, int *overflow, void *stream) {
+    const int rc = cubert_attention_fused_split_pairs_f32(q, k, v, ld, mask, scale, h(split_ctx), alpha, batch, heads, seq,
+                                                          head_size, overflow, stream);
+    if (rc == CUBERT_UNSUPPORTED) return false;
+    CUBERT_CHECK(rc);
+    return true;
+}
+inline void dense_pairs(int tokens, int features, int in, const half *x, const half *w, const float *bias, bool gelu, float alpha,
+                        float scale, float *out, int ldo, int *overflow, void *stream) {
+    CUBERT_CHECK(cubert_dense_pairs_f32(stream, tokens, features, in, h(x), h(w), bias, gelu, alpha, scale, out, ldo, overflow));
+}
 inline void bias_gelu_split3(const float *in, const float *bias, int rows, int width, float scale, half *out,
                              int *overflow, void *stream) {
     CUBERT_CHECK(cubert_bias_gelu_split3_f32(in, bias, rows, width, scale, h(out), overflow, stream));

@@ -65,10 +65,11 @@ struct SplitOut {
     int width = 0;            // halves per part of a row [hi | hi | lo]
     float scale = 1.f;        // applied before the value is taken apart
     int *overflow = nullptr;  // set to 1 when a scaled value is outside the fp16 range (or not a number); may be null
+    bool pairs = false;       // high and low terms in turn, 32 of each, instead of [hi | hi | lo]
 };
 
 // One element of the attention context.  split.width = 0: ctx[row, col] in the storage type.  split.width = W > 0
-// (fp32 only): `ctx` is really a buffer of halves with rows [hi | hi | lo] of W each, the two-term form of
+// (fp32 only): `ctx` is really a buffer of halves with rows [hi | hi | lo] of W each (or of W pairs), the two-term form of
 // split.scale * v that the Dense GEMM on the fp16 matrix cores reads (hi = fp16(.), lo = fp16(. - hi), clamped to
 // the fp16 range; a value that had to be clamped raises split.overflow, and the caller recomputes in fp32).
 // (SPLIT is a compile-time choice so that the plain kernels are exactly what they were without it.)
@@ -79,13 +80,20 @@ __device__ __forceinline__ void store_context(T *ctx, int ld_ctx, size_t row, in
         // fuses a product that made v into the subtraction below, and lo would belong to the unrounded value)
         asm volatile("" : "+v"(v));
         v *= split.scale;
-        half_t *p = reinterpret_cast<half_t *>(ctx) + row * 3 * split.width + col;
         half_t hi, lo;
         split_two_terms(v, hi, lo);
         if (two_term_overflow(v) && split.overflow != nullptr) *split.overflow = 1;
-        p[0] = hi;
-        p[split.width] = hi;
-        p[2 * split.width] = lo;
+        half_t *p = reinterpret_cast<half_t *>(ctx);
+        if (split.pairs) {  // (uniform)
+            p += row * 2 * split.width + pair_at(col);
+            p[0] = hi;
+            p[kPairBlock] = lo;
+        } else {
+            p += row * 3 * split.width + col;
+            p[0] = hi;
+            p[split.width] = hi;
+            p[2 * split.width] = lo;
+        }
     } else {
         ctx[row * ld_ctx + col] = from_f32<T>(v);
     }
@@ -1796,6 +1804,16 @@ extern "C" int cubert_attention_fused_split3_f32(const float *q, const float *k,
     const int hidden = heads * head_size;
     return cubert::attention_fused<float>(q, k, v, ld, mask, reinterpret_cast<float *>(split_ctx), hidden, alpha, batch,
                                           heads, seq_length, head_size, stream, cubert::SplitOut{hidden, scale, overflow});
+}
+
+extern "C" int cubert_attention_fused_split_pairs_f32(const float *q, const float *k, const float *v, int ld,
+                                                      const int8_t *mask, float scale, cubert_half *split_ctx, float alpha,
+                                                      int batch, int heads, int seq_length, int head_size, int *overflow,
+                                                      void *stream) {
+    const int hidden = heads * head_size;
+    if ((split_ctx != nullptr && !cubert::is_aligned(split_ctx, 2)) || hidden % cubert::kPairBlock != 0) return CUBERT_BAD_ARGUMENT;
+    return cubert::attention_fused<float>(q, k, v, ld, mask, reinterpret_cast<float *>(split_ctx), hidden, alpha, batch,
+                                          heads, seq_length, head_size, stream, cubert::SplitOut{hidden, scale, overflow, true});
 }
 
 extern "C" int cubert_attention_fused_f16(const cubert_half *q, const cubert_half *k, const cubert_half *v, int ld,

@@ -1,0 +1,355 @@
+// Dense layers of hundreds to thousands of tokens whose fp32 operands come as pairs of fp16 numbers:
+//   C[token, feature] = alpha * sum_k x[token, k] w[feature, k] (+ bias) (, GELU),   x = xh + xl, w = wh + wl  (see split.hip)
+// A row of X or W holds, for every 32 values of K, their 32 high terms and then their 32 low terms: 128 bytes, a whole line.
+// The library's form of the same sum is one fp16 GEMM over [hi | hi | lo] rows, which reads the high terms twice and multiplies
+// each operand it reads once; here an operand that has come to LDS takes part in three products of one step, high x low, low x
+// high and high x high, so the 40 bytes per cycle that a compute unit gets from its L2 (measured: 128-byte row pieces; 64-byte
+// pieces 23) feed the matrix cores, which such a GEMM otherwise waits for.
+//
+// What bounds it: the matrix cores, which throttle the clock to 1.7 to 2.1 GHz while they are busy; a step of the 256 x 192 tile
+// is 2304 cycles of products and takes some 2900.  What it took to get there, each measured at 4096 tokens, 768 -> 2304:
+//   - two rings in LDS, X two steps deep and W three: the next step's X is asked for when its slot has been read, W earlier;
+//   - requests go out between the products of a phase: asked for in one go after the barrier, a wavefront stands at its
+//     requests while its matrix core idles;
+//   - LDS reads of the next phase also go out between the products, one by one (in one go in front of them: 54.5 us, 47.5);
+//   - one barrier per step, in front of its last phase, whose operands are in registers by then.
+// 32 x 32 blocks of C per wavefront; a finished part of C passes through LDS of its wavefront and leaves in whole row segments.
+#include "activations.h"
+#include "cubert_kernels.h"
+#include "device_common.h"
+
+namespace cubert {
+namespace {
+
+typedef float v16f32 __attribute__((ext_vector_type(16)));
+typedef _Float16 v8f16 __attribute__((ext_vector_type(8)));
+
+constexpr int kRowBytes = 128;              // of a row of X or W that a step takes
+constexpr int kPairStep = kRowBytes / 4;    // values of K in them
+constexpr int kPhases = 2, kTerms = 2;      // of a step, 16 values of K each; high and low
+
+// 16 bytes per lane from memory to LDS at `base` + 16 * lane, without passing through registers
+__device__ __forceinline__ void load_to_lds(const void *src, void *base) {
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *) src,
+                                     (__attribute__((address_space(3))) void *) base, 16, 0, 0);
+}
+
+template <int N>
+__device__ __forceinline__ void wait_loads() {  // at most N vector-memory requests of this wavefront outstanding
+    __builtin_amdgcn_s_waitcnt(0x0f70 | (N & 15) | ((N >> 4) << 14));
+}
+
+// the LDS accesses of this wavefront in front of it are done before those behind it start
+__device__ __forceinline__ void order_lds() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+
+// What leaves the kernel: alpha * product + bias as fp32, or GELU of that, times scale, as operand rows of the next layer.
+enum PairOutput { kPairFloat = 0, kPairGelu = 1 };
+
+// TM tokens x TN features by WM x WN wavefronts, rings of XS steps of X and WS steps of W
+template <int TM, int TN, int WM, int WN, int XS, int WS>
+struct PairShape {
+    static constexpr int kWaves = WM * WN, kThreads = kWaves * kWave;
+    static constexpr int kTB = TM / WM / 32, kFB = TN / WN / 32;  // 32 x 32 blocks of a wavefront
+    static constexpr int kXBytes = TM * kRowBytes, kWBytes = TN * kRowBytes;
+    static constexpr int kXLoads = TM / 8 / kWaves, kWLoads = TN / 8 / kWaves;  // requests of a wavefront per step
+    static constexpr int kOutRow = kFB * 32 * 4;  // bytes of a token in a wavefront's part of C
+    static constexpr int kOutPitch = kOutRow + 16, kOutBytes = 32 * kOutPitch;
+    static constexpr int kRings = XS * kXBytes + WS * kWBytes, kOut = kWaves * kOutBytes + TN * 4;
+    static constexpr int kLdsBytes = kRings > kOut ? kRings : kOut;
+    static_assert(kXLoads * kWaves * 8 == TM && kWLoads * kWaves * 8 == TN, "whole requests");
+    static_assert(XS >= 2 && WS >= XS, "weights are further ahead, or as far");
+    static_assert(TN <= kThreads && kLdsBytes <= 160 * 1024, "a thread per bias, LDS of a compute unit");
+};
+
+template <int TM, int TN, int WM, int WN, int XS, int WS, int OUT>
+__global__ __launch_bounds__(WM * WN * kWave) void dense_pairs_kernel(
+        const half_t *__restrict__ W, const half_t *__restrict__ X, const float *__restrict__ bias, float *__restrict__ C,
+        int ldc, int tokens, int features, int steps, int token_tiles, int feature_tiles, float alpha, float scale,
+        int *__restrict__ overflow) {
+    typedef PairShape<TM, TN, WM, WN, XS, WS> S;
+    constexpr int TB = S::kTB, FB = S::kFB;
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int lane = threadIdx.x & (kWave - 1), wave = wave_in_block();
+    const int r = lane & 31, hh = lane >> 5;
+    const int wm = wave / WN, wn = wave % WN;
+
+    // Workgroups are handed to the eight dies in turn; each die gets a contiguous run of tiles, which go down groups of eight
+    // token tiles and then across features: the 32 tiles that a die works on at a time are about 8 x 4 of them.
+    const int die = blockIdx.x & 7, die_share = gridDim.x >> 3, extra = gridDim.x & 7;
+    const int index = die * die_share + (die < extra ? die : extra) + (int) (blockIdx.x >> 3);
+    const int per_group = 8 * feature_tiles;
+    const int first = index / per_group * 8, in_group = index % per_group;
+    const int height = token_tiles - first < 8 ? token_tiles - first : 8;
+    const int ft = in_group / height, tt = first + in_group - ft * height;
+    const int m0 = tt * TM, n0 = ft * TN;
+
+    // the bias of a feature per thread, on its way before the first operands; read where it is used, behind the products
+    const int my_feature = n0 + (int) threadIdx.x;
+    const float b = bias != nullptr && threadIdx.x < TN && my_feature < features ? bias[my_feature] : 0.f;
+
+    // lane l of a request brings the 16-byte unit l % 8 of row l / 8 of eight rows to unit (l % 8) ^ (row / 2 % 8), which
+    // spreads the operand reads over all banks; rows past the end are read from the last one
+    const unsigned row_bytes = (unsigned) steps * kRowBytes;
+    const char *xbase = reinterpret_cast<const char *>(X) + (size_t) m0 * row_bytes;
+    const char *wbase = reinterpret_cast<const char *>(W) + (size_t) n0 * row_bytes;
+    unsigned xo[S::kXLoads], wo[S::kWLoads];
+    auto offset_of = [&](int i, int rows_left) {
+        const int row = (wave + i * S::kWaves) * 8 + (lane >> 3);
+        return (unsigned) (row < rows_left ? row : rows_left - 1) * row_bytes + ((lane & 7) ^ ((row >> 1) & 7)) * 16;
+    };
+#pragma unroll
+    for (int i = 0; i < S::kXLoads; ++i) xo[i] = offset_of(i, tokens - m0);
+#pragma unroll
+    for (int i = 0; i < S::kWLoads; ++i) wo[i] = offset_of(i, features - n0);
+
+    // request number i of a step's: X of a step, then W of one
+    constexpr int kRequests = S::kXLoads + S::kWLoads;
+    auto request = [&](int i, int xslot, bool with_x, int wslot, bool with_w) {
+        if (i < S::kXLoads) {
+            if (with_x) load_to_lds(xbase + xo[i], smem + xslot * S::kXBytes + (wave + i * S::kWaves) * 1024);
+            if (with_x && i == S::kXLoads - 1) xbase += kRowBytes;
+        } else {
+            const int j = i - S::kXLoads;
+            if (with_w) {
+                load_to_lds(wbase + wo[j], smem + XS * S::kXBytes + wslot * S::kWBytes + (wave + j * S::kWaves) * 1024);
+            }
+            if (with_w && i == kRequests - 1) wbase += kRowBytes;
+        }
+    };
+
+    v16f32 acc[TB][FB];
+#pragma unroll
+    for (int t = 0; t < TB; ++t)
+#pragma unroll
+        for (int f = 0; f < FB; ++f) acc[t][f] = v16f32{};
+
+    // operand number j of a phase: the blocks of W, then those of X, low terms first
+    constexpr int kReads = kTerms * (TB + FB);
+    const int xoff = (wm * TB * 32 + r) * kRowBytes, woff = XS * S::kXBytes + (wn * FB * 32 + r) * kRowBytes;
+    v8f16 x[kPhases][kTerms][TB], w[kPhases][kTerms][FB];
+    auto read = [&](int j, int xslot, int wslot, int phase) {
+        const int term = kTerms - 1 - j / (TB + FB), k = j % (TB + FB);
+        const int unit = ((term * 4 + phase * 2 + hh) ^ ((r >> 1) & 7)) * 16;
+        const unsigned char *at = k < FB ? smem + wslot * S::kWBytes + woff + k * 32 * kRowBytes
+                                         : smem + xslot * S::kXBytes + xoff + (k - FB) * 32 * kRowBytes;
+        (k < FB ? w[phase][term][k < FB ? k : 0] : x[phase][term][k < FB ? 0 : k - FB]) =
+                *reinterpret_cast<const v8f16 *>(at + unit);
+    };
+
+    int xslot = 0, wslot = 0, xfree = 0, wfree = 0;  // slots of the next operands, and those that were read last
+    bool more_x = false, more_w = false;
+    // The products of a phase; in between go the reads of the next phase, in the first three quarters, and this phase's share
+    // of the requests into the free slots, which starts with the last phase of a step.
+    auto multiply = [&](int phase) {
+        constexpr int kProducts = 3 * TB * FB;
+        const int next = (phase + 1) % kPhases;
+        const int from = next * kRequests / kPhases, until = (next + 1) * kRequests / kPhases;
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+        for (int m = 0; m < kProducts; ++m) {
+            const int kind = m / (TB * FB), t = m / FB % TB, f = m % FB;  // low x high, high x low, high x high
+            acc[t][f] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w[phase][kind == 0 ? 1 : 0][f], x[phase][kind == 1 ? 1 : 0][t],
+                                                               acc[t][f], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int j = 0; j < kReads; ++j) {
+                if (j * kProducts * 3 / (4 * kReads) == m) read(j, xslot, wslot, next);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < kRequests; ++i) {
+                if (i >= from && i < until && (i - from) * kProducts / (until - from) == m) {
+                    request(i, xfree, more_x, wfree, more_w);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+        }
+        __builtin_amdgcn_s_setprio(0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+
+#pragma unroll
+    for (int d = 0; d < WS; ++d)
+#pragma unroll
+        for (int i = 0; i < kRequests; ++i) request(i, d, d < XS && d < steps, d, d < steps);
+    if (steps >= WS) {
+        wait_loads<(WS - 1) * S::kWLoads + (XS - 1) * S::kXLoads>();
+    } else {
+        wait_loads<0>();
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < kReads; ++j) read(j, 0, 0, 0);
+    for (int s = 0; s < steps; ++s) {
+        multiply(0);
+        xfree = xslot, wfree = wslot;
+        xslot = xslot + 1 < XS ? xslot + 1 : 0, wslot = wslot + 1 < WS ? wslot + 1 : 0;
+        more_x = s + XS < steps, more_w = s + WS < steps;
+        if (s + 1 < steps) {
+            // The next step has landed.  Younger than it: X of XS - 2 steps, and W of as many, or of one more where the ring
+            // of W is the deeper one (W of step j + WS follows X of step j + XS).  In the last steps nothing is.
+            constexpr int kYounger = (XS - 2) * S::kXLoads + (XS == WS ? XS - 2 : XS - 1) * S::kWLoads;
+            if (s + WS <= steps) {
+                wait_loads<kYounger>();
+            } else {
+                wait_loads<0>();
+            }
+            __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wavefront has read this step
+            __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_s_barrier();
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        multiply(1);  // (behind the last step it reads a slot that holds nothing of use, for a phase that does not follow)
+    }
+
+    __syncthreads();
+    float *bias_lds = reinterpret_cast<float *>(smem + S::kWaves * S::kOutBytes);
+    if (threadIdx.x < TN) bias_lds[threadIdx.x] = b;
+    __syncthreads();
+    // 32 tokens at a time: a lane owns a token and, per four accumulator registers, four consecutive features
+    unsigned char *out = smem + wave * S::kOutBytes;
+    const int col0 = n0 + wn * FB * 32;
+    bool over = false;
+#pragma unroll
+    for (int t = 0; t < TB; ++t) {
+        unsigned char *at = out + r * S::kOutPitch;
+#pragma unroll
+        for (int f = 0; f < FB; ++f)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const int col = g * 8 + hh * 4;
+                const Vec<float, 4> bv = load_vec<float, 4>(bias_lds + (wn * FB + f) * 32 + col);
+                Vec<float, 4> y;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) y.v[e] = fmaf(acc[t][f][g * 4 + e], alpha, bv.v[e]);
+                if constexpr (OUT == kPairGelu) {
+                    Vec<half_t, 4> hi, lo;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float v = GeluOp<float>()(y.v[e]) * scale;
+                        split_two_terms(v, hi.v[e], lo.v[e]);
+                        const int token = m0 + (wm * TB + t) * 32 + r;
+                        over = over || (two_term_overflow(v) && token < tokens && col0 + f * 32 < features);
+                    }
+                    store_vec<half_t, 4>(reinterpret_cast<half_t *>(at) + f * 64 + col, hi);
+                    store_vec<half_t, 4>(reinterpret_cast<half_t *>(at) + f * 64 + 32 + col, lo);
+                } else {
+                    store_vec<float, 4>(reinterpret_cast<float *>(at) + f * 32 + col, y);
+                }
+            }
+        order_lds();
+        constexpr int kPieces = S::kOutRow / 16;
+        const int token0 = m0 + (wm * TB + t) * 32;
+        float *rows = C + (size_t) token0 * ldc + col0;
+#pragma unroll
+        for (int i = 0; i < 32 * kPieces / kWave; ++i) {
+            const int item = i * kWave + lane, row = item / kPieces, piece = item - row * kPieces;
+            const Vec<float, 4> v = load_vec<float, 4>(reinterpret_cast<const float *>(out + row * S::kOutPitch + piece * 16));
+            if (token0 + row < tokens && col0 + piece * 4 < features) store_vec<float, 4>(rows + (size_t) row * ldc + piece * 4, v);
+        }
+        order_lds();
+    }
+    if (OUT == kPairGelu && over && overflow != nullptr) *overflow = 1;
+}
+
+template <int TM, int TN, int WM, int WN, int XS, int WS, int OUT>
+int launch_pairs(const half_t *W, const half_t *X, const float *bias, float *C, int ldc, int tokens, int features, int steps,
+                 float alpha, float scale, int *overflow, hipStream_t stream) {
+    typedef PairShape<TM, TN, WM, WN, XS, WS> S;
+    static std::atomic<unsigned long long> raised{0};  // per kernel
+    auto kernel = dense_pairs_kernel<TM, TN, WM, WN, XS, WS, OUT>;
+    if (!allow_large_lds(kernel, raised)) return CUBERT_UNSUPPORTED;
+    const int token_tiles = (tokens + TM - 1) / TM, feature_tiles = (features + TN - 1) / TN;
+    return launch_lds(kernel, dim3((unsigned) (token_tiles * feature_tiles)), dim3(S::kThreads), (unsigned) S::kLdsBytes,
+                      stream, W, X, bias, C, ldc, tokens, features, steps, token_tiles, feature_tiles, alpha, scale, overflow);
+}
+
+// The tile, by a model of the launch time in microseconds, fitted to 768 and 3072 inputs, 384 to 16384 tokens and 768 to 3072
+// features.  With u tiles per compute unit a launch takes what a tile takes by itself, slowed down by the others', or what the
+// tiles of a compute unit take one after the other; for the two larger tiles rounds are whole.  Measured at 768 -> 2304 /
+// 768 -> 768 / 768 -> 3072 with GELU / 3072 -> 768, the tile that is taken first:
+//    384 tokens  64 x 64    10 / 9.4 / 14 / 28         128 x 96   16 / 15 / 18 / 56     256 x 192  35 / 33 / 42 / 117
+//   1280         128 x 96   19 / 16 / 28 / 57          128 x 128  19 / 16 / 24 / 57     64 x 64    21 / 10 / 27 / 30
+//   4096         256 x 192  45 / 36 / 60 / 120         128 x 96   46 / 19 / 64 / 63     64 x 64    57 / 21 / 80 / 74
+//  16384         256 x 192  155 / 54 / 238 / 188       128 x 128  163 / 57 / 237 / 210  64 x 64    225 / 74 / 328 / 281
+struct PairTile {
+    int tm, tn;
+    float alone, alone_step, crowd, each, each_step, start;
+    int round;  // tiles per compute unit that run as one round (0: no rounds)
+};
+
+constexpr PairTile kPairTiles[4] = {
+        {256, 192, 7.5f, 1.14f, 0.55f, 11.2f, 1.71f, 0.f, 1},
+        {128, 128, 2.3f, 0.556f, 0.25f, 0.8f, 0.72f, 7.f, 0},
+        {128, 96, 1.6f, 0.57f, 0.12f, 0.6f, 0.55f, 5.f, 2},
+        {64, 64, 3.1f, 0.258f, 0.12f, 0.37f, 0.239f, 4.f, 0},
+};
+
+int plan_pairs(int tokens, int features, int steps, bool gelu) {
+    int best = 0;
+    float best_us = 0.f;
+    for (int i = 0; i < 4; ++i) {
+        const PairTile &t = kPairTiles[i];
+        const long long tiles = (long long) ((tokens + t.tm - 1) / t.tm) * ((features + t.tn - 1) / t.tn);
+        const float u = (float) tiles / 256.f;
+        const float alone = t.alone + t.alone_step * steps, each = t.each + t.each_step * steps;
+        float us = 0.f, left = u;
+        if (t.round > 0) {
+            const float rounds = (float) (tiles / (256 * t.round));
+            left = u - rounds * t.round;
+            us = rounds * t.round * each + (rounds > 0.f ? t.start : 0.f);
+        }
+        if (left > 0.f) {
+            const float crowded = alone * (1.f + t.crowd * (t.round == 1 ? left * left : left));
+            const float in_turn = t.start + each * left;
+            us += left > 1.f && in_turn > crowded ? in_turn : crowded;
+        }
+        if (gelu) us += 2.f + u * (t.tm * t.tn) * 0.12e-3f;
+        if (i == 0 || us < best_us) best = i, best_us = us;
+    }
+    return best;
+}
+
+template <int OUT>
+int launch_tile(int tile, const half_t *W, const half_t *X, const float *bias, float *C, int ldc, int tokens, int features,
+                int steps, float alpha, float scale, int *overflow, hipStream_t s) {
+    switch (tile) {
+        case 0: return launch_pairs<256, 192, 4, 2, 2, 3, OUT>(W, X, bias, C, ldc, tokens, features, steps, alpha, scale, overflow, s);
+        case 1: return launch_pairs<128, 128, 4, 2, 2, 3, OUT>(W, X, bias, C, ldc, tokens, features, steps, alpha, scale, overflow, s);
+        case 2: return launch_pairs<128, 96, 4, 1, 2, 3, OUT>(W, X, bias, C, ldc, tokens, features, steps, alpha, scale, overflow, s);
+        default: return launch_pairs<64, 64, 2, 2, 4, 4, OUT>(W, X, bias, C, ldc, tokens, features, steps, alpha, scale, overflow, s);
+    }
+}
+
+}  // namespace
+
+int dense_pairs(int tokens, int features, int in, const half_t *x, const half_t *w, const float *bias, int activation,
+                float alpha, float scale, float *out, int ldo, int *overflow, hipStream_t stream) {
+    if (!x || !w || !out || tokens < 0 || features < 0 || in < 0 || ldo < features || (activation != 0 && activation != 1)) {
+        return CUBERT_BAD_ARGUMENT;
+    }
+    // (an offset inside a tile's rows has 32 bits)
+    if (in == 0 || in % kPairStep != 0 || in > (1 << 20) || features % (activation == 1 ? kPairBlock : 4) != 0 || ldo % 4 != 0 ||
+        (activation == 1 && ldo != features) || !is_aligned(x, 16) || !is_aligned(w, 16) || !is_aligned(out, 16) ||
+        ((long long) tokens / 64 + 1) * (features / 64 + 1) > 0x7fffffffLL) {
+        return CUBERT_UNSUPPORTED;
+    }
+    if (tokens == 0 || features == 0) return 0;
+    const int steps = in / kPairStep, tile = plan_pairs(tokens, features, steps, activation == 1);
+    return activation == 1
+                   ? launch_tile<kPairGelu>(tile, w, x, bias, out, ldo, tokens, features, steps, alpha, scale, overflow, stream)
+                   : launch_tile<kPairFloat>(tile, w, x, bias, out, ldo, tokens, features, steps, alpha, scale, overflow, stream);
+}
+
+int dense_pairs_plan(int tokens, int features, int in, int activation, int *tile_tokens, int *tile_features) {
+    if (tokens <= 0 || features <= 0 || in <= 0 || !tile_tokens || !tile_features) return CUBERT_BAD_ARGUMENT;
+    if (in % kPairStep != 0) return CUBERT_UNSUPPORTED;
+    const PairTile &t = kPairTiles[plan_pairs(tokens, features, in / kPairStep, activation == 1)];
+    *tile_tokens = t.tm, *tile_features = t.tn;
+    return 0;
+}
+
+}  // namespace cubert

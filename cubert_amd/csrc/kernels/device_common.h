@@ -53,6 +53,11 @@ __device__ __forceinline__ void split_two_terms(float x, half_t &hi, half_t &lo)
 // consumes them must be told (the kernels that write two-term rows raise a flag the caller looks at).
 __device__ __forceinline__ bool two_term_overflow(float x) { return !(fabsf(x) <= 65504.f); }
 
+// Where the two terms of a row's element stand in the operand rows of the own Dense kernel: 32 high terms, then the 32 low ones,
+// for every 32 elements (the low term kPairBlock behind the high one).
+constexpr int kPairBlock = 32;
+__host__ __device__ __forceinline__ int pair_at(int col) { return col / kPairBlock * (2 * kPairBlock) + col % kPairBlock; }
+
 // x when keep, +0.f otherwise, as a bit operation: a select between a loaded value and zero invites the compiler to
 // put the load itself under a branch, where it is waited for on the spot.
 __device__ __forceinline__ float keep_or_zero(float x, bool keep) {

@@ -44,13 +44,14 @@ __device__ __forceinline__ int uniform_i8(const int8_t *__restrict__ p, int inde
 
 // Normalise the row held in x[][] and store it.  gamma/beta were loaded before
 // the reduction so their latency overlaps it.
-// With `split_row` the stored values, times split_scale, also go out as two-term fp16 rows [hi | hi | lo] (hi = fp16(y),
-// lo = fp16(y - hi), clamped to the fp16 range), the token operand of a Dense GEMM on the fp16 matrix cores (see split.hip).
+// With `split_row` the stored values, times split_scale, also go out as two-term fp16 rows (hi = fp16(y), lo = fp16(y - hi),
+// clamped to the fp16 range), [hi | hi | lo] or, with `pairs`, high and low terms in turn: the token operand of a Dense layer on
+// the fp16 matrix cores (see split.hip).
 template <typename T, int VEC, int CHUNKS>
 __device__ __forceinline__ void ln_finish(float (&x)[CHUNKS][VEC], float sum, float sumsq, const Vec<T, VEC> (&g)[CHUNKS],
                                           const Vec<T, VEC> (&b)[CHUNKS], T *__restrict__ out_row, int lane,
                                           half_t *__restrict__ split_row = nullptr, float split_scale = 1.f,
-                                          int *__restrict__ overflow = nullptr) {
+                                          int *__restrict__ overflow = nullptr, bool pairs = false) {
     constexpr int H = kWave * VEC * CHUNKS;
     float mean, rstd;
     ln_stats(sum, sumsq, H, mean, rstd);
@@ -72,10 +73,15 @@ __device__ __forceinline__ void ln_finish(float (&x)[CHUNKS][VEC], float sum, fl
                 over = over || two_term_overflow(y);
             }
             if (over && overflow != nullptr) *overflow = 1;  // the caller recomputes in fp32
-            half_t *at = split_row + (c * kWave + lane) * VEC;
-            store_vec<half_t, VEC>(at, hi);
-            store_vec<half_t, VEC>(at + H, hi);
-            store_vec<half_t, VEC>(at + 2 * H, lo);
+            const int col = (c * kWave + lane) * VEC;
+            if (pairs) {  // (uniform)
+                store_vec<half_t, VEC>(split_row + pair_at(col), hi);
+                store_vec<half_t, VEC>(split_row + pair_at(col) + kPairBlock, lo);
+            } else {
+                store_vec<half_t, VEC>(split_row + col, hi);
+                store_vec<half_t, VEC>(split_row + H + col, hi);
+                store_vec<half_t, VEC>(split_row + 2 * H + col, lo);
+            }
         }
     }
 }
@@ -85,7 +91,7 @@ __global__ __launch_bounds__(kBlock) void bias_res_ln_kernel(T *__restrict__ ino
                                                              const T *__restrict__ bias, const T *__restrict__ beta,
                                                              const T *__restrict__ gamma, int rows,
                                                              half_t *__restrict__ split_out, float split_scale,
-                                                             int *__restrict__ overflow) {
+                                                             int *__restrict__ overflow, bool pairs) {
     constexpr int H = kWave * VEC * CHUNKS;
     const int row = blockIdx.x * kRowsPerBlock + wave_in_block();
     if (row >= rows) return;
@@ -123,8 +129,8 @@ __global__ __launch_bounds__(kBlock) void bias_res_ln_kernel(T *__restrict__ ino
             sumsq += v * v;
         }
     }
-    ln_finish<T, VEC, CHUNKS>(x, sum, sumsq, g, be, io, lane, SPLIT ? split_out + (size_t) row * 3 * H : nullptr,
-                              split_scale, overflow);
+    ln_finish<T, VEC, CHUNKS>(x, sum, sumsq, g, be, io, lane,
+                              SPLIT ? split_out + (size_t) row * (pairs ? 2 : 3) * H : nullptr, split_scale, overflow, pairs);
 }
 
 // N consecutive floats (N = 2, 4 or 8) with 16-byte loads where N allows.
@@ -466,9 +472,9 @@ int bias_res_ln(T *inout, const T *residual, const T *bias, const T *beta, const
     if (hidden == kWave * VEC * CHUNKS && vector_ok<T>(hidden, VEC, {inout, residual, bias, beta, gamma})) { \
         if (bias != nullptr)                                                                             \
             return launch(bias_res_ln_kernel<T, VEC, CHUNKS, true>, grid, block, s, inout, residual, bias, beta, gamma, \
-                          rows, nullptr, 1.f, nullptr);                                                  \
+                          rows, nullptr, 1.f, nullptr, false);                                                  \
         return launch(bias_res_ln_kernel<T, VEC, CHUNKS, false>, grid, block, s, inout, residual, bias, beta, gamma, \
-                      rows, nullptr, 1.f, nullptr);                                                      \
+                      rows, nullptr, 1.f, nullptr, false);                                                      \
     }
     CUBERT_LN_CASE(V, 1)
     CUBERT_LN_CASE(V, 2)
@@ -532,7 +538,7 @@ int bias_res_ln_partials(T *out, const float *partials, int slices, int pitch, c
 // bias + residual + LayerNorm of fp32 rows, in place, and the result again as two-term fp16 rows in split_out
 // [rows, 3 * hidden]; only the register-resident shapes (hidden = 256 k), anything else is declined.
 int bias_res_ln_split3(float *inout, const float *residual, const float *bias, const float *beta, const float *gamma,
-                       int rows, int hidden, float scale, half_t *split_out, int *overflow, void *stream) {
+                       int rows, int hidden, float scale, half_t *split_out, int *overflow, bool pairs, void *stream) {
     if (rows < 0 || hidden <= 0 || !inout || !residual || !beta || !gamma || !split_out) return CUBERT_BAD_ARGUMENT;
     if (rows == 0) return 0;
     hipStream_t s = (hipStream_t) stream;
@@ -542,9 +548,9 @@ int bias_res_ln_split3(float *inout, const float *residual, const float *bias, c
     if (hidden == kWave * 4 * CHUNKS && vector_ok<float>(hidden, 4, {inout, residual, bias, beta, gamma})) {         \
         if (bias != nullptr)                                                                                          \
             return launch(bias_res_ln_kernel<float, 4, CHUNKS, true, true>, grid, block, s, inout, residual, bias, beta, \
-                          gamma, rows, split_out, scale, overflow);                                                   \
+                          gamma, rows, split_out, scale, overflow, pairs);                                            \
         return launch(bias_res_ln_kernel<float, 4, CHUNKS, false, true>, grid, block, s, inout, residual, bias, beta,  \
-                      gamma, rows, split_out, scale, overflow);                                                       \
+                      gamma, rows, split_out, scale, overflow, pairs);                                                \
     }
     CUBERT_LN_SPLIT_CASE(1)
     CUBERT_LN_SPLIT_CASE(2)
@@ -610,7 +616,14 @@ extern "C" int cubert_bias_res_ln_split3_f32(float *inout, const float *residual
                                              const float *gamma, int rows, int hidden, float scale,
                                              cubert_half *split_out, int *overflow, void *stream) {
     return cubert::bias_res_ln_split3(inout, residual, bias, beta, gamma, rows, hidden, scale,
-                                      (cubert::half_t *) split_out, overflow, stream);
+                                      (cubert::half_t *) split_out, overflow, false, stream);
+}
+
+extern "C" int cubert_bias_res_ln_split_pairs_f32(float *inout, const float *residual, const float *bias, const float *beta,
+                                                  const float *gamma, int rows, int hidden, float scale,
+                                                  cubert_half *split_out, int *overflow, void *stream) {
+    return cubert::bias_res_ln_split3(inout, residual, bias, beta, gamma, rows, hidden, scale,
+                                      (cubert::half_t *) split_out, overflow, true, stream);
 }
 
 extern "C" int cubert_bias_res_ln_f16(cubert_half *inout, const cubert_half *residual, const cubert_half *bias,

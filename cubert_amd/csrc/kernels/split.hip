@@ -14,6 +14,7 @@
 // apart (`scale`, exact, taken out again by the GEMM's alpha): weights per matrix, so that the largest is in
 // [512, 1024) and their size does not matter; activations by a fixed factor chosen by the caller (the host classes
 // use 16: full accuracy for rows whose entries are of order 2^-7 to 2^12), clamped to the fp16 range beyond it.
+// Rows for the library's own kernel (dense_pairs.hip) hold every term once, [hi | lo] for every 32 elements.
 // A value that had to be clamped (or is not a number) no longer equals its two terms: every kernel that writes
 // two-term rows takes an `overflow` pointer (may be null) and stores 1 there when that happens -- an ordinary store by
 // the lanes concerned, nothing otherwise -- so that the caller can recompute in fp32 instead of using a wrong product.
@@ -29,14 +30,17 @@ struct IdentityOp {
     __device__ __forceinline__ float operator()(float x) const { return x; }
 };
 
-// out[row] = [hi | hi | lo] (LO_IN_MIDDLE: [hi | lo | hi]) of scale * f(in[row] + bias), each part `width` halves.
+// the order of a row's terms: [hi | hi | lo], [hi | lo | hi], or high and low terms in turn, 32 of each
+enum TermOrder { kLoLast = 0, kLoInMiddle = 1, kPairs = 2 };
+
+// out[row] = the terms of scale * f(in[row] + bias) in the given order.
 // One workgroup per row, threads walk the columns 8 at a time: two 16-byte loads, three 16-byte stores.
-template <typename Op, bool LO_IN_MIDDLE>
+template <typename Op, int ORDER>
 __global__ __launch_bounds__(kBlock) void split3_kernel(const float *__restrict__ in, const float *__restrict__ bias,
                                                          int width, float scale, half_t *__restrict__ out,
                                                          int *__restrict__ overflow) {
     const float *row = in + (size_t) blockIdx.x * width;
-    half_t *dst = out + (size_t) blockIdx.x * 3 * width;
+    half_t *dst = out + (size_t) blockIdx.x * (ORDER == kPairs ? 2 : 3) * width;
     Op op;
     bool over = false;
     for (int col = threadIdx.x * 8; col < width; col += blockDim.x * 8) {
@@ -54,20 +58,25 @@ __global__ __launch_bounds__(kBlock) void split3_kernel(const float *__restrict_
             split_two_terms(y1, hi.v[4 + i], lo.v[4 + i]);
             over = over || two_term_overflow(y0) || two_term_overflow(y1);
         }
-        store_vec<half_t, 8>(dst + col, hi);
-        store_vec<half_t, 8>(dst + width + col, LO_IN_MIDDLE ? lo : hi);
-        store_vec<half_t, 8>(dst + 2 * width + col, LO_IN_MIDDLE ? hi : lo);
+        if constexpr (ORDER == kPairs) {
+            store_vec<half_t, 8>(dst + pair_at(col), hi);
+            store_vec<half_t, 8>(dst + pair_at(col) + kPairBlock, lo);
+        } else {
+            store_vec<half_t, 8>(dst + col, hi);
+            store_vec<half_t, 8>(dst + width + col, ORDER == kLoInMiddle ? lo : hi);
+            store_vec<half_t, 8>(dst + 2 * width + col, ORDER == kLoInMiddle ? hi : lo);
+        }
     }
     if (over && overflow != nullptr) *overflow = 1;
 }
 
 // any width and alignment
-template <typename Op, bool LO_IN_MIDDLE>
+template <typename Op, int ORDER>
 __global__ __launch_bounds__(kBlock) void split3_scalar_kernel(const float *__restrict__ in,
                                                                 const float *__restrict__ bias, int width, float scale,
                                                                 half_t *__restrict__ out, int *__restrict__ overflow) {
     const float *row = in + (size_t) blockIdx.x * width;
-    half_t *dst = out + (size_t) blockIdx.x * 3 * width;
+    half_t *dst = out + (size_t) blockIdx.x * (ORDER == kPairs ? 2 : 3) * width;
     Op op;
     bool over = false;
     for (int col = threadIdx.x; col < width; col += blockDim.x) {
@@ -75,14 +84,19 @@ __global__ __launch_bounds__(kBlock) void split3_scalar_kernel(const float *__re
         const float y = op(row[col] + (bias != nullptr ? bias[col] : 0.f)) * scale;
         split_two_terms(y, hi, lo);
         over = over || two_term_overflow(y);
-        dst[col] = hi;
-        dst[width + col] = LO_IN_MIDDLE ? lo : hi;
-        dst[2 * width + col] = LO_IN_MIDDLE ? hi : lo;
+        if constexpr (ORDER == kPairs) {
+            dst[pair_at(col)] = hi;
+            dst[pair_at(col) + kPairBlock] = lo;
+        } else {
+            dst[col] = hi;
+            dst[width + col] = ORDER == kLoInMiddle ? lo : hi;
+            dst[2 * width + col] = ORDER == kLoInMiddle ? hi : lo;
+        }
     }
     if (over && overflow != nullptr) *overflow = 1;
 }
 
-template <typename Op, bool LO_IN_MIDDLE>
+template <typename Op, int ORDER>
 int split3(const float *in, const float *bias, int rows, int width, float scale, half_t *out, int *overflow,
            void *stream) {
     if (rows < 0 || width <= 0 || !in || !out) return CUBERT_BAD_ARGUMENT;
@@ -91,10 +105,10 @@ int split3(const float *in, const float *bias, int rows, int width, float scale,
     if (width % 8 == 0 && is_aligned(in, 16) && is_aligned(out, 16) && (bias == nullptr || is_aligned(bias, 16))) {
         const int vectors = width / 8;
         const int threads = vectors >= kBlock ? kBlock : ((vectors + kWave - 1) / kWave) * kWave;
-        return launch(split3_kernel<Op, LO_IN_MIDDLE>, dim3(rows), dim3(threads), s, in, bias, width, scale, out,
+        return launch(split3_kernel<Op, ORDER>, dim3(rows), dim3(threads), s, in, bias, width, scale, out,
                       overflow);
     }
-    return launch(split3_scalar_kernel<Op, LO_IN_MIDDLE>, dim3(rows), dim3(kBlock), s, in, bias, width, scale, out,
+    return launch(split3_scalar_kernel<Op, ORDER>, dim3(rows), dim3(kBlock), s, in, bias, width, scale, out,
                   overflow);
 }
 
@@ -104,12 +118,19 @@ int split3(const float *in, const float *bias, int rows, int width, float scale,
 extern "C" int cubert_split3_f32(const float *in, int rows, int width, float scale, int lo_in_middle, cubert_half *out,
                                  int *overflow, void *stream) {
     using namespace cubert;
-    return lo_in_middle ? split3<IdentityOp, true>(in, nullptr, rows, width, scale, (half_t *) out, overflow, stream)
-                        : split3<IdentityOp, false>(in, nullptr, rows, width, scale, (half_t *) out, overflow, stream);
+    return lo_in_middle ? split3<IdentityOp, kLoInMiddle>(in, nullptr, rows, width, scale, (half_t *) out, overflow, stream)
+                        : split3<IdentityOp, kLoLast>(in, nullptr, rows, width, scale, (half_t *) out, overflow, stream);
+}
+
+extern "C" int cubert_split_pairs_f32(const float *in, int rows, int width, float scale, cubert_half *out, int *overflow,
+                                      void *stream) {
+    using namespace cubert;
+    if (width % kPairBlock != 0) return CUBERT_BAD_ARGUMENT;
+    return split3<IdentityOp, kPairs>(in, nullptr, rows, width, scale, (half_t *) out, overflow, stream);
 }
 
 extern "C" int cubert_bias_gelu_split3_f32(const float *in, const float *bias, int rows, int width, float scale,
                                            cubert_half *out, int *overflow, void *stream) {
     using namespace cubert;
-    return split3<GeluOp<float>, false>(in, bias, rows, width, scale, (half_t *) out, overflow, stream);
+    return split3<GeluOp<float>, kLoLast>(in, bias, rows, width, scale, (half_t *) out, overflow, stream);
 }

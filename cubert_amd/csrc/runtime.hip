@@ -44,6 +44,10 @@ int dense_mid_slices(int tokens, int features, int in, const T *X, int ldx, cons
                      size_t partial_floats, int *slices, hipStream_t stream);
 template <typename T>
 int dense_mid_plan(int tokens, int features, int in, bool as_slices, size_t partial_floats, int *tile, int *depth, int *slices);
+// kernels/dense_pairs.hip
+int dense_pairs(int tokens, int features, int in, const half_t *x, const half_t *w, const float *bias, int activation,
+                float alpha, float scale, float *out, int ldo, int *overflow, hipStream_t stream);
+int dense_pairs_plan(int tokens, int features, int in, int activation, int *tile_tokens, int *tile_features);
 // kernels/gemm_batch.hip
 template <typename T>
 int gemm_batch(int transA, int transB, int M, int N, int K, float alpha, const T *const *A_array, int lda,
@@ -737,6 +741,18 @@ int cubert_dense_plan(int half_precision, int tokens, int features, int in, int 
                                                                    depth, slices)
                           : cubert::dense_mid_plan<float>(tokens, features, in, as_slices != 0, partial_floats, tile, depth,
                                                           slices);
+}
+
+int cubert_dense_pairs_f32(void *stream, int tokens, int features, int in, const cubert_half *x, const cubert_half *w,
+                           const float *bias, int activation, float alpha, float scale, float *out, int ldo, int *overflow) {
+    if (library_gemm_only() || force_naive_gemm()) return CUBERT_UNSUPPORTED;
+    return cubert::dense_pairs(tokens, features, in, (const cubert::half_t *) x, (const cubert::half_t *) w, bias, activation,
+                               alpha, scale, out, ldo, overflow, (hipStream_t) stream);
+}
+
+int cubert_dense_pairs_plan(int tokens, int features, int in, int activation, int *tile_tokens, int *tile_features) {
+    if (library_gemm_only() || force_naive_gemm()) return CUBERT_UNSUPPORTED;
+    return cubert::dense_pairs_plan(tokens, features, in, activation, tile_tokens, tile_features);
 }
 
 int cubert_gemm_strided_batch_f32(void *handle, int transA, int transB, int M, int N, int K, float alpha,

@@ -156,6 +156,20 @@ def attention_fused_split3(qkv, mask, batch, heads, seq, head_size, alpha, scale
     return ctx
 
 
+def attention_fused_split_pairs(qkv, mask, batch, heads, seq, head_size, alpha, scale=1.0, overflow=None):
+    """attention_fused_split3 with rows as split_pairs writes them, [B*S, 2*H]."""
+    hidden = heads * head_size
+    flat = qkv.view(-1)
+    ctx = torch.empty((batch * seq, 2 * hidden), dtype=torch.float16, device=qkv.device)
+    rc = lib().cubert_attention_fused_split_pairs_f32(_ptr(flat), _ptr(flat[hidden:]), _ptr(flat[2 * hidden:]), 3 * hidden,
+                                                      _ptr(mask), float(scale), _ptr(ctx), float(alpha), batch, heads, seq,
+                                                      head_size, _ptr(overflow), _stream())
+    if rc == -2:
+        return None
+    _check(rc, "cubert_attention_fused_split_pairs_f32")
+    return ctx
+
+
 def attention_context(probs, qkv, batch, heads, seq, head_size):
     """ctx[B*S, H] = P V with V the third column block of the packed projection."""
     hidden = heads * head_size
@@ -204,6 +218,37 @@ def classifier_head_(pooled, pooler_bias, weights, out_bias):
     return logits, probs
 
 
+def split_pairs(x, scale=1.0, overflow=None):
+    """fp32 rows [rows, width] as fp16 rows [rows, 2 * width]: for every 32 elements their high and then their low terms."""
+    rows, width = x.shape
+    out = torch.empty((rows, 2 * width), dtype=torch.float16, device=x.device)
+    _check(lib().cubert_split_pairs_f32(_ptr(x), rows, width, float(scale), _ptr(out), _ptr(overflow), _stream()),
+           "cubert_split_pairs_f32")
+    return out
+
+
+def dense_pairs(x, w, bias=None, gelu=False, alpha=1.0, scale=1.0, ldo=None, overflow=None):
+    """alpha * x w^T + bias of operands from split_pairs, as fp32 [tokens, features]; with gelu, scale * GELU of that as rows like
+    the operands'; None when declined."""
+    (tokens, width), features = x.shape, w.shape[0]
+    ldo = features if ldo is None else ldo
+    out = torch.empty((tokens, ldo), dtype=torch.float32, device=x.device)
+    rc = lib().cubert_dense_pairs_f32(_stream(), tokens, features, width // 2, _ptr(x), _ptr(w), _ptr(bias), int(gelu),
+                                      float(alpha), float(scale), _ptr(out), ldo, _ptr(overflow))
+    if rc == -2:
+        return None
+    _check(rc, "cubert_dense_pairs_f32")
+    return out.view(torch.float16) if gelu else out[:, :features]
+
+
+def dense_pairs_plan(tokens, features, width, gelu=False):
+    """(tokens, features) of the tile that dense_pairs takes for a shape."""
+    tm, tn = ctypes.c_int(), ctypes.c_int()
+    _check(lib().cubert_dense_pairs_plan(tokens, features, width, int(gelu), ctypes.byref(tm), ctypes.byref(tn)),
+           "cubert_dense_pairs_plan")
+    return tm.value, tn.value
+
+
 def split3(x, scale=1.0, lo_in_middle=False, overflow=None):
     """fp32 rows [rows, width] as fp16 rows [rows, 3 * width]: hi | hi | lo (lo_in_middle: hi | lo | hi)."""
     rows, width = x.shape
@@ -233,6 +278,18 @@ def bias_res_ln_split3_(inout, residual, bias, beta, gamma, scale=1.0, overflow=
     if rc == -2:
         return None
     _check(rc, "cubert_bias_res_ln_split3_f32")
+    return out
+
+
+def bias_res_ln_split_pairs_(inout, residual, bias, beta, gamma, scale=1.0, overflow=None):
+    """bias_res_ln_split3_ with rows as split_pairs writes them."""
+    rows, hidden = inout.shape
+    out = torch.empty((rows, 2 * hidden), dtype=torch.float16, device=inout.device)
+    rc = lib().cubert_bias_res_ln_split_pairs_f32(_ptr(inout), _ptr(residual), _ptr(bias), _ptr(beta), _ptr(gamma), rows,
+                                                  hidden, float(scale), _ptr(out), _ptr(overflow), _stream())
+    if rc == -2:
+        return None
+    _check(rc, "cubert_bias_res_ln_split_pairs_f32")
     return out
 
 

@@ -319,6 +319,28 @@ int cubert_bias_res_ln_split3_f32(float *inout, const float *residual, const flo
                                   const float *gamma, int rows, int hidden, float scale, cubert_half *split_out,
                                   int *overflow, void *stream);
 
+/* The same operands and layers with every term stored once: a row of `width` values (a multiple of 32) is, for every 32 of
+ * them, their 32 high terms and then their 32 low terms, on the token and on the weight side.  The three kernels above that
+ * write rows, in this order, with the same values and return codes; */
+int cubert_split_pairs_f32(const float *in, int rows, int width, float scale, cubert_half *out, int *overflow, void *stream);
+int cubert_attention_fused_split_pairs_f32(const float *q, const float *k, const float *v, int ld, const int8_t *mask,
+                                           float scale, cubert_half *split_ctx, float alpha, int batch, int heads,
+                                           int seq_length, int head_size, int *overflow, void *stream);
+int cubert_bias_res_ln_split_pairs_f32(float *inout, const float *residual, const float *bias, const float *beta,
+                                       const float *gamma, int rows, int hidden, float scale, cubert_half *split_out,
+                                       int *overflow, void *stream);
+/* and the Dense layer over them, out[token, feature] = alpha * sum_k x[token, k] w[feature, k] + bias[feature] (bias may be NULL)
+ * as high * low + low * high + high * high products on the fp16 matrix cores in fp32 sums.  activation 0: `out` holds floats,
+ * rows `ldo` apart.  activation 1: out = GELU of that, times `scale`, as such rows again (features a multiple of 32, ldo =
+ * features floats: as many bytes), with `overflow` as above.  x is [tokens, in] and w [features, in] in that form, in a multiple
+ * of 32, features of 4, operands 16-byte aligned; other shapes (and CUBERT_GEMM=library or naive
+ * in the environment) return CUBERT_UNSUPPORTED and launch nothing.
+ * replaces: Dense<float>::compute, reference src/cuBERT/op/Dense.cpp:47-57, and gelu<float>, op/GELU.h:6-7, in their opt-in form. */
+int cubert_dense_pairs_f32(void *stream, int tokens, int features, int in, const cubert_half *x, const cubert_half *w,
+                           const float *bias, int activation, float alpha, float scale, float *out, int ldo, int *overflow);
+/* the tile of tokens x features that cubert_dense_pairs_f32 takes for a shape */
+int cubert_dense_pairs_plan(int tokens, int features, int in, int activation, int *tile_tokens, int *tile_features);
+
 /* C = alpha * A * B + bias for N <= 64 columns (no transposes, beta = 0): the Dense layer of a request with at
  * most 64 tokens, where A is the [in, out] weight matrix (M = out, K = in) and each column of B one token.
  * One pass over the weights on the matrix cores with every load in flight at once (from 33 tokens on a wavefront

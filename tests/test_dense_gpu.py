@@ -119,3 +119,101 @@ def test_dense_declines_what_it_cannot_do(K, name):
     assert K.dense(*operands_of(128, 64, pad=1)) is None    # rows of unaligned pitch
     assert K.dense_slices(*operands_of(128, 64)) is None    # too short to cut
     assert K.dense_slices(*operands_of(1024, 64), partial_floats=8 * 64) is None  # no room for two slices
+
+
+# ---- fp32 operands as pairs of fp16 numbers (kernels/dense_pairs.hip) ------------------------------------------
+
+def dev(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+def _pairs(x, scale):
+    """The operand rows by numpy: for every 32 values their high terms and then their low terms."""
+    y = x.astype(np.float32) * np.float32(scale)
+    hi = np.clip(y, -65504, 65504).astype(np.float16)
+    lo = np.clip(y - hi.astype(np.float32), -65504, 65504).astype(np.float16)
+    rows, width = x.shape
+    return np.stack([hi.reshape(rows, -1, 32), lo.reshape(rows, -1, 32)], axis=2).reshape(rows, 2 * width)
+
+
+@pytest.mark.parametrize("rows,width", [(5, 768), (3, 32), (2, 96)])
+def test_rows_of_pairs_bit_exact(K, rows, width):
+    rng = np.random.default_rng(rows + width)
+    x = rng.normal(0, 1, (rows, width)).astype(np.float32)
+    x.flat[::5] *= 1e-4
+    x.flat[0] = 70000.0
+    got = K.split_pairs(dev(x), 4.0).cpu().numpy()
+    assert np.array_equal(got.view(np.uint16), _pairs(x, 4.0).view(np.uint16))
+    # element path: an input that is not 16-byte aligned
+    base = torch.zeros(rows * width + 1, device="cuda")
+    base[1:] = dev(x).flatten()
+    assert np.array_equal(K.split_pairs(base[1:].view(rows, width), 4.0).cpu().numpy().view(np.uint16), got.view(np.uint16))
+    if width % 256 == 0:
+        res = dev(rng.normal(0, 1, (rows, width)).astype(np.float32))
+        beta, gamma = dev(np.zeros(width, np.float32)), dev(np.ones(width, np.float32))
+        plain = K.bias_res_ln_(dev(x), res, None, beta, gamma)
+        inout = dev(x)
+        terms = K.bias_res_ln_split_pairs_(inout, res, None, beta, gamma, scale=16.0)
+        assert torch.equal(inout, plain) and torch.equal(terms, K.split_pairs(plain, 16.0))
+
+
+@pytest.mark.parametrize("batch,heads,seq,d", [(1, 12, 32, 64), (24, 12, 32, 64), (3, 4, 100, 64), (2, 3, 200, 32), (1, 2, 512, 64)])
+def test_attention_rows_of_pairs(K, batch, heads, seq, d):
+    rng = np.random.default_rng(batch + seq)
+    qkv = dev(rng.normal(0, 1, (batch * seq, 3 * heads * d)).astype(np.float32))
+    mask = (rng.random((batch, seq)) < 0.7).astype(np.int8)
+    mask[:, 0] = 1
+    plain = K.attention_fused(qkv, dev(mask), batch, heads, seq, d, d ** -0.5)
+    got = K.attention_fused_split_pairs(qkv, dev(mask), batch, heads, seq, d, d ** -0.5, scale=16.0)
+    assert torch.equal(got, K.split_pairs(plain, 16.0))
+
+
+# every tile, one and fewer steps than the rings hold, tokens and features that end inside a tile
+PAIR_SHAPES = [(1, 4, 32), (65, 68, 64), (129, 36, 160), (400, 768, 96), (1283, 2308, 768), (1281, 3072, 800), (4090, 2308, 768)]
+
+
+@pytest.mark.parametrize("tokens,features,width", PAIR_SHAPES)
+@pytest.mark.parametrize("gelu", [False, True])
+def test_dense_pairs(K, tokens, features, width, gelu):
+    features = (features + 31) // 32 * 32 if gelu else features
+    rng = np.random.default_rng(tokens + width)
+    x = dev(rng.normal(0, 1, (tokens, width)).astype(np.float32))
+    w = dev(rng.normal(0, 0.05, (features, width)).astype(np.float32))
+    bias = dev(rng.normal(0, 0.5, features).astype(np.float32)) if width != 160 else None
+    ldo = features if gelu else features + 8
+    got = K.dense_pairs(K.split_pairs(x, 16.0), K.split_pairs(w, 8192.0), bias, gelu, 1 / (16.0 * 8192.0), 16.0, ldo)
+    assert got is not None
+    want, size = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    if bias is not None:
+        want, size = want + bias.double(), size + bias.double().abs()
+    # 3 width / 16 additions of 16 products each, every one rounded once relative to what has been added so far, and the dropped
+    # low x low terms and representation errors (2^-22 of a product together); GELU has a slope of at most 1.13
+    bound = size * ((3 * width / 16 + 16) * 2.0 ** -23 + 2.0 ** -22)
+    if gelu:
+        want = 0.5 * want * (1 + torch.erf(want / 2 ** 0.5))
+        terms = got.double().view(tokens, -1, 2, 32)
+        got = (terms[:, :, 0] + terms[:, :, 1]).reshape(tokens, features) / 16
+        bound = 1.13 * bound + 5e-7 * (1 + want.abs())  # (the approximation of erf, and the two terms)
+    assert bool(torch.isfinite(got).all()) and bool(((got.double() - want).abs() <= bound).all())
+
+
+def test_dense_pairs_takes_every_tile(K):
+    tiles = {K.dense_pairs_plan(t, f, w, g) for t, f, w in PAIR_SHAPES for g in (False, True)}
+    assert tiles == {(64, 64), (128, 96), (128, 128), (256, 192)}
+
+
+def test_dense_pairs_overflow_and_refusals(K):
+    flag = torch.zeros(1, dtype=torch.int32, device="cuda")
+    x, w = torch.zeros(70, 64, device="cuda"), torch.zeros(96, 64, device="cuda")
+    xs, ws = K.split_pairs(x, 16.0), K.split_pairs(w, 16.0)
+    bias = torch.full((96,), 4000.0, device="cuda")
+    assert K.dense_pairs(xs, ws, bias, True, 1 / 256, 16.0, overflow=flag) is not None
+    torch.cuda.synchronize()
+    assert int(flag.item()) == 0       # 16 * 4000 fits, also in the rows of a tile that are past the last token
+    bias[95] = 4100.0
+    assert K.dense_pairs(xs, ws, bias, True, 1 / 256, 16.0, overflow=flag) is not None
+    torch.cuda.synchronize()
+    assert int(flag.item()) == 1
+    assert K.dense_pairs(xs, ws[:94].contiguous(), None, True) is None      # rows of pairs need whole blocks of 32
+    assert K.dense_pairs(xs, ws[:94].contiguous(), None) is None            # four features per store
+    assert K.dense_pairs(xs, ws, None, ldo=98) is None
