@@ -55,9 +55,9 @@ Transformer<T>::Transformer(void *cublas, const std::string &var_prefix,
                   max_batch_size * seq_length >= kTwoTermMinTokens;
 
     // (also where the library's own kernel is switched off by CUBERT_GEMM the rows are the ones of the library GEMM)
-    int tile_tokens = 0, tile_features = 0;
+    int tile = 0, tile_tokens = 0, tile_features = 0;
     pair_dense = split_dense && H % 32 == 0 && I % 32 == 0 &&
-                 cubert_dense_pairs_plan(1, (int) H, (int) H, 0, &tile_tokens, &tile_features) == 0;
+                 cubert_dense_pairs_plan(1, (int) H, (int) H, 0, &tile, &tile_tokens, &tile_features) == 0;
 
     if (split_dense) {
         split_overflow = static_cast<int *>(cubert_malloc_host(64));

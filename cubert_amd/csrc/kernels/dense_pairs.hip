@@ -45,33 +45,39 @@ __device__ __forceinline__ void order_lds() { asm volatile("s_waitcnt lgkmcnt(0)
 // What leaves the kernel: alpha * product + bias as fp32, or GELU of that, times scale, as operand rows of the next layer.
 enum PairOutput { kPairFloat = 0, kPairGelu = 1 };
 
-// TM tokens x TN features by WM x WN wavefronts, rings of XS steps of X and WS steps of W
-template <int TM, int TN, int WM, int WN, int XS, int WS>
+// TM tokens x TN features by WM x WN wavefronts, or twice as many that take a half of each step (KW = 2); rings of XS steps of X
+// and WS steps of W
+template <int TM, int TN, int WM, int WN, int KW, int XS, int WS>
 struct PairShape {
-    static constexpr int kWaves = WM * WN, kThreads = kWaves * kWave;
+    static constexpr int kTileWaves = WM * WN, kWaves = kTileWaves * KW, kThreads = kWaves * kWave;
     static constexpr int kTB = TM / WM / 32, kFB = TN / WN / 32;  // 32 x 32 blocks of a wavefront
     static constexpr int kXBytes = TM * kRowBytes, kWBytes = TN * kRowBytes;
-    static constexpr int kXLoads = TM / 8 / kWaves, kWLoads = TN / 8 / kWaves;  // requests of a wavefront per step
+    // requests of a wavefront per step, eight rows each; some wavefronts may have one of W less
+    static constexpr int kXLoads = TM / 8 / kWaves, kWLoads = (TN / 8 + kWaves - 1) / kWaves, kWLoadsAtLeast = TN / 8 / kWaves;
     static constexpr int kOutRow = kFB * 32 * 4;  // bytes of a token in a wavefront's part of C
     static constexpr int kOutPitch = kOutRow + 16, kOutBytes = 32 * kOutPitch;
-    static constexpr int kRings = XS * kXBytes + WS * kWBytes, kOut = kWaves * kOutBytes + TN * 4;
+    // of a wavefront at the end: its rows on their way out, and before them what the second half of the wavefronts hands over
+    static constexpr int kHalfBytes = KW == 2 ? kTB * kFB * 16 * kWave * 4 : 0;
+    static constexpr int kPart = kOutBytes > kHalfBytes ? kOutBytes : kHalfBytes;
+    static constexpr int kRings = XS * kXBytes + WS * kWBytes, kOut = kTileWaves * kPart + TN * 4;
     static constexpr int kLdsBytes = kRings > kOut ? kRings : kOut;
-    static_assert(kXLoads * kWaves * 8 == TM && kWLoads * kWaves * 8 == TN, "whole requests");
+    static_assert(kXLoads * kWaves * 8 == TM && TN % 32 == 0 && kWLoadsAtLeast > 0, "whole requests");
     static_assert(XS >= 2 && WS >= XS, "weights are further ahead, or as far");
     static_assert(TN <= kThreads && kLdsBytes <= 160 * 1024, "a thread per bias, LDS of a compute unit");
 };
 
-template <int TM, int TN, int WM, int WN, int XS, int WS, int OUT>
-__global__ __launch_bounds__(WM * WN * kWave) void dense_pairs_kernel(
+template <int TM, int TN, int WM, int WN, int KW, int XS, int WS, int OUT>
+__global__ __launch_bounds__(WM * WN * KW * kWave) void dense_pairs_kernel(
         const half_t *__restrict__ W, const half_t *__restrict__ X, const float *__restrict__ bias, float *__restrict__ C,
         int ldc, int tokens, int features, int steps, int token_tiles, int feature_tiles, float alpha, float scale,
         int *__restrict__ overflow) {
-    typedef PairShape<TM, TN, WM, WN, XS, WS> S;
+    typedef PairShape<TM, TN, WM, WN, KW, XS, WS> S;
     constexpr int TB = S::kTB, FB = S::kFB;
     extern __shared__ __align__(16) unsigned char smem[];
     const int lane = threadIdx.x & (kWave - 1), wave = wave_in_block();
     const int r = lane & 31, hh = lane >> 5;
-    const int wm = wave / WN, wn = wave % WN;
+    const int tile_wave = wave % S::kTileWaves, half = wave / S::kTileWaves;
+    const int wm = tile_wave / WN, wn = tile_wave % WN;
 
     // Workgroups are handed to the eight dies in turn; each die gets a contiguous run of tiles, which go down groups of eight
     // token tiles and then across features: the 32 tiles that a die works on at a time are about 8 x 4 of them.
@@ -110,7 +116,7 @@ __global__ __launch_bounds__(WM * WN * kWave) void dense_pairs_kernel(
             if (with_x && i == S::kXLoads - 1) xbase += kRowBytes;
         } else {
             const int j = i - S::kXLoads;
-            if (with_w) {
+            if (with_w && (j < S::kWLoadsAtLeast || wave + j * S::kWaves < TN / 8)) {
                 load_to_lds(wbase + wo[j], smem + XS * S::kXBytes + wslot * S::kWBytes + (wave + j * S::kWaves) * 1024);
             }
             if (with_w && i == kRequests - 1) wbase += kRowBytes;
@@ -126,35 +132,36 @@ __global__ __launch_bounds__(WM * WN * kWave) void dense_pairs_kernel(
     // operand number j of a phase: the blocks of W, then those of X, low terms first
     constexpr int kReads = kTerms * (TB + FB);
     const int xoff = (wm * TB * 32 + r) * kRowBytes, woff = XS * S::kXBytes + (wn * FB * 32 + r) * kRowBytes;
-    v8f16 x[kPhases][kTerms][TB], w[kPhases][kTerms][FB];
-    auto read = [&](int j, int xslot, int wslot, int phase) {
+    v8f16 x[2][kTerms][TB], w[2][kTerms][FB];
+    auto read = [&](int j, int xslot, int wslot, int phase, int buffer) {
         const int term = kTerms - 1 - j / (TB + FB), k = j % (TB + FB);
         const int unit = ((term * 4 + phase * 2 + hh) ^ ((r >> 1) & 7)) * 16;
         const unsigned char *at = k < FB ? smem + wslot * S::kWBytes + woff + k * 32 * kRowBytes
                                          : smem + xslot * S::kXBytes + xoff + (k - FB) * 32 * kRowBytes;
-        (k < FB ? w[phase][term][k < FB ? k : 0] : x[phase][term][k < FB ? 0 : k - FB]) =
+        (k < FB ? w[buffer][term][k < FB ? k : 0] : x[buffer][term][k < FB ? 0 : k - FB]) =
                 *reinterpret_cast<const v8f16 *>(at + unit);
     };
 
     int xslot = 0, wslot = 0, xfree = 0, wfree = 0;  // slots of the next operands, and those that were read last
     bool more_x = false, more_w = false;
-    // The products of a phase; in between go the reads of the next phase, in the first three quarters, and this phase's share
-    // of the requests into the free slots, which starts with the last phase of a step.
-    auto multiply = [&](int phase) {
+    // The products of a phase; in between go the reads of the wavefront's next phase, in the first three quarters, and this
+    // phase's share of the requests into the free slots, which starts with the last phase of a step.
+    constexpr int kMyPhases = kPhases / KW;
+    auto multiply = [&](int phase, int buffer) {
         constexpr int kProducts = 3 * TB * FB;
-        const int next = (phase + 1) % kPhases;
-        const int from = next * kRequests / kPhases, until = (next + 1) * kRequests / kPhases;
+        const int next = (phase + 1) % kMyPhases;
+        const int from = next * kRequests / kMyPhases, until = (next + 1) * kRequests / kMyPhases;
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_setprio(1);
 #pragma unroll
         for (int m = 0; m < kProducts; ++m) {
             const int kind = m / (TB * FB), t = m / FB % TB, f = m % FB;  // low x high, high x low, high x high
-            acc[t][f] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w[phase][kind == 0 ? 1 : 0][f], x[phase][kind == 1 ? 1 : 0][t],
+            acc[t][f] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w[buffer][kind == 0 ? 1 : 0][f], x[buffer][kind == 1 ? 1 : 0][t],
                                                                acc[t][f], 0, 0, 0);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int j = 0; j < kReads; ++j) {
-                if (j * kProducts * 3 / (4 * kReads) == m) read(j, xslot, wslot, next);
+                if (j * kProducts * 3 / (4 * kReads) == m) read(j, xslot, wslot, KW == 1 ? next : half, buffer ^ 1);
             }
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -174,7 +181,7 @@ __global__ __launch_bounds__(WM * WN * kWave) void dense_pairs_kernel(
 #pragma unroll
         for (int i = 0; i < kRequests; ++i) request(i, d, d < XS && d < steps, d, d < steps);
     if (steps >= WS) {
-        wait_loads<(WS - 1) * S::kWLoads + (XS - 1) * S::kXLoads>();
+        wait_loads<(WS - 1) * S::kWLoadsAtLeast + (XS - 1) * S::kXLoads>();
     } else {
         wait_loads<0>();
     }
@@ -182,16 +189,16 @@ __global__ __launch_bounds__(WM * WN * kWave) void dense_pairs_kernel(
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int j = 0; j < kReads; ++j) read(j, 0, 0, 0);
-    for (int s = 0; s < steps; ++s) {
-        multiply(0);
+    for (int j = 0; j < kReads; ++j) read(j, 0, 0, KW == 1 ? 0 : half, 0);
+    auto step = [&](int s, int buffer) {
+        if constexpr (KW == 1) multiply(0, 0);
         xfree = xslot, wfree = wslot;
         xslot = xslot + 1 < XS ? xslot + 1 : 0, wslot = wslot + 1 < WS ? wslot + 1 : 0;
         more_x = s + XS < steps, more_w = s + WS < steps;
         if (s + 1 < steps) {
             // The next step has landed.  Younger than it: X of XS - 2 steps, and W of as many, or of one more where the ring
             // of W is the deeper one (W of step j + WS follows X of step j + XS).  In the last steps nothing is.
-            constexpr int kYounger = (XS - 2) * S::kXLoads + (XS == WS ? XS - 2 : XS - 1) * S::kWLoads;
+            constexpr int kYounger = (XS - 2) * S::kXLoads + (XS == WS ? XS - 2 : XS - 1) * S::kWLoadsAtLeast;
             if (s + WS <= steps) {
                 wait_loads<kYounger>();
             } else {
@@ -202,22 +209,56 @@ __global__ __launch_bounds__(WM * WN * kWave) void dense_pairs_kernel(
             __builtin_amdgcn_s_barrier();
             __builtin_amdgcn_sched_barrier(0);
         }
-        multiply(1);  // (behind the last step it reads a slot that holds nothing of use, for a phase that does not follow)
+        // (behind the last step this reads a slot that holds nothing of use, for a phase that does not follow)
+        multiply(kMyPhases - 1, KW == 1 ? 1 : buffer);
+    };
+    for (int s = 0; s < steps; s += KW) {
+        step(s, 0);
+        if (KW == 2 && s + 1 < steps) step(s + 1, 1);
     }
 
     __syncthreads();
-    float *bias_lds = reinterpret_cast<float *>(smem + S::kWaves * S::kOutBytes);
+    float *bias_lds = reinterpret_cast<float *>(smem + S::kTileWaves * S::kPart);
     if (threadIdx.x < TN) bias_lds[threadIdx.x] = b;
-    __syncthreads();
+    if constexpr (KW == 2) {
+        float *other = reinterpret_cast<float *>(smem + tile_wave * S::kPart) + lane * 4;
+        if (half == 1) {
+#pragma unroll
+            for (int t = 0; t < TB; ++t)
+#pragma unroll
+                for (int f = 0; f < FB; ++f)
+#pragma unroll
+                    for (int g = 0; g < 4; ++g) {
+                        const Vec<float, 4> v = {acc[t][f][g * 4], acc[t][f][g * 4 + 1], acc[t][f][g * 4 + 2], acc[t][f][g * 4 + 3]};
+                        store_vec<float, 4>(other + ((t * FB + f) * 4 + g) * (4 * kWave), v);
+                    }
+        }
+        __syncthreads();
+        if (half == 1) return;
+#pragma unroll
+        for (int t = 0; t < TB; ++t)
+#pragma unroll
+            for (int f = 0; f < FB; ++f)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    const Vec<float, 4> v = load_vec<float, 4>(other + ((t * FB + f) * 4 + g) * (4 * kWave));
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) acc[t][f][g * 4 + e] += v.v[e];
+                }
+        order_lds();
+    } else {
+        __syncthreads();
+    }
     // 32 tokens at a time: a lane owns a token and, per four accumulator registers, four consecutive features
-    unsigned char *out = smem + wave * S::kOutBytes;
+    unsigned char *out = smem + tile_wave * S::kPart;
     const int col0 = n0 + wn * FB * 32;
     bool over = false;
 #pragma unroll
     for (int t = 0; t < TB; ++t) {
         unsigned char *at = out + r * S::kOutPitch;
 #pragma unroll
-        for (int f = 0; f < FB; ++f)
+        for (int f = 0; f < FB; ++f) {
+            bool fits = true;
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 const int col = g * 8 + hh * 4;
@@ -229,10 +270,12 @@ __global__ __launch_bounds__(WM * WN * kWave) void dense_pairs_kernel(
                     Vec<half_t, 4> hi, lo;
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
+                        // (as split_two_terms; GELU is never below -0.2, and a low term that does not fit is one of a value
+                        // that raises the flag)
                         const float v = GeluOp<float>()(y.v[e]) * scale;
-                        split_two_terms(v, hi.v[e], lo.v[e]);
-                        const int token = m0 + (wm * TB + t) * 32 + r;
-                        over = over || (two_term_overflow(v) && token < tokens && col0 + f * 32 < features);
+                        hi.v[e] = (half_t) fminf(v, 65504.f);
+                        lo.v[e] = (half_t) fmaf(-1.f, (float) hi.v[e], v);
+                        fits = fits && fabsf(v) <= 65504.f;
                     }
                     store_vec<half_t, 4>(reinterpret_cast<half_t *>(at) + f * 64 + col, hi);
                     store_vec<half_t, 4>(reinterpret_cast<half_t *>(at) + f * 64 + 32 + col, lo);
@@ -240,6 +283,8 @@ __global__ __launch_bounds__(WM * WN * kWave) void dense_pairs_kernel(
                     store_vec<float, 4>(reinterpret_cast<float *>(at) + f * 32 + col, y);
                 }
             }
+            over = over || (!fits && m0 + (wm * TB + t) * 32 + r < tokens && col0 + f * 32 < features);
+        }
         order_lds();
         constexpr int kPieces = S::kOutRow / 16;
         const int token0 = m0 + (wm * TB + t) * 32;
@@ -255,12 +300,12 @@ __global__ __launch_bounds__(WM * WN * kWave) void dense_pairs_kernel(
     if (OUT == kPairGelu && over && overflow != nullptr) *overflow = 1;
 }
 
-template <int TM, int TN, int WM, int WN, int XS, int WS, int OUT>
+template <int TM, int TN, int WM, int WN, int KW, int XS, int WS, int OUT>
 int launch_pairs(const half_t *W, const half_t *X, const float *bias, float *C, int ldc, int tokens, int features, int steps,
                  float alpha, float scale, int *overflow, hipStream_t stream) {
-    typedef PairShape<TM, TN, WM, WN, XS, WS> S;
+    typedef PairShape<TM, TN, WM, WN, KW, XS, WS> S;
     static std::atomic<unsigned long long> raised{0};  // per kernel
-    auto kernel = dense_pairs_kernel<TM, TN, WM, WN, XS, WS, OUT>;
+    auto kernel = dense_pairs_kernel<TM, TN, WM, WN, KW, XS, WS, OUT>;
     if (!allow_large_lds(kernel, raised)) return CUBERT_UNSUPPORTED;
     const int token_tiles = (tokens + TM - 1) / TM, feature_tiles = (features + TN - 1) / TN;
     return launch_lds(kernel, dim3((unsigned) (token_tiles * feature_tiles)), dim3(S::kThreads), (unsigned) S::kLdsBytes,
@@ -269,29 +314,35 @@ int launch_pairs(const half_t *W, const half_t *X, const float *bias, float *C, 
 
 // The tile, by a model of the launch time in microseconds, fitted to 768 and 3072 inputs, 384 to 16384 tokens and 768 to 3072
 // features.  With u tiles per compute unit a launch takes what a tile takes by itself, slowed down by the others', or what the
-// tiles of a compute unit take one after the other; for the two larger tiles rounds are whole.  Measured at 768 -> 2304 /
-// 768 -> 768 / 768 -> 3072 with GELU / 3072 -> 768, the tile that is taken first:
-//    384 tokens  64 x 64    10 / 9.4 / 14 / 28         128 x 96   16 / 15 / 18 / 56     256 x 192  35 / 33 / 42 / 117
-//   1280         128 x 96   19 / 16 / 28 / 57          128 x 128  19 / 16 / 24 / 57     64 x 64    21 / 10 / 27 / 30
-//   4096         256 x 192  45 / 36 / 60 / 120         128 x 96   46 / 19 / 64 / 63     64 x 64    57 / 21 / 80 / 74
-//  16384         256 x 192  155 / 54 / 238 / 188       128 x 128  163 / 57 / 237 / 210  64 x 64    225 / 74 / 328 / 281
+// tiles of a compute unit take one after the other; where one or two tiles fill a compute unit, rounds are whole.  Two halves of
+// the wavefronts take a half of each step where a tile would otherwise have one wavefront per matrix core or little to do.
+// Measured at 768 -> 2304 / 768 -> 768 / 768 -> 3072 with GELU / 3072 -> 768, in halves marked *:
+//   tokens   256 x 192            128 x 128            128 x 96           *128 x 96            *64 x 64
+//      384   35 / 34 / 43 / 117   17 / 15 / 20 / 56    16 / 15 / 19 / 60    15 / 15 / 19 / 44   10 / 8.9 / 14 / 26
+//     1280   36 / 34 / 45 / 116   19 / 16 / 24 / 57    20 / 16 / 29 / 59    18 / 16 / 35 / 45   21 / 10 / 27 / 28
+//     2080   38 / 35 / 46 / 116   30 / 17 / 36 / 56    27 / 18 / 48 / 59    31 / 16 / 52 / 45   31 / 13 / 46 / 40
+//     3072   38 / 35 / 52 / 116   34 / 18 / 55 / 59    43 / 19 / 50 / 61    45 / 16 / 57 / 49   42 / 20 / 59 / 65
+//     4096   44 / 35 / 59 / 121   48 / 19 / 60 / 64    44 / 19 / 61 / 67    48 / 18 / 76 / 58   55 / 20 / 86 / 71
+//     8192   87 / 41 / 116 / 131  83 / 32 / 114 / 115  83 / 30 / 122 / 105  94 / 34 / 155 / 113  108 / 37 / 164 / 135
 struct PairTile {
     int tm, tn;
     float alone, alone_step, crowd, each, each_step, start;
     int round;  // tiles per compute unit that run as one round (0: no rounds)
 };
 
-constexpr PairTile kPairTiles[4] = {
+constexpr int kPairTileCount = 5;
+constexpr PairTile kPairTiles[kPairTileCount] = {
         {256, 192, 7.5f, 1.14f, 0.55f, 11.2f, 1.71f, 0.f, 1},
         {128, 128, 2.3f, 0.556f, 0.25f, 0.8f, 0.72f, 7.f, 0},
         {128, 96, 1.6f, 0.57f, 0.12f, 0.6f, 0.55f, 5.f, 2},
-        {64, 64, 3.1f, 0.258f, 0.12f, 0.37f, 0.239f, 4.f, 0},
+        {128, 96, 5.4f, 0.407f, 0.22f, 4.f, 0.54f, 0.f, 1},
+        {64, 64, 3.2f, 0.237f, 0.12f, 0.33f, 0.236f, 4.f, 0},
 };
 
 int plan_pairs(int tokens, int features, int steps, bool gelu) {
     int best = 0;
     float best_us = 0.f;
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < kPairTileCount; ++i) {
         const PairTile &t = kPairTiles[i];
         const long long tiles = (long long) ((tokens + t.tm - 1) / t.tm) * ((features + t.tn - 1) / t.tn);
         const float u = (float) tiles / 256.f;
@@ -316,12 +367,16 @@ int plan_pairs(int tokens, int features, int steps, bool gelu) {
 template <int OUT>
 int launch_tile(int tile, const half_t *W, const half_t *X, const float *bias, float *C, int ldc, int tokens, int features,
                 int steps, float alpha, float scale, int *overflow, hipStream_t s) {
+#define CUBERT_PAIR_TILE(...) \
+    launch_pairs<__VA_ARGS__, OUT>(W, X, bias, C, ldc, tokens, features, steps, alpha, scale, overflow, s)
     switch (tile) {
-        case 0: return launch_pairs<256, 192, 4, 2, 2, 3, OUT>(W, X, bias, C, ldc, tokens, features, steps, alpha, scale, overflow, s);
-        case 1: return launch_pairs<128, 128, 4, 2, 2, 3, OUT>(W, X, bias, C, ldc, tokens, features, steps, alpha, scale, overflow, s);
-        case 2: return launch_pairs<128, 96, 4, 1, 2, 3, OUT>(W, X, bias, C, ldc, tokens, features, steps, alpha, scale, overflow, s);
-        default: return launch_pairs<64, 64, 2, 2, 4, 4, OUT>(W, X, bias, C, ldc, tokens, features, steps, alpha, scale, overflow, s);
+        case 0: return CUBERT_PAIR_TILE(256, 192, 4, 2, 1, 2, 3);
+        case 1: return CUBERT_PAIR_TILE(128, 128, 4, 2, 1, 2, 3);
+        case 2: return CUBERT_PAIR_TILE(128, 96, 4, 1, 1, 2, 3);
+        case 3: return CUBERT_PAIR_TILE(128, 96, 4, 1, 2, 3, 3);
+        default: return CUBERT_PAIR_TILE(64, 64, 2, 2, 2, 4, 4);
     }
+#undef CUBERT_PAIR_TILE
 }
 
 }  // namespace
@@ -344,11 +399,12 @@ int dense_pairs(int tokens, int features, int in, const half_t *x, const half_t 
                    : launch_tile<kPairFloat>(tile, w, x, bias, out, ldo, tokens, features, steps, alpha, scale, overflow, stream);
 }
 
-int dense_pairs_plan(int tokens, int features, int in, int activation, int *tile_tokens, int *tile_features) {
-    if (tokens <= 0 || features <= 0 || in <= 0 || !tile_tokens || !tile_features) return CUBERT_BAD_ARGUMENT;
+// the tile's number, 0 to 4, and its size
+int dense_pairs_plan(int tokens, int features, int in, int activation, int *tile, int *tile_tokens, int *tile_features) {
+    if (tokens <= 0 || features <= 0 || in <= 0 || !tile || !tile_tokens || !tile_features) return CUBERT_BAD_ARGUMENT;
     if (in % kPairStep != 0) return CUBERT_UNSUPPORTED;
-    const PairTile &t = kPairTiles[plan_pairs(tokens, features, in / kPairStep, activation == 1)];
-    *tile_tokens = t.tm, *tile_features = t.tn;
+    *tile = plan_pairs(tokens, features, in / kPairStep, activation == 1);
+    *tile_tokens = kPairTiles[*tile].tm, *tile_features = kPairTiles[*tile].tn;
     return 0;
 }
 

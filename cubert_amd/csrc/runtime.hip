@@ -47,7 +47,7 @@ int dense_mid_plan(int tokens, int features, int in, bool as_slices, size_t part
 // kernels/dense_pairs.hip
 int dense_pairs(int tokens, int features, int in, const half_t *x, const half_t *w, const float *bias, int activation,
                 float alpha, float scale, float *out, int ldo, int *overflow, hipStream_t stream);
-int dense_pairs_plan(int tokens, int features, int in, int activation, int *tile_tokens, int *tile_features);
+int dense_pairs_plan(int tokens, int features, int in, int activation, int *tile, int *tile_tokens, int *tile_features);
 // kernels/gemm_batch.hip
 template <typename T>
 int gemm_batch(int transA, int transB, int M, int N, int K, float alpha, const T *const *A_array, int lda,
@@ -750,9 +750,9 @@ int cubert_dense_pairs_f32(void *stream, int tokens, int features, int in, const
                                alpha, scale, out, ldo, overflow, (hipStream_t) stream);
 }
 
-int cubert_dense_pairs_plan(int tokens, int features, int in, int activation, int *tile_tokens, int *tile_features) {
+int cubert_dense_pairs_plan(int tokens, int features, int in, int activation, int *tile, int *tile_tokens, int *tile_features) {
     if (library_gemm_only() || force_naive_gemm()) return CUBERT_UNSUPPORTED;
-    return cubert::dense_pairs_plan(tokens, features, in, activation, tile_tokens, tile_features);
+    return cubert::dense_pairs_plan(tokens, features, in, activation, tile, tile_tokens, tile_features);
 }
 
 int cubert_gemm_strided_batch_f32(void *handle, int transA, int transB, int M, int N, int K, float alpha,

@@ -242,11 +242,11 @@ def dense_pairs(x, w, bias=None, gelu=False, alpha=1.0, scale=1.0, ldo=None, ove
 
 
 def dense_pairs_plan(tokens, features, width, gelu=False):
-    """(tokens, features) of the tile that dense_pairs takes for a shape."""
-    tm, tn = ctypes.c_int(), ctypes.c_int()
-    _check(lib().cubert_dense_pairs_plan(tokens, features, width, int(gelu), ctypes.byref(tm), ctypes.byref(tn)),
-           "cubert_dense_pairs_plan")
-    return tm.value, tn.value
+    """(number, tokens, features) of the tile that dense_pairs takes for a shape."""
+    tile, tm, tn = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
+    _check(lib().cubert_dense_pairs_plan(tokens, features, width, int(gelu), ctypes.byref(tile), ctypes.byref(tm),
+                                         ctypes.byref(tn)), "cubert_dense_pairs_plan")
+    return tile.value, tm.value, tn.value
 
 
 def split3(x, scale=1.0, lo_in_middle=False, overflow=None):

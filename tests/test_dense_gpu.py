@@ -169,7 +169,8 @@ def test_attention_rows_of_pairs(K, batch, heads, seq, d):
 
 
 # every tile, one and fewer steps than the rings hold, tokens and features that end inside a tile
-PAIR_SHAPES = [(1, 4, 32), (65, 68, 64), (129, 36, 160), (400, 768, 96), (1283, 2308, 768), (1281, 3072, 800), (4090, 2308, 768)]
+PAIR_SHAPES = [(1, 4, 32), (65, 68, 64), (129, 36, 160), (400, 768, 96), (1283, 2308, 768), (1281, 3072, 768), (2080, 2304, 768),
+               (3071, 772, 3072), (4090, 2308, 768)]
 
 
 @pytest.mark.parametrize("tokens,features,width", PAIR_SHAPES)
@@ -199,7 +200,7 @@ def test_dense_pairs(K, tokens, features, width, gelu):
 
 def test_dense_pairs_takes_every_tile(K):
     tiles = {K.dense_pairs_plan(t, f, w, g) for t, f, w in PAIR_SHAPES for g in (False, True)}
-    assert tiles == {(64, 64), (128, 96), (128, 128), (256, 192)}
+    assert tiles == {(0, 256, 192), (1, 128, 128), (2, 128, 96), (3, 128, 96), (4, 64, 64)}
 
 
 def test_dense_pairs_overflow_and_refusals(K):
