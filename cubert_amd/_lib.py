@@ -112,7 +112,8 @@ SIGNATURES = {
     "cubert_attention_fused_split_pairs_f32": (ci, [vp, vp, vp, ci, vp, cf, vp, cf, ci, ci, ci, ci, vp, vp]),
     "cubert_bias_res_ln_split_pairs_f32": (ci, [vp, vp, vp, vp, vp, ci, ci, cf, vp, vp, vp]),
     "cubert_dense_pairs_f32": (ci, [vp, ci, ci, ci, vp, vp, vp, ci, cf, cf, vp, ci, vp]),
-    "cubert_dense_pairs_plan": (ci, [ci, ci, ci, ci, ctypes.POINTER(ci), ctypes.POINTER(ci), ctypes.POINTER(ci)]),
+    "cubert_dense_large_f16": (ci, [vp, ci, ci, ci, vp, vp, vp, ci, vp, ci]),
+    "cubert_dense_large_plan": (ci, [ci, ci, ci, ci, ci, ctypes.POINTER(ci), ctypes.POINTER(ci), ctypes.POINTER(ci)]),
     "cubert_blas_create": (vp, []),
     "cubert_blas_destroy": (ci, [vp]),
     "cubert_blas_set_stream": (ci, [vp, vp]),

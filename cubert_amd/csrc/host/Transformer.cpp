@@ -57,7 +57,7 @@ Transformer<T>::Transformer(void *cublas, const std::string &var_prefix,
     // (also where the library's own kernel is switched off by CUBERT_GEMM the rows are the ones of the library GEMM)
     int tile = 0, tile_tokens = 0, tile_features = 0;
     pair_dense = split_dense && H % 32 == 0 && I % 32 == 0 &&
-                 cubert_dense_pairs_plan(1, (int) H, (int) H, 0, &tile, &tile_tokens, &tile_features) == 0;
+                 cubert_dense_large_plan(1, 1, (int) H, (int) H, 0, &tile, &tile_tokens, &tile_features) == 0;
 
     if (split_dense) {
         split_overflow = static_cast<int *>(cubert_malloc_host(64));
@@ -368,6 +368,27 @@ bool own_dense_is_best(bool half_precision, int tokens, int out_features, int in
     return products <= (use == DenseUse::kPlain ? 4.7e8 : use == DenseUse::kGelu ? 7.6e8 : 7.0e8);
 }
 
+// Whether a half Dense layer runs on the library's own kernel for large requests (kernels/dense_large.hip), which applies bias
+// and GELU, instead of the one for small requests or a library GEMM (with its GELU pass).  Small or library against large, us:
+//   Q|K|V           768 in: 384 tokens 6.2 / 7.2, 512 8.5 / 7.5, 1280 10.7 / 10, 2080 13.8 / 13.1, 2560 16.9 / 16.3, 3072 16.5 /
+//                   16.5, 4096 20.0 / 20.5; 1024 in: 128 4.9 / 7.8, 256 8.7 / 8.3, 1024 12.5 / 11.3, 1536 15.6 / 15.8
+//   intermediate    768 in: 384 9.0 / 8.4, 512 8.9 / 8.8, 768 13.3 / 11, 1280 17.1 / 12.3, 2080 23.7 / 19.3, 4096 33.3 / 27.0,
+//                   8192 66.3 / 52.5, 16384 104 / 94.6; 1024 in: 256 7.9 / 9.7, 384 10.7 / 10, 1024 20.4 / 14.1, 16384 157 / 152
+//   attention out   768: 1280 (small) 5.9 / 7.2, 1536 7.9 / 7.2, 2560 9.1 / 7.8, 4096 11.4 / 9.5, 4992 16.8 / 10.6, 6144 13.6 /
+//                   13.2, 8192 14.6 / 15.4; 1024: 1536 9.5 / 8.8, 4096 13.9 / 12.7, 6144 17.8 / 20.5
+//   output          3072 in: 2080 20.0 / 19.6, 2560 24.9 / 21.1, 3072 21.9 / 29.8, 4096 26.0 / 30.1: left to the library
+// (weights from the Infinity Cache; where a model's weights come from memory the small kernel, which asks for all of its operands
+// at once, is ahead for longer: requests of 256 tokens through BERT-large with Q|K|V on the large one 1070 instead of 1011 us)
+static bool large_dense_is_best(int tokens, int out_features, int in_features, DenseUse use) {
+    const double products = (double) tokens * out_features * in_features;
+    if (tokens < 512) return false;
+    switch (use) {
+        case DenseUse::kPlain: return products > 7.5e8 && products <= 4.6e9;
+        case DenseUse::kGelu: return products > 1.2e9 && products <= 7e10;
+        default: return in_features <= out_features && products <= 4.4e9;
+    }
+}
+
 // CUBERT_FEW_TOKEN_SLICES=0 in the environment keeps the Dense kernels of small requests adding their own K slices.
 static bool few_token_slices_enabled() {
     static const bool on = [] {
@@ -377,13 +398,16 @@ static bool few_token_slices_enabled() {
     return on;
 }
 
+static DenseUse use_of(Profiler::Kind kind) {
+    return kind == Profiler::kDenseQkv            ? DenseUse::kPlain
+           : kind == Profiler::kDenseIntermediate ? DenseUse::kGelu
+                                                  : DenseUse::kNorm;
+}
+
 template <typename T>
 bool Transformer<T>::own_dense_takes(int tokens, int out_features, int in_features, Profiler::Kind kind) const {
     if (!own_dense) return false;
-    const DenseUse use = kind == Profiler::kDenseQkv            ? DenseUse::kPlain
-                         : kind == Profiler::kDenseIntermediate ? DenseUse::kGelu
-                                                                : DenseUse::kNorm;
-    return own_dense_is_best(sizeof(T) == 2, tokens, out_features, in_features, use,
+    return own_dense_is_best(sizeof(T) == 2, tokens, out_features, in_features, use_of(kind),
                              own_slices_to_norm && few_token_slices_enabled());
 }
 
@@ -396,7 +420,18 @@ bool Transformer<T>::dense(int out_features, int tokens, int in_features, const 
     void *stream = cuBERT::blas_get_stream(cublas);
     Timed t(profiler, profiler != nullptr ? profiler->dense_kind(kind) : Profiler::kDenseGemm, stream);
     if (ld_out == 0) ld_out = out_features;
-    if (own_dense_takes(tokens, out_features, in_features, kind)) {
+    const bool small = own_dense_takes(tokens, out_features, in_features, kind);
+    if constexpr (sizeof(T) == 2) {
+        const DenseUse use = use_of(kind);
+        if (own_dense && !(small && use == DenseUse::kNorm) && large_dense_is_best(tokens, out_features, in_features, use)) {
+            const bool with_bias = bias_in_gemm || gelu;
+            if (cuBERT::dense_large(tokens, out_features, in_features, in, kernel, with_bias ? bias : nullptr, gelu, out, ld_out,
+                                    stream)) {
+                return with_bias;
+            }
+        }
+    }
+    if (small) {
         const bool with_bias = bias_in_gemm || gelu;
         if (cuBERT::dense_mid(tokens, out_features, in_features, in, in_features, kernel,
                               transposed_kernels ? in_features : out_features, with_bias ? bias : nullptr, gelu, out, ld_out,

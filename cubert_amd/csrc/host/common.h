@@ -228,7 +228,7 @@ inline bool attention_fused_split3(const float *q, const float *k, const float *
     CUBERT_CHECK(rc);
     return true;
 }
-// the same operands in rows of pairs (the library's own Dense kernel, kernels/dense_pairs.hip)
+// the same operands in rows of pairs (the library's own Dense kernel, kernels/dense_large.hip)
 inline void split_pairs(const float *in, int rows, int width, float scale, half *out, int *overflow, void *stream) {
     CUBERT_CHECK(cubert_split_pairs_f32(in, rows, width, scale, h(out), overflow, stream));
 }
@@ -253,6 +253,14 @@ inline bool attention_fused_split_pairs(const float *q, const float *k, const fl
 inline void dense_pairs(int tokens, int features, int in, const half *x, const half *w, const float *bias, bool gelu, float alpha,
                         float scale, float *out, int ldo, int *overflow, void *stream) {
     CUBERT_CHECK(cubert_dense_pairs_f32(stream, tokens, features, in, h(x), h(w), bias, gelu, alpha, scale, out, ldo, overflow));
+}
+// the same kernel over plain half operands; false when the shape is not taken
+inline bool dense_large(int tokens, int features, int in, const half *x, const half *w, const half *bias, bool gelu, half *out,
+                        int ldo, void *stream) {
+    const int rc = cubert_dense_large_f16(stream, tokens, features, in, h(x), h(w), h(bias), gelu, h(out), ldo);
+    if (rc == CUBERT_UNSUPPORTED) return false;
+    CUBERT_CHECK(rc);
+    return true;
 }
 inline void bias_gelu_split3(const float *in, const float *bias, int rows, int width, float scale, half *out,
                              int *overflow, void *stream) {

@@ -1,17 +1,19 @@
-// Dense layers of hundreds to thousands of tokens whose fp32 operands come as pairs of fp16 numbers:
-//   C[token, feature] = alpha * sum_k x[token, k] w[feature, k] (+ bias) (, GELU),   x = xh + xl, w = wh + wl  (see split.hip)
-// A row of X or W holds, for every 32 values of K, their 32 high terms and then their 32 low terms: 128 bytes, a whole line.
-// The library's form of the same sum is one fp16 GEMM over [hi | hi | lo] rows, which reads the high terms twice and multiplies
-// each operand it reads once; here an operand that has come to LDS takes part in three products of one step, high x low, low x
-// high and high x high, so the 40 bytes per cycle that a compute unit gets from its L2 (measured: 128-byte row pieces; 64-byte
-// pieces 23) feed the matrix cores, which such a GEMM otherwise waits for.
+// Dense layers of hundreds to thousands of tokens on the fp16 matrix cores, C[token, feature] = sum_k x[token, k] w[feature, k],
+// in two forms:
+//   - halves: fp16 rows of X and W, C = fp16(sum + bias) or fp16(GELU(sum + bias)); a step takes 64 values of K;
+//   - pairs: fp32 operands as pairs of fp16 numbers, x = xh + xl, w = wh + wl (see split.hip).  A row of X or W holds, for every
+//     32 values of K, their 32 high terms and then their 32 low terms, a step.  The library's form of the same sum is one fp16
+//     GEMM over [hi | hi | lo] rows, which reads the high terms twice and multiplies each operand it reads once; here an operand
+//     that has come to LDS takes part in three products of one step, high x low, low x high and high x high.
+// Either way a step takes 128 bytes of a row, a whole line: a compute unit gets 40 bytes per cycle from its L2 in such pieces and
+// 23 in pieces of 64 (measured without any products).
 //
-// What bounds it: the matrix cores, which throttle the clock to 1.7 to 2.1 GHz while they are busy; a step of the 256 x 192 tile
-// is 2304 cycles of products and takes some 2900.  What it took to get there, each measured at 4096 tokens, 768 -> 2304:
+// What bounds it: the matrix cores, which throttle the clock to 1.7 to 2.1 GHz while they are busy, and which both forms keep
+// busy for some 60 (halves) to 80 % (pairs) of a step.  What it took to get there, each measured at 4096 tokens, 768 -> 2304:
 //   - two rings in LDS, X two steps deep and W three: the next step's X is asked for when its slot has been read, W earlier;
 //   - requests go out between the products of a phase: asked for in one go after the barrier, a wavefront stands at its
-//     requests while its matrix core idles;
-//   - LDS reads of the next phase also go out between the products, one by one (in one go in front of them: 54.5 us, 47.5);
+//     requests while its matrix core idles (halves 28.1 -> 25.3 us at 256 x 256);
+//   - LDS reads of the next phase also go out between the products, one by one (in one go in front of them: pairs 54.5 us, 47.5);
 //   - one barrier per step, in front of its last phase, whose operands are in registers by then.
 // 32 x 32 blocks of C per wavefront; a finished part of C passes through LDS of its wavefront and leaves in whole row segments.
 #include "activations.h"
@@ -24,9 +26,9 @@ namespace {
 typedef float v16f32 __attribute__((ext_vector_type(16)));
 typedef _Float16 v8f16 __attribute__((ext_vector_type(8)));
 
-constexpr int kRowBytes = 128;              // of a row of X or W that a step takes
-constexpr int kPairStep = kRowBytes / 4;    // values of K in them
-constexpr int kPhases = 2, kTerms = 2;      // of a step, 16 values of K each; high and low
+constexpr int kRowBytes = 128;             // of a row of X or W that a step takes
+constexpr int kHalfStep = kRowBytes / 2;   // values of K in them
+constexpr int kPairStep = kRowBytes / 4;
 
 // 16 bytes per lane from memory to LDS at `base` + 16 * lane, without passing through registers
 __device__ __forceinline__ void load_to_lds(const void *src, void *base) {
@@ -42,19 +44,27 @@ __device__ __forceinline__ void wait_loads() {  // at most N vector-memory reque
 // the LDS accesses of this wavefront in front of it are done before those behind it start
 __device__ __forceinline__ void order_lds() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
-// What leaves the kernel: alpha * product + bias as fp32, or GELU of that, times scale, as operand rows of the next layer.
-enum PairOutput { kPairFloat = 0, kPairGelu = 1 };
+// What the kernel reads and what leaves it.  Pairs: alpha * sum + bias as fp32, or GELU of that, times scale, as operand rows of
+// the next layer.
+enum DenseForm { kHalves = 0, kHalvesGelu = 1, kPairsFloat = 2, kPairsGelu = 3 };
+constexpr bool has_pairs(int form) { return form >= kPairsFloat; }
+template <int FORM>
+struct FormTypes { typedef float Value; };  // of bias and C
+template <>
+struct FormTypes<kHalves> { typedef half_t Value; };
+template <>
+struct FormTypes<kHalvesGelu> { typedef half_t Value; };
 
 // TM tokens x TN features by WM x WN wavefronts, or twice as many that take a half of each step (KW = 2); rings of XS steps of X
 // and WS steps of W
-template <int TM, int TN, int WM, int WN, int KW, int XS, int WS>
-struct PairShape {
+template <int FORM, int TM, int TN, int WM, int WN, int KW, int XS, int WS>
+struct TileShape {
     static constexpr int kTileWaves = WM * WN, kWaves = kTileWaves * KW, kThreads = kWaves * kWave;
     static constexpr int kTB = TM / WM / 32, kFB = TN / WN / 32;  // 32 x 32 blocks of a wavefront
     static constexpr int kXBytes = TM * kRowBytes, kWBytes = TN * kRowBytes;
     // requests of a wavefront per step, eight rows each; some wavefronts may have one of W less
     static constexpr int kXLoads = TM / 8 / kWaves, kWLoads = (TN / 8 + kWaves - 1) / kWaves, kWLoadsAtLeast = TN / 8 / kWaves;
-    static constexpr int kOutRow = kFB * 32 * 4;  // bytes of a token in a wavefront's part of C
+    static constexpr int kOutRow = kFB * 32 * (has_pairs(FORM) ? 4 : 2);  // bytes of a token in a wavefront's part of C
     static constexpr int kOutPitch = kOutRow + 16, kOutBytes = 32 * kOutPitch;
     // of a wavefront at the end: its rows on their way out, and before them what the second half of the wavefronts hands over
     static constexpr int kHalfBytes = KW == 2 ? kTB * kFB * 16 * kWave * 4 : 0;
@@ -66,13 +76,16 @@ struct PairShape {
     static_assert(TN <= kThreads && kLdsBytes <= 160 * 1024, "a thread per bias, LDS of a compute unit");
 };
 
-template <int TM, int TN, int WM, int WN, int KW, int XS, int WS, int OUT>
-__global__ __launch_bounds__(WM * WN * KW * kWave) void dense_pairs_kernel(
-        const half_t *__restrict__ W, const half_t *__restrict__ X, const float *__restrict__ bias, float *__restrict__ C,
-        int ldc, int tokens, int features, int steps, int token_tiles, int feature_tiles, float alpha, float scale,
-        int *__restrict__ overflow) {
-    typedef PairShape<TM, TN, WM, WN, KW, XS, WS> S;
+template <int FORM, int TM, int TN, int WM, int WN, int KW, int XS, int WS>
+__global__ __launch_bounds__(WM * WN * KW * kWave) void dense_large_kernel(
+        const half_t *__restrict__ W, const half_t *__restrict__ X, const typename FormTypes<FORM>::Value *__restrict__ bias,
+        typename FormTypes<FORM>::Value *__restrict__ C, int ldc, int tokens, int features, int steps, int token_tiles,
+        int feature_tiles, float alpha, float scale, int *__restrict__ overflow) {
+    typedef TileShape<FORM, TM, TN, WM, WN, KW, XS, WS> S;
     constexpr int TB = S::kTB, FB = S::kFB;
+    constexpr bool kPairs = has_pairs(FORM);
+    constexpr int kTerms = kPairs ? 2 : 1, kPhases = kPairs ? 2 : 4;  // high and low; phases of a step, 16 values of K each
+    typedef typename FormTypes<FORM>::Value Value;
     extern __shared__ __align__(16) unsigned char smem[];
     const int lane = threadIdx.x & (kWave - 1), wave = wave_in_block();
     const int r = lane & 31, hh = lane >> 5;
@@ -89,9 +102,11 @@ __global__ __launch_bounds__(WM * WN * KW * kWave) void dense_pairs_kernel(
     const int ft = in_group / height, tt = first + in_group - ft * height;
     const int m0 = tt * TM, n0 = ft * TN;
 
-    // the bias of a feature per thread, on its way before the first operands; read where it is used, behind the products
+    // The bias of a feature per thread, on its way before the first operands and looked at behind the products.  (Read without a
+    // branch, from any valid address where there is none: a branch would end with the wait for it.)
     const int my_feature = n0 + (int) threadIdx.x;
-    const float b = bias != nullptr && threadIdx.x < TN && my_feature < features ? bias[my_feature] : 0.f;
+    const bool has_bias = bias != nullptr && threadIdx.x < TN && my_feature < features;
+    const Value b = *(has_bias ? bias + my_feature : reinterpret_cast<const Value *>(W));
 
     // lane l of a request brings the 16-byte unit l % 8 of row l / 8 of eight rows to unit (l % 8) ^ (row / 2 % 8), which
     // spreads the operand reads over all banks; rows past the end are read from the last one
@@ -147,8 +162,9 @@ __global__ __launch_bounds__(WM * WN * KW * kWave) void dense_pairs_kernel(
     // The products of a phase; in between go the reads of the wavefront's next phase, in the first three quarters, and this
     // phase's share of the requests into the free slots, which starts with the last phase of a step.
     constexpr int kMyPhases = kPhases / KW;
+    const int my_first = half * kMyPhases;
     auto multiply = [&](int phase, int buffer) {
-        constexpr int kProducts = 3 * TB * FB;
+        constexpr int kProducts = (kPairs ? 3 : 1) * TB * FB;
         const int next = (phase + 1) % kMyPhases;
         const int from = next * kRequests / kMyPhases, until = (next + 1) * kRequests / kMyPhases;
         __builtin_amdgcn_sched_barrier(0);
@@ -156,12 +172,12 @@ __global__ __launch_bounds__(WM * WN * KW * kWave) void dense_pairs_kernel(
 #pragma unroll
         for (int m = 0; m < kProducts; ++m) {
             const int kind = m / (TB * FB), t = m / FB % TB, f = m % FB;  // low x high, high x low, high x high
-            acc[t][f] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w[buffer][kind == 0 ? 1 : 0][f], x[buffer][kind == 1 ? 1 : 0][t],
-                                                               acc[t][f], 0, 0, 0);
+            acc[t][f] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w[buffer][kPairs && kind == 0 ? 1 : 0][f],
+                                                               x[buffer][kPairs && kind == 1 ? 1 : 0][t], acc[t][f], 0, 0, 0);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int j = 0; j < kReads; ++j) {
-                if (j * kProducts * 3 / (4 * kReads) == m) read(j, xslot, wslot, KW == 1 ? next : half, buffer ^ 1);
+                if (j * kProducts * 3 / (4 * kReads) == m) read(j, xslot, wslot, my_first + next, buffer ^ 1);
             }
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -189,9 +205,10 @@ __global__ __launch_bounds__(WM * WN * KW * kWave) void dense_pairs_kernel(
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int j = 0; j < kReads; ++j) read(j, 0, 0, KW == 1 ? 0 : half, 0);
+    for (int j = 0; j < kReads; ++j) read(j, 0, 0, my_first, 0);
     auto step = [&](int s, int buffer) {
-        if constexpr (KW == 1) multiply(0, 0);
+#pragma unroll
+        for (int q = 0; q + 1 < kMyPhases; ++q) multiply(q, (buffer + q) & 1);
         xfree = xslot, wfree = wslot;
         xslot = xslot + 1 < XS ? xslot + 1 : 0, wslot = wslot + 1 < WS ? wslot + 1 : 0;
         more_x = s + XS < steps, more_w = s + WS < steps;
@@ -210,16 +227,17 @@ __global__ __launch_bounds__(WM * WN * KW * kWave) void dense_pairs_kernel(
             __builtin_amdgcn_sched_barrier(0);
         }
         // (behind the last step this reads a slot that holds nothing of use, for a phase that does not follow)
-        multiply(kMyPhases - 1, KW == 1 ? 1 : buffer);
+        multiply(kMyPhases - 1, (buffer + kMyPhases - 1) & 1);
     };
-    for (int s = 0; s < steps; s += KW) {
+    constexpr int kUnroll = kMyPhases % 2 == 0 ? 1 : 2;  // the operand registers alternate
+    for (int s = 0; s < steps; s += kUnroll) {
         step(s, 0);
-        if (KW == 2 && s + 1 < steps) step(s + 1, 1);
+        if (kUnroll == 2 && s + 1 < steps) step(s + 1, 1);
     }
 
     __syncthreads();
     float *bias_lds = reinterpret_cast<float *>(smem + S::kTileWaves * S::kPart);
-    if (threadIdx.x < TN) bias_lds[threadIdx.x] = b;
+    if (threadIdx.x < TN) bias_lds[threadIdx.x] = to_f32(keep_or_zero(b, has_bias));
     if constexpr (KW == 2) {
         float *other = reinterpret_cast<float *>(smem + tile_wave * S::kPart) + lane * 4;
         if (half == 1) {
@@ -265,8 +283,8 @@ __global__ __launch_bounds__(WM * WN * KW * kWave) void dense_pairs_kernel(
                 const Vec<float, 4> bv = load_vec<float, 4>(bias_lds + (wn * FB + f) * 32 + col);
                 Vec<float, 4> y;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) y.v[e] = fmaf(acc[t][f][g * 4 + e], alpha, bv.v[e]);
-                if constexpr (OUT == kPairGelu) {
+                for (int e = 0; e < 4; ++e) y.v[e] = kPairs ? fmaf(acc[t][f][g * 4 + e], alpha, bv.v[e]) : acc[t][f][g * 4 + e] + bv.v[e];
+                if constexpr (FORM == kPairsGelu) {
                     Vec<half_t, 4> hi, lo;
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
@@ -279,44 +297,71 @@ __global__ __launch_bounds__(WM * WN * KW * kWave) void dense_pairs_kernel(
                     }
                     store_vec<half_t, 4>(reinterpret_cast<half_t *>(at) + f * 64 + col, hi);
                     store_vec<half_t, 4>(reinterpret_cast<half_t *>(at) + f * 64 + 32 + col, lo);
-                } else {
+                } else if constexpr (FORM == kPairsFloat) {
                     store_vec<float, 4>(reinterpret_cast<float *>(at) + f * 32 + col, y);
+                } else {
+                    Vec<half_t, 4> v;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v.v[e] = from_f32<half_t>(FORM == kHalvesGelu ? GeluOp<half_t>()(y.v[e]) : y.v[e]);
+                    store_vec<half_t, 4>(reinterpret_cast<half_t *>(at) + f * 32 + col, v);
                 }
             }
             over = over || (!fits && m0 + (wm * TB + t) * 32 + r < tokens && col0 + f * 32 < features);
         }
         order_lds();
-        constexpr int kPieces = S::kOutRow / 16;
+        constexpr int kPieces = S::kOutRow / 16, kPiece = 16 / sizeof(Value);
         const int token0 = m0 + (wm * TB + t) * 32;
-        float *rows = C + (size_t) token0 * ldc + col0;
+        Value *rows = C + (size_t) token0 * ldc + col0;
 #pragma unroll
         for (int i = 0; i < 32 * kPieces / kWave; ++i) {
             const int item = i * kWave + lane, row = item / kPieces, piece = item - row * kPieces;
-            const Vec<float, 4> v = load_vec<float, 4>(reinterpret_cast<const float *>(out + row * S::kOutPitch + piece * 16));
-            if (token0 + row < tokens && col0 + piece * 4 < features) store_vec<float, 4>(rows + (size_t) row * ldc + piece * 4, v);
+            const auto v = load_vec<Value, kPiece>(reinterpret_cast<const Value *>(out + row * S::kOutPitch + piece * 16));
+            if (token0 + row < tokens && col0 + piece * kPiece < features) {
+                store_vec<Value, kPiece>(rows + (size_t) row * ldc + piece * kPiece, v);
+            }
         }
         order_lds();
     }
-    if (OUT == kPairGelu && over && overflow != nullptr) *overflow = 1;
+    if (FORM == kPairsGelu && over && overflow != nullptr) *overflow = 1;
 }
 
-template <int TM, int TN, int WM, int WN, int KW, int XS, int WS, int OUT>
-int launch_pairs(const half_t *W, const half_t *X, const float *bias, float *C, int ldc, int tokens, int features, int steps,
-                 float alpha, float scale, int *overflow, hipStream_t stream) {
-    typedef PairShape<TM, TN, WM, WN, KW, XS, WS> S;
+// the arguments of a launch
+template <typename Value>
+struct DenseCall {
+    const half_t *W, *X;
+    const Value *bias;
+    Value *C;
+    int ldc, tokens, features, steps;
+    float alpha, scale;
+    int *overflow;
+    hipStream_t stream;
+};
+
+template <int FORM, int TM, int TN, int WM, int WN, int KW, int XS, int WS>
+int launch_large(const DenseCall<typename FormTypes<FORM>::Value> &c) {
+    typedef TileShape<FORM, TM, TN, WM, WN, KW, XS, WS> S;
     static std::atomic<unsigned long long> raised{0};  // per kernel
-    auto kernel = dense_pairs_kernel<TM, TN, WM, WN, KW, XS, WS, OUT>;
+    auto kernel = dense_large_kernel<FORM, TM, TN, WM, WN, KW, XS, WS>;
     if (!allow_large_lds(kernel, raised)) return CUBERT_UNSUPPORTED;
-    const int token_tiles = (tokens + TM - 1) / TM, feature_tiles = (features + TN - 1) / TN;
+    const int token_tiles = (c.tokens + TM - 1) / TM, feature_tiles = (c.features + TN - 1) / TN;
     return launch_lds(kernel, dim3((unsigned) (token_tiles * feature_tiles)), dim3(S::kThreads), (unsigned) S::kLdsBytes,
-                      stream, W, X, bias, C, ldc, tokens, features, steps, token_tiles, feature_tiles, alpha, scale, overflow);
+                      c.stream, c.W, c.X, c.bias, c.C, c.ldc, c.tokens, c.features, c.steps, token_tiles, feature_tiles, c.alpha,
+                      c.scale, c.overflow);
 }
 
 // The tile, by a model of the launch time in microseconds, fitted to 768 and 3072 inputs, 384 to 16384 tokens and 768 to 3072
 // features.  With u tiles per compute unit a launch takes what a tile takes by itself, slowed down by the others', or what the
-// tiles of a compute unit take one after the other; where one or two tiles fill a compute unit, rounds are whole.  Two halves of
-// the wavefronts take a half of each step where a tile would otherwise have one wavefront per matrix core or little to do.
-// Measured at 768 -> 2304 / 768 -> 768 / 768 -> 3072 with GELU / 3072 -> 768, in halves marked *:
+// tiles of a compute unit take one after the other; where one or two tiles fill a compute unit, rounds are whole.
+struct TileModel {
+    int tm, tn;
+    float alone, alone_step, crowd, each, each_step, start;
+    int round;  // tiles per compute unit that run as one round (0: no rounds)
+};
+
+constexpr int kTiles = 5;
+
+// Pairs.  Two halves of the wavefronts take a half of each step where a tile would otherwise have one wavefront per matrix core
+// or little to do.  Measured at 768 -> 2304 / 768 -> 768 / 768 -> 3072 with GELU / 3072 -> 768, in halves marked *:
 //   tokens   256 x 192            128 x 128            128 x 96           *128 x 96            *64 x 64
 //      384   35 / 34 / 43 / 117   17 / 15 / 20 / 56    16 / 15 / 19 / 60    15 / 15 / 19 / 44   10 / 8.9 / 14 / 26
 //     1280   36 / 34 / 45 / 116   19 / 16 / 24 / 57    20 / 16 / 29 / 59    18 / 16 / 35 / 45   21 / 10 / 27 / 28
@@ -324,14 +369,7 @@ int launch_pairs(const half_t *W, const half_t *X, const float *bias, float *C, 
 //     3072   38 / 35 / 52 / 116   34 / 18 / 55 / 59    43 / 19 / 50 / 61    45 / 16 / 57 / 49   42 / 20 / 59 / 65
 //     4096   44 / 35 / 59 / 121   48 / 19 / 60 / 64    44 / 19 / 61 / 67    48 / 18 / 76 / 58   55 / 20 / 86 / 71
 //     8192   87 / 41 / 116 / 131  83 / 32 / 114 / 115  83 / 30 / 122 / 105  94 / 34 / 155 / 113  108 / 37 / 164 / 135
-struct PairTile {
-    int tm, tn;
-    float alone, alone_step, crowd, each, each_step, start;
-    int round;  // tiles per compute unit that run as one round (0: no rounds)
-};
-
-constexpr int kPairTileCount = 5;
-constexpr PairTile kPairTiles[kPairTileCount] = {
+constexpr TileModel kPairTiles[kTiles] = {
         {256, 192, 7.5f, 1.14f, 0.55f, 11.2f, 1.71f, 0.f, 1},
         {128, 128, 2.3f, 0.556f, 0.25f, 0.8f, 0.72f, 7.f, 0},
         {128, 96, 1.6f, 0.57f, 0.12f, 0.6f, 0.55f, 5.f, 2},
@@ -339,11 +377,29 @@ constexpr PairTile kPairTiles[kPairTileCount] = {
         {64, 64, 3.2f, 0.237f, 0.12f, 0.33f, 0.236f, 4.f, 0},
 };
 
-int plan_pairs(int tokens, int features, int steps, bool gelu) {
+// Halves, measured in the same way at 768 -> 2304 / 768 -> 768 / 768 -> 3072 with GELU, in halves of a step marked *:
+//   tokens   256 x 256          256 x 192          128 x 128          128 x 96           *128 x 64
+//      512   19 / 18 / 24       16 / 15 / 20       8.7 / 8.1 / 10     8.7 / 8.2 / 10     7.5 / 6.9 / 8.8
+//     1280   20 / 19 / 26       16 / 16 / 22       10 / 8.9 / 12      10 / 8.4 / 15      11 / 7.2 / 13
+//     2080   20 / 19 / 26       18 / 16 / 22       17 / 8.9 / 19      13 / 8.8 / 24      16 / 7.5 / 22
+//     3072   22 / 19 / 28       19 / 16 / 24       17 / 9.2 / 27      22 / 9.8 / 26      21 / 10 / 29
+//     4096   24 / 20 / 30       21 / 16 / 27       24 / 9.6 / 29      23 / 9.5 / 31      26 / 11 / 34
+//     4992   25 / 20 / 32       22 / 17 / 44       25 / 11 / 36       26 / 12 / 39       30 / 11 / 43
+//     8192   45 / 22 / 59       38 / 18 / 53       39 / 16 / 53       38 / 15 / 59       45 / 17 / 66
+//    16384   71 / 25 / 95       65 / 23 / 100      75 / 26 / 102      73 / 27 / 113      92 / 32 / 132
+constexpr TileModel kHalfTiles[kTiles] = {
+        {256, 256, 6.3f, 1.015f, 0.55f, 8.5f, 1.4f, 0.f, 1},
+        {256, 192, 4.8f, 0.858f, 0.55f, 6.7f, 1.24f, 0.f, 1},
+        {128, 128, 1.3f, 0.567f, 0.25f, 2.4f, 0.434f, 5.f, 0},
+        {128, 96, 0.8f, 0.61f, 0.15f, 1.0f, 0.408f, 4.f, 2},
+        {128, 64, 3.0f, 0.322f, 0.18f, 1.3f, 0.306f, 4.f, 0},
+};
+
+int plan_large(int form, int tokens, int features, int steps) {
     int best = 0;
     float best_us = 0.f;
-    for (int i = 0; i < kPairTileCount; ++i) {
-        const PairTile &t = kPairTiles[i];
+    for (int i = 0; i < kTiles; ++i) {
+        const TileModel &t = has_pairs(form) ? kPairTiles[i] : kHalfTiles[i];
         const long long tiles = (long long) ((tokens + t.tm - 1) / t.tm) * ((features + t.tn - 1) / t.tn);
         const float u = (float) tiles / 256.f;
         const float alone = t.alone + t.alone_step * steps, each = t.each + t.each_step * steps;
@@ -358,53 +414,80 @@ int plan_pairs(int tokens, int features, int steps, bool gelu) {
             const float in_turn = t.start + each * left;
             us += left > 1.f && in_turn > crowded ? in_turn : crowded;
         }
-        if (gelu) us += 2.f + u * (t.tm * t.tn) * 0.12e-3f;
+        if (form == kPairsGelu) us += 2.f + u * (t.tm * t.tn) * 0.12e-3f;
+        if (form == kHalvesGelu) us += 0.6f + u * (t.tm * t.tn) * 0.08e-3f;
         if (i == 0 || us < best_us) best = i, best_us = us;
     }
     return best;
 }
 
-template <int OUT>
-int launch_tile(int tile, const half_t *W, const half_t *X, const float *bias, float *C, int ldc, int tokens, int features,
-                int steps, float alpha, float scale, int *overflow, hipStream_t s) {
-#define CUBERT_PAIR_TILE(...) \
-    launch_pairs<__VA_ARGS__, OUT>(W, X, bias, C, ldc, tokens, features, steps, alpha, scale, overflow, s)
-    switch (tile) {
-        case 0: return CUBERT_PAIR_TILE(256, 192, 4, 2, 1, 2, 3);
-        case 1: return CUBERT_PAIR_TILE(128, 128, 4, 2, 1, 2, 3);
-        case 2: return CUBERT_PAIR_TILE(128, 96, 4, 1, 1, 2, 3);
-        case 3: return CUBERT_PAIR_TILE(128, 96, 4, 1, 2, 3, 3);
-        default: return CUBERT_PAIR_TILE(64, 64, 2, 2, 2, 4, 4);
+template <int FORM>
+int launch_tile(const DenseCall<typename FormTypes<FORM>::Value> &c) {
+    const int tile = plan_large(FORM, c.tokens, c.features, c.steps);
+    if constexpr (has_pairs(FORM)) {
+        switch (tile) {
+            case 0: return launch_large<FORM, 256, 192, 4, 2, 1, 2, 3>(c);
+            case 1: return launch_large<FORM, 128, 128, 4, 2, 1, 2, 3>(c);
+            case 2: return launch_large<FORM, 128, 96, 4, 1, 1, 2, 3>(c);
+            case 3: return launch_large<FORM, 128, 96, 4, 1, 2, 3, 3>(c);
+            default: return launch_large<FORM, 64, 64, 2, 2, 2, 4, 4>(c);
+        }
+    } else {
+        switch (tile) {
+            case 0: return launch_large<FORM, 256, 256, 2, 4, 1, 2, 3>(c);
+            case 1: return launch_large<FORM, 256, 192, 4, 2, 1, 2, 3>(c);
+            case 2: return launch_large<FORM, 128, 128, 4, 2, 1, 2, 3>(c);
+            case 3: return launch_large<FORM, 128, 96, 4, 1, 1, 2, 3>(c);
+            default: return launch_large<FORM, 128, 64, 4, 1, 2, 3, 3>(c);
+        }
     }
-#undef CUBERT_PAIR_TILE
+}
+
+// (an offset inside a tile's rows has 32 bits, a grid 31)
+bool fits_large(int tokens, int features, int in, int step) {
+    return in > 0 && in % step == 0 && in <= (1 << 20) && ((long long) tokens / 64 + 1) * (features / 64 + 1) <= 0x7fffffffLL;
 }
 
 }  // namespace
+
+// C = fp16(X W^T + bias), or GELU of it; CUBERT_UNSUPPORTED (and nothing launched) where it does not fit.
+int dense_large(int tokens, int features, int in, const half_t *x, const half_t *w, const half_t *bias, int activation,
+                half_t *out, int ldo, hipStream_t stream) {
+    if (!x || !w || !out || tokens < 0 || features < 0 || in < 0 || ldo < features || (activation != 0 && activation != 1)) {
+        return CUBERT_BAD_ARGUMENT;
+    }
+    if (!fits_large(tokens, features, in, kHalfStep) || features % 8 != 0 || ldo % 8 != 0 || !is_aligned(x, 16) ||
+        !is_aligned(w, 16) || !is_aligned(out, 16)) {
+        return CUBERT_UNSUPPORTED;
+    }
+    if (tokens == 0 || features == 0) return 0;
+    const DenseCall<half_t> c = {w, x, bias, out, ldo, tokens, features, in / kHalfStep, 1.f, 1.f, nullptr, stream};
+    return activation == 1 ? launch_tile<kHalvesGelu>(c) : launch_tile<kHalves>(c);
+}
 
 int dense_pairs(int tokens, int features, int in, const half_t *x, const half_t *w, const float *bias, int activation,
                 float alpha, float scale, float *out, int ldo, int *overflow, hipStream_t stream) {
     if (!x || !w || !out || tokens < 0 || features < 0 || in < 0 || ldo < features || (activation != 0 && activation != 1)) {
         return CUBERT_BAD_ARGUMENT;
     }
-    // (an offset inside a tile's rows has 32 bits)
-    if (in == 0 || in % kPairStep != 0 || in > (1 << 20) || features % (activation == 1 ? kPairBlock : 4) != 0 || ldo % 4 != 0 ||
-        (activation == 1 && ldo != features) || !is_aligned(x, 16) || !is_aligned(w, 16) || !is_aligned(out, 16) ||
-        ((long long) tokens / 64 + 1) * (features / 64 + 1) > 0x7fffffffLL) {
+    if (!fits_large(tokens, features, in, kPairStep) || features % (activation == 1 ? kPairBlock : 4) != 0 || ldo % 4 != 0 ||
+        (activation == 1 && ldo != features) || !is_aligned(x, 16) || !is_aligned(w, 16) || !is_aligned(out, 16)) {
         return CUBERT_UNSUPPORTED;
     }
     if (tokens == 0 || features == 0) return 0;
-    const int steps = in / kPairStep, tile = plan_pairs(tokens, features, steps, activation == 1);
-    return activation == 1
-                   ? launch_tile<kPairGelu>(tile, w, x, bias, out, ldo, tokens, features, steps, alpha, scale, overflow, stream)
-                   : launch_tile<kPairFloat>(tile, w, x, bias, out, ldo, tokens, features, steps, alpha, scale, overflow, stream);
+    const DenseCall<float> c = {w, x, bias, out, ldo, tokens, features, in / kPairStep, alpha, scale, overflow, stream};
+    return activation == 1 ? launch_tile<kPairsGelu>(c) : launch_tile<kPairsFloat>(c);
 }
 
 // the tile's number, 0 to 4, and its size
-int dense_pairs_plan(int tokens, int features, int in, int activation, int *tile, int *tile_tokens, int *tile_features) {
+int dense_large_plan(int pairs, int tokens, int features, int in, int activation, int *tile, int *tile_tokens,
+                     int *tile_features) {
     if (tokens <= 0 || features <= 0 || in <= 0 || !tile || !tile_tokens || !tile_features) return CUBERT_BAD_ARGUMENT;
-    if (in % kPairStep != 0) return CUBERT_UNSUPPORTED;
-    *tile = plan_pairs(tokens, features, in / kPairStep, activation == 1);
-    *tile_tokens = kPairTiles[*tile].tm, *tile_features = kPairTiles[*tile].tn;
+    const int step = pairs ? kPairStep : kHalfStep;
+    if (in % step != 0) return CUBERT_UNSUPPORTED;
+    *tile = plan_large((pairs ? kPairsFloat : kHalves) + (activation == 1), tokens, features, in / step);
+    const TileModel &t = pairs ? kPairTiles[*tile] : kHalfTiles[*tile];
+    *tile_tokens = t.tm, *tile_features = t.tn;
     return 0;
 }
 

@@ -14,7 +14,7 @@
 // apart (`scale`, exact, taken out again by the GEMM's alpha): weights per matrix, so that the largest is in
 // [512, 1024) and their size does not matter; activations by a fixed factor chosen by the caller (the host classes
 // use 16: full accuracy for rows whose entries are of order 2^-7 to 2^12), clamped to the fp16 range beyond it.
-// Rows for the library's own kernel (dense_pairs.hip) hold every term once, [hi | lo] for every 32 elements.
+// Rows for the library's own kernel (dense_large.hip) hold every term once, [hi | lo] for every 32 elements.
 // A value that had to be clamped (or is not a number) no longer equals its two terms: every kernel that writes
 // two-term rows takes an `overflow` pointer (may be null) and stores 1 there when that happens -- an ordinary store by
 // the lanes concerned, nothing otherwise -- so that the caller can recompute in fp32 instead of using a wrong product.

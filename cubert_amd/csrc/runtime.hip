@@ -44,10 +44,13 @@ int dense_mid_slices(int tokens, int features, int in, const T *X, int ldx, cons
                      size_t partial_floats, int *slices, hipStream_t stream);
 template <typename T>
 int dense_mid_plan(int tokens, int features, int in, bool as_slices, size_t partial_floats, int *tile, int *depth, int *slices);
-// kernels/dense_pairs.hip
+// kernels/dense_large.hip
 int dense_pairs(int tokens, int features, int in, const half_t *x, const half_t *w, const float *bias, int activation,
                 float alpha, float scale, float *out, int ldo, int *overflow, hipStream_t stream);
-int dense_pairs_plan(int tokens, int features, int in, int activation, int *tile, int *tile_tokens, int *tile_features);
+int dense_large(int tokens, int features, int in, const half_t *x, const half_t *w, const half_t *bias, int activation,
+                half_t *out, int ldo, hipStream_t stream);
+int dense_large_plan(int pairs, int tokens, int features, int in, int activation, int *tile, int *tile_tokens,
+                     int *tile_features);
 // kernels/gemm_batch.hip
 template <typename T>
 int gemm_batch(int transA, int transB, int M, int N, int K, float alpha, const T *const *A_array, int lda,
@@ -750,9 +753,17 @@ int cubert_dense_pairs_f32(void *stream, int tokens, int features, int in, const
                                alpha, scale, out, ldo, overflow, (hipStream_t) stream);
 }
 
-int cubert_dense_pairs_plan(int tokens, int features, int in, int activation, int *tile, int *tile_tokens, int *tile_features) {
+int cubert_dense_large_f16(void *stream, int tokens, int features, int in, const cubert_half *x, const cubert_half *w,
+                           const cubert_half *bias, int activation, cubert_half *out, int ldo) {
     if (library_gemm_only() || force_naive_gemm()) return CUBERT_UNSUPPORTED;
-    return cubert::dense_pairs_plan(tokens, features, in, activation, tile, tile_tokens, tile_features);
+    return cubert::dense_large(tokens, features, in, (const cubert::half_t *) x, (const cubert::half_t *) w,
+                               (const cubert::half_t *) bias, activation, (cubert::half_t *) out, ldo, (hipStream_t) stream);
+}
+
+int cubert_dense_large_plan(int pairs, int tokens, int features, int in, int activation, int *tile, int *tile_tokens,
+                            int *tile_features) {
+    if (library_gemm_only() || force_naive_gemm()) return CUBERT_UNSUPPORTED;
+    return cubert::dense_large_plan(pairs, tokens, features, in, activation, tile, tile_tokens, tile_features);
 }
 
 int cubert_gemm_strided_batch_f32(void *handle, int transA, int transB, int M, int N, int K, float alpha,

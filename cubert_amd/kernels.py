@@ -241,11 +241,23 @@ def dense_pairs(x, w, bias=None, gelu=False, alpha=1.0, scale=1.0, ldo=None, ove
     return out.view(torch.float16) if gelu else out[:, :features]
 
 
-def dense_pairs_plan(tokens, features, width, gelu=False):
-    """(number, tokens, features) of the tile that dense_pairs takes for a shape."""
+def dense_large(x, w, bias=None, gelu=False, ldo=None):
+    """x w^T + bias of fp16 rows (, GELU), for hundreds to thousands of tokens; None when declined."""
+    (tokens, width), features = x.shape, w.shape[0]
+    ldo = features if ldo is None else ldo
+    out = torch.empty((tokens, ldo), dtype=torch.float16, device=x.device)
+    rc = lib().cubert_dense_large_f16(_stream(), tokens, features, width, _ptr(x), _ptr(w), _ptr(bias), int(gelu), _ptr(out), ldo)
+    if rc == -2:
+        return None
+    _check(rc, "cubert_dense_large_f16")
+    return out[:, :features]
+
+
+def dense_large_plan(pairs, tokens, features, width, gelu=False):
+    """(number, tokens, features) of the tile that dense_pairs (pairs) or dense_large takes for a shape."""
     tile, tm, tn = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
-    _check(lib().cubert_dense_pairs_plan(tokens, features, width, int(gelu), ctypes.byref(tile), ctypes.byref(tm),
-                                         ctypes.byref(tn)), "cubert_dense_pairs_plan")
+    _check(lib().cubert_dense_large_plan(int(pairs), tokens, features, width, int(gelu), ctypes.byref(tile), ctypes.byref(tm),
+                                         ctypes.byref(tn)), "cubert_dense_large_plan")
     return tile.value, tm.value, tn.value
 
 

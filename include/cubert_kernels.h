@@ -338,8 +338,15 @@ int cubert_bias_res_ln_split_pairs_f32(float *inout, const float *residual, cons
  * replaces: Dense<float>::compute, reference src/cuBERT/op/Dense.cpp:47-57, and gelu<float>, op/GELU.h:6-7, in their opt-in form. */
 int cubert_dense_pairs_f32(void *stream, int tokens, int features, int in, const cubert_half *x, const cubert_half *w,
                            const float *bias, int activation, float alpha, float scale, float *out, int ldo, int *overflow);
-/* the tile, by its number and size, that cubert_dense_pairs_f32 takes for a shape */
-int cubert_dense_pairs_plan(int tokens, int features, int in, int activation, int *tile, int *tile_tokens, int *tile_features);
+/* The same kernel over plain fp16 operands, x [tokens, in] and w [features, in]: out = fp16(x w^T + bias) (bias may be NULL), or,
+ * with activation 1, GELU of that, sums, bias and GELU in fp32.  in a multiple of 64, features and ldo of 8, operands 16-byte
+ * aligned; otherwise (and with CUBERT_GEMM=library or naive) CUBERT_UNSUPPORTED.  For hundreds to thousands of tokens;
+ * replaces: Dense<half>::compute, reference src/cuBERT/op/Dense.cpp:47-57, and gelu<half>, op/GELU.h:6-7. */
+int cubert_dense_large_f16(void *stream, int tokens, int features, int in, const cubert_half *x, const cubert_half *w,
+                           const cubert_half *bias, int activation, cubert_half *out, int ldo);
+/* the tile, by its number and size, that cubert_dense_pairs_f32 (pairs = 1) or cubert_dense_large_f16 takes for a shape */
+int cubert_dense_large_plan(int pairs, int tokens, int features, int in, int activation, int *tile, int *tile_tokens,
+                            int *tile_features);
 
 /* C = alpha * A * B + bias for N <= 64 columns (no transposes, beta = 0): the Dense layer of a request with at
  * most 64 tokens, where A is the [in, out] weight matrix (M = out, K = in) and each column of B one token.

@@ -121,7 +121,7 @@ def test_dense_declines_what_it_cannot_do(K, name):
     assert K.dense_slices(*operands_of(1024, 64), partial_floats=8 * 64) is None  # no room for two slices
 
 
-# ---- fp32 operands as pairs of fp16 numbers (kernels/dense_pairs.hip) ------------------------------------------
+# ---- large requests (kernels/dense_large.hip): fp32 operands as pairs of fp16 numbers --------------------------
 
 def dev(a):
     return torch.from_numpy(np.ascontiguousarray(a)).cuda()
@@ -199,7 +199,7 @@ def test_dense_pairs(K, tokens, features, width, gelu):
 
 
 def test_dense_pairs_takes_every_tile(K):
-    tiles = {K.dense_pairs_plan(t, f, w, g) for t, f, w in PAIR_SHAPES for g in (False, True)}
+    tiles = {K.dense_large_plan(True, t, f, w, g) for t, f, w in PAIR_SHAPES for g in (False, True)}
     assert tiles == {(0, 256, 192), (1, 128, 128), (2, 128, 96), (3, 128, 96), (4, 64, 64)}
 
 
@@ -218,3 +218,40 @@ def test_dense_pairs_overflow_and_refusals(K):
     assert K.dense_pairs(xs, ws[:94].contiguous(), None, True) is None      # rows of pairs need whole blocks of 32
     assert K.dense_pairs(xs, ws[:94].contiguous(), None) is None            # four features per store
     assert K.dense_pairs(xs, ws, None, ldo=98) is None
+
+
+# ---- large requests: half operands ----------------------------------------------------------------------------
+
+LARGE_SHAPES = [(1, 8, 64), (129, 72, 128), (130, 64, 192), (700, 768, 256), (1537, 2304, 768), (2083, 3080, 768), (4090, 2312, 768),
+                (4990, 3072, 768), (3001, 776, 3072), (2080, 2304, 768)]
+
+
+@pytest.mark.parametrize("tokens,features,width", LARGE_SHAPES)
+@pytest.mark.parametrize("gelu", [False, True])
+def test_dense_large(K, tokens, features, width, gelu):
+    rng = np.random.default_rng(tokens + width)
+    x = dev(rng.normal(0, 1, (tokens, width)).astype(np.float16))
+    w = dev(rng.normal(0, 0.05, (features, width)).astype(np.float16))
+    bias = dev(rng.normal(0, 0.5, features).astype(np.float16)) if width != 192 else None
+    got = K.dense_large(x, w, bias, gelu, features + 8)
+    assert got is not None
+    want, size = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    if bias is not None:
+        want, size = want + bias.double(), size + bias.double().abs()
+    bound = size * (width / 16 + 16) * 2.0 ** -23  # additions of 16 products each, rounded relative to what has been added
+    if gelu:
+        want = 0.5 * want * (1 + torch.erf(want / 2 ** 0.5))
+        bound = 1.13 * bound + 7.2e-7 * (1 + want.abs())  # (the approximation of erf)
+    bound = bound + want.abs() * 2.0 ** -11 + 2.0 ** -25  # the store
+    assert bool(torch.isfinite(got).all()) and bool(((got.double() - want).abs() <= bound).all())
+
+
+def test_dense_large_tiles_and_refusals(K):
+    tiles = {K.dense_large_plan(False, t, f, w, g) for t, f, w in LARGE_SHAPES for g in (False, True)}
+    assert tiles == {(0, 256, 256), (1, 256, 192), (2, 128, 128), (3, 128, 96), (4, 128, 64)}
+    x, w = torch.zeros(64, 128, dtype=torch.float16, device="cuda"), torch.zeros(64, 128, dtype=torch.float16, device="cuda")
+    assert K.dense_large(x[:, :96].contiguous(), w[:, :96].contiguous()) is None  # whole lines of K
+    assert K.dense_large(x, w[:60].contiguous()) is None                          # eight features per store
+    assert K.dense_large(x, w, ldo=68) is None
+    base = torch.zeros(64 * 128 + 1, dtype=torch.float16, device="cuda")
+    assert K.dense_large(base[1:].view(64, 128), w) is None                       # 16-byte requests
