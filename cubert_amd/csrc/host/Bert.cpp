@@ -134,6 +134,14 @@ Bert<T>::Bert(const std::unordered_map<std::string, T *> &var, size_t max_batch_
         if (input_staging == nullptr) throw std::runtime_error("no page-locked host memory for the request inputs");
         output_staging = static_cast<unsigned char *>(cubert_malloc_host(kOutputStagingBytes));
         if (output_staging == nullptr) throw std::runtime_error("no page-locked host memory for the outputs");
+        if (max_batch_size * seq_length * H * sizeof(T) > kOutputStagingBytes) {
+            output_ring = static_cast<unsigned char *>(cubert_malloc_host(kOutputSlots * kOutputPieceBytes));
+            if (output_ring == nullptr) throw std::runtime_error("no page-locked host memory for the outputs");
+            for (void *&event : slot_filled) {
+                event = cubert_copy_event_create();
+                if (event == nullptr) throw std::runtime_error("no event for the output copies");
+            }
+        }
 
         for (size_t batch : open_warmup_batches(std::getenv("CUBERT_OPEN_WARMUP"), max_batch_size)) _pre_compute(batch);
     } catch (...) {
@@ -152,10 +160,15 @@ void Bert<T>::release() noexcept {
     if (stream != nullptr) cubert_stream_synchronize(stream);
     cubert_free_host(input_staging);  // null is accepted
     cubert_free_host(output_staging);
+    cubert_free_host(output_ring);
+    for (void *&event : slot_filled) {
+        if (event != nullptr) cubert_event_destroy(event);
+        event = nullptr;
+    }
     delete transformer;
     if (cublas != nullptr) cubert_blas_destroy(cublas);
     if (stream != nullptr) cubert_stream_destroy(stream);
-    input_staging = nullptr, output_staging = nullptr, transformer = nullptr, cublas = nullptr, stream = nullptr;
+    input_staging = nullptr, output_staging = nullptr, output_ring = nullptr, transformer = nullptr, cublas = nullptr, stream = nullptr;
 }
 
 template <typename T>
@@ -232,13 +245,36 @@ void Bert<T>::enqueue_fetch(void *dst, const void *src, size_t bytes) {
         cuBERT::memcpyAsync(output_staging + at, src, bytes, 2, stream);
         staged.push_back(StagedOutput{dst, at, bytes});
         staged_bytes = at + bytes;
+    } else if (output_ring != nullptr && !cubert_is_page_locked(dst)) {
+        for (size_t done = 0; done < bytes; done += kOutputPieceBytes) {
+            pieces.push_back(OutputPiece{static_cast<unsigned char *>(dst) + done, static_cast<const unsigned char *>(src) + done,
+                                         bytes - done < kOutputPieceBytes ? bytes - done : kOutputPieceBytes});
+        }
     } else {
         cuBERT::memcpyAsync(dst, src, bytes, 2, stream);
     }
 }
 
 template <typename T>
+void Bert<T>::drain_pieces() {
+    auto request = [&](size_t i) {
+        const size_t slot = i % kOutputSlots;
+        cuBERT::memcpyAsync(output_ring + slot * kOutputPieceBytes, pieces[i].src, pieces[i].bytes, 2, stream);
+        CUBERT_CHECK(cubert_event_record(slot_filled[slot], stream));
+    };
+    for (size_t i = 0; i < pieces.size() && i < kOutputSlots; ++i) request(i);
+    for (size_t i = 0; i < pieces.size(); ++i) {
+        const size_t slot = i % kOutputSlots;
+        CUBERT_CHECK(cubert_event_synchronize(slot_filled[slot]));
+        std::memcpy(pieces[i].dst, output_ring + slot * kOutputPieceBytes, pieces[i].bytes);
+        if (i + kOutputSlots < pieces.size()) request(i + kOutputSlots);
+    }
+    pieces.clear();
+}
+
+template <typename T>
 void Bert<T>::finish_outputs() {
+    drain_pieces();
     synchronize();
     // An fp32 model in the two-term fp16 Dense form (opt-in): an activation beyond what two fp16 terms can hold
     // raised a flag while the request ran.  Its results are not to be trusted: the same request, whose inputs are
@@ -249,6 +285,7 @@ void Bert<T>::finish_outputs() {
         staged.clear();
         staged_bytes = 0;
         for (const RequestedOutput &o : requested) enqueue_fetch(o.dst, o.src, o.bytes);
+        drain_pieces();
         synchronize();
         (void) transformer->two_term_overflowed();  // (the fp32 pass writes no two-term rows; nothing to clear)
     }

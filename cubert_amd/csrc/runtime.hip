@@ -526,6 +526,24 @@ void *cubert_event_create(void) {
     return e;
 }
 
+void *cubert_copy_event_create(void) {
+    hipEvent_t e = nullptr;
+    if (hipEventCreateWithFlags(&e, hipEventDisableTiming | hipEventReleaseToSystem) != hipSuccess) {
+        (void) hipGetLastError();
+        return nullptr;
+    }
+    return e;
+}
+
+int cubert_is_page_locked(const void *p) {
+    hipPointerAttribute_t attributes;
+    if (hipPointerGetAttributes(&attributes, p) != hipSuccess) {
+        (void) hipGetLastError();  // memory the runtime does not know
+        return 0;
+    }
+    return attributes.type == hipMemoryTypeHost ? 1 : 0;
+}
+
 void *cubert_malloc_host(size_t size) {
     void *p = nullptr;
     if (hipHostMalloc(&p, size, hipHostMallocDefault) != hipSuccess) {

@@ -752,3 +752,30 @@ def test_concurrent_callers_share_one_model(cb, small_pb, monkeypatch, models_pe
     [t.join() for t in threads]
     model.close()
     assert not errors, errors
+
+
+@pytest.mark.parametrize("batch,seq", [(1, 33), (3, 85), (64, 128), (130, 126), (200, 128)])
+def test_large_outputs_reach_pageable_and_page_locked_arrays(cb, batch, seq):
+    """Outputs beyond the small staging block come in pieces of 4 MB through two slots: less than a piece, one whole piece, a
+    remainder, and more pieces than slots; into ordinary and into page-locked arrays, together with small ones,
+    twice in a row.  hidden 128 fp32: 512 bytes a token."""
+    cfg = dict(vocab=211, hidden=128, layers=1, heads=4, intermediate=256, max_position=128, type_vocab=2)
+    from cubert_amd.testing import random_bert_weights, random_inputs
+    torch = pytest.importorskip("torch")
+    w = random_bert_weights(seed=3, labels=2, ln_random=True, **cfg)
+    bert = cb.Bert(w, batch, seq, cfg["layers"], cfg["heads"])
+    for seed in (1, 2):
+        ids, mask, seg = random_inputs(seed=seed, batch=batch, seq_length=seq, vocab=cfg["vocab"], min_valid=1)
+        want = oracle.bert_forward(w, ids, mask, seg, cfg["layers"], cfg["heads"])
+        for locked in (False, True):
+            o = cb.Output()
+            keep = {}
+            for k, shape in (("sequence_output", (batch, seq, 128)), ("embedding_output", (batch, seq, 128)),
+                             ("pooled_output", (batch, 128))):
+                keep[k] = torch.full(shape, float("nan"), pin_memory=locked).numpy()
+                setattr(o, k, keep[k])
+            bert.compute(ids, mask, seg)
+            bert.output(batch, o)
+            for k, got in keep.items():
+                assert_close(got, want[k], FP32_TOL, "%s %s" % (k, locked))
+    bert.close()
