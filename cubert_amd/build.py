@@ -22,11 +22,8 @@ INCLUDES = ["-I" + os.path.join(ROOT, "include"), "-I" + os.path.join(CSRC, "ker
 # -amdgpu-mfma-vgpr-form: matrix-core accumulators stay in ordinary vector registers.  The default puts them in the
 # accumulation registers and copies every result out before the first ordinary instruction can touch it (96 copies
 # per wavefront in the one-launch attention kernel) and, with both files in use, holds fewer wavefronts per SIMD.
-# -amdgpu-kernarg-preload-count: a kernel's first arguments arrive in scalar registers with the dispatch instead of by a
-# load that every wavefront starts with and waits for, 0.1 us of each of the some 87 dependent launches of a small request
-# (whole request, without / with: 1 x 32 fp32 476.9 / 466.3 us, 1 x 128 fp16 401.9 / 394.7, 5 x 24 fp32 657.2 / 651.2).
 DEVICE_FLAGS = ["--offload-arch=" + ARCH, "-O3", "-std=c++17", "-fPIC", "-Xclang", "-target-feature", "-Xclang",
-                "-packed-fp32-ops", "-mllvm", "-amdgpu-mfma-vgpr-form=1", "-mllvm", "-amdgpu-kernarg-preload-count=16", "-Wno-unused-command-line-argument"]
+                "-packed-fp32-ops", "-mllvm", "-amdgpu-mfma-vgpr-form=1", "-Wno-unused-command-line-argument"]
 HOST_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-command-line-argument"]
 
 DEVICE_SOURCES = ["kernels/layernorm.hip", "kernels/softmax.hip", "kernels/elementwise.hip", "kernels/attention.hip", "kernels/gemm_skinny.hip", "kernels/dense_mid.hip", "kernels/dense_large.hip", "kernels/gemm_batch.hip", "kernels/split.hip",
