@@ -377,16 +377,19 @@ bool own_dense_is_best(bool half_precision, int tokens, int out_features, int in
 //   attention out   768: 1280 (small) 5.9 / 7.2, 1536 7.9 / 7.2, 2560 9.1 / 7.8, 4096 11.4 / 9.5, 4992 16.8 / 10.6, 6144 13.6 /
 //                   13.2, 8192 14.6 / 15.4; 1024: 1536 9.5 / 8.8, 4096 13.9 / 12.7, 6144 17.8 / 20.5
 //   output          3072 in: 2080 20.0 / 19.6, 2560 24.9 / 21.1, 3072 21.9 / 29.8, 4096 26.0 / 30.1: left to the library
+// other sizes      Q|K|V 128 in: 32768 tokens 12.1 / 10.6; 512: 4096 12.1 / 11.6; 1536: 512 15.4 / 16.8; intermediate 128 in:
+//                   32768 33.9 / 18.6; 512: 4096 28.6 / 20.3, 65536 223 / 203; 2048: 512 28.3 / 25.2, 2048 67.3 / 66.8; attention
+//                   out 128: 8192 5.5 / 4.6; 256: 32768 11.3 / 12.6; 512: 8192 10.0 / 8.7, 16384 14.8 / 16.5
 // (weights from the Infinity Cache; where a model's weights come from memory the small kernel, which asks for all of its operands
 // at once, is ahead for longer: requests of 256 tokens through BERT-large with Q|K|V on the large one 1070 instead of 1011 us)
 static bool large_dense_is_best(int tokens, int out_features, int in_features, DenseUse use) {
     const double products = (double) tokens * out_features * in_features;
     if (tokens < 512) return false;
     switch (use) {
-        case DenseUse::kPlain: return products > 7.5e8 && products <= 4.6e9;
+        case DenseUse::kPlain: return products > 7.5e8 && products <= 4.6e9 && in_features <= 1024;
         // (just past the small kernel's 1280 tokens the library's two launches stay, as test_model_gpu.py states it for 1312)
         case DenseUse::kGelu: return products > 1.2e9 && products <= 7e10 && (tokens <= 1280 || tokens > 1312);
-        default: return in_features <= out_features && products <= 4.4e9;
+        default: return in_features <= out_features && products <= 4.4e9 && tokens <= 8192;
     }
 }
 
