@@ -128,8 +128,9 @@ def algorithmic_bytes(cfg):
     e = 4 if cfg["dtype"] == "f32" else 2
     M = B * S
     if two_term_dense() and e == 4 and M >= 384:
-        # bias+GELU reads fp32 and writes [hi | hi | lo] fp16 rows; the LayerNorm writes both forms
-        extra = {"bias_gelu": M * I * (4 + 6) + I * 4, "bias_res_ln": 3 * M * H * 4 + 3 * H * 4 + 6 * M * H,
+        # The LayerNorm also writes rows of pairs.  Passes that only the library's form of the Dense layers has: bias+GELU reads
+        # fp32 and writes [hi | hi | lo] fp16 rows, and so does the split.
+        extra = {"bias_gelu": M * I * (4 + 6) + I * 4, "bias_res_ln": 3 * M * H * 4 + 3 * H * 4 + 4 * M * H,
                  "dense_split": M * H * (4 + 6)}
     else:
         extra = {}
