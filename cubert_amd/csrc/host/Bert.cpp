@@ -296,6 +296,16 @@ void Bert<T>::finish_outputs() {
 }
 
 template <typename T>
+void Bert<T>::forget_outputs() noexcept {
+    // (requested is empty behind a call that ended well)  Copies may be on their way into arrays that the caller is about to free.
+    if (!requested.empty()) (void) cubert_stream_synchronize(stream);
+    requested.clear();
+    pieces.clear();
+    staged.clear();
+    staged_bytes = 0;
+}
+
+template <typename T>
 void Bert<T>::compute(size_t batch_size, int *input_ids, int8_t *input_mask, int8_t *segment_ids) {
     if (batch_size > max_batch_size) {
         throw std::invalid_argument("batch_size > max_batch_size");
@@ -387,6 +397,7 @@ void Bert<T>::forward(size_t batch_size) {
 
 template <typename T>
 void Bert<T>::logits(size_t batch_size, T *logits, T *probs) {
+    const OutputCall call{this};
     if (!has_classifier) {
         std::cerr << "model does not have additional_output_layer, the output logits is wrong." << std::endl;
     }
@@ -401,24 +412,28 @@ void Bert<T>::logits(size_t batch_size, T *logits, T *probs) {
 
 template <typename T>
 void Bert<T>::pooled_output(size_t batch_size, T *pooled_output) {
+    const OutputCall call{this};
     fetch(pooled_output, _pooled_output, sizeof(T) * batch_size * hidden_size);
     finish_outputs();
 }
 
 template <typename T>
 void Bert<T>::sequence_output(size_t batch_size, T *sequence_output) {
+    const OutputCall call{this};
     fetch(sequence_output, _sequence_output, sizeof(T) * batch_size * seq_length * hidden_size);
     finish_outputs();
 }
 
 template <typename T>
 void Bert<T>::embedding_output(size_t batch_size, T *embedding_output) {
+    const OutputCall call{this};
     fetch(embedding_output, _embedding_output, sizeof(T) * batch_size * seq_length * hidden_size);
     finish_outputs();
 }
 
 template <typename T>
 void Bert<T>::output(size_t batch_size, cuBERT_Output *output) {
+    const OutputCall call{this};
     const size_t tokens = batch_size * seq_length * hidden_size;
     if (output->logits != nullptr && has_classifier) {
         fetch(output->logits, _logits, sizeof(T) * batch_size * num_labels);

@@ -82,6 +82,7 @@ private:
     void enqueue_fetch(void *dst, const void *src, size_t bytes);
     void drain_pieces();      // the large outputs, piece by piece
     void finish_outputs();    // drain the stream and hand staged outputs to the caller's arrays
+    void forget_outputs() noexcept;  // what is left of an output call that threw: nothing may name its caller's arrays
     void release() noexcept;  // everything the constructor acquired so far (also run when it throws)
     void layout_weights(size_t vocab_size, size_t type_vocab_size);
     void layout_buffers();
@@ -138,6 +139,11 @@ private:
         size_t bytes;
     };
     std::vector<RequestedOutput> requested;
+    // in scope while an output method runs, however it ends
+    struct OutputCall {
+        Bert *bert;
+        ~OutputCall() { bert->forget_outputs(); }
+    };
     size_t last_batch = 0;               // batch size of the forward pass whose results the buffers hold
     bool input_copy_pending = false;     // a copy out of input_staging was queued and the stream not drained since
     int *input_ids_buf;
