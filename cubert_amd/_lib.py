@@ -93,7 +93,7 @@ SIGNATURES = {
     "cubert_event_synchronize": (ci, [vp]),
     "cubert_event_create": (vp, []),
     "cubert_copy_event_create": (vp, []),
-    "cubert_is_page_locked": (ci, [vp]),
+    "cubert_is_pageable": (ci, [vp]),
     "cubert_event_destroy": (ci, [vp]),
     "cubert_event_record": (ci, [vp, vp]),
     "cubert_event_elapsed_ms": (ci, [vp, vp, ctypes.POINTER(cf)]),

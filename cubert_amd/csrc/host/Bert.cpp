@@ -245,7 +245,7 @@ void Bert<T>::enqueue_fetch(void *dst, const void *src, size_t bytes) {
         cuBERT::memcpyAsync(output_staging + at, src, bytes, 2, stream);
         staged.push_back(StagedOutput{dst, at, bytes});
         staged_bytes = at + bytes;
-    } else if (output_ring != nullptr && !cubert_is_page_locked(dst)) {
+    } else if (output_ring != nullptr && cubert_is_pageable(dst)) {
         for (size_t done = 0; done < bytes; done += kOutputPieceBytes) {
             pieces.push_back(OutputPiece{static_cast<unsigned char *>(dst) + done, static_cast<const unsigned char *>(src) + done,
                                          bytes - done < kOutputPieceBytes ? bytes - done : kOutputPieceBytes});

@@ -535,13 +535,14 @@ void *cubert_copy_event_create(void) {
     return e;
 }
 
-int cubert_is_page_locked(const void *p) {
+int cubert_is_pageable(const void *p) {
+    if (p == nullptr) return 0;
     hipPointerAttribute_t attributes;
     if (hipPointerGetAttributes(&attributes, p) != hipSuccess) {
         (void) hipGetLastError();  // memory the runtime does not know
-        return 0;
+        return 1;
     }
-    return attributes.type == hipMemoryTypeHost ? 1 : 0;
+    return attributes.type == hipMemoryTypeUnregistered ? 1 : 0;
 }
 
 void *cubert_malloc_host(size_t size) {

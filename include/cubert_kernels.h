@@ -247,8 +247,9 @@ int cubert_free_host(void *ptr);
  * kernels of a forward pass where they run and tell the host when a staging buffer may be written again. */
 void *cubert_event_create(void);
 void *cubert_copy_event_create(void); /* an event without a time, behind which copies to host memory can be read */
-/* 1 when `p` is page-locked host memory (cubert_malloc_host, hipHostMalloc), which copies reach directly, else 0 */
-int cubert_is_page_locked(const void *p);
+/* 1 when `p` is ordinary host memory, which the runtime knows nothing of; 0 for NULL and for page-locked host, device and managed
+ * memory, to which it copies by itself */
+int cubert_is_pageable(const void *p);
 int cubert_event_synchronize(void *event); /* blocks the calling thread until the event has completed */
 int cubert_event_destroy(void *event);
 int cubert_event_record(void *event, void *stream);

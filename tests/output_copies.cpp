@@ -43,6 +43,7 @@ struct Copy {
 static bool g_late = false;
 static std::vector<Copy> *g_copies = nullptr;  // asked for, in order
 static size_t g_copied = 0;                    // of them carried out
+static const void *g_known = nullptr;          // an array that is not ordinary host memory
 static size_t g_events[64];                    // copies in front of each event
 
 static void carry_out(size_t until) {
@@ -69,7 +70,7 @@ int cubert_memcpy_async(void *dst, const void *src, size_t n, int kind, void *) 
     if (!g_late || kind != 2) carry_out(g_copies->size());
     return 0;
 }
-int cubert_is_page_locked(const void *) { return 0; }
+int cubert_is_pageable(const void *p) { return p != nullptr && p != g_known; }
 void *cubert_event_create(void) {
     static size_t next = 0;
     return &g_events[next++ % 64];
@@ -186,6 +187,25 @@ static void arrive() {
     }
 }
 
+// an array that only the runtime can write to: one copy, to its address
+static void leave_to_the_runtime() {
+    for (size_t batch : {2, 200}) {
+        Model m(batch);
+        Arrays a(batch);
+        cuBERT_Output o = a.output();
+        g_known = a.sequence.data();
+        m.request();
+        const size_t before = g_copies->size();
+        m.bert->output(batch, &o);
+        size_t direct = 0;
+        for (size_t i = before; i < g_copies->size(); ++i) {
+            if ((*g_copies)[i].dst == g_known) direct += (*g_copies)[i].bytes == a.sequence.size() * sizeof(float);
+        }
+        EXPECT(direct == 1);
+        a.expect_request();
+    }
+}
+
 // an output call that throws half-way, with arrays that are gone before the next one
 static void throw_half_way() {
     for (size_t batch : {1, 3, 200}) {
@@ -223,6 +243,7 @@ int main(int argc, char **argv) {
         g_late = late;
         if (what == "arrive") arrive();
         else if (what == "throw") throw_half_way();
+        else if (what == "known") leave_to_the_runtime();
         else return 2;
     }
     printf("output_copies ok\n");

@@ -779,3 +779,24 @@ def test_large_outputs_reach_pageable_and_page_locked_arrays(cb, batch, seq):
             for k, got in keep.items():
                 assert_close(got, want[k], FP32_TOL, "%s %s" % (k, locked))
     bert.close()
+
+
+def test_large_output_into_device_memory(cb):
+    """An output that is no host array is the runtime's to write, whatever its size; NULL is no ordinary memory either."""
+    from cubert_amd._lib import lib
+    from cubert_amd.testing import random_bert_weights, random_inputs
+    torch = pytest.importorskip("torch")
+    cfg = dict(vocab=211, hidden=128, layers=1, heads=4, intermediate=256, max_position=128, type_vocab=2)
+    w = random_bert_weights(seed=3, labels=2, ln_random=True, **cfg)
+    bert = cb.Bert(w, 200, 128, cfg["layers"], cfg["heads"])
+    ids, mask, seg = random_inputs(seed=1, batch=200, seq_length=128, vocab=cfg["vocab"], min_valid=1)
+    want = bert.forward(ids, mask, seg)["sequence_output"]
+    device = torch.full((200, 128, 128), float("nan"), device="cuda")
+    locked, plain = torch.empty(16, pin_memory=True), np.empty(16, np.float32)
+    assert [lib().cubert_is_pageable(p) for p in (None, device.data_ptr(), locked.data_ptr(), plain.ctypes.data)] == [0, 0, 0, 1]
+    torch.cuda.synchronize()
+    o = cb.Output()
+    o._c.sequence_output = device.data_ptr()
+    bert.output(200, o)
+    assert np.array_equal(device.cpu().numpy(), want)
+    bert.close()
