@@ -134,14 +134,6 @@ Bert<T>::Bert(const std::unordered_map<std::string, T *> &var, size_t max_batch_
         if (input_staging == nullptr) throw std::runtime_error("no page-locked host memory for the request inputs");
         output_staging = static_cast<unsigned char *>(cubert_malloc_host(kOutputStagingBytes));
         if (output_staging == nullptr) throw std::runtime_error("no page-locked host memory for the outputs");
-        if (max_batch_size * seq_length * H * sizeof(T) > kOutputStagingBytes) {
-            output_ring = static_cast<unsigned char *>(cubert_malloc_host(kOutputSlots * kOutputPieceBytes));
-            if (output_ring == nullptr) throw std::runtime_error("no page-locked host memory for the outputs");
-            for (void *&event : slot_filled) {
-                event = cubert_copy_event_create();
-                if (event == nullptr) throw std::runtime_error("no event for the output copies");
-            }
-        }
 
         for (size_t batch : open_warmup_batches(std::getenv("CUBERT_OPEN_WARMUP"), max_batch_size)) _pre_compute(batch);
     } catch (...) {
@@ -245,7 +237,7 @@ void Bert<T>::enqueue_fetch(void *dst, const void *src, size_t bytes) {
         cuBERT::memcpyAsync(output_staging + at, src, bytes, 2, stream);
         staged.push_back(StagedOutput{dst, at, bytes});
         staged_bytes = at + bytes;
-    } else if (output_ring != nullptr && cubert_is_pageable(dst)) {
+    } else if (cubert_is_pageable(dst) && have_output_ring()) {
         for (size_t done = 0; done < bytes; done += kOutputPieceBytes) {
             pieces.push_back(OutputPiece{static_cast<unsigned char *>(dst) + done, static_cast<const unsigned char *>(src) + done,
                                          bytes - done < kOutputPieceBytes ? bytes - done : kOutputPieceBytes});
@@ -253,6 +245,17 @@ void Bert<T>::enqueue_fetch(void *dst, const void *src, size_t bytes) {
     } else {
         cuBERT::memcpyAsync(dst, src, bytes, 2, stream);
     }
+}
+
+// The slots of the large outputs, made for the first of them; false: no memory, the runtime copies by itself.
+template <typename T>
+bool Bert<T>::have_output_ring() {
+    for (void *&event : slot_filled) {
+        if (event == nullptr) event = cubert_copy_event_create();
+        if (event == nullptr) return false;
+    }
+    if (output_ring == nullptr) output_ring = static_cast<unsigned char *>(cubert_malloc_host(kOutputSlots * kOutputPieceBytes));
+    return output_ring != nullptr;
 }
 
 template <typename T>

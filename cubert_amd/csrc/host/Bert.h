@@ -80,6 +80,7 @@ private:
     void synchronize();       // drains the stream
     void fetch(void *dst, const void *src, size_t bytes);  // queue one device-to-host output copy and remember it
     void enqueue_fetch(void *dst, const void *src, size_t bytes);
+    bool have_output_ring();
     void drain_pieces();      // the large outputs, piece by piece
     void finish_outputs();    // drain the stream and hand staged outputs to the caller's arrays
     void forget_outputs() noexcept;  // what is left of an output call that threw: nothing may name its caller's arrays

@@ -44,6 +44,7 @@ static bool g_late = false;
 static std::vector<Copy> *g_copies = nullptr;  // asked for, in order
 static size_t g_copied = 0;                    // of them carried out
 static const void *g_known = nullptr;          // an array that is not ordinary host memory
+static size_t g_locked_bytes = 0, g_locked_limit = (size_t) 1 << 40;  // page-locked memory: asked for so far, to be had
 static size_t g_events[64];                    // copies in front of each event
 
 static void carry_out(size_t until) {
@@ -59,7 +60,11 @@ int cubert_blas_destroy(void *h) { return std::free(h), 0; }
 int cubert_blas_set_stream(void *, void *) { return 0; }
 void *cubert_malloc(size_t n) { return std::malloc(n); }
 int cubert_free(void *p) { return std::free(p), 0; }
-void *cubert_malloc_host(size_t n) { return std::malloc(n); }
+void *cubert_malloc_host(size_t n) {
+    if (g_locked_bytes + n > g_locked_limit) return nullptr;
+    g_locked_bytes += n;
+    return std::malloc(n);
+}
 int cubert_free_host(void *p) { return std::free(p), 0; }
 int cubert_memcpy(void *dst, const void *src, size_t n, int) { return std::memcpy(dst, src, n), 0; }
 int cubert_memcpy_async(void *dst, const void *src, size_t n, int kind, void *) {
@@ -206,6 +211,29 @@ static void leave_to_the_runtime() {
     }
 }
 
+// page-locked memory for large outputs: only where one is asked for, and the runtime's copy where there is none
+static void lock_on_demand() {
+    const size_t batch = 200;
+    g_locked_bytes = 0;
+    Model m(batch);
+    Arrays a(batch);
+    cuBERT_Output o = a.output();
+    m.request();
+    m.bert->pooled_output(1, a.pooled.data());
+    EXPECT(g_locked_bytes < (1 << 20));
+    const size_t limit = g_locked_limit;
+    g_locked_limit = g_locked_bytes;
+    m.bert->output(batch, &o);
+    a.expect_request();
+    g_locked_limit = limit;
+    for (int repeat = 0; repeat < 2; ++repeat) {
+        m.request();
+        m.bert->output(batch, &o);
+        a.expect_request();
+        EXPECT(g_locked_bytes > (8 << 20) && g_locked_bytes < (9 << 20));
+    }
+}
+
 // an output call that throws half-way, with arrays that are gone before the next one
 static void throw_half_way() {
     for (size_t batch : {1, 3, 200}) {
@@ -244,6 +272,7 @@ int main(int argc, char **argv) {
         if (what == "arrive") arrive();
         else if (what == "throw") throw_half_way();
         else if (what == "known") leave_to_the_runtime();
+        else if (what == "lock") lock_on_demand();
         else return 2;
     }
     printf("output_copies ok\n");

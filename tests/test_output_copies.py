@@ -25,8 +25,9 @@ def driver(tmp_path_factory):
 
 
 # arrive: from less than a piece to several pieces and a remainder; throw: an output call that throws half-way leaves nothing that
-# names its caller's arrays, which are freed before the next call; known: what is not ordinary host memory is left to the runtime's copy
-@pytest.mark.parametrize("what", ["arrive", "throw", "known"])
+# names its caller's arrays, which are freed before the next call; known: what is not ordinary host memory is left to the runtime's copy;
+# lock: page-locked memory of some size only for a caller of large outputs, who is also served where there is none
+@pytest.mark.parametrize("what", ["arrive", "throw", "known", "lock"])
 def test_outputs(driver, what):
     run = subprocess.run([driver, what], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=300)
     assert run.returncode == 0 and "output_copies ok" in run.stdout, run.stdout[-4000:]
