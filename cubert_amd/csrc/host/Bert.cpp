@@ -235,7 +235,7 @@ void Bert<T>::enqueue_fetch(void *dst, const void *src, size_t bytes) {
     const size_t at = round_up_16(staged_bytes);
     if (output_staging != nullptr && at + bytes <= kOutputStagingBytes) {
         cuBERT::memcpyAsync(output_staging + at, src, bytes, 2, stream);
-        staged.push_back(StagedOutput{dst, at, bytes});
+        staged.push_back(StagedOutput{dst, output_staging + at, bytes});
         staged_bytes = at + bytes;
     } else if (cubert_is_pageable(dst) && have_output_ring()) {
         for (size_t done = 0; done < bytes; done += kOutputPieceBytes) {
@@ -260,6 +260,18 @@ bool Bert<T>::have_output_ring() {
 
 template <typename T>
 void Bert<T>::drain_pieces() {
+    size_t together = 0;
+    for (const OutputPiece &p : pieces) together += round_up_16(p.bytes);
+    if (together <= kOutputPieceBytes) {  // staged, as small outputs are
+        size_t at = 0;
+        for (const OutputPiece &p : pieces) {
+            cuBERT::memcpyAsync(output_ring + at, p.src, p.bytes, 2, stream);
+            staged.push_back(StagedOutput{p.dst, output_ring + at, p.bytes});
+            at += round_up_16(p.bytes);
+        }
+        pieces.clear();
+        return;
+    }
     auto request = [&](size_t i) {
         const size_t slot = i % kOutputSlots;
         cuBERT::memcpyAsync(output_ring + slot * kOutputPieceBytes, pieces[i].src, pieces[i].bytes, 2, stream);
@@ -292,7 +304,7 @@ void Bert<T>::finish_outputs() {
         synchronize();
         (void) transformer->two_term_overflowed();  // (the fp32 pass writes no two-term rows; nothing to clear)
     }
-    for (const StagedOutput &o : staged) std::memcpy(o.dst, output_staging + o.offset, o.bytes);
+    for (const StagedOutput &o : staged) std::memcpy(o.dst, o.from, o.bytes);
     staged.clear();
     staged_bytes = 0;
     requested.clear();

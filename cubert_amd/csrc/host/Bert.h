@@ -115,13 +115,18 @@ private:
     static constexpr size_t kOutputStagingBytes = 32 * 1024;
     struct StagedOutput {
         void *dst;
-        size_t offset, bytes;
+        const unsigned char *from;  // page-locked
+        size_t bytes;
     };
     unsigned char *output_staging = nullptr;
-    // Larger outputs come in pieces through two page-locked slots: while the copy engine fills one the host moves the other's
-    // piece to the caller's array.  Pieces this large because a copy costs some 20 us besides its bytes (7.3 MB through pieces of
-    // 0.5 MB 383 us, 1 MB 278, 2 MB 219, 4 MB 166; 25 MB 1218, 854, 676, 592).  A copy into pageable memory by the runtime takes
-    // 482 us for 7.3 MB and 1695 for 25.
+    // Larger outputs that fit one page-locked slot together land there in the same way: one wait for the whole call.  Waiting for
+    // an event behind each costs some 20 us more (1 x 48 tokens of 768 floats, a kept array and a new one, one layer, us a request:
+    // runtime's copy 111 / 114, events 115 / 115, one wait 94 / 94; 1 x 250 tokens 204 / 204, 208 / 207, 184 / 185; 1 x 500 tokens,
+    // 1.5 MB, 279 / 278, 277 / 270, 256 / 252).
+    // More than that comes in pieces through two such slots: while the copy engine fills one the host moves the other's
+    // piece to the caller's array.  Pieces this large because a copy costs some 20 us besides its bytes (the copy alone, repeated,
+    // 7.3 MB through pieces of 0.5 MB 383 us, 1 MB 278, 2 MB 219, 4 MB 166; 25 MB 1218, 854, 676, 592; the runtime's copy into
+    // pageable memory 482 and 1695).
     static constexpr size_t kOutputPieceBytes = 4 << 20, kOutputSlots = 2;
     unsigned char *output_ring = nullptr;
     void *slot_filled[kOutputSlots] = {};  // events
@@ -131,7 +136,7 @@ private:
         const unsigned char *src;
         size_t bytes;
     };
-    std::vector<OutputPiece> pieces;
+    std::vector<OutputPiece> pieces;     // of this call's large outputs, none longer than a slot
     size_t staged_bytes = 0;
     // every copy an output call has asked for, so that the call can be repeated after the request was recomputed
     struct RequestedOutput {

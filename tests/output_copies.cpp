@@ -45,6 +45,7 @@ static std::vector<Copy> *g_copies = nullptr;  // asked for, in order
 static size_t g_copied = 0;                    // of them carried out
 static const void *g_known = nullptr;          // an array that is not ordinary host memory
 static size_t g_locked_bytes = 0, g_locked_limit = (size_t) 1 << 40;  // page-locked memory: asked for so far, to be had
+static size_t g_records = 0;                   // of events
 static size_t g_events[64];                    // copies in front of each event
 
 static void carry_out(size_t until) {
@@ -82,7 +83,7 @@ void *cubert_event_create(void) {
 }
 void *cubert_copy_event_create(void) { return cubert_event_create(); }
 int cubert_event_destroy(void *) { return 0; }
-int cubert_event_record(void *e, void *) { return *static_cast<size_t *>(e) = g_copies->size(), 0; }
+int cubert_event_record(void *e, void *) { return ++g_records, *static_cast<size_t *>(e) = g_copies->size(), 0; }
 int cubert_event_synchronize(void *e) { return carry_out(*static_cast<size_t *>(e)), 0; }
 int cubert_event_elapsed_ms(void *, void *, float *) { return 0; }
 int cubert_time_next_launch(void *, void *) { return 0; }
@@ -178,16 +179,18 @@ struct Arrays {
     }
 };
 
-// from less than a piece to several pieces and a remainder, two requests each
+// from less than a piece to several pieces and a remainder, two requests each; what fits one slot waits for no event
 static void arrive() {
-    for (size_t batch : {1, 2, 3, 40, 127, 128, 129, 300, 384, 385}) {
+    for (size_t batch : {1, 2, 3, 40, 64, 65, 127, 128, 129, 300, 384, 385}) {
         Model m(batch);
         for (int repeat = 0; repeat < 2; ++repeat) {
             Arrays a(batch);
             cuBERT_Output o = a.output();
             m.request();
+            g_records = 0;
             m.bert->output(batch, &o);
             a.expect_request();
+            EXPECT((g_records == 0) == (2 * a.sequence.size() * sizeof(float) <= (4 << 20)));
         }
     }
 }

@@ -754,10 +754,10 @@ def test_concurrent_callers_share_one_model(cb, small_pb, monkeypatch, models_pe
     assert not errors, errors
 
 
-@pytest.mark.parametrize("batch,seq", [(1, 33), (3, 85), (64, 128), (130, 126), (200, 128)])
+@pytest.mark.parametrize("batch,seq", [(1, 33), (3, 85), (32, 128), (33, 128), (64, 128), (130, 126), (200, 128)])
 def test_large_outputs_reach_pageable_and_page_locked_arrays(cb, batch, seq):
-    """Outputs beyond the small staging block come in pieces of 4 MB through two slots: less than a piece, one whole piece, a
-    remainder, and more pieces than slots; into ordinary and into page-locked arrays, together with small ones,
+    """Outputs beyond the small staging block: together less than a slot of 4 MB, more than one (pieces through two slots), a
+    whole piece each, a remainder, and more pieces than slots; into ordinary and into page-locked arrays, together with small ones,
     twice in a row.  hidden 128 fp32: 512 bytes a token."""
     cfg = dict(vocab=211, hidden=128, layers=1, heads=4, intermediate=256, max_position=128, type_vocab=2)
     from cubert_amd.testing import random_bert_weights, random_inputs
