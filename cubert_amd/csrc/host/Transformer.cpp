@@ -387,8 +387,7 @@ static bool large_dense_is_best(int tokens, int out_features, int in_features, D
     if (tokens < 512) return false;
     switch (use) {
         case DenseUse::kPlain: return products > 7.5e8 && products <= 4.6e9 && in_features <= 1024;
-        // (just past the small kernel's 1280 tokens the library's two launches stay, as test_model_gpu.py states it for 1312)
-        case DenseUse::kGelu: return products > 1.2e9 && products <= 7e10 && (tokens <= 1280 || tokens > 1312);
+        case DenseUse::kGelu: return products > 1.2e9 && products <= 7e10;
         default: return in_features <= out_features && products <= 4.4e9 && tokens <= 8192;
     }
 }

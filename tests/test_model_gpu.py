@@ -176,10 +176,11 @@ def test_requests_of_33_to_64_tokens(cb, compute_type, seq_length, batches, mode
 
 
 @pytest.mark.parametrize("compute_type,batches", [(0, ((8, True), (10, True), (11, False))),
-                                                  (1, ((17, True), (28, True), (37, True), (40, True), (41, False)))])
+                                                  (1, ((17, True), (28, True), (37, True), (40, True), (41, True)))])
 def test_requests_around_the_switch_to_the_library(cb, compute_type, batches):
     """Two layers of BERT-base's width, 32 tokens a sequence, on either side of the token counts where a Dense layer goes
-    over to the library's GEMM (whose GELU is a launch of its own); between them some layers run on one and some on the
+    over to the library's GEMM (whose GELU is a launch of its own), or in half precision to the own kernel for large
+    requests (whose epilogue applies it); between them some layers run on one and some on the
     other.  Against the oracle, the first and the last sequences of each batch."""
     from cubert_amd.testing import random_bert_weights, random_inputs
     m = dict(vocab=97, hidden=768, layers=2, heads=12, intermediate=3072, max_position=64, type_vocab=2)
