@@ -45,6 +45,7 @@ SIGNATURES = {
     "cubert_model_info": (ci, [vp, ci, ctypes.POINTER(ci), ctypes.POINTER(ci), ctypes.POINTER(ci)]),
     "cubert_check_input_range": (ci, [vp, vp, ctypes.c_size_t, ctypes.c_size_t, ctypes.c_size_t]),
     "cubert_dense_is_best": (ci, [ci, ci, ci, ci, ci, ci]),
+    "cubert_dense_route": (ci, [ci, ci, ci, ci, ci, ci]),
     "cubert_open_warmup_batches": (cll, [ctypes.c_char_p, ctypes.c_size_t, ctypes.POINTER(ctypes.c_size_t),
                                          ctypes.c_size_t]),
     "cubert_graph_open": (ci, [ctypes.c_char_p, ci, ctypes.POINTER(vp)]),

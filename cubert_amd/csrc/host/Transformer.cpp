@@ -369,27 +369,42 @@ bool own_dense_is_best(bool half_precision, int tokens, int out_features, int in
 }
 
 // Whether a half Dense layer runs on the library's own kernel for large requests (kernels/dense_large.hip), which applies bias
-// and GELU, instead of the one for small requests or a library GEMM (with its GELU pass).  Small or library against large, us:
-//   Q|K|V           768 in: 384 tokens 6.2 / 7.2, 512 8.5 / 7.5, 1280 10.7 / 10, 2080 13.8 / 13.1, 2560 16.9 / 16.3, 3072 16.5 /
-//                   16.5, 4096 20.0 / 20.5; 1024 in: 128 4.9 / 7.8, 256 8.7 / 8.3, 1024 12.5 / 11.3, 1536 15.6 / 15.8
-//   intermediate    768 in: 384 9.0 / 8.4, 512 8.9 / 8.8, 768 13.3 / 11, 1280 17.1 / 12.3, 2080 23.7 / 19.3, 4096 33.3 / 27.0,
-//                   8192 66.3 / 52.5, 16384 104 / 94.6; 1024 in: 256 7.9 / 9.7, 384 10.7 / 10, 1024 20.4 / 14.1, 16384 157 / 152
-//   attention out   768: 1280 (small) 5.9 / 7.2, 1536 7.9 / 7.2, 2560 9.1 / 7.8, 4096 11.4 / 9.5, 4992 16.8 / 10.6, 6144 13.6 /
-//                   13.2, 8192 14.6 / 15.4; 1024: 1536 9.5 / 8.8, 4096 13.9 / 12.7, 6144 17.8 / 20.5
-//   output          3072 in: 2080 20.0 / 19.6, 2560 24.9 / 21.1, 3072 21.9 / 29.8, 4096 26.0 / 30.1: left to the library
-// other sizes      Q|K|V 128 in: 32768 tokens 12.1 / 10.6; 512: 4096 12.1 / 11.6; 1536: 512 15.4 / 16.8; intermediate 128 in:
-//                   32768 33.9 / 18.6; 512: 4096 28.6 / 20.3, 65536 223 / 203; 2048: 512 28.3 / 25.2, 2048 67.3 / 66.8; attention
-//                   out 128: 8192 5.5 / 4.6; 256: 32768 11.3 / 12.6; 512: 8192 10.0 / 8.7, 16384 14.8 / 16.5
-// (weights from the Infinity Cache; where a model's weights come from memory the small kernel, which asks for all of its operands
-// at once, is ahead for longer: requests of 256 tokens through BERT-large with Q|K|V on the large one 1070 instead of 1011 us)
+// and GELU, instead of the one for small requests or a library GEMM (with its GELU pass).  What that saves, us a layer (negative:
+// what it costs), by whole requests of 12 layers (1024 inputs: 24) with the one layer on the one kernel or the other in
+// alternation.  Against the small kernel one figure; against the library's GEMM two, hipBLASLt 1.2 of ROCm 7.2 / the copy that a
+// PyTorch for ROCm 7.0 brings and that a process uses that has loaded PyTorch first: their choices differ by more than the lines.
+//   Q|K|V           512 in: 1024 tokens -0.9, 1280 -0.3, 1408 2.3 / 4.8, 4096 0.9 / 3.8, 5120 -0.4 / 2.2; 576: 1024 1.3, 1152 -0.7,
+//                   1280 1.7; 640: 640 1.5, 3072 0.0 / 1.4, 3584 -0.8 / 0.4; 768: 512 1.5, 640 1.1, 1280 1.0, 1312 3.5 / 1.9, 2048
+//                   1.9 / 5.0, 2560 0.2 / 2.4, 2816 -0.3 / -1.2, 4096 0.4 / 0.6, 8192 -4.9 / -2.8; 1024: 512 0.8, 1152 -1.4 / 0.1,
+//                   1408 0.6 / 1.2, 2048 -1.9 / -1.2; 1536: 512 -4.6 / -1.2; 256: 16384 2.6 / 9.2; 128: 65536 13 / 5.9
+//   intermediate    512 in: 1024 -1.5, 1152 1.0, 1536 5.0 / 7.2, 3072 0.4 / 2.1, 32768 20 / 11; 640: 640 0.8; 768: 512 0.3, 768 1.0,
+//                   1280 4.2 / 3.4, 1312 6.2 / 7.3, 4096 6.8 / 8.5, 16384 16 / 11, 24576 15 / 21, 32768 14 / 12; 1024: 512 1.0, 1024
+//                   4.6 / 6.4, 2048 0.2 / 2.0, 8192 5.7 / 2.9, 14336 -1.0 / 1.4, 16384 -1.1 / 4.7, 32768 0.4 / 5.7; 1536: 512 -0.2 /
+//                   2.2, 6144 8.0 / 9.1; 2048: 512 5.9 / 4.7, 1024 -0.1 / 2.9, 2048 1.8 / 2.3, 2304 -0.9 / -2.1, 2560 -14 / -4.9, 3072
+//                   -10 / -6.2, 4096 1.1 / 5.4; 256: 8192 3.8 / 5.4; 128: 32768 14 / 9.6
+//   attention out   512 in: 1280 -2.3, 1408 0.8 / 2.3, 3072 -0.5 / 0.9, 4096 -0.5 / 1.9, 8192 0.4 / 2.4, 16384 -4.1 / -0.8; 640: 3072
+//                   0.8 / 1.8, 3584 -0.8 / 0.3, 8192 -0.1 / 1.7; 768: 1280 -0.6, 1312 1.7 / 0.5, 2048 1.2 / 1.8, 2688 1.0 / 1.5, 3072
+//                   -1.1 / 0.8, 4096 -0.5 / 1.5, 4992 -0.1 / 1.6, 6144 -0.7 / 1.6, 12288 -2.9 / 8.0, 20480 -3.4 / -4.4; 896: 1408
+//                   -0.5 / 1.5, 2048 0.6 / 2.6; 1024: 1312 0.2 / 3.4, 1536 -1.0 / 2.5, 2048 0.2 / 2.8, 4096 -0.8 / 2.4, 6144 -1.7 /
+//                   -0.5; 256: 8192 1.5 / 3.9; 128: 8192 2.4 / 1.2
+//   output          3072 in: 1536 -1.8 / -1.4, 2048 -1.3 / -0.5, 2560 -0.2 / 0.5, 4096 -2.7 / -3.0, 8192 -7.2 / -6.7: left to the library
+// The lines are where the sum of the two changes sign.
 static bool large_dense_is_best(int tokens, int out_features, int in_features, DenseUse use) {
     const double products = (double) tokens * out_features * in_features;
     if (tokens < 512) return false;
     switch (use) {
-        case DenseUse::kPlain: return products > 7.5e8 && products <= 4.6e9 && in_features <= 1024;
-        case DenseUse::kGelu: return products > 1.2e9 && products <= 7e10;
+        // (narrow layers: the small kernel is ahead for all of its 1280 tokens)
+        case DenseUse::kPlain: return products > 7.5e8 && products <= 4.6e9 && in_features <= 1024 && (in_features > 512 || tokens > 1280);
+        case DenseUse::kGelu: return products > 1.2e9 && products <= (in_features <= 1536 ? 7e10 : 3.5e10);
         default: return in_features <= out_features && products <= 4.4e9 && tokens <= 8192;
     }
+}
+
+DenseRoute dense_route(bool half_precision, int tokens, int out_features, int in_features, DenseUse use, bool as_slices) {
+    const bool small = own_dense_is_best(half_precision, tokens, out_features, in_features, use, as_slices);
+    const bool large = half_precision && !(small && use == DenseUse::kNorm) &&
+                       large_dense_is_best(tokens, out_features, in_features, use);
+    return large ? DenseRoute::kLarge : small ? DenseRoute::kSmall : DenseRoute::kOther;
 }
 
 // CUBERT_FEW_TOKEN_SLICES=0 in the environment keeps the Dense kernels of small requests adding their own K slices.
@@ -408,10 +423,10 @@ static DenseUse use_of(Profiler::Kind kind) {
 }
 
 template <typename T>
-bool Transformer<T>::own_dense_takes(int tokens, int out_features, int in_features, Profiler::Kind kind) const {
-    if (!own_dense) return false;
-    return own_dense_is_best(sizeof(T) == 2, tokens, out_features, in_features, use_of(kind),
-                             own_slices_to_norm && few_token_slices_enabled());
+DenseRoute Transformer<T>::route_of(int tokens, int out_features, int in_features, Profiler::Kind kind) const {
+    if (!own_dense) return DenseRoute::kOther;
+    return dense_route(sizeof(T) == 2, tokens, out_features, in_features, use_of(kind),
+                       own_slices_to_norm && few_token_slices_enabled());
 }
 
 // One Dense layer.  The bias goes into the GEMM only where the caller asks for it (bias_in_gemm: the Q/K/V
@@ -423,18 +438,15 @@ bool Transformer<T>::dense(int out_features, int tokens, int in_features, const 
     void *stream = cuBERT::blas_get_stream(cublas);
     Timed t(profiler, profiler != nullptr ? profiler->dense_kind(kind) : Profiler::kDenseGemm, stream);
     if (ld_out == 0) ld_out = out_features;
-    const bool small = own_dense_takes(tokens, out_features, in_features, kind);
+    const DenseRoute route = route_of(tokens, out_features, in_features, kind);
     if constexpr (sizeof(T) == 2) {
-        const DenseUse use = use_of(kind);
-        if (own_dense && !(small && use == DenseUse::kNorm) && large_dense_is_best(tokens, out_features, in_features, use)) {
-            const bool with_bias = bias_in_gemm || gelu;
-            if (cuBERT::dense_large(tokens, out_features, in_features, in, kernel, with_bias ? bias : nullptr, gelu, out, ld_out,
-                                    stream)) {
-                return with_bias;
-            }
+        const bool with_bias = bias_in_gemm || gelu;
+        if (route == DenseRoute::kLarge && cuBERT::dense_large(tokens, out_features, in_features, in, kernel,
+                                                               with_bias ? bias : nullptr, gelu, out, ld_out, stream)) {
+            return with_bias;
         }
     }
-    if (small) {
+    if (route == DenseRoute::kSmall) {
         const bool with_bias = bias_in_gemm || gelu;
         if (cuBERT::dense_mid(tokens, out_features, in_features, in, in_features, kernel,
                               transposed_kernels ? in_features : out_features, with_bias ? bias : nullptr, gelu, out, ld_out,
@@ -525,7 +537,7 @@ void Transformer<T>::dense_norm(int tokens, int in_features, const T *kernel, co
                                 const T *residual, const T *beta, const T *gamma, T *out, Profiler::Kind kind) {
     void *stream = cuBERT::blas_get_stream(cublas);
     const int H = (int) hidden_size;
-    if (own_dense_takes(tokens, H, in_features, kind) && own_slices_to_norm && few_token_slices_enabled()) {
+    if (route_of(tokens, H, in_features, kind) == DenseRoute::kSmall && own_slices_to_norm && few_token_slices_enabled()) {
         int slices = 0;
         bool done = false;
         {

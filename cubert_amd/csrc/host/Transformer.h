@@ -4,15 +4,16 @@
 // with device pointers, returning a device pointer to [batch, seq, hidden].
 //
 // Inside, a layer is 8 launches (7 for small requests, whose intermediate Dense applies its GELU and whose two Dense
-// layers in front of a LayerNorm may leave their K slices to it; which of the own Dense kernel, the few-token kernel and
-// the library's GEMM a layer runs on: own_dense_is_best, few_token_limit):
+// layers in front of a LayerNorm may leave their K slices to it, and for large half ones, whose intermediate Dense applies its
+// GELU too; which of the own Dense kernels, the few-token kernel and the library's GEMM a layer runs on: dense_route,
+// few_token_limit):
 //   qkv   = x * [Wq|Wk|Wv] + [bq|bk|bv]          one GEMM, bias in its epilogue
 //   ctx   = softmax((1/sqrt d) Q K^T + mask) V    one attention kernel (scores stay in registers); where its
 //                                                 shape limits do not hold: scores kernel or batched GEMM into
 //                                                 scores[B, A, S, S], mask_scale_softmax_, context kernel or GEMM
 //   a     = LN(ctx * Wo + bo + x)                 GEMM, then layer_norm_   (fused kernel)
-//   i     = GELU(a * Wi + bi)                     GEMM, then gelu          (fused kernel; one launch for both in
-//                                                 small requests)
+//   i     = GELU(a * Wi + bi)                     GEMM, then gelu          (fused kernel; one launch for both on
+//                                                 the own Dense kernels)
 //   out   = LN(i * Wout + bout + a)               GEMM, then layer_norm_   (fused kernel)
 // Activation buffers are shared by all layers (the reference keeps four private
 // buffers per layer); weights live in one device allocation.  A half-precision model of seq_length
@@ -43,8 +44,12 @@ namespace cuBERT {
 // What follows a Dense layer: nothing (its bias is added in the GEMM), bias + GELU, or bias + residual + LayerNorm.
 enum class DenseUse { kPlain, kGelu, kNorm };
 
-// Whether the library's own Dense kernel is the best one for a layer of this size whose sizes it takes; as_slices: the
+// What a Dense layer of this size runs on where its sizes are whole steps of the own Dense kernels: the one for small requests
+// (kernels/dense_mid.hip), the one for large requests (dense_large.hip), or the few-token kernel or a library GEMM; as_slices: the
 // LayerNorm that follows can add K slices.
+enum class DenseRoute { kOther, kSmall, kLarge };
+DenseRoute dense_route(bool half_precision, int tokens, int out_features, int in_features, DenseUse use, bool as_slices);
+// ... and whether the one for small requests is better than the few-token kernel and the library's GEMM
 bool own_dense_is_best(bool half_precision, int tokens, int out_features, int in_features, DenseUse use, bool as_slices);
 
 template <typename T>
@@ -135,8 +140,8 @@ private:
     void dense_norm(int tokens, int in_features, const T *kernel, const T *packed, const T *in, const T *bias,
                     const T *residual, const T *beta, const T *gamma, T *out, Profiler::Kind kind);
 
-    // own_dense_is_best for a layer of this model
-    bool own_dense_takes(int tokens, int out_features, int in_features, Profiler::Kind kind) const;
+    // dense_route for a layer of this model
+    DenseRoute route_of(int tokens, int out_features, int in_features, Profiler::Kind kind) const;
 
     // up to how many tokens the Dense layer of this kind runs on the few-token kernel (32 or 64)
     int few_token_limit(Profiler::Kind kind) const;

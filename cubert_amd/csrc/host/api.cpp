@@ -441,6 +441,10 @@ int cubert_dense_is_best(int dtype, int tokens, int out_features, int in_feature
     return cuBERT::own_dense_is_best(dtype == 1, tokens, out_features, in_features, (cuBERT::DenseUse) use, as_slices != 0);
 }
 
+int cubert_dense_route(int dtype, int tokens, int out_features, int in_features, int use, int as_slices) {
+    return (int) cuBERT::dense_route(dtype == 1, tokens, out_features, in_features, (cuBERT::DenseUse) use, as_slices != 0);
+}
+
 int cubert_graph_open(const char *model_file, int dtype, void **graph) {
     return guarded([&] {
         if (graph == nullptr || model_file == nullptr) throw std::invalid_argument("null argument");

@@ -62,10 +62,13 @@ int cubert_check_input_range(const int *input_ids, const int8_t *segment_ids, si
  * max_batch_size, e.g. "1,8,max".  Entries outside [1, max_batch_size] are named on stderr and skipped.  Writes up
  * to `capacity` sizes to `batches` in the order they will run and returns how many there are.  CPU only. */
 long long cubert_open_warmup_batches(const char *setting, size_t max_batch_size, size_t *batches, size_t capacity);
-/* 1 where a model runs a Dense layer of this size on cubert_dense_* / cubert_dense_slices_* rather than on cubert_gemm_* or
- * the few-token kernel (dtype as below; use: 0 = bias only, 1 = bias + GELU follow, 2 = bias + residual + LayerNorm
+/* 1 where cubert_dense_* / cubert_dense_slices_* is a better choice for a Dense layer of this size than cubert_gemm_* or the
+ * few-token kernel (dtype as below; use: 0 = bias only, 1 = bias + GELU follow, 2 = bias + residual + LayerNorm
  * follow; as_slices: that LayerNorm takes K slices), 0 otherwise.  CPU only. */
 int cubert_dense_is_best(int dtype, int tokens, int out_features, int in_features, int use, int as_slices);
+/* What a model runs such a layer on: 1 = cubert_dense_* / cubert_dense_slices_*, 2 = cubert_dense_large_f16, 0 = cubert_gemm_* or
+ * the few-token kernel.  CPU only. */
+int cubert_dense_route(int dtype, int tokens, int out_features, int in_features, int use, int as_slices);
 /* replaces: cuBERT_close, reference src/cuBERT.cpp:92-102 */
 int cubert_try_close(void *model, int compute_type);
 /* Shape facts of an opened model (hidden size, labels, seq_length) for sizing output arrays. */

@@ -330,16 +330,46 @@ def test_which_dense_layers_keep_to_short_sums():
 
 
 @pytest.mark.parametrize("dtype,use,layer,last,first", [
-    # the last token count measured ahead of the library's GEMM and the first one measured behind it
+    # the last token count at which the own kernel for small requests measured ahead of the library's GEMM and the first behind it
     (1, 0, (768, 2304), 896, 1024), (1, 0, (1024, 3072), 512, 640), (1, 0, (1536, 4608), 128, 320), (1, 0, (512, 1536), 1280, 1281), (1, 0, (640, 1920), 1024, 1152),
     (1, 2, (1024, 1024), 1280, 1281), (1, 2, (1536, 1536), 640, 768), (1, 2, (2048, 2048), 320, 640),
     (1, 1, (768, 3072), 1280, 1281), (1, 1, (1024, 4096), 640, 1280), (1, 2, (3072, 768), 1280, 1281),
     (0, 0, (768, 2304), 264, 300), (0, 0, (1024, 3072), 128, 160), (0, 2, (768, 768), 320, 321),
     (0, 1, (768, 3072), 320, 321), (0, 1, (1024, 4096), 160, 320), (0, 2, (3072, 768), 256, 320)])
 def test_where_the_library_gemm_takes_over(dtype, use, layer, last, first):
+    """... from the own kernel for small requests; the one for large ones, where that is ahead of both, is in the next test."""
     from cubert_amd._lib import lib
     best = lib().cubert_dense_is_best
     assert best(dtype, last, layer[1], layer[0], use, 1) and not best(dtype, first, layer[1], layer[0], use, 1)
+
+
+OTHER, SMALL, LARGE = 0, 1, 2
+
+
+@pytest.mark.parametrize("use,layer,expected", [
+    # Q|K|V: the small kernel, then the large one, then the library
+    (0, (512, 1536), ((953, SMALL), (1280, SMALL), (1281, LARGE), (5849, LARGE), (5850, OTHER))),
+    (0, (576, 1728), ((753, SMALL), (754, LARGE), (1281, LARGE))),
+    (0, (768, 2304), ((511, SMALL), (512, LARGE), (1312, LARGE), (2599, LARGE), (2600, OTHER))),
+    (0, (1024, 3072), ((511, SMALL), (512, LARGE), (1462, LARGE), (1463, OTHER))),
+    (0, (1536, 4608), ((128, SMALL), (512, OTHER), (4096, OTHER))),
+    (0, (128, 384), ((1281, OTHER), (15258, OTHER), (15259, LARGE), (93587, LARGE), (93588, OTHER))),
+    # intermediate, with GELU
+    (1, (512, 2048), ((1144, SMALL), (1145, LARGE), (66757, LARGE), (66758, OTHER))),
+    (1, (768, 3072), ((511, SMALL), (512, LARGE), (1280, LARGE), (1281, LARGE), (1312, LARGE), (1313, LARGE), (29669, LARGE), (29670, OTHER))),
+    (1, (1536, 6144), ((511, OTHER), (512, LARGE), (7417, LARGE), (7418, OTHER))),
+    (1, (2048, 8192), ((511, OTHER), (512, LARGE), (2086, LARGE), (2087, OTHER), (3072, OTHER))),
+    # attention output: the small kernel as long as that is ahead
+    (2, (512, 512), ((1280, SMALL), (1281, LARGE), (8192, LARGE), (8193, OTHER))),
+    (2, (768, 768), ((1280, SMALL), (1281, LARGE), (7459, LARGE), (7460, OTHER))),
+    (2, (1024, 1024), ((1280, SMALL), (1281, LARGE), (4196, LARGE), (4197, OTHER))),
+    # output: never
+    (2, (3072, 768), ((1280, SMALL), (1281, OTHER), (4096, OTHER)))])
+def test_what_half_dense_layers_run_on(use, layer, expected):
+    from cubert_amd._lib import lib
+    for tokens, route in expected:
+        assert lib().cubert_dense_route(1, tokens, layer[1], layer[0], use, 1) == route, tokens
+        assert lib().cubert_dense_route(0, tokens, layer[1], layer[0], use, 1) != LARGE
 
 
 def test_the_dense_tests_run_every_tile_a_model_does():
