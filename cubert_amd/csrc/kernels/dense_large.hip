@@ -30,17 +30,6 @@ constexpr int kRowBytes = 128;             // of a row of X or W that a step tak
 constexpr int kHalfStep = kRowBytes / 2;   // values of K in them
 constexpr int kPairStep = kRowBytes / 4;
 
-// 16 bytes per lane from memory to LDS at `base` + 16 * lane, without passing through registers
-__device__ __forceinline__ void load_to_lds(const void *src, void *base) {
-    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *) src,
-                                     (__attribute__((address_space(3))) void *) base, 16, 0, 0);
-}
-
-template <int N>
-__device__ __forceinline__ void wait_loads() {  // at most N vector-memory requests of this wavefront outstanding
-    __builtin_amdgcn_s_waitcnt(0x0f70 | (N & 15) | ((N >> 4) << 14));
-}
-
 // the LDS accesses of this wavefront in front of it are done before those behind it start
 __device__ __forceinline__ void order_lds() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 

@@ -27,17 +27,6 @@ constexpr int kMidWaves = 4;
 constexpr int kMidThreads = kMidWaves * kWave;
 constexpr int kStepBytes = 128;  // of a row of X that a wavefront consumes per step
 
-// 16 bytes per lane from memory to LDS at `base` + 16 * lane, without passing through registers
-__device__ __forceinline__ void load_to_lds(const void *src, void *base) {
-    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *) src,
-                                     (__attribute__((address_space(3))) void *) base, 16, 0, 0);
-}
-
-template <int N>
-__device__ __forceinline__ void wait_loads() {  // at most N vector-memory requests of this wavefront outstanding
-    __builtin_amdgcn_s_waitcnt(0x0f70 | (N & 15) | ((N >> 4) << 14));
-}
-
 template <typename T, int TM, int TN, int DEPTH>
 struct MidShape {
     static constexpr int kStep = kStepBytes / sizeof(T);           // K values per step

@@ -31,6 +31,17 @@ __device__ __forceinline__ void store_vec(T *p, const Vec<T, N> &x) {
     *reinterpret_cast<Vec<T, N> *>(p) = x;
 }
 
+// 16 bytes per lane from memory to LDS at `base` + 16 * lane, without passing through registers
+__device__ __forceinline__ void load_to_lds(const void *src, void *base) {
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *) src,
+                                     (__attribute__((address_space(3))) void *) base, 16, 0, 0);
+}
+
+template <int N>
+__device__ __forceinline__ void wait_loads() {  // at most N vector-memory requests of this wavefront outstanding
+    __builtin_amdgcn_s_waitcnt(0x0f70 | (N & 15) | ((N >> 4) << 14));
+}
+
 __device__ __forceinline__ float to_f32(float x) { return x; }
 __device__ __forceinline__ float to_f32(half_t x) { return (float) x; }
 
