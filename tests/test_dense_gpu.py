@@ -210,7 +210,7 @@ def test_dense_pairs_overflow_and_refusals(K):
     bias = torch.full((96,), 4000.0, device="cuda")
     assert K.dense_pairs(xs, ws, bias, True, 1 / 256, 16.0, overflow=flag) is not None
     torch.cuda.synchronize()
-    assert int(flag.item()) == 0       # 16 * 4000 fits, also in the rows of a tile that are past the last token
+    assert int(flag.item()) == 0       # 16 * 4000 fits
     bias[95] = 4100.0
     assert K.dense_pairs(xs, ws, bias, True, 1 / 256, 16.0, overflow=flag) is not None
     torch.cuda.synchronize()
@@ -218,6 +218,26 @@ def test_dense_pairs_overflow_and_refusals(K):
     assert K.dense_pairs(xs, ws[:94].contiguous(), None, True) is None      # rows of pairs need whole blocks of 32
     assert K.dense_pairs(xs, ws[:94].contiguous(), None) is None            # four features per store
     assert K.dense_pairs(xs, ws, None, ldo=98) is None
+
+
+@pytest.mark.parametrize("tokens,features,width,tile", [(4000, 2976, 128, 0), (900, 3104, 64, 1), (70, 32, 64, 2), (900, 3008, 768, 3),
+                                                        (70, 32, 256, 4)])
+def test_dense_pairs_overflow_past_the_last_feature(K, tokens, features, width, tile):
+    """Past the last feature a tile multiplies that feature's weights again, without its bias: a sum that only the bias brings
+    into range does not raise the flag there, whatever the tile."""
+    number, _, tile_features = K.dense_large_plan(True, tokens, features, width, True)
+    assert number == tile and features % tile_features != 0
+    flag = torch.zeros(1, dtype=torch.int32, device="cuda")
+    x, w, bias = torch.ones(tokens, width, device="cuda"), torch.zeros(features, width, device="cuda"), torch.zeros(features, device="cuda")
+    w[-1] = 8192.0 / width  # 16 * 8192 is out of range
+    xs, ws = K.split_pairs(x, 16.0), K.split_pairs(w, 16.0)
+    for last, raised in ((-6144.0, 0), (0.0, 1)):
+        bias[-1] = last
+        out = K.dense_pairs(xs, ws, bias, True, 1 / 256, 16.0, overflow=flag)
+        torch.cuda.synchronize()
+        assert int(flag.item()) == raised
+        if not raised:
+            assert bool((out[:, 2 * features - 33] == 16 * 2048.0).all())  # the last feature's high terms
 
 
 # ---- large requests: half operands ----------------------------------------------------------------------------
@@ -255,3 +275,36 @@ def test_dense_large_tiles_and_refusals(K):
     assert K.dense_large(x, w, ldo=68) is None
     base = torch.zeros(64 * 128 + 1, dtype=torch.float16, device="cuda")
     assert K.dense_large(base[1:].view(64, 128), w) is None                       # 16-byte requests
+
+
+def _beyond(out, tokens, features):
+    """What a launch has left in the rows behind the last token and in the columns between `features` and the row pitch."""
+    return torch.cat([out[tokens:].flatten(), out[:tokens, features:].flatten()])
+
+
+# (256 rows more than there are tokens: what any tile could write to)
+@pytest.mark.parametrize("gelu", [False, True])
+@pytest.mark.parametrize("tokens,features,width", PAIR_SHAPES)
+def test_dense_pairs_writes_nothing_else(K, tokens, features, width, gelu):
+    from cubert_amd._lib import lib
+    features = (features + 31) // 32 * 32 if gelu else features
+    ldo = features if gelu else features + 200
+    out = torch.full((tokens + 256, ldo), 7.0, device="cuda")
+    x = K.split_pairs(torch.ones(tokens, width, device="cuda"), 16.0)
+    w = K.split_pairs(torch.full((features, width), 3.0, device="cuda"), 16.0)
+    assert lib().cubert_dense_pairs_f32(torch.cuda.current_stream().cuda_stream, tokens, features, width, x.data_ptr(), w.data_ptr(), None,
+                                        int(gelu), 1 / 256, 16.0, out.data_ptr(), ldo, None) == 0
+    assert bool((_beyond(out, tokens, features) == 7).all()) and not bool((out[:tokens, :features] == 7).any())
+
+
+@pytest.mark.parametrize("gelu", [False, True])
+@pytest.mark.parametrize("tokens,features,width", LARGE_SHAPES)
+def test_dense_large_writes_nothing_else(K, tokens, features, width, gelu):
+    from cubert_amd._lib import lib
+    ldo = features + 264
+    out = torch.full((tokens + 256, ldo), 7.0, dtype=torch.float16, device="cuda")
+    x = torch.ones(tokens, width, dtype=torch.float16, device="cuda")
+    w = torch.full((features, width), 3.0, dtype=torch.float16, device="cuda")
+    assert lib().cubert_dense_large_f16(torch.cuda.current_stream().cuda_stream, tokens, features, width, x.data_ptr(), w.data_ptr(), None,
+                                        int(gelu), out.data_ptr(), ldo) == 0
+    assert bool((_beyond(out, tokens, features) == 7).all()) and bool((out[:tokens, :features] == 3 * width).all())
