@@ -51,46 +51,46 @@ TRAFFIC_PROFILE = "profiles/traffic_pmc.md"
 TRAFFIC_SOURCE = {  # kernel kind -> (source file under cubert_amd/csrc/kernels, first 16 hex digits of its SHA-256)
     "bias_gelu": ("elementwise.hip", "59dcc33f61344079"),
     "bias_tanh": ("elementwise.hip", "59dcc33f61344079"),
-    "bias_res_ln": ("layernorm.hip", "63cfef94a6b85850"),
-    "embed_ln": ("layernorm.hip", "63cfef94a6b85850"),
+    "bias_res_ln": ("layernorm.hip", "560bea195e2fb7ea"),
+    "embed_ln": ("layernorm.hip", "560bea195e2fb7ea"),
     "mask_scale_softmax": ("softmax.hip", "90a529eac55169fa"),
     "mean_pool": ("elementwise.hip", "59dcc33f61344079"),
     "classifier_head": ("elementwise.hip", "59dcc33f61344079"),
-    "attention_fused": ("attention.hip", "4d44df3fda986cf4"),
+    "attention_fused": ("attention.hip", "af161662ae4c499d"),
 }
 MEASURED_TRAFFIC = {
     "C1": {
-        "embed_ln": 25327834,
-        "attention_fused": 50081947,
-        "bias_res_ln": 37631060,
-        "bias_gelu": 100340726,
-        "classifier_head": 934419,
-        "mask_scale_softmax": 12589780
+        "embed_ln": 25320144,
+        "attention_fused": 50085885,
+        "bias_res_ln": 37630949,
+        "bias_gelu": 100340646,
+        "classifier_head": 934323,
+        "mask_scale_softmax": 12589727
     },
     "C2": {
-        "embed_ln": 12897102,
-        "attention_fused": 25138619,
-        "bias_res_ln": 18850804,
-        "bias_gelu": 50185082,
-        "mean_pool": 6325077,
-        "classifier_head": 147249,
-        "mask_scale_softmax": 25117480
+        "embed_ln": 12907297,
+        "attention_fused": 25138702,
+        "bias_res_ln": 18866010,
+        "bias_gelu": 50185812,
+        "mean_pool": 6325424,
+        "classifier_head": 147198,
+        "mask_scale_softmax": 25117472
     },
     "C3": {
-        "embed_ln": 99732176,
-        "attention_fused": 128669549,
-        "bias_res_ln": 150191566,
-        "bias_gelu": 400908911,
-        "classifier_head": 308694,
-        "mask_scale_softmax": 801926098
+        "embed_ln": 99598184,
+        "attention_fused": 124666044,
+        "bias_res_ln": 150205903,
+        "bias_gelu": 400907571,
+        "classifier_head": 308598,
+        "mask_scale_softmax": 801925456
     },
     "C4": {
-        "embed_ln": 133757147,
-        "attention_fused": 267267773,
-        "bias_res_ln": 200203032,
-        "bias_gelu": 534519157,
-        "classifier_head": 1199518,
-        "mask_scale_softmax": 267503966
+        "embed_ln": 133692287,
+        "attention_fused": 267267510,
+        "bias_res_ln": 200204325,
+        "bias_gelu": 534518728,
+        "classifier_head": 1199422,
+        "mask_scale_softmax": 267503753
     }
 }
 
@@ -127,10 +127,13 @@ def algorithmic_bytes(cfg):
     H, I, A = m["hidden"], m["intermediate"], m["heads"]
     e = 4 if cfg["dtype"] == "f32" else 2
     M = B * S
-    if two_term_dense() and e == 4 and M >= 384:
-        # The LayerNorm also writes rows of pairs.  Passes that only the library's form of the Dense layers has: bias+GELU reads
-        # fp32 and writes [hi | hi | lo] fp16 rows, and so does the split.
-        extra = {"bias_gelu": M * I * (4 + 6) + I * 4, "bias_res_ln": 3 * M * H * 4 + 3 * H * 4 + 4 * M * H,
+    if two_term_dense() and e == 4 and M >= 384 and H % 32 == 0 and I % 32 == 0 and \
+            os.environ.get("CUBERT_GEMM") not in ("library", "naive"):
+        # the own Dense kernel: the LayerNorm and the split also write rows of pairs, bias+GELU is in the Dense launch
+        extra = {"bias_res_ln": 3 * M * H * 4 + 3 * H * 4 + 4 * M * H, "dense_split": M * H * (4 + 4)}
+    elif two_term_dense() and e == 4 and M >= 384:
+        # the library's GEMM: LayerNorm, bias+GELU and split write [hi | hi | lo] fp16 rows
+        extra = {"bias_gelu": M * I * (4 + 6) + I * 4, "bias_res_ln": 3 * M * H * 4 + 3 * H * 4 + 6 * M * H,
                  "dense_split": M * H * (4 + 6)}
     else:
         extra = {}

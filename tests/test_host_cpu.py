@@ -304,12 +304,20 @@ def test_bench_algorithmic_bytes_follow_the_published_formulas():
                                            ("C4", 536.9, 201.3, 268.5, 134.7)):
         assert abs(mb[name]["bias_gelu"] - gelu) < 0.06 and abs(mb[name]["bias_res_ln"] - ln) < 0.06
         assert abs(mb[name]["mask_scale_softmax"] - softmax) < 0.06 and abs(mb[name]["embed_ln"] - embed) < 0.06
+    kept = os.environ.pop("CUBERT_GEMM", None)
     os.environ["CUBERT_FP32_DENSE"] = "f16x3"
     try:
-        two_term = bench.algorithmic_bytes(CONFIGS["C1"])
+        pairs = bench.algorithmic_bytes(CONFIGS["C1"])
         half_model = bench.algorithmic_bytes(CONFIGS["C3"])
+        os.environ["CUBERT_GEMM"] = "library"
+        two_term = bench.algorithmic_bytes(CONFIGS["C1"])
     finally:
-        del os.environ["CUBERT_FP32_DENSE"]
+        del os.environ["CUBERT_FP32_DENSE"], os.environ["CUBERT_GEMM"]
+        if kept is not None:
+            os.environ["CUBERT_GEMM"] = kept
+    # on the own kernel every term is written once and GELU is no pass of its own; on the library's GEMM the high term twice
+    assert pairs["bias_gelu"] == 2 * 4096 * 3072 * 4 + 3072 * 4 and pairs["dense_split"] == 4096 * 768 * 8
+    assert pairs["bias_res_ln"] == 4096 * 768 * 16 + 768 * 12 and two_term["bias_res_ln"] == 4096 * 768 * 18 + 768 * 12
     assert two_term["bias_gelu"] == 4096 * 3072 * 10 + 3072 * 4 and two_term["dense_split"] == 4096 * 768 * 10
     assert half_model["bias_gelu"] == bench.algorithmic_bytes(CONFIGS["C3"])["bias_gelu"]  # fp16 models: unchanged
 
