@@ -124,9 +124,10 @@ private:
     // runtime's copy 111 / 114, events 115 / 115, one wait 94 / 94; 1 x 250 tokens 204 / 204, 208 / 207, 184 / 185; 1 x 500 tokens,
     // 1.5 MB, 279 / 278, 277 / 270, 256 / 252).
     // More than that comes in pieces through two such slots: while the copy engine fills one the host moves the other's
-    // piece to the caller's array.  Pieces this large because a copy costs some 20 us besides its bytes (the copy alone, repeated,
-    // 7.3 MB through pieces of 0.5 MB 383 us, 1 MB 278, 2 MB 219, 4 MB 166; 25 MB 1218, 854, 676, 592; the runtime's copy into
-    // pageable memory 482 and 1695).
+    // piece to the caller's array.  Pieces this large because a copy costs some 20 us besides its bytes (the copies by themselves,
+    // in a loop, 7.3 MB through pieces of 0.5 MB 383 us, 1 MB 278, 2 MB 219, 4 MB 166; 25 MB 1218, 854, 676, 592; the runtime's copy
+    // into pageable memory 482 and 1695).  In an output call 7.7 MB take 355 us (runtime's copy some 450): 86 until the first piece has
+    // come, at 49 GB/s, then 150 and 114 for the host to move the two, at 28 to 30 GB/s, which is what bounds it.
     static constexpr size_t kOutputPieceBytes = 4 << 20, kOutputSlots = 2;
     unsigned char *output_ring = nullptr;
     void *slot_filled[kOutputSlots] = {};  // events

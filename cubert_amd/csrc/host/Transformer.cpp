@@ -588,8 +588,10 @@ T *Transformer<T>::_in_compute(size_t batch_size, T *input_gpu, int8_t *attentio
     void *stream = cuBERT::blas_get_stream(cublas);
     const int M = (int) (batch_size * seq_length), H = (int) hidden_size, I = (int) intermediate_size;
 
-    // (small requests are bound by the pass over the weights, which are 6 bytes per parameter in two-term form and 4
-    // in fp32: they keep the fp32 kernels)
+    // (Below 384 tokens the fp32 kernels stay: the tiles of the two-term kernel are too few to fill the chip, and a request takes
+    // what it takes at 300 tokens.  BERT-base, us a request, two-term / fp32: 128 tokens 942 / 639, 256 954 / 827, 320 967 / 912, 384
+    // 1025 / 1135, 640 1147 / 1334; BERT-large 384 2555 / 2734; hidden 512 384 714 / 748.  On the library's GEMM 256 1019, 320 1012,
+    // 384 1150.)
     const bool split = split_dense && (size_t) M >= kTwoTermMinTokens && !fp32_dense_once;
     fp32_dense_once = false;
     bool operand_ready = false;

@@ -21,9 +21,10 @@
 // GEMM kernel's own order.
 //
 // CUBERT_FP32_DENSE=f16x3 in the environment when an fp32 model is opened makes its Dense layers run on the fp16
-// matrix cores for requests of at least 384 tokens (measured break-even at BERT-base: below it the GEMMs are bound
-// by reading the weights, and two-term weights are the larger ones): every fp32 operand is written as the sum of two fp16 numbers and the
-// product as hi*hi + hi*lo + lo*hi with fp32 accumulation (one GEMM over three times the reduction length), which
+// matrix cores for requests of at least 384 tokens (measured break-even, _in_compute): every fp32 operand is written as the sum of
+// two fp16 numbers and the product as hi*hi + hi*lo + lo*hi with fp32 accumulation (one pass of the own kernel for large requests,
+// kernels/dense_large.hip, which also applies GELU; for layer sizes that are no multiple of 32 one library GEMM over three times the
+// reduction length), which
 // keeps the error of an fp32 GEMM for activations up to 2^12 in size (see kernels/split.hip).
 // Everything between the GEMMs stays fp32.  The default is the fp32 GEMM.
 #ifndef CUBERT_HOST_TRANSFORMER_H
