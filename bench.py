@@ -456,7 +456,7 @@ def main():
     roofline = {"bound": "hbm", "kernel": dominant, "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic, "traffic_source": traffic_source,
                 "algorithmic_bytes_per_launch": alg[dominant], "avg_launch_us": round(avg_us, 2), "launches": launches,
-                "timing": EVENT_PAIR_NOTE + "; launches inside the timed steps"}
+                "timing": EVENT_PAIR_NOTE + "; launches inside the timed steps" if dominant in prof else alone["note"]}
 
     # ---- every kernel kind, in extra untimed passes (reported, not part of `value`)
     table_passes = max(5, args.steps // 5)
@@ -605,7 +605,8 @@ def main():
     if concurrent is not None:
         line["concurrent_instances"] = concurrent
     for k, row in kernels.items():
-        row["traffic"], _ = recorded_traffic(args.workload, k)
+        # (no counter values are recorded for the two-term form, whose kernels move other bytes)
+        row["traffic"] = None if two_term_dense() and not half else recorded_traffic(args.workload, k)[0]
     line["kernels"] = kernels
     line["kernel_timing"] = EVENT_PAIR_NOTE
     line["gemm"] = gemm
