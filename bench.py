@@ -116,7 +116,7 @@ def recorded_traffic(workload, kind):
 
 def two_term_dense():
     """CUBERT_FP32_DENSE=f16x3 in the environment: fp32 models run their Dense layers (requests of at least 384 tokens) on the
-    fp16 matrix cores from two-term operands (opt-in; the default is the fp32 GEMM)."""
+    fp16 matrix cores from two-term operands (as models opened without the variable do; this bench's `value` is the fp32 GEMM)."""
     return os.environ.get("CUBERT_FP32_DENSE") == "f16x3"
 
 
@@ -379,7 +379,7 @@ def main():
                     help="instead of the model: 10 launches of a plain row copy of known size (100 MB read, 100 MB "
                          "written), the yardstick for hardware traffic counters")
     ap.add_argument("--no-two-term", action="store_true",
-                    help="skip the extra leg that repeats the steps with CUBERT_FP32_DENSE=f16x3 (fp32 workloads)")
+                    help="skip the extra leg that repeats the steps on a model opened without CUBERT_FP32_DENSE (fp32 workloads)")
     ap.add_argument("--device-only", action="store_true",
                     help="only the device-resident steps (no host-path / batch-1 latency loops): for profiler runs")
     ap.add_argument("--instances", type=int, default=0,
@@ -387,13 +387,13 @@ def main():
                          "the workload's batch through the host path (what CUBERT_MODELS_PER_GPU gives concurrent "
                          "callers of cuBERT_compute); reported as `concurrent_instances`")
     ap.add_argument("--fp32-dense", choices=["f32", "f16x3"], default=None,
-                    help="f16x3: open the model with CUBERT_FP32_DENSE=f16x3 (the opt-in two-term fp16 Dense form of fp32 "
-                         "models); default: whatever the environment says, normally the fp32 GEMM")
+                    help="f16x3: open the model with CUBERT_FP32_DENSE=f16x3 (the two-term fp16 Dense form of fp32 models); "
+                         "default: whatever the environment says, else f32, the fp32 GEMM")
     args = ap.parse_args()
     if args.fp32_dense == "f16x3":
         os.environ["CUBERT_FP32_DENSE"] = "f16x3"
-    elif args.fp32_dense == "f32":
-        os.environ.pop("CUBERT_FP32_DENSE", None)
+    elif args.fp32_dense == "f32" or not os.environ.get("CUBERT_FP32_DENSE"):
+        os.environ["CUBERT_FP32_DENSE"] = "f32"  # `value` is products of fp32 operands; the library's default is a leg of its own
     if args.gpus != 1 or int(os.environ.get("WORLD_SIZE", "1")) != 1:
         print("bench.py: this build measures one GPU only (replicas on several GPUs share nothing); "
               "run with --gpus 1", file=sys.stderr)
@@ -522,14 +522,15 @@ def main():
                  "ms_per_step": round(ms3, 4), "sequences_per_s": round(c3["batch"] / (ms3 * 1e-3), 1), "steps": 10,
                  "kernels": table3, "gemm": gemm3, "kernel_timing": EVENT_PAIR_NOTE}
 
-    # ---- the same steps with the opt-in two-term fp16 Dense form of fp32 models (reported beside `value`, never as it)
+    # ---- the same steps on a model as the library opens it by itself: fp32 Dense layers as two-term fp16 operands (reported
+    # beside `value`, never as it)
     two_term = None
     if not half and B * S >= 384 and not two_term_dense() and not args.device_only and not args.no_two_term:
-        os.environ["CUBERT_FP32_DENSE"] = "f16x3"  # read when a model is opened
+        kept = os.environ.pop("CUBERT_FP32_DENSE")  # read when a model is opened
         try:
             other = cubert_amd.Bert(w, B, S, m["layers"], m["heads"], 0)
         finally:
-            del os.environ["CUBERT_FP32_DENSE"]
+            os.environ["CUBERT_FP32_DENSE"] = kept
         other.compute(ids, mask, seg)
         other.synchronize()
         for _ in range(args.warmup):
@@ -543,7 +544,7 @@ def main():
         other.close()
         two_term = {"value": round(B / (ms * 1e-3), 1), "unit": "sequences/s", "ms_per_step": round(ms, 4),
                     "dtype": "f32 storage and accumulation; Dense products as three f16 matrix-core products of two-term "
-                             "operands (CUBERT_FP32_DENSE=f16x3, opt-in)"}
+                             "operands (what a model opened without CUBERT_FP32_DENSE runs)"}
 
     # ---- several instances on the one GPU, one caller thread each (host arrays in, pooled output out)
     concurrent = None

@@ -125,6 +125,10 @@ Bert<T>::Bert(const std::unordered_map<std::string, T *> &var, size_t max_batch_
         this->transformer = new Transformer<T>(cublas, "bert/encoder", var, max_batch_size, seq_length, hidden_size,
                                                num_hidden_layers, num_attention_heads, intermediate_size);
         this->transformer->set_profiler(&profiler);
+        if constexpr (sizeof(T) == 4) {
+            this->transformer->set_input_bound(norm_bound(var.at("bert/embeddings/LayerNorm/gamma"),
+                                                          var.at("bert/embeddings/LayerNorm/beta"), H));
+        }
 
         layout_buffers();
         buffers.allocate();
@@ -291,7 +295,7 @@ template <typename T>
 void Bert<T>::finish_outputs() {
     drain_pieces();
     synchronize();
-    // An fp32 model in the two-term fp16 Dense form (opt-in): an activation beyond what two fp16 terms can hold
+    // An fp32 model in the two-term fp16 Dense form: an activation beyond what two fp16 terms can hold
     // raised a flag while the request ran.  Its results are not to be trusted: the same request, whose inputs are
     // still on the device, runs again on the fp32 GEMMs, and the copies this call asked for are made again.
     if (transformer != nullptr && transformer->two_term_overflowed() && last_batch > 0 && input_ids_buf != nullptr) {

@@ -46,18 +46,21 @@ Transformer<T>::Transformer(void *cublas, const std::string &var_prefix,
     // 32768 tokens on every Dense shape of BERT-base and BERT-large, same bits out); its fp32 GEMMs do not care.
     // Half-precision models therefore keep their Dense kernels [out, in], transposed once here.
     transposed_kernels = sizeof(T) == 2;
-    const char *dense_mode = std::getenv("CUBERT_FP32_DENSE");
-    if (dense_mode != nullptr && std::string(dense_mode) != "f16x3" && std::string(dense_mode) != "f32" &&
-        std::string(dense_mode) != "") {
-        fprintf(stderr, "cuBERT: CUBERT_FP32_DENSE=%s is not understood (f32 or f16x3); using f32\n", dense_mode);
+    if constexpr (sizeof(T) == 4) {
+        const char *setting = std::getenv("CUBERT_FP32_DENSE");
+        const std::string dense_mode = setting != nullptr ? setting : "";
+        if (dense_mode != "f16x3" && dense_mode != "f32" && dense_mode != "") {
+            fprintf(stderr, "cuBERT: CUBERT_FP32_DENSE=%s is not understood (f32 or f16x3); using f32\n", setting);
+        }
+        // (where the library's own kernel is switched off by CUBERT_GEMM the rows are the ones of the library GEMM)
+        int tile = 0, tile_tokens = 0, tile_features = 0;
+        pair_dense = H % 32 == 0 && I % 32 == 0 &&
+                     cubert_dense_large_plan(1, 1, (int) H, (int) H, 0, &tile, &tile_tokens, &tile_features) == 0;
+        split_asked = dense_mode == "f16x3";
+        split_dense = max_batch_size * seq_length >= kTwoTermMinTokens && (split_asked || (dense_mode == "" && pair_dense));
+        if (split_dense && !two_term_scales(var_prefix, var) && !split_asked) split_dense = false;
+        pair_dense = pair_dense && split_dense;
     }
-    split_dense = sizeof(T) == 4 && dense_mode != nullptr && std::string(dense_mode) == "f16x3" &&
-                  max_batch_size * seq_length >= kTwoTermMinTokens;
-
-    // (also where the library's own kernel is switched off by CUBERT_GEMM the rows are the ones of the library GEMM)
-    int tile = 0, tile_tokens = 0, tile_features = 0;
-    pair_dense = split_dense && H % 32 == 0 && I % 32 == 0 &&
-                 cubert_dense_large_plan(1, 1, (int) H, (int) H, 0, &tile, &tile_tokens, &tile_features) == 0;
 
     if (split_dense) {
         split_overflow = static_cast<int *>(cubert_malloc_host(64));
@@ -87,8 +90,16 @@ Transformer<T>::Transformer(void *cublas, const std::string &var_prefix,
         if constexpr (sizeof(T) == 4) {
             if (split_dense) {
                 // a power of two that brings the largest weight to [512, 1024): far from fp16's subnormals and its limit
-                float largest_weight = 0.f;
-                for (size_t i = 0; i < in * out; ++i) largest_weight = std::fmax(largest_weight, std::fabs(host[i]));
+                // (non-negative numbers are in the order of their bits, which is a loop over whole vectors)
+                uint32_t largest_bits = 0;
+                for (size_t i = 0; i < in * out; ++i) {
+                    uint32_t bits;
+                    std::memcpy(&bits, host + i, 4);
+                    bits &= 0x7fffffffu;
+                    largest_bits = bits > largest_bits ? bits : largest_bits;
+                }
+                float largest_weight;
+                std::memcpy(&largest_weight, &largest_bits, 4);
                 int exponent = 0;
                 if (largest_weight > 0.f && std::isfinite(largest_weight)) {
                     (void) std::frexp(largest_weight, &exponent);  // largest = f * 2^exponent, f in [0.5, 1)
@@ -156,6 +167,61 @@ bool Transformer<T>::two_term_overflowed() {
     if (split_overflow == nullptr || *static_cast<volatile int *>(split_overflow) == 0) return false;
     *split_overflow = 0;
     return true;
+}
+
+// Bounds of what a layer's Dense kernels are given, || || the 2-norm:
+//   - a LayerNorm's result: norm_bound;
+//   - the context, an average of rows of V: ||row|| times the norm of the value kernel's largest column, + its largest |bias|;
+//   - GELU's result: the same with the intermediate kernel.
+// Each operand's scale is the largest power of two that keeps its bound inside fp16.  Values down to 2^-18 of the bound then have
+// both their terms in full, whatever sizes the weights of neighbouring layers trade with each other.  (The bounds allow 1 %
+// for rounding.  A variance that cancellation makes too small can still leave them: the overflow flag stays.)
+template <typename T>
+bool Transformer<T>::two_term_scales(const std::string &var_prefix, const std::unordered_map<std::string, T *> &var) {
+    if constexpr (sizeof(T) == 4) {
+        const size_t H = hidden_size, I = intermediate_size;
+        auto of_norm = [&](const std::string &name) { return norm_bound(var.at(name + "/gamma"), var.at(name + "/beta"), H); };
+        std::vector<float> squares;
+        struct DenseBound { double column, bias; };
+        auto of_dense = [&](const std::string &name, size_t out) {
+            const T *kernel = var.at(name + "/kernel"), *bias = var.at(name + "/bias");
+            squares.assign(out, 0.f);
+            for (size_t i = 0; i < H; ++i)
+                for (size_t j = 0; j < out; ++j) squares[j] += kernel[i * out + j] * kernel[i * out + j];
+            double column = 0, largest_bias = 0;
+            for (size_t j = 0; j < out; ++j) {
+                column = larger_or_nan(column, squares[j]);
+                largest_bias = larger_or_nan(largest_bias, std::fabs((double) bias[j]));
+            }
+            return DenseBound{std::sqrt(column), largest_bias};
+        };
+        bool fits = true;
+        auto set = [&](float &scale, double bound) {
+            const float s = two_term_scale(bound);
+            fits = fits && s >= kTwoTermActivationScale;
+            scale = s >= kTwoTermActivationScale ? s : kTwoTermActivationScale;
+        };
+        NormBound input;
+        for (size_t l = 0; l < num_hidden_layers; ++l) {
+            const std::string p = var_prefix + "/layer_" + std::to_string(l);
+            Layer &w = layers[l];
+            const DenseBound value = of_dense(p + "/attention/self/value", H);
+            if (l > 0) {
+                set(w.input_scale, input.element);
+                set(w.context_scale, input.row * value.column + value.bias);
+            } else {
+                first_value_norm = value.column, first_value_bias = value.bias;
+            }
+            const NormBound attention_norm = of_norm(p + "/attention/output/LayerNorm");
+            const DenseBound inner = of_dense(p + "/intermediate/dense", I);
+            set(w.norm_scale, attention_norm.element);
+            set(w.inner_scale, attention_norm.row * inner.column + inner.bias);
+            input = of_norm(p + "/output/LayerNorm");
+        }
+        return fits;
+    } else {
+        return false;
+    }
 }
 
 template <typename T>
@@ -261,7 +327,7 @@ bool Transformer<T>::three_step_attention_is_faster(size_t batch_size) const {
 // problems have two strides (b: seq*3H, a: d), a strided-batched GEMM has one, so the shorter of the two
 // axes is looped on the host and the longer one is the GEMM batch.
 template <typename T>
-bool Transformer<T>::attention(size_t batch_size, const T *qkv, const int8_t *mask, half *split_context) {
+bool Transformer<T>::attention(size_t batch_size, const T *qkv, const int8_t *mask, half *split_context, float scale) {
     void *stream = cuBERT::blas_get_stream(cublas);
     const int S = (int) seq_length, A = (int) num_attention_heads, H = (int) hidden_size, d = H / A;
     const int B = (int) batch_size, ld = (int) qkv_ld;
@@ -282,10 +348,10 @@ bool Transformer<T>::attention(size_t batch_size, const T *qkv, const int8_t *ma
         Timed t(profiler, Profiler::kAttentionFused, stream);
         if constexpr (sizeof(T) == 4) {
             if (split_context != nullptr &&
-                (pair_dense ? cuBERT::attention_fused_split_pairs(Q, K, V, ld, mask, kTwoTermActivationScale, split_context,
-                                                                  alpha, B, A, S, d, split_overflow, stream)
-                            : cuBERT::attention_fused_split3(Q, K, V, ld, mask, kTwoTermActivationScale, split_context, alpha,
-                                                             B, A, S, d, split_overflow, stream))) {
+                (pair_dense ? cuBERT::attention_fused_split_pairs(Q, K, V, ld, mask, scale, split_context, alpha, B, A, S, d,
+                                                                  split_overflow, stream)
+                            : cuBERT::attention_fused_split3(Q, K, V, ld, mask, scale, split_context, alpha, B, A, S, d,
+                                                             split_overflow, stream))) {
                 return true;
             }
         }
@@ -470,31 +536,29 @@ bool Transformer<T>::dense(int out_features, int tokens, int in_features, const 
 }
 
 template <typename T>
-void Transformer<T>::dense_split(int out_features, int tokens, int in_features, const SplitKernel &kernel, const T *in,
-                                 T *out, const T *bias, Profiler::Kind kind, int ld_out) {
+void Transformer<T>::dense_split(int out_features, int tokens, int in_features, const SplitKernel &kernel, float scale,
+                                 const T *in, T *out, const T *bias, Profiler::Kind kind, int ld_out, float inner_scale) {
     if (ld_out == 0) ld_out = out_features;
     if constexpr (sizeof(T) == 4) {
         void *stream = cuBERT::blas_get_stream(cublas);
         if (in != nullptr) {
             Timed t(profiler, Profiler::kDenseSplit, stream);
             if (pair_dense) {
-                cuBERT::split_pairs(in, tokens, in_features, kTwoTermActivationScale, split_operand, split_overflow, stream);
+                cuBERT::split_pairs(in, tokens, in_features, scale, split_operand, split_overflow, stream);
             } else {
-                cuBERT::split3(in, tokens, in_features, kTwoTermActivationScale, false, split_operand, split_overflow,
-                               stream);
+                cuBERT::split3(in, tokens, in_features, scale, false, split_operand, split_overflow, stream);
             }
         }
         Timed t(profiler, profiler != nullptr ? profiler->dense_kind(kind) : Profiler::kDenseGemm, stream);
         if (pair_dense) {
             const bool gelu = kind == Profiler::kDenseIntermediate;
             cuBERT::dense_pairs(tokens, out_features, in_features, kind == Profiler::kDenseOutput ? split_intermediate : split_operand,
-                                kernel.weights, bias, gelu, kernel.unscale / kTwoTermActivationScale, kTwoTermActivationScale,
+                                kernel.weights, bias, gelu, kernel.unscale / scale, inner_scale,
                                 gelu ? reinterpret_cast<float *>(split_intermediate) : out, ld_out, split_overflow, stream);
             return;
         }
         cuBERT::blas_gemm_f16_f32(cublas, true, false, out_features, tokens, 3 * in_features,
-                                  kernel.unscale / kTwoTermActivationScale,
-                                  kernel.weights, 3 * in_features, split_operand, 3 * in_features, 0.f, out,
+                                  kernel.unscale / scale, kernel.weights, 3 * in_features, split_operand, 3 * in_features, 0.f, out,
                                   ld_out, bias);
     } else {
         throw std::logic_error("the two-term fp16 Dense form is for fp32 models");
@@ -502,17 +566,30 @@ void Transformer<T>::dense_split(int out_features, int tokens, int in_features, 
 }
 
 template <typename T>
-bool Transformer<T>::norm_split(const T *residual, T *inout, int tokens, const T *bias, const T *beta, const T *gamma) {
+bool Transformer<T>::norm_split(const T *residual, T *inout, int tokens, const T *bias, const T *beta, const T *gamma,
+                               float scale) {
     if constexpr (sizeof(T) == 4) {
         void *stream = cuBERT::blas_get_stream(cublas);
         const int H = (int) hidden_size;
-        return pair_dense ? cuBERT::layer_norm_split_pairs(residual, inout, tokens, H, bias, beta, gamma, kTwoTermActivationScale,
-                                                           split_operand, split_overflow, stream)
-                          : cuBERT::layer_norm_split3(residual, inout, tokens, H, bias, beta, gamma, kTwoTermActivationScale,
-                                                      split_operand, split_overflow, stream);
+        return pair_dense ? cuBERT::layer_norm_split_pairs(residual, inout, tokens, H, bias, beta, gamma, scale, split_operand,
+                                                           split_overflow, stream)
+                          : cuBERT::layer_norm_split3(residual, inout, tokens, H, bias, beta, gamma, scale, split_operand,
+                                                      split_overflow, stream);
     } else {
         throw std::logic_error("the two-term fp16 Dense form is for fp32 models");
     }
+}
+
+template <typename T>
+bool Transformer<T>::norm_to_operand(const T *residual, T *inout, int tokens, const T *bias, const T *beta, const T *gamma,
+                                     float scale) {
+    Timed t(profiler, Profiler::kBiasResLayerNorm, cuBERT::blas_get_stream(cublas));
+    if (scale > 0.f && norm_writes_operand) {
+        if (norm_split(residual, inout, tokens, bias, beta, gamma, scale)) return true;
+        norm_writes_operand = false;  // the hidden size is fixed per model: do not ask again
+    }
+    cuBERT::layer_norm_(residual, inout, tokens, (int) hidden_size, bias, beta, gamma, cuBERT::blas_get_stream(cublas));
+    return false;
 }
 
 // Up to how many tokens a Dense layer that the own Dense kernel does not take runs on the few-token kernel.  32 for all of
@@ -588,11 +665,14 @@ T *Transformer<T>::_in_compute(size_t batch_size, T *input_gpu, int8_t *attentio
     void *stream = cuBERT::blas_get_stream(cublas);
     const int M = (int) (batch_size * seq_length), H = (int) hidden_size, I = (int) intermediate_size;
 
-    // (Below 384 tokens the fp32 kernels stay: the tiles of the two-term kernel are too few to fill the chip, and a request takes
-    // what it takes at 300 tokens.  BERT-base, us a request, two-term / fp32: 128 tokens 942 / 639, 256 954 / 827, 320 967 / 912, 384
-    // 1025 / 1135, 640 1147 / 1334; BERT-large 384 2555 / 2734; hidden 512 384 714 / 748.  On the library's GEMM 256 1019, 320 1012,
-    // 384 1150.)
-    const bool split = split_dense && (size_t) M >= kTwoTermMinTokens && !fp32_dense_once;
+    // Below 384 tokens the fp32 kernels stay: the tiles of the two-term kernel are too few there to fill the chip, and a request
+    // takes what it takes at 300 tokens (BERT-base, us a request, two-term / fp32: 128 tokens 942 / 639, 256 954 / 827, 320 967 / 912,
+    // 384 1025 / 1135, 640 1147 / 1334; BERT-large 384 2555 / 2734).  So they do where the layers are too narrow for their products to
+    // count: four layers of hidden 128 1312 tokens 189 / 153, 4096 214 / 217, 16384 408 / 452; 256 384 171 / 159, 1312 204 / 215, 4096
+    // 274 / 374; 384 384 228 / 215, 1312 274 / 302; 512 384 234 / 237, 1312 320 / 421; 768 384 303 / 340, 1312 464 / 739, 4096 912 /
+    // 1877, 16384 3112 / 6956; hidden 64 16384 277 / 273.
+    const bool split = split_dense && (size_t) M >= kTwoTermMinTokens && !fp32_dense_once &&
+                       (split_asked || (double) M * H * H >= 6.7e7);
     fp32_dense_once = false;
     bool operand_ready = false;
 
@@ -611,42 +691,35 @@ T *Transformer<T>::_in_compute(size_t batch_size, T *input_gpu, int8_t *attentio
             if constexpr (sizeof(T) == 4) {
                 // split_operand holds the two-term rows of the next Dense input whenever the kernel before it could
                 // write them itself (LayerNorm, GELU); otherwise dense_split makes them from the fp32 rows
-                dense_split(3 * H, M, H, w.qkv_split, operand_ready ? nullptr : layer_input, qkv_out, w.qkv_bias,
-                            Profiler::kDenseQkv, (int) qkv_ld);
-                const bool context_ready = attention(batch_size, qkv_out, attention_mask, split_operand);
-                dense_split(H, M, H, w.attention_output_split, context_ready ? nullptr : context_out, attention_output,
-                            nullptr, Profiler::kDenseAttentionOutput);
-                {
-                    Timed t(profiler, Profiler::kBiasResLayerNorm, stream);
-                    operand_ready = norm_writes_operand &&
-                                    norm_split(layer_input, attention_output, M, w.attention_output_bias,
-                                               w.attention_norm_beta, w.attention_norm_gamma);
-                    if (!operand_ready) {
-                        norm_writes_operand = false;  // the hidden size is fixed per model: do not ask again
-                        cuBERT::layer_norm_(layer_input, attention_output, M, H, w.attention_output_bias,
-                                            w.attention_norm_beta, w.attention_norm_gamma, stream);
-                    }
+                if (l == 0 && !input_bounded && !split_asked) {
+                    dense(3 * H, M, H, w.qkv_kernel, w.qkv_packed, layer_input, qkv_out, w.qkv_bias, true, false,
+                          Profiler::kDenseQkv, (int) qkv_ld);
+                    attention(batch_size, qkv_out, attention_mask);
+                    dense(H, M, H, w.attention_output_kernel, w.attention_output_packed, context_out, attention_output,
+                          w.attention_output_bias, false, false, Profiler::kDenseAttentionOutput);
+                } else {
+                    dense_split(3 * H, M, H, w.qkv_split, w.input_scale, operand_ready ? nullptr : layer_input, qkv_out,
+                                w.qkv_bias, Profiler::kDenseQkv, (int) qkv_ld);
+                    const bool context_ready = attention(batch_size, qkv_out, attention_mask, split_operand, w.context_scale);
+                    dense_split(H, M, H, w.attention_output_split, w.context_scale, context_ready ? nullptr : context_out,
+                                attention_output, nullptr, Profiler::kDenseAttentionOutput);
                 }
-                dense_split(I, M, H, w.intermediate_split, operand_ready ? nullptr : attention_output,
-                            intermediate_output, pair_dense ? w.intermediate_bias : nullptr, Profiler::kDenseIntermediate);
+                operand_ready = norm_to_operand(layer_input, attention_output, M, w.attention_output_bias,
+                                                w.attention_norm_beta, w.attention_norm_gamma, w.norm_scale);
+                dense_split(I, M, H, w.intermediate_split, w.norm_scale, operand_ready ? nullptr : attention_output,
+                            intermediate_output, pair_dense ? w.intermediate_bias : nullptr, Profiler::kDenseIntermediate, 0,
+                            w.inner_scale);
                 if (!pair_dense) {
                     // bias + GELU straight into the two-term rows the output Dense reads
                     Timed t(profiler, Profiler::kBiasGelu, stream);
-                    cuBERT::bias_gelu_split3(intermediate_output, w.intermediate_bias, M, I, kTwoTermActivationScale,
-                                             split_operand, split_overflow, stream);
+                    cuBERT::bias_gelu_split3(intermediate_output, w.intermediate_bias, M, I, w.inner_scale, split_operand,
+                                             split_overflow, stream);
                 }
-                dense_split(H, M, I, w.output_split, nullptr, out, nullptr, Profiler::kDenseOutput);
-                {
-                    Timed t(profiler, Profiler::kBiasResLayerNorm, stream);
-                    operand_ready = norm_writes_operand &&
-                                    norm_split(attention_output, out, M, w.output_bias, w.output_norm_beta,
-                                               w.output_norm_gamma);
-                    if (!operand_ready) {
-                        norm_writes_operand = false;
-                        cuBERT::layer_norm_(attention_output, out, M, H, w.output_bias, w.output_norm_beta,
-                                            w.output_norm_gamma, stream);
-                    }
-                }
+                dense_split(H, M, I, w.output_split, w.inner_scale, nullptr, out, nullptr, Profiler::kDenseOutput);
+                // (nobody reads the last layer's result as an operand)
+                const bool last = l + 1 == num_hidden_layers;
+                operand_ready = norm_to_operand(attention_output, out, M, w.output_bias, w.output_norm_beta, w.output_norm_gamma,
+                                                last ? 0.f : layers[l + 1].input_scale);
             }
             prev_output = out;
             continue;

@@ -20,16 +20,19 @@
 // <= 64 whose layer sizes are not whole steps of the own Dense kernel also keeps its four Dense kernels in the few-token
 // GEMM kernel's own order.
 //
-// CUBERT_FP32_DENSE=f16x3 in the environment when an fp32 model is opened makes its Dense layers run on the fp16
-// matrix cores for requests of at least 384 tokens (measured break-even, _in_compute): every fp32 operand is written as the sum of
-// two fp16 numbers and the product as hi*hi + hi*lo + lo*hi with fp32 accumulation (one pass of the own kernel for large requests,
-// kernels/dense_large.hip, which also applies GELU; for layer sizes that are no multiple of 32 one library GEMM over three times the
-// reduction length), which
-// keeps the error of an fp32 GEMM for activations up to 2^12 in size (see kernels/split.hip).
-// Everything between the GEMMs stays fp32.  The default is the fp32 GEMM.
+// The Dense layers of an fp32 model run on the fp16 matrix cores for requests of at least 384 tokens (measured break-even,
+// _in_compute): every fp32 operand is written as the sum of two fp16 numbers and the product as hi*hi + hi*lo + lo*hi with fp32
+// accumulation (one pass of the own kernel for large requests, kernels/dense_large.hip, which also applies GELU).  Everything
+// between them stays fp32.  The error is smaller than that of the fp32 GEMM (BERT-base against float64, relative 2-norm of the
+// tokens, two-term / fp32 GEMM: 1 x 384 6.3e-7 / 12.9e-7, 20 x 100 6.7 / 12.7, 128 x 32 6.8 / 13.0, 16 x 128 6.7 / 12.7) as long as
+// both terms are inside the range of fp16, which the weights decide when the model is opened: two_term_scales().
+// CUBERT_FP32_DENSE in the environment at that time: f32 keeps the fp32 GEMM, f16x3 takes the two-term form also where the
+// weights prove no range (a request that leaves it is recomputed in fp32) and, for layer sizes that are no multiple of 32, as one
+// library GEMM over three times the reduction length.
 #ifndef CUBERT_HOST_TRANSFORMER_H
 #define CUBERT_HOST_TRANSFORMER_H
 
+#include <cmath>
 #include <cstddef>
 #include <cstdint>
 #include <string>
@@ -52,6 +55,26 @@ enum class DenseRoute { kOther, kSmall, kLarge };
 DenseRoute dense_route(bool half_precision, int tokens, int out_features, int in_features, DenseUse use, bool as_slices);
 // ... and whether the one for small requests is better than the few-token kernel and the library's GEMM
 bool own_dense_is_best(bool half_precision, int tokens, int out_features, int in_features, DenseUse use, bool as_slices);
+
+// What a LayerNorm's result cannot exceed: an element |gamma_j| sqrt(H) + |beta_j| (no value is further than sqrt(H - 1)
+// standard deviations from the mean), a row max |gamma| sqrt(H) + ||beta|| in 2-norm.  Not a number where one of them is not.
+struct NormBound {
+    double element = 0, row = 0;
+};
+// the larger one, or whichever is not a number
+inline double larger_or_nan(double a, double b) { return a >= b || a != a ? a : b; }
+template <typename T>
+NormBound norm_bound(const T *gamma, const T *beta, size_t hidden_size) {
+    const double root = std::sqrt((double) hidden_size);
+    double element = 0, largest_gamma = 0, beta_squares = 0;
+    for (size_t j = 0; j < hidden_size; ++j) {
+        const double g = std::fabs((double) gamma[j]), b = std::fabs((double) beta[j]);
+        element = larger_or_nan(element, g * root + b);
+        largest_gamma = larger_or_nan(largest_gamma, g);
+        beta_squares += b * b;
+    }
+    return NormBound{element, largest_gamma * root + std::sqrt(beta_squares)};
+}
 
 template <typename T>
 class Transformer {
@@ -77,21 +100,37 @@ public:
     // Optional per-kernel timing (owned by the caller; null = off).
     void set_profiler(Profiler *p) { profiler = p; }
 
-    // Two-term fp16 Dense form only (CUBERT_FP32_DENSE=f16x3).  An activation beyond the fp16 range (|16 x| > 65504)
-    // cannot be written as two fp16 terms; the kernels that write two-term rows then raise a flag instead of
+    // Two-term fp16 Dense form only.  An activation beyond the fp16 range (times its scale) cannot be written as two fp16 terms; the kernels that write two-term rows then raise a flag instead of
     // handing a clamped operand to the GEMM in silence.  Once the stream has drained, two_term_overflowed() says
     // whether any request since the last call raised it (and clears it); the caller then runs the request again
     // after use_fp32_dense_once(), which makes the next _in_compute take the fp32 GEMMs whatever its size.
     bool two_term_overflowed();
     void use_fp32_dense_once() { fp32_dense_once = true; }
 
+    // What _in_compute's input cannot exceed (two-term form; where this is not known layer 0 of a model that was not asked for
+    // the form by name has its attention in fp32).
+    void set_input_bound(const NormBound &bound) {
+        if (!split_dense || layers.empty()) return;
+        const float input = two_term_scale(bound.element),
+                    context = two_term_scale(bound.row * first_value_norm + first_value_bias);
+        if (input < kTwoTermActivationScale || context < kTwoTermActivationScale) return;
+        input_bounded = true, layers[0].input_scale = input, layers[0].context_scale = context;
+    }
+
 private:
     // A Dense kernel for the two-term fp16 form: rows of pairs of scale * W^T, [out, 2 * in], or, for the library's GEMM, rows
     // [hi | lo | hi], [out, 3 * in]; unscale = 1 / scale
     static constexpr size_t kTwoTermMinTokens = 384;
-    // activations are multiplied by this before they are taken apart (undone by the GEMM's alpha): rows whose
-    // entries are of order 2^-7 .. 2^12 keep full accuracy (fp16 subnormals below, clamping above)
+    // Activations are multiplied by a power of two before they are taken apart (undone by the GEMM's alpha).  At this one, the
+    // smallest that is used, entries of 2^-7 to 2^12 keep full accuracy (fp16 subnormals below, clamping above).
     static constexpr float kTwoTermActivationScale = 16.f;
+    // the largest power of two that leaves `bound` inside the range of fp16 (0: there is none)
+    static float two_term_scale(double bound) {
+        if (!(bound >= 0) || !std::isfinite(bound)) return 0.f;
+        int exponent = 0;
+        (void) std::frexp(65504.0 / (1.01 * bound + 1e-6), &exponent);  // f * 2^exponent, f in [0.5, 1)
+        return (float) std::ldexp(1.0, exponent - 1 < 20 ? exponent - 1 : 20);
+    }
     struct SplitKernel {
         half *weights = nullptr;
         float unscale = 1.f;
@@ -109,7 +148,13 @@ private:
         T *qkv_packed = nullptr, *attention_output_packed = nullptr, *intermediate_packed = nullptr,
           *output_packed = nullptr;
         SplitKernel qkv_split, attention_output_split, intermediate_split, output_split;  // (null when not kept)
+        // of the four operands: what the layer is given, context, attention output behind its LayerNorm, GELU's result
+        float input_scale = kTwoTermActivationScale, context_scale = kTwoTermActivationScale,
+              norm_scale = kTwoTermActivationScale, inner_scale = kTwoTermActivationScale;
     };
+
+    // The scales of every layer's operands from bounds that its weights give; whether every bound allows the smallest scale.
+    bool two_term_scales(const std::string &var_prefix, const std::unordered_map<std::string, T *> &var);
 
     void layout_weights();
     void layout_buffers();
@@ -123,7 +168,7 @@ private:
     bool three_step_attention_is_faster(size_t batch_size) const;
     // context_out = attention(qkv); with `split_context` (fp32 models in the two-term Dense form) the one-launch
     // kernel writes the context there as two-term rows instead and true is returned
-    bool attention(size_t batch_size, const T *qkv, const int8_t *mask, half *split_context = nullptr);
+    bool attention(size_t batch_size, const T *qkv, const int8_t *mask, half *split_context = nullptr, float scale = 1.f);
     // out[tokens, out_features] = in[tokens, in_features] * kernel (+ bias) (, GELU); returns whether bias and
     // activation were applied (false: the caller's fused kernel still has to).
     bool dense(int out_features, int tokens, int in_features, const T *kernel, const T *packed, const T *in, T *out,
@@ -131,10 +176,13 @@ private:
     // The same on the fp16 matrix cores from two-term operands (fp32 models only): `in` is split into
     // split_operand first, or, when null, split_operand already holds its two-term rows.  `bias` may be null.  With pair_dense
     // the intermediate layer applies GELU and leaves two-term rows in split_intermediate, where the output layer finds them.
-    void dense_split(int out_features, int tokens, int in_features, const SplitKernel &kernel, const T *in, T *out,
-                     const T *bias, Profiler::Kind kind, int ld_out = 0);
+    // scale: of the operand; inner_scale: of the intermediate layer's result
+    void dense_split(int out_features, int tokens, int in_features, const SplitKernel &kernel, float scale, const T *in, T *out,
+                     const T *bias, Profiler::Kind kind, int ld_out = 0, float inner_scale = 1.f);
     // inout = LayerNorm(inout + bias + residual), and its two-term rows in split_operand; false: the hidden size is declined
-    bool norm_split(const T *residual, T *inout, int tokens, const T *bias, const T *beta, const T *gamma);
+    bool norm_split(const T *residual, T *inout, int tokens, const T *bias, const T *beta, const T *gamma, float scale);
+    // the same, or without the rows where they are declined or nobody asks for them (scale 0); whether they were written
+    bool norm_to_operand(const T *residual, T *inout, int tokens, const T *bias, const T *beta, const T *gamma, float scale);
     // out = LayerNorm(in * kernel + bias + residual): dense(), then layer_norm_; for a small request the Dense kernel
     // leaves its K slices in few_token_partials and the LayerNorm kernel adds them while it loads (no hand-over between
     // the GEMM's workgroups).
@@ -155,7 +203,10 @@ private:
     bool own_slices_to_norm = true;    // cleared when the LayerNorm over its slices declines the hidden size
     bool keep_packed = false;          // Dense kernels are also kept in the few-token kernel's order
     bool transposed_kernels = false;   // Dense kernels are stored [out, in] instead of [in, out] (half precision)
-    bool split_dense = false;          // fp32 model with Dense layers in the two-term fp16 form (opt-in)
+    bool split_dense = false;          // fp32 model with Dense layers in the two-term fp16 form
+    bool split_asked = false;          // ... because it was asked for by name (CUBERT_FP32_DENSE=f16x3)
+    bool input_bounded = false;        // set_input_bound gave layer 0 its scales
+    double first_value_norm = 0, first_value_bias = 0;  // of layer 0: the largest column of the value kernel, and bias
     bool pair_dense = false;           // ... on the library's own kernel, whose operand rows hold every term once
     bool fp32_dense_once = false;      // the next request takes the fp32 GEMMs (set after a two-term overflow)
     int *split_overflow = nullptr;     // page-locked host word the two-term kernels set to 1 on overflow (split_dense)

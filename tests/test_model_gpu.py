@@ -635,6 +635,98 @@ def test_two_term_dense_falls_back_to_fp32_when_an_activation_does_not_fit(cb, m
         bert.close()
 
 
+def scaled_layers(w, factors):
+    """The model with the named tensors of every layer multiplied by their factors."""
+    out = dict(w)
+    for name in w:
+        for part, factor in factors.items():
+            if name.endswith(part) and "/layer_" in name:
+                out[name] = (w[name] * np.float32(factor)).astype(np.float32)
+    return out
+
+
+@pytest.mark.parametrize("factors", [
+    {},
+    {"value/kernel": 2.0 ** -12, "value/bias": 2.0 ** -12, "attention/output/dense/kernel": 2.0 ** 12},  # the same function
+    {"LayerNorm/gamma": 2.0 ** -9, "LayerNorm/beta": 2.0 ** -9},
+    {"LayerNorm/gamma": 2.0 ** 4, "LayerNorm/beta": 2.0 ** 4, "intermediate/dense/kernel": 2.0 ** -4}], ids=str)
+def test_two_term_scales_follow_the_weights(cb, monkeypatch, factors):
+    """An fp32 model opened without CUBERT_FP32_DENSE runs requests of enough tokens in the two-term form, with operand scales
+    that its weights prove to be safe: however sizes are shared out between neighbouring tensors, the result is no further
+    from float64 than the fp32 GEMM's."""
+    from cubert_amd.testing import random_bert_weights, random_inputs
+    m = dict(vocab=97, hidden=512, layers=2, heads=8, intermediate=2048, max_position=64, type_vocab=2)
+    w = scaled_layers(random_bert_weights(seed=61, labels=2, pooler=True, classifier=True, ln_random=True, **m), factors)
+    ids, mask, seg = random_inputs(seed=62, batch=20, seq_length=32, vocab=97, min_valid=3, segment_split=9)
+    want = float64_tokens(w, ids, mask, seg, 2, 8)
+    error = {}
+    for mode in ("f32", ""):
+        monkeypatch.setenv("CUBERT_FP32_DENSE", mode)
+        bert = cb.Bert(w, 20, 32, 2, 8, 0)
+        bert.profile(["dense_split", "bias_gelu"])
+        got = bert.forward(ids, mask, seg)["sequence_output"]
+        assert ("dense_split" in bert.profile_read()) == (mode == "")
+        bert.close()
+        error[mode] = np.linalg.norm(got - want) / np.linalg.norm(want)
+    print("\nrelative error against float64: fp32 GEMM %.2e, two-term %.2e" % (error["f32"], error[""]))
+    assert error[""] <= error["f32"]
+
+
+def float64_tokens(w, ids, mask, seg, layers, heads):
+    """The encoder's output in float64."""
+    from scipy.special import erf
+    w = {k: v.astype(np.float64) for k, v in w.items()}
+
+    def norm(x, p):
+        return (x - x.mean(-1, keepdims=True)) / np.sqrt(x.var(-1, keepdims=True) + 1e-12) * w[p + "/gamma"] + w[p + "/beta"]
+    e = "bert/embeddings/"
+    x = w[e + "word_embeddings"][ids] + w[e + "position_embeddings"][:ids.shape[1]] + w[e + "token_type_embeddings"][seg]
+    x = norm(x, e + "LayerNorm")
+    B, S, H = x.shape
+    for layer in range(layers):
+        p = "bert/encoder/layer_%d" % layer
+
+        def dense(y, name):
+            return y @ w[p + name + "/kernel"] + w[p + name + "/bias"]
+        q, k, v = (dense(x, "/attention/self/" + n).reshape(B, S, heads, H // heads).transpose(0, 2, 1, 3)
+                   for n in ("query", "key", "value"))
+        s = q @ k.transpose(0, 1, 3, 2) / np.sqrt(H // heads) - 10000.0 * (1 - mask[:, None, None, :].astype(np.float64))
+        s = np.exp(s - s.max(-1, keepdims=True))
+        c = (s / s.sum(-1, keepdims=True) @ v).transpose(0, 2, 1, 3).reshape(B, S, H)
+        a = norm(dense(c, "/attention/output/dense") + x, p + "/attention/output/LayerNorm")
+        h = dense(a, "/intermediate/dense")
+        x = norm(dense(0.5 * h * (1 + erf(h / np.sqrt(2))), "/output/dense") + a, p + "/output/LayerNorm")
+    return x
+
+
+def test_two_term_form_is_left_alone_where_nothing_bounds_the_input(cb, monkeypatch):
+    """The encoder by itself, on inputs of any size: layer 0's attention, whose operands no weight bounds, is computed in fp32;
+    tiny and huge rows come out as from the fp32 GEMM.  A model with a weight that is not a number keeps the fp32 GEMM."""
+    from cubert_amd.testing import random_bert_weights, random_inputs
+    m = dict(vocab=97, hidden=512, layers=2, heads=8, intermediate=2048, max_position=64, type_vocab=2)
+    w = random_bert_weights(seed=63, labels=2, pooler=True, classifier=True, ln_random=True, **m)
+    rng = np.random.default_rng(64)
+    mask = np.ones((13, 32), np.int8)
+    for size in (1e-6, 1e6):
+        x = (rng.standard_normal((13, 32, 512)) * size).astype(np.float32)
+        got = cb.transformer_run(w, "bert/encoder", x, mask, 2, 8, 2048, 0)
+        monkeypatch.setenv("CUBERT_FP32_DENSE", "f32")
+        plain = cb.transformer_run(w, "bert/encoder", x, mask, 2, 8, 2048, 0)
+        monkeypatch.delenv("CUBERT_FP32_DENSE")
+        assert np.isfinite(got).all() and not np.array_equal(got, plain)
+        assert np.abs(got - plain).max() <= FP32_TOL * np.abs(plain).max()
+    ids, mask, seg = random_inputs(seed=65, batch=13, seq_length=32, vocab=97, min_valid=3, segment_split=9)
+    bad = dict(w)
+    name = "bert/encoder/layer_1/attention/output/LayerNorm/beta"
+    bad[name] = w[name].copy()
+    bad[name][0] = np.nan
+    bert = cb.Bert(bad, 13, 32, 2, 8, 0)
+    bert.profile(["dense_split"])
+    bert.forward(ids, mask, seg)
+    assert "dense_split" not in bert.profile_read()
+    bert.close()
+
+
 def test_first_request_does_not_pay_for_gemm_planning(cb):
     """The constructor runs one forward pass at max_batch_size (Bert<T>::_pre_compute), so the GEMM shapes of that
     batch size are planned and timed before the first request: BERT-base width, 2 layers, batch 128 x seq 32 (Dense
