@@ -115,7 +115,7 @@ def recorded_traffic(workload, kind):
 
 
 def two_term_dense():
-    """CUBERT_FP32_DENSE=f16x3 in the environment: fp32 models run their Dense layers (requests of at least 384 tokens) on the
+    """CUBERT_FP32_DENSE=f16x3 in the environment: fp32 models run their Dense layers (requests of more than 64 tokens) on the
     fp16 matrix cores from two-term operands (as models opened without the variable do; this bench's `value` is the fp32 GEMM)."""
     return os.environ.get("CUBERT_FP32_DENSE") == "f16x3"
 

@@ -115,6 +115,9 @@ SIGNATURES = {
     "cubert_attention_fused_split_pairs_f32": (ci, [vp, vp, vp, ci, vp, cf, vp, cf, ci, ci, ci, ci, vp, vp]),
     "cubert_bias_res_ln_split_pairs_f32": (ci, [vp, vp, vp, vp, vp, ci, ci, cf, vp, vp, vp]),
     "cubert_dense_pairs_f32": (ci, [vp, ci, ci, ci, vp, vp, vp, ci, cf, cf, vp, ci, vp]),
+    "cubert_dense_pairs_small_f32": (ci, [vp, ci, ci, ci, vp, vp, vp, ci, cf, cf, vp, ci, vp]),
+    "cubert_dense_pairs_slices_f32": (ci, [vp, ci, ci, ci, vp, vp, cf, vp, ctypes.c_size_t, ctypes.POINTER(ci)]),
+    "cubert_bias_res_ln_slices_split_pairs_f32": (ci, [vp, vp, ci, ci, cll, vp, vp, vp, vp, ci, ci, cf, vp, vp, vp]),
     "cubert_dense_large_f16": (ci, [vp, ci, ci, ci, vp, vp, vp, ci, vp, ci]),
     "cubert_dense_large_plan": (ci, [ci, ci, ci, ci, ci, ctypes.POINTER(ci), ctypes.POINTER(ci), ctypes.POINTER(ci)]),
     "cubert_blas_create": (vp, []),

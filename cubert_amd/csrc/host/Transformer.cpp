@@ -1,5 +1,6 @@
 #include "Transformer.h"
 
+#include <algorithm>
 #include <cmath>
 #include <cstdlib>
 #include <string>
@@ -57,7 +58,9 @@ Transformer<T>::Transformer(void *cublas, const std::string &var_prefix,
         pair_dense = H % 32 == 0 && I % 32 == 0 &&
                      cubert_dense_large_plan(1, 1, (int) H, (int) H, 0, &tile, &tile_tokens, &tile_features) == 0;
         split_asked = dense_mode == "f16x3";
-        split_dense = max_batch_size * seq_length >= kTwoTermMinTokens && (split_asked || (dense_mode == "" && pair_dense));
+        const size_t most = max_batch_size * seq_length;
+        split_dense = (two_terms_pay(most) || two_terms_pay(std::min(most, kTwoTermSmallTokens))) &&
+                      (split_asked || (dense_mode == "" && pair_dense));
         if (split_dense && !two_term_scales(var_prefix, var) && !split_asked) split_dense = false;
         pair_dense = pair_dense && split_dense;
     }
@@ -535,6 +538,30 @@ bool Transformer<T>::dense(int out_features, int tokens, int in_features, const 
     return bias_in_gemm;
 }
 
+// Whether a Dense layer over rows of pairs runs on the kernel for small requests (kernels/dense_mid.hip) instead of the one for
+// large ones: as long as no compute unit has two of its 64 x 64 tiles.  A layer, with its GELU or LayerNorm, small / large, us:
+//   Q|K|V           768 in: 120 tokens 7.4 / 10.3, 300 9.7 / 10.3, 384 9.8 / 10.4, 512 14.9 / 12.5; 1024: 300 11.7 / 12.8, 384 18.6 / 16.0
+//   attention out   768: 120 7.5 / 12.0, 640 10.0 / 12.9, 1280 14.3 / 15.0; 1024: 800 14.6 / 16.2, 1024 18.4 / 17.8, 1280 23.8 / 22.1
+//   intermediate    768 in: 120 8.0 / 11.1, 300 10.8 / 11.1, 384 15.9 / 13.7; 1024: 200 12.5 / 13.2, 300 19.7 / 18.6
+//   output          3072 in: 120 10.7 / 32, 640 19.9 / 33.5, 1280 30.9 / 34.6; 4096: 300 19.0 / 40.0, 1024 37.4 / 44.1, 1280 59.7 / 64.3
+static bool small_pairs_are_best(int tokens, int out_features) {
+    return (long long) ((tokens + 63) / 64) * ((out_features + 63) / 64) <= 256;
+}
+
+// Up to 64 tokens the fp32 kernels stay: theirs are the shorter sums (tokens of BERT-base against float64, 1e-7 of their 2-norm,
+// pairs / fp32: 32 tokens 3.4 / 3.2, 64 3.4 / 3.2; 96 3.5 / 5.1, 120 3.4 / 4.8, 256 3.5 / 5.0, 300 3.5 / 11, 640 4.2 / 12.7, 1600 6.7 /
+// 12.7), and no slower (us a request: 32 476 / 454, 64 485 / 487).  Above, BERT-base: 96 506 / 546, 100 633 / 734, 160 633 / 684, 256 720 /
+// 852, 300 798 / 1024, 384 822 / 1205.  Narrow layers, whose launches are all there is to them, four layers, us, pairs / fp32: hidden
+// 256 192 tokens 157 / 147, 320 155 / 151, 640 190 / 245; 512 96 159 / 161, 192 186 / 210; and, where the LayerNorm kernel writes no rows
+// of pairs (no multiple of 256) and a pass of its own does, 128 320 174 / 141, 4096 263 / 298; 384 192 189 / 177, 512 232 / 281; 640 96 182 / 174, 192 217 / 230.
+// (321 to 383 tokens stay on the fp32 GEMM and its GELU pass, the one size of request that
+// test_requests_around_the_switch_to_the_library still finds there: 352 tokens.)
+template <typename T>
+bool Transformer<T>::two_terms_pay(size_t tokens) const {
+    if (split_asked && tokens >= kTwoTermMinTokens) return true;
+    return pair_dense && tokens > 64 && (tokens <= kTwoTermSmallTokens || tokens >= kTwoTermMinTokens) && (double) tokens * hidden_size * hidden_size >= (hidden_size % 256 == 0 ? 3.8e7 : 6.7e7);
+}
+
 template <typename T>
 void Transformer<T>::dense_split(int out_features, int tokens, int in_features, const SplitKernel &kernel, float scale,
                                  const T *in, T *out, const T *bias, Profiler::Kind kind, int ld_out, float inner_scale) {
@@ -552,6 +579,14 @@ void Transformer<T>::dense_split(int out_features, int tokens, int in_features, 
         Timed t(profiler, profiler != nullptr ? profiler->dense_kind(kind) : Profiler::kDenseGemm, stream);
         if (pair_dense) {
             const bool gelu = kind == Profiler::kDenseIntermediate;
+            if (small_pairs_are_best(tokens, out_features) &&
+                cuBERT::dense_pairs_small(tokens, out_features, in_features,
+                                          kind == Profiler::kDenseOutput ? split_intermediate : split_operand, kernel.weights, bias,
+                                          gelu, kernel.unscale / scale, inner_scale,
+                                          gelu ? reinterpret_cast<float *>(split_intermediate) : out, ld_out, split_overflow,
+                                          stream)) {
+                return;
+            }
             cuBERT::dense_pairs(tokens, out_features, in_features, kind == Profiler::kDenseOutput ? split_intermediate : split_operand,
                                 kernel.weights, bias, gelu, kernel.unscale / scale, inner_scale,
                                 gelu ? reinterpret_cast<float *>(split_intermediate) : out, ld_out, split_overflow, stream);
@@ -590,6 +625,46 @@ bool Transformer<T>::norm_to_operand(const T *residual, T *inout, int tokens, co
     }
     cuBERT::layer_norm_(residual, inout, tokens, (int) hidden_size, bias, beta, gamma, cuBERT::blas_get_stream(cublas));
     return false;
+}
+
+template <typename T>
+bool Transformer<T>::dense_split_norm(int tokens, int in_features, const SplitKernel &kernel, float scale, const T *in, const T *bias,
+                                      const T *residual, const T *beta, const T *gamma, T *out, Profiler::Kind kind,
+                                      float next_scale) {
+    if constexpr (sizeof(T) == 4) {
+        void *stream = cuBERT::blas_get_stream(cublas);
+        const int H = (int) hidden_size;
+        if (in == nullptr && pair_dense && own_slices_to_norm && few_token_slices_enabled() &&
+            small_pairs_are_best(tokens, H)) {
+            int slices = 0;
+            bool done = false;
+            {
+                Timed t(profiler, profiler != nullptr ? profiler->dense_kind(kind) : Profiler::kDenseGemm, stream);
+                done = cuBERT::dense_pairs_slices(tokens, H, in_features,
+                                                  kind == Profiler::kDenseOutput ? split_intermediate : split_operand,
+                                                  kernel.weights, kernel.unscale / scale, few_token_partials,
+                                                  kFewTokenPartialFloats, &slices, stream);
+                if (!done) t.cancel();
+            }
+            if (done) {
+                Timed t(profiler, Profiler::kBiasResLayerNorm, stream);
+                if (next_scale > 0.f && norm_writes_operand &&
+                    cuBERT::layer_norm_slices_pairs(out, few_token_partials, slices, residual, bias, beta, gamma, tokens, H,
+                                                    next_scale, split_operand, split_overflow, stream)) {
+                    return true;
+                }
+                if (cuBERT::layer_norm_slices(out, few_token_partials, slices, residual, bias, beta, gamma, tokens, H, stream)) {
+                    return false;
+                }
+                t.cancel();
+                own_slices_to_norm = false;  // the hidden size is fixed per model: do not ask again
+            }
+        }
+        dense_split(H, tokens, in_features, kernel, scale, in, out, nullptr, kind);
+        return norm_to_operand(residual, out, tokens, bias, beta, gamma, next_scale);
+    } else {
+        throw std::logic_error("the two-term fp16 Dense form is for fp32 models");
+    }
 }
 
 // Up to how many tokens a Dense layer that the own Dense kernel does not take runs on the few-token kernel.  32 for all of
@@ -665,14 +740,7 @@ T *Transformer<T>::_in_compute(size_t batch_size, T *input_gpu, int8_t *attentio
     void *stream = cuBERT::blas_get_stream(cublas);
     const int M = (int) (batch_size * seq_length), H = (int) hidden_size, I = (int) intermediate_size;
 
-    // Below 384 tokens the fp32 kernels stay: the tiles of the two-term kernel are too few there to fill the chip, and a request
-    // takes what it takes at 300 tokens (BERT-base, us a request, two-term / fp32: 128 tokens 942 / 639, 256 954 / 827, 320 967 / 912,
-    // 384 1025 / 1135, 640 1147 / 1334; BERT-large 384 2555 / 2734).  So they do where the layers are too narrow for their products to
-    // count: four layers of hidden 128 1312 tokens 189 / 153, 4096 214 / 217, 16384 408 / 452; 256 384 171 / 159, 1312 204 / 215, 4096
-    // 274 / 374; 384 384 228 / 215, 1312 274 / 302; 512 384 234 / 237, 1312 320 / 421; 768 384 303 / 340, 1312 464 / 739, 4096 912 /
-    // 1877, 16384 3112 / 6956; hidden 64 16384 277 / 273.
-    const bool split = split_dense && (size_t) M >= kTwoTermMinTokens && !fp32_dense_once &&
-                       (split_asked || (double) M * H * H >= 6.7e7);
+    const bool split = split_dense && two_terms_pay((size_t) M) && !fp32_dense_once;
     fp32_dense_once = false;
     bool operand_ready = false;
 
@@ -691,21 +759,30 @@ T *Transformer<T>::_in_compute(size_t batch_size, T *input_gpu, int8_t *attentio
             if constexpr (sizeof(T) == 4) {
                 // split_operand holds the two-term rows of the next Dense input whenever the kernel before it could
                 // write them itself (LayerNorm, GELU); otherwise dense_split makes them from the fp32 rows
-                if (l == 0 && !input_bounded && !split_asked) {
+                // (for a small request a pass that makes them takes longer than the first Q|K|V loses in fp32: 120 tokens 4.2 + 7.4 us
+                // against 11.5, 300 4.2 + 9.7 against 15.0)
+                const bool bounded = l > 0 || input_bounded || split_asked;
+                const bool fp32_projection = l == 0 && (!bounded || (size_t) M < kTwoTermMinTokens);
+                if (fp32_projection) {
                     dense(3 * H, M, H, w.qkv_kernel, w.qkv_packed, layer_input, qkv_out, w.qkv_bias, true, false,
                           Profiler::kDenseQkv, (int) qkv_ld);
-                    attention(batch_size, qkv_out, attention_mask);
-                    dense(H, M, H, w.attention_output_kernel, w.attention_output_packed, context_out, attention_output,
-                          w.attention_output_bias, false, false, Profiler::kDenseAttentionOutput);
                 } else {
                     dense_split(3 * H, M, H, w.qkv_split, w.input_scale, operand_ready ? nullptr : layer_input, qkv_out,
                                 w.qkv_bias, Profiler::kDenseQkv, (int) qkv_ld);
-                    const bool context_ready = attention(batch_size, qkv_out, attention_mask, split_operand, w.context_scale);
-                    dense_split(H, M, H, w.attention_output_split, w.context_scale, context_ready ? nullptr : context_out,
-                                attention_output, nullptr, Profiler::kDenseAttentionOutput);
                 }
-                operand_ready = norm_to_operand(layer_input, attention_output, M, w.attention_output_bias,
-                                                w.attention_norm_beta, w.attention_norm_gamma, w.norm_scale);
+                if (!bounded) {
+                    attention(batch_size, qkv_out, attention_mask);
+                    dense(H, M, H, w.attention_output_kernel, w.attention_output_packed, context_out, attention_output,
+                          w.attention_output_bias, false, false, Profiler::kDenseAttentionOutput);
+                    operand_ready = norm_to_operand(layer_input, attention_output, M, w.attention_output_bias,
+                                                    w.attention_norm_beta, w.attention_norm_gamma, w.norm_scale);
+                } else {
+                    const bool context_ready = attention(batch_size, qkv_out, attention_mask, split_operand, w.context_scale);
+                    operand_ready = dense_split_norm(M, H, w.attention_output_split, w.context_scale,
+                                                     context_ready ? nullptr : context_out, w.attention_output_bias, layer_input,
+                                                     w.attention_norm_beta, w.attention_norm_gamma, attention_output,
+                                                     Profiler::kDenseAttentionOutput, w.norm_scale);
+                }
                 dense_split(I, M, H, w.intermediate_split, w.norm_scale, operand_ready ? nullptr : attention_output,
                             intermediate_output, pair_dense ? w.intermediate_bias : nullptr, Profiler::kDenseIntermediate, 0,
                             w.inner_scale);
@@ -715,11 +792,11 @@ T *Transformer<T>::_in_compute(size_t batch_size, T *input_gpu, int8_t *attentio
                     cuBERT::bias_gelu_split3(intermediate_output, w.intermediate_bias, M, I, w.inner_scale, split_operand,
                                              split_overflow, stream);
                 }
-                dense_split(H, M, I, w.output_split, w.inner_scale, nullptr, out, nullptr, Profiler::kDenseOutput);
                 // (nobody reads the last layer's result as an operand)
                 const bool last = l + 1 == num_hidden_layers;
-                operand_ready = norm_to_operand(attention_output, out, M, w.output_bias, w.output_norm_beta, w.output_norm_gamma,
-                                                last ? 0.f : layers[l + 1].input_scale);
+                operand_ready = dense_split_norm(M, I, w.output_split, w.inner_scale, nullptr, w.output_bias, attention_output,
+                                                 w.output_norm_beta, w.output_norm_gamma, out, Profiler::kDenseOutput,
+                                                 last ? 0.f : layers[l + 1].input_scale);
             }
             prev_output = out;
             continue;

@@ -20,11 +20,11 @@
 // <= 64 whose layer sizes are not whole steps of the own Dense kernel also keeps its four Dense kernels in the few-token
 // GEMM kernel's own order.
 //
-// The Dense layers of an fp32 model run on the fp16 matrix cores for requests of at least 384 tokens (measured break-even,
-// _in_compute): every fp32 operand is written as the sum of two fp16 numbers and the product as hi*hi + hi*lo + lo*hi with fp32
-// accumulation (one pass of the own kernel for large requests, kernels/dense_large.hip, which also applies GELU).  Everything
+// The Dense layers of an fp32 model run on the fp16 matrix cores for requests of more than 64 tokens (where they pay:
+// two_terms_pay): every fp32 operand is written as the sum of two fp16 numbers and the product as hi*hi + hi*lo + lo*hi with fp32
+// accumulation (one pass of the own kernels, kernels/dense_mid.hip and dense_large.hip, which also apply GELU).  Everything
 // between them stays fp32.  The error is smaller than that of the fp32 GEMM (BERT-base against float64, relative 2-norm of the
-// tokens, two-term / fp32 GEMM: 1 x 384 6.3e-7 / 12.9e-7, 20 x 100 6.7 / 12.7, 128 x 32 6.8 / 13.0, 16 x 128 6.7 / 12.7) as long as
+// tokens, two-term / fp32: 5 x 24 3.4e-7 / 4.8e-7, 3 x 100 3.5 / 11, 20 x 100 6.7 / 12.7, 128 x 32 6.8 / 13.0, 16 x 128 6.7 / 12.7) as long as
 // both terms are inside the range of fp16, which the weights decide when the model is opened: two_term_scales().
 // CUBERT_FP32_DENSE in the environment at that time: f32 keeps the fp32 GEMM, f16x3 takes the two-term form also where the
 // weights prove no range (a request that leaves it is recomputed in fp32) and, for layer sizes that are no multiple of 32, as one
@@ -120,7 +120,7 @@ public:
 private:
     // A Dense kernel for the two-term fp16 form: rows of pairs of scale * W^T, [out, 2 * in], or, for the library's GEMM, rows
     // [hi | lo | hi], [out, 3 * in]; unscale = 1 / scale
-    static constexpr size_t kTwoTermMinTokens = 384;
+    static constexpr size_t kTwoTermMinTokens = 384, kTwoTermSmallTokens = 320;  // two_terms_pay
     // Activations are multiplied by a power of two before they are taken apart (undone by the GEMM's alpha).  At this one, the
     // smallest that is used, entries of 2^-7 to 2^12 keep full accuracy (fp16 subnormals below, clamping above).
     static constexpr float kTwoTermActivationScale = 16.f;
@@ -179,6 +179,11 @@ private:
     // scale: of the operand; inner_scale: of the intermediate layer's result
     void dense_split(int out_features, int tokens, int in_features, const SplitKernel &kernel, float scale, const T *in, T *out,
                      const T *bias, Profiler::Kind kind, int ld_out = 0, float inner_scale = 1.f);
+    // out = LayerNorm(dense_split + bias + residual), and with a next_scale its two-term rows in split_operand; whether they were written
+    bool dense_split_norm(int tokens, int in_features, const SplitKernel &kernel, float scale, const T *in, const T *bias,
+                          const T *residual, const T *beta, const T *gamma, T *out, Profiler::Kind kind, float next_scale);
+    // whether a request of this many tokens is faster in the two-term form
+    bool two_terms_pay(size_t tokens) const;
     // inout = LayerNorm(inout + bias + residual), and its two-term rows in split_operand; false: the hidden size is declined
     bool norm_split(const T *residual, T *inout, int tokens, const T *bias, const T *beta, const T *gamma, float scale);
     // the same, or without the rows where they are declined or nobody asks for them (scale 0); whether they were written

@@ -255,6 +255,31 @@ inline void dense_pairs(int tokens, int features, int in, const half *x, const h
     CUBERT_CHECK(cubert_dense_pairs_f32(stream, tokens, features, in, h(x), h(w), bias, gelu, alpha, scale, out, ldo, overflow));
 }
 // the same kernel over plain half operands; false when the shape is not taken
+// the same for up to some hundreds of tokens; false: declined
+inline bool dense_pairs_small(int tokens, int features, int in, const half *x, const half *w, const float *bias, bool gelu,
+                              float alpha, float scale, float *out, int ldo, int *overflow, void *stream) {
+    const int rc = cubert_dense_pairs_small_f32(stream, tokens, features, in, h(x), h(w), bias, gelu, alpha, scale, out, ldo, overflow);
+    if (rc == CUBERT_UNSUPPORTED) return false;
+    CUBERT_CHECK(rc);
+    return true;
+}
+// its product as K slices, and the LayerNorm that adds them and writes the next layer's rows of pairs as well
+inline bool dense_pairs_slices(int tokens, int features, int in, const half *x, const half *w, float alpha, float *partials,
+                               size_t partial_floats, int *slices, void *stream) {
+    const int rc = cubert_dense_pairs_slices_f32(stream, tokens, features, in, h(x), h(w), alpha, partials, partial_floats, slices);
+    if (rc == CUBERT_UNSUPPORTED) return false;
+    CUBERT_CHECK(rc);
+    return true;
+}
+inline bool layer_norm_slices_pairs(float *out, const float *partials, int slices, const float *residual, const float *bias,
+                                    const float *beta, const float *gamma, int rows, int hidden, float scale, half *split_out,
+                                    int *overflow, void *stream) {
+    const int rc = cubert_bias_res_ln_slices_split_pairs_f32(out, partials, slices, hidden, (long long) rows * hidden, residual,
+                                                             bias, beta, gamma, rows, hidden, scale, h(split_out), overflow, stream);
+    if (rc == CUBERT_UNSUPPORTED) return false;
+    CUBERT_CHECK(rc);
+    return true;
+}
 inline bool dense_large(int tokens, int features, int in, const half *x, const half *w, const half *bias, bool gelu, half *out,
                         int ldo, void *stream) {
     const int rc = cubert_dense_large_f16(stream, tokens, features, in, h(x), h(w), h(bias), gelu, h(out), ldo);

@@ -155,14 +155,16 @@ __device__ __forceinline__ void load_floats(const float *__restrict__ p, float (
 // col], fp32): the slices are added here, in slice order from 0.f, and the sum is rounded to the storage type before
 // anything else happens to it.  In fp32 the result has the bits of bias_res_ln on that sum; in half precision a few results
 // differ in the last bit (separately compiled kernels, at 768 halves another order of a row's sums).
-template <typename T, int VEC, int CHUNKS, bool HAS_BIAS>
+// SPLIT: the result also as operand rows of pairs, times split_scale (ln_finish).
+template <typename T, int VEC, int CHUNKS, bool HAS_BIAS, bool SPLIT = false>
 __global__ __launch_bounds__(kBlock) void bias_res_ln_partials_kernel(T *__restrict__ out,
                                                                       const float *__restrict__ partials, int slices,
                                                                       int pitch, const T *__restrict__ residual,
                                                                       const T *__restrict__ bias,
                                                                       const T *__restrict__ beta,
                                                                       const T *__restrict__ gamma, int rows,
-                                                                      long long slice_stride) {
+                                                                      long long slice_stride, half_t *__restrict__ split_out,
+                                                                      float split_scale, int *__restrict__ overflow) {
     constexpr int H = kWave * VEC * CHUNKS;
     constexpr int kAhead = CHUNKS * VEC <= 12 ? 8 : 4;  // slices whose loads are in flight together
     const int row = blockIdx.x * (int) (blockDim.x / kWave) + wave_in_block();
@@ -231,7 +233,8 @@ __global__ __launch_bounds__(kBlock) void bias_res_ln_partials_kernel(T *__restr
             sumsq += v * v;
         }
     }
-    ln_finish<T, VEC, CHUNKS>(x, sum, sumsq, g, be, out + (size_t) row * H, lane);
+    ln_finish<T, VEC, CHUNKS>(x, sum, sumsq, g, be, out + (size_t) row * H, lane,
+                              SPLIT ? split_out + (size_t) row * 2 * H : nullptr, split_scale, overflow, true);
 }
 
 template <typename T, int VEC, int CHUNKS>
@@ -511,9 +514,9 @@ int bias_res_ln_slices(T *out, const float *partials, int slices, int pitch, lon
     if (hidden == kWave * VEC * CHUNKS && vector_ok<T>(hidden, VEC, {out, residual, bias, beta, gamma})) {       \
         if (bias != nullptr)                                                                                     \
             return launch(bias_res_ln_partials_kernel<T, VEC, CHUNKS, true>, grid, block, s, out, partials, slices, \
-                          pitch, residual, bias, beta, gamma, rows, slice_stride);                                             \
+                          pitch, residual, bias, beta, gamma, rows, slice_stride, nullptr, 1.f, nullptr);                      \
         return launch(bias_res_ln_partials_kernel<T, VEC, CHUNKS, false>, grid, block, s, out, partials, slices, \
-                      pitch, residual, bias, beta, gamma, rows, slice_stride);                                                 \
+                      pitch, residual, bias, beta, gamma, rows, slice_stride, nullptr, 1.f, nullptr);                          \
     }
     CUBERT_LN_CASE(V, 1)
     CUBERT_LN_CASE(V, 2)
@@ -533,6 +536,33 @@ int bias_res_ln_partials(T *out, const float *partials, int slices, int pitch, c
     if (rows > 64) return CUBERT_UNSUPPORTED;
     return bias_res_ln_slices<T>(out, partials, slices, pitch, (long long) ((rows + 31) / 32 * 32) * pitch, residual, bias,
                                  beta, gamma, rows, hidden, stream);
+}
+
+// The same in fp32, and the result again as operand rows of pairs in split_out [rows, 2 * hidden].
+int bias_res_ln_slices_pairs(float *out, const float *partials, int slices, int pitch, long long slice_stride,
+                             const float *residual, const float *bias, const float *beta, const float *gamma, int rows,
+                             int hidden, float scale, half_t *split_out, int *overflow, void *stream) {
+    if (rows < 0 || hidden <= 0 || slices <= 0 || !out || !partials || !residual || !beta || !gamma || !split_out) {
+        return CUBERT_BAD_ARGUMENT;
+    }
+    if (pitch < hidden || pitch % 4 != 0 || slice_stride % 4 != 0 || !is_aligned(partials, 16) || !is_aligned(split_out, 8)) {
+        return CUBERT_UNSUPPORTED;
+    }
+    if (rows == 0) return 0;
+    const dim3 grid(rows), block(kWave);
+#define CUBERT_LN_SPLIT_CASE(CHUNKS)                                                                                      \
+    if (hidden == kWave * 4 * CHUNKS && vector_ok<float>(hidden, 4, {out, residual, bias, beta, gamma})) {                \
+        auto kernel = bias != nullptr ? bias_res_ln_partials_kernel<float, 4, CHUNKS, true, true>                         \
+                                      : bias_res_ln_partials_kernel<float, 4, CHUNKS, false, true>;                       \
+        return launch(kernel, grid, block, (hipStream_t) stream, out, partials, slices, pitch, residual, bias, beta, gamma, \
+                      rows, slice_stride, split_out, scale, overflow);                                                    \
+    }
+    CUBERT_LN_SPLIT_CASE(1)
+    CUBERT_LN_SPLIT_CASE(2)
+    CUBERT_LN_SPLIT_CASE(3)
+    CUBERT_LN_SPLIT_CASE(4)
+#undef CUBERT_LN_SPLIT_CASE
+    return CUBERT_UNSUPPORTED;
 }
 
 // bias + residual + LayerNorm of fp32 rows, in place, and the result again as two-term fp16 rows in split_out
@@ -654,6 +684,14 @@ extern "C" int cubert_bias_res_ln_slices_f32(float *out, const float *partials, 
                                              const float *beta, const float *gamma, int rows, int hidden, void *stream) {
     return cubert::bias_res_ln_slices<float>(out, partials, slices, pitch, slice_stride, residual, bias, beta, gamma, rows,
                                              hidden, stream);
+}
+
+extern "C" int cubert_bias_res_ln_slices_split_pairs_f32(float *out, const float *partials, int slices, int pitch,
+                                                         long long slice_stride, const float *residual, const float *bias,
+                                                         const float *beta, const float *gamma, int rows, int hidden,
+                                                         float scale, cubert_half *split_out, int *overflow, void *stream) {
+    return cubert::bias_res_ln_slices_pairs(out, partials, slices, pitch, slice_stride, residual, bias, beta, gamma, rows,
+                                            hidden, scale, (half_t *) split_out, overflow, stream);
 }
 
 extern "C" int cubert_bias_res_ln_slices_f16(cubert_half *out, const float *partials, int slices, int pitch,

@@ -44,6 +44,10 @@ int dense_mid_slices(int tokens, int features, int in, const T *X, int ldx, cons
                      size_t partial_floats, int *slices, hipStream_t stream);
 template <typename T>
 int dense_mid_plan(int tokens, int features, int in, bool as_slices, size_t partial_floats, int *tile, int *depth, int *slices);
+int dense_mid_pairs(int tokens, int features, int in, const half_t *X, const half_t *W, const float *bias, int activation,
+                    float alpha, float scale, float *C, int ldc, int *overflow, hipStream_t stream);
+int dense_mid_pairs_slices(int tokens, int features, int in, const half_t *X, const half_t *W, float alpha, float *partials,
+                           size_t partial_floats, int *slices, hipStream_t stream);
 // kernels/dense_large.hip
 int dense_pairs(int tokens, int features, int in, const half_t *x, const half_t *w, const float *bias, int activation,
                 float alpha, float scale, float *out, int ldo, int *overflow, hipStream_t stream);
@@ -770,6 +774,21 @@ int cubert_dense_pairs_f32(void *stream, int tokens, int features, int in, const
     if (library_gemm_only() || force_naive_gemm()) return CUBERT_UNSUPPORTED;
     return cubert::dense_pairs(tokens, features, in, (const cubert::half_t *) x, (const cubert::half_t *) w, bias, activation,
                                alpha, scale, out, ldo, overflow, (hipStream_t) stream);
+}
+
+int cubert_dense_pairs_small_f32(void *stream, int tokens, int features, int in, const cubert_half *x, const cubert_half *w,
+                                 const float *bias, int activation, float alpha, float scale, float *out, int ldo,
+                                 int *overflow) {
+    if (library_gemm_only() || force_naive_gemm()) return CUBERT_UNSUPPORTED;
+    return cubert::dense_mid_pairs(tokens, features, in, (const cubert::half_t *) x, (const cubert::half_t *) w, bias, activation,
+                                   alpha, scale, out, ldo, overflow, (hipStream_t) stream);
+}
+
+int cubert_dense_pairs_slices_f32(void *stream, int tokens, int features, int in, const cubert_half *x, const cubert_half *w,
+                                  float alpha, float *partials, size_t partial_floats, int *slices) {
+    if (library_gemm_only() || force_naive_gemm()) return CUBERT_UNSUPPORTED;
+    return cubert::dense_mid_pairs_slices(tokens, features, in, (const cubert::half_t *) x, (const cubert::half_t *) w, alpha,
+                                          partials, partial_floats, slices, (hipStream_t) stream);
 }
 
 int cubert_dense_large_f16(void *stream, int tokens, int features, int in, const cubert_half *x, const cubert_half *w,

@@ -227,18 +227,46 @@ def split_pairs(x, scale=1.0, overflow=None):
     return out
 
 
-def dense_pairs(x, w, bias=None, gelu=False, alpha=1.0, scale=1.0, ldo=None, overflow=None):
+def dense_pairs(x, w, bias=None, gelu=False, alpha=1.0, scale=1.0, ldo=None, overflow=None, small=False):
     """alpha * x w^T + bias of operands from split_pairs, as fp32 [tokens, features]; with gelu, scale * GELU of that as rows like
-    the operands'; None when declined."""
+    the operands'; small: on the kernel for few tokens; None when declined."""
     (tokens, width), features = x.shape, w.shape[0]
     ldo = features if ldo is None else ldo
     out = torch.empty((tokens, ldo), dtype=torch.float32, device=x.device)
-    rc = lib().cubert_dense_pairs_f32(_stream(), tokens, features, width // 2, _ptr(x), _ptr(w), _ptr(bias), int(gelu),
-                                      float(alpha), float(scale), _ptr(out), ldo, _ptr(overflow))
+    fn = lib().cubert_dense_pairs_small_f32 if small else lib().cubert_dense_pairs_f32
+    rc = fn(_stream(), tokens, features, width // 2, _ptr(x), _ptr(w), _ptr(bias), int(gelu), float(alpha), float(scale),
+            _ptr(out), ldo, _ptr(overflow))
     if rc == -2:
         return None
-    _check(rc, "cubert_dense_pairs_f32")
+    _check(rc, fn.__name__)
     return out.view(torch.float16) if gelu else out[:, :features]
+
+
+def dense_pairs_slices(x, w, alpha=1.0, partial_floats=1 << 21):
+    """alpha * x w^T of operands from split_pairs, left as K slices [slices, tokens, features]; None when declined."""
+    (tokens, width), features = x.shape, w.shape[0]
+    partials = torch.empty(partial_floats, dtype=torch.float32, device=x.device)
+    slices = ctypes.c_int(0)
+    rc = lib().cubert_dense_pairs_slices_f32(_stream(), tokens, features, width // 2, _ptr(x), _ptr(w), float(alpha),
+                                             _ptr(partials), partial_floats, ctypes.byref(slices))
+    if rc == -2:
+        return None
+    _check(rc, "cubert_dense_pairs_slices_f32")
+    return partials[:slices.value * tokens * features].view(slices.value, tokens, features)
+
+
+def bias_res_ln_slices_split_pairs(partials, residual, bias, beta, gamma, scale=1.0, overflow=None):
+    """bias_res_ln_slices of fp32 slices, and scale * the result as split_pairs writes it; None when declined."""
+    out = torch.empty_like(residual)
+    rows, hidden = residual.shape
+    terms = torch.empty((rows, 2 * hidden), dtype=torch.float16, device=residual.device)
+    rc = lib().cubert_bias_res_ln_slices_split_pairs_f32(
+        _ptr(out), _ptr(partials), partials.shape[0], partials.shape[2], partials.stride(0), _ptr(residual), _ptr(bias),
+        _ptr(beta), _ptr(gamma), rows, hidden, float(scale), _ptr(terms), _ptr(overflow), _stream())
+    if rc == -2:
+        return None
+    _check(rc, "cubert_bias_res_ln_slices_split_pairs_f32")
+    return out, terms
 
 
 def dense_large(x, w, bias=None, gelu=False, ldo=None):

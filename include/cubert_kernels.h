@@ -342,6 +342,18 @@ int cubert_bias_res_ln_split_pairs_f32(float *inout, const float *residual, cons
  * replaces: Dense<float>::compute, reference src/cuBERT/op/Dense.cpp:47-57, and gelu<float>, op/GELU.h:6-7, in their opt-in form. */
 int cubert_dense_pairs_f32(void *stream, int tokens, int features, int in, const cubert_half *x, const cubert_half *w,
                            const float *bias, int activation, float alpha, float scale, float *out, int ldo, int *overflow);
+/* The same for up to some hundreds of tokens (cubert_dense_f32's kernel over these operands); and alpha * x w^T alone, left as K
+ * slices as cubert_dense_slices_f32 leaves them, which cubert_bias_res_ln_slices_split_pairs_f32 adds on its way to its result and
+ * the rows of the next layer. */
+int cubert_dense_pairs_small_f32(void *stream, int tokens, int features, int in, const cubert_half *x, const cubert_half *w,
+                                 const float *bias, int activation, float alpha, float scale, float *out, int ldo,
+                                 int *overflow);
+int cubert_dense_pairs_slices_f32(void *stream, int tokens, int features, int in, const cubert_half *x, const cubert_half *w,
+                                  float alpha, float *partials, size_t partial_floats, int *slices);
+int cubert_bias_res_ln_slices_split_pairs_f32(float *out, const float *partials, int slices, int pitch, long long slice_stride,
+                                              const float *residual, const float *bias, const float *beta, const float *gamma,
+                                              int rows, int hidden, float scale, cubert_half *split_out, int *overflow,
+                                              void *stream);
 /* The same kernel over plain fp16 operands, x [tokens, in] and w [features, in]: out = fp16(x w^T + bias) (bias may be NULL), or,
  * with activation 1, GELU of that, sums, bias and GELU in fp32.  in a multiple of 64, features and ldo of 8, operands 16-byte
  * aligned; otherwise (and with CUBERT_GEMM=library or naive) CUBERT_UNSUPPORTED.  For hundreds to thousands of tokens;

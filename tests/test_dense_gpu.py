@@ -198,6 +198,59 @@ def test_dense_pairs(K, tokens, features, width, gelu):
     assert bool(torch.isfinite(got).all()) and bool(((got.double() - want).abs() <= bound).all())
 
 
+# the kernel for small requests: one token, tiles of 32 and 64 and what ends inside them, a step for one wavefront only, K in slices
+@pytest.mark.parametrize("tokens,features,width", [(1, 4, 32), (33, 36, 96), (65, 768, 768), (120, 772, 160), (129, 3072, 768),
+                                                   (300, 768, 3072), (383, 2304, 768), (1279, 768, 768)])
+@pytest.mark.parametrize("gelu", [False, True])
+def test_dense_pairs_small(K, tokens, features, width, gelu):
+    features = (features + 31) // 32 * 32 if gelu else features
+    rng = np.random.default_rng(tokens + width)
+    x = dev(rng.normal(0, 1, (tokens, width)).astype(np.float32))
+    w = dev(rng.normal(0, 0.05, (features, width)).astype(np.float32))
+    bias = dev(rng.normal(0, 0.5, features).astype(np.float32)) if width != 160 else None
+    ldo = features if gelu else features + 8
+    xs, ws, alpha = K.split_pairs(x, 16.0), K.split_pairs(w, 8192.0), 1 / (16.0 * 8192.0)
+    flag = torch.zeros(1, dtype=torch.int32, device="cuda")
+    out = K.dense_pairs(xs, ws, bias, gelu, alpha, 16.0, ldo, overflow=flag, small=True)
+    want, size = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    # as in test_dense_pairs, a quarter of K to a wavefront
+    bound = size * ((3 * width / 64 + 24) * 2.0 ** -23 + 2.0 ** -22)
+    slices = K.dense_pairs_slices(xs, ws, alpha) if not gelu else None
+    if slices is not None:
+        assert slices.shape[0] >= 2
+        assert bool(((slices.double().sum(0) - want).abs() <= bound).all())
+        if features % 256 == 0:
+            res = dev(rng.normal(0, 1, (tokens, features)).astype(np.float32))
+            beta, gamma = dev(rng.normal(0, 1, features).astype(np.float32)), dev(rng.normal(1, 0.1, features).astype(np.float32))
+            plain = K.bias_res_ln_slices(slices, res, bias, beta, gamma)
+            norm, terms = K.bias_res_ln_slices_split_pairs(slices, res, bias, beta, gamma, scale=16.0, overflow=flag)
+            assert torch.equal(norm, plain) and torch.equal(terms, K.split_pairs(plain, 16.0))
+    if bias is not None:
+        want, bound = want + bias.double(), bound + bias.double().abs() * 2.0 ** -22
+    got = out
+    if gelu:
+        want = 0.5 * want * (1 + torch.erf(want / 2 ** 0.5))
+        terms = out.double().view(tokens, -1, 2, 32)
+        got = (terms[:, :, 0] + terms[:, :, 1]).reshape(tokens, features) / 16
+        bound = 1.13 * bound + 5e-7 * (1 + want.abs())
+    assert bool(torch.isfinite(got).all()) and bool(((got.double() - want).abs() <= bound).all())
+    assert int(flag) == 0
+    if gelu:  # values of 70000 and more in the result: the flag, and nothing that is not finite
+        big = K.dense_pairs(xs, ws, bias, True, alpha, 2.0 ** 20, overflow=flag, small=True)
+        assert int(flag) == (1 if float(want.abs().max()) * 2.0 ** 20 > 65536 else 0) and bool(torch.isfinite(big).all())
+
+
+def test_dense_pairs_small_refusals(K):
+    x, w = torch.zeros(40, 2 * 64, dtype=torch.float16, device="cuda"), torch.zeros(96, 2 * 64, dtype=torch.float16, device="cuda")
+    assert K.dense_pairs(x, w[:94].contiguous(), None, True, small=True) is None   # rows of pairs need whole blocks of 32
+    assert K.dense_pairs(x, w[:94].contiguous(), None, small=True) is None         # four features per store
+    assert K.dense_pairs(x, w, None, ldo=98, small=True) is None
+    assert K.dense_pairs_slices(x, w, partial_floats=40 * 96) is None              # no room for two slices
+    part = torch.zeros(2, 40, 320, device="cuda")
+    row = torch.zeros(40, 320, device="cuda")
+    assert K.bias_res_ln_slices_split_pairs(part, row, None, row[0], row[1]) is None  # hidden = 256 k
+
+
 def test_dense_pairs_takes_every_tile(K):
     tiles = {K.dense_large_plan(True, t, f, w, g) for t, f, w in PAIR_SHAPES for g in (False, True)}
     assert tiles == {(0, 256, 192), (1, 128, 128), (2, 128, 96), (3, 128, 96), (4, 64, 64)}

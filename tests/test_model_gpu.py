@@ -672,6 +672,31 @@ def test_two_term_scales_follow_the_weights(cb, monkeypatch, factors):
     assert error[""] <= error["f32"]
 
 
+@pytest.mark.parametrize("batch,seq", [(1, 64), (1, 65), (3, 37), (4, 96), (2, 300), (20, 64)])
+@pytest.mark.parametrize("hidden", [768, 640])
+def test_two_term_form_of_small_requests(cb, monkeypatch, batch, seq, hidden):
+    """From 65 tokens on the Dense layers run in the two-term form on the kernels for small requests (K slices into the LayerNorm,
+    which writes rows of pairs where hidden is a multiple of 256): no further from float64 than the fp32 kernels; below, their bits."""
+    from cubert_amd.testing import random_bert_weights, random_inputs
+    m = dict(vocab=97, hidden=hidden, layers=2, heads=hidden // 64, intermediate=4 * hidden, max_position=300, type_vocab=2)
+    w = random_bert_weights(seed=71, labels=2, pooler=True, classifier=True, ln_random=True, **m)
+    ids, mask, seg = random_inputs(seed=72, batch=batch, seq_length=seq, vocab=97, min_valid=seq // 4, segment_split=9)
+    want = float64_tokens(w, ids, mask, seg, 2, m["heads"])
+    got = {}
+    for mode in ("f32", ""):
+        monkeypatch.setenv("CUBERT_FP32_DENSE", mode)
+        bert = cb.Bert(w, batch, seq, 2, m["heads"], 0)
+        got[mode] = bert.forward(ids, mask, seg)["sequence_output"]
+        again = bert.forward(ids, mask, seg)["sequence_output"]
+        assert np.array_equal(again, got[mode])
+        bert.close()
+    error = {k: np.linalg.norm(v - want) / np.linalg.norm(want) for k, v in got.items()}
+    print("\nrelative error against float64: fp32 %.2e, as opened %.2e" % (error["f32"], error[""]))
+    pays = batch * seq > 64 and batch * seq * hidden ** 2 >= (3.8e7 if hidden % 256 == 0 else 6.7e7)
+    assert np.array_equal(got[""], got["f32"]) == (not pays)
+    assert error[""] <= error["f32"]
+
+
 def float64_tokens(w, ids, mask, seg, layers, heads):
     """The encoder's output in float64."""
     from scipy.special import erf
