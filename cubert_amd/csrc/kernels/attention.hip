@@ -68,26 +68,36 @@ struct SplitOut {
     bool pairs = false;       // high and low terms in turn, 32 of each, instead of [hi | hi | lo]
 };
 
+enum ContextForm { kPlain = 0, kThirdRows = 1, kPairRows = 2 };  // floats or halves; [hi | hi | lo]; pairs
+
 // One element of the attention context.  split.width = 0: ctx[row, col] in the storage type.  split.width = W > 0
 // (fp32 only): `ctx` is really a buffer of halves with rows [hi | hi | lo] of W each (or of W pairs), the two-term form of
 // split.scale * v that the Dense GEMM on the fp16 matrix cores reads (hi = fp16(.), lo = fp16(. - hi), clamped to
 // the fp16 range; a value that had to be clamped raises split.overflow, and the caller recomputes in fp32).
-// (SPLIT is a compile-time choice so that the plain kernels are exactly what they were without it.)
-template <typename T, bool SPLIT>
-__device__ __forceinline__ void store_context(T *ctx, int ld_ctx, size_t row, int col, float v, const SplitOut &split) {
-    if constexpr (SPLIT) {
+// (SPLIT is a compile-time choice: the plain kernels are exactly what they were without it, and no branch stands between stores.)
+// Neighbouring lanes, 2 i and 2 i + 1, come with the columns 2 j and 2 j + 1 of one row.  In rows of pairs they trade halves, so that
+// the even lane stores both high terms and the odd one both low terms, a word each (two stores of two bytes per lane, and a branch
+// per value for the flag, in its place: 128 x 12 problems of 32 keys 14.7 us, 13.6 so, 32 x 12 7.3 and 6.3, 20 x 12 of 100 17.4 and 16.3).  `over` collects what
+// flag_overflow passes on at the end.
+template <typename T, int SPLIT>
+__device__ __forceinline__ void store_context(T *ctx, int ld_ctx, size_t row, int col, float v, const SplitOut &split, bool &over) {
+    if constexpr (SPLIT != kPlain) {
         // v as the plain kernel would store it: rounded to fp32 before it is taken apart (without this the compiler
         // fuses a product that made v into the subtraction below, and lo would belong to the unrounded value)
         asm volatile("" : "+v"(v));
         v *= split.scale;
         half_t hi, lo;
         split_two_terms(v, hi, lo);
-        if (two_term_overflow(v) && split.overflow != nullptr) *split.overflow = 1;
+        over = over || two_term_overflow(v);
         half_t *p = reinterpret_cast<half_t *>(ctx);
-        if (split.pairs) {  // (uniform)
-            p += row * 2 * split.width + pair_at(col);
-            p[0] = hi;
-            p[kPairBlock] = lo;
+        if constexpr (SPLIT == kPairRows) {
+            typedef uint32_t Word __attribute__((aligned(2)));
+            const bool odd = col & 1;
+            const uint32_t own = __builtin_bit_cast(uint16_t, hi) | (uint32_t) __builtin_bit_cast(uint16_t, lo) << 16;
+            const uint32_t other = (uint32_t) __builtin_amdgcn_update_dpp((int) own, (int) own, kDppQuadXor1, 0xf, 0xf, false);
+            // bytes 0 to 3 are own's, 4 to 7 the other lane's
+            const uint32_t both = __builtin_amdgcn_perm(other, own, odd ? 0x03020706u : 0x05040100u);
+            *reinterpret_cast<Word *>(p + row * 2 * split.width + pair_at(col & ~1) + (odd ? kPairBlock : 0)) = both;
         } else {
             p += row * 3 * split.width + col;
             p[0] = hi;
@@ -97,6 +107,10 @@ __device__ __forceinline__ void store_context(T *ctx, int ld_ctx, size_t row, in
     } else {
         ctx[row * ld_ctx + col] = from_f32<T>(v);
     }
+}
+template <int SPLIT>
+__device__ __forceinline__ void flag_overflow(const SplitOut &split, bool over) {
+    if (SPLIT != kPlain && over && split.overflow != nullptr) *split.overflow = 1;
 }
 
 // grid = (seq / 32 query tiles, key super-tiles, batch * heads); a wavefront computes 32 queries x (32 * NT) keys.
@@ -382,7 +396,7 @@ constexpr size_t fused_lds_bytes() {
 }
 
 // grid = batch * heads workgroups of KT wavefronts; seq = 32 * KT, or with RAGGED 32 * (KT - 1) < seq_ragged < 32 * KT.
-template <typename T, int D, int KT, bool SPLIT, bool RAGGED>
+template <typename T, int D, int KT, int SPLIT, bool RAGGED>
 __global__ __launch_bounds__(KT * kWave) void attention_fused_kernel(const T *__restrict__ q, const T *__restrict__ k,
                                                                      const T *__restrict__ v, int ld,
                                                                      const int8_t *__restrict__ mask,
@@ -523,14 +537,16 @@ __global__ __launch_bounds__(KT * kWave) void attention_fused_kernel(const T *__
     }
     // lane holds output column jt*32 + r and 16 query rows
     const size_t first_row = (size_t) b * seq + qt * 32;
+    bool over = false;
 #pragma unroll
     for (int jt = 0; jt < kColTiles; ++jt) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
             if (RAGGED && qt * 32 + acc_row(i, hh) >= seq) continue;
-            store_context<T, SPLIT>(ctx, ld_ctx, first_row + acc_row(i, hh), h * D + jt * 32 + r, out[jt][i], split);
+            store_context<T, SPLIT>(ctx, ld_ctx, first_row + acc_row(i, hh), h * D + jt * 32 + r, out[jt][i], split, over);
         }
     }
+    flag_overflow<SPLIT>(split, over);
 }
 
 // ---- the same for fp16 storage with the ordinary-instruction work cut down ----
@@ -807,7 +823,7 @@ __global__ __launch_bounds__(KT * kWave) void attention_fused_half_kernel(const 
 // used by one lane only), the four partial score tiles are added in wavefront order through LDS, every
 // wavefront repeats the (cheap) softmax, and P V is split into (column tile, key half), the two key halves
 // meeting in LDS again.  Same arithmetic and rounding as attention_fused_kernel, other summation order.
-template <typename T, bool SPLIT, bool RAGGED>
+template <typename T, int SPLIT, bool RAGGED>
 __global__ __launch_bounds__(4 * kWave) void attention_small_kernel(const T *__restrict__ q, const T *__restrict__ k,
                                                                     const T *__restrict__ v, int ld,
                                                                     const int8_t *__restrict__ mask,
@@ -908,12 +924,14 @@ __global__ __launch_bounds__(4 * kWave) void attention_small_kernel(const T *__r
     }
     __syncthreads();
     if (kh == 0) {
+        bool over = false;
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
             if (RAGGED && acc_row(i, hh) >= seq) continue;
             store_context<T, SPLIT>(ctx, ld_ctx, (size_t) row0 + acc_row(i, hh), h * D + jt * 32 + r,
-                             out[i] + s_part[jt][i * kWave + lane], split);
+                                    out[i] + s_part[jt][i * kWave + lane], split, over);
         }
+        flag_overflow<SPLIT>(split, over);
     }
 }
 
@@ -934,7 +952,7 @@ __global__ __launch_bounds__(4 * kWave) void attention_small_kernel(const T *__r
 // RAGGED it is read as bytes, otherwise every tile is computed.
 // RAGGED: seq is not a multiple of 32 (with the clamped rows and guarded stores in every launch: 13 x 384, 12 heads, fp16
 // 20.3 instead of 19.5 us, 32 x 256 18.5 instead of 17.1).
-template <typename T, int D, bool SPLIT, bool RAGGED>
+template <typename T, int D, int SPLIT, bool RAGGED>
 __global__ __launch_bounds__(1024) void attention_flash_kernel(const T *__restrict__ q, const T *__restrict__ k,
                                                                const T *__restrict__ v, int ld,
                                                                const int8_t *__restrict__ mask, T *__restrict__ ctx,
@@ -1134,6 +1152,7 @@ __global__ __launch_bounds__(1024) void attention_flash_kernel(const T *__restri
     __builtin_amdgcn_s_waitcnt(0xc07f);
     __builtin_amdgcn_wave_barrier();
     const size_t first_row = (size_t) b * seq + qt * 32;
+    bool over = false;
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
         const Vec<float, 4> fr = load_vec<float, 4>(factor + g * 8 + hh * 4);
@@ -1143,10 +1162,11 @@ __global__ __launch_bounds__(1024) void attention_flash_kernel(const T *__restri
             for (int e = 0; e < 4; ++e) {
                 if (RAGGED && qt * 32 + acc_row(g * 4 + e, hh) >= seq) continue;
                 store_context<T, SPLIT>(ctx, ld_ctx, first_row + acc_row(g * 4 + e, hh), h * D + jt * 32 + r,
-                                 out[jt][g * 4 + e] * fr.v[e], split);
+                                        out[jt][g * 4 + e] * fr.v[e], split, over);
             }
         }
     }
+    flag_overflow<SPLIT>(split, over);
 }
 
 // ---- seq 512 with the keys staged a group at a time ----
@@ -1158,7 +1178,7 @@ __global__ __launch_bounds__(1024) void attention_flash_kernel(const T *__restri
 // and, since the LDS no longer grows with the sequence, fp32 fits as well.  Measured at batch 64, 12 heads, ~4 live
 // tiles per sequence: 54.6 against 59.5 us; groups of 2 or 8 tiles are slower.  Arithmetic and rounding are those of
 // attention_flash_kernel.
-template <typename T, int D, bool SPLIT, bool ANY_SEQ>
+template <typename T, int D, int SPLIT, bool ANY_SEQ>
 __global__ __launch_bounds__(1024) void attention_flash_grouped_kernel(
     const T *__restrict__ q, const T *__restrict__ k, const T *__restrict__ v, int ld, const int8_t *__restrict__ mask,
     T *__restrict__ ctx, int ld_ctx, float alpha, int heads, int any_seq, int skip_masked_tiles, SplitOut split,
@@ -1386,6 +1406,7 @@ __global__ __launch_bounds__(1024) void attention_flash_grouped_kernel(
     __builtin_amdgcn_s_waitcnt(0xc07f);
     __builtin_amdgcn_wave_barrier();
     const size_t first_row = (size_t) b * seq + qt * 32;
+    bool over = false;
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
         const Vec<float, 4> fr = load_vec<float, 4>(factor + g * 8 + hh * 4);
@@ -1395,10 +1416,11 @@ __global__ __launch_bounds__(1024) void attention_flash_grouped_kernel(
             for (int e = 0; e < 4; ++e) {
                 if (ANY_SEQ && qt * 32 + acc_row(g * 4 + e, hh) >= seq) continue;
                 store_context<T, SPLIT>(ctx, ld_ctx, first_row + acc_row(g * 4 + e, hh), h * D + jt * 32 + r,
-                                        out[jt][g * 4 + e] * fr.v[e], split);
+                                        out[jt][g * 4 + e] * fr.v[e], split, over);
             }
         }
     }
+    flag_overflow<SPLIT>(split, over);
 }
 
 // ---- longest sequences first ----
@@ -1605,8 +1627,10 @@ int launch_fused_kt(const T *q, const T *k, const T *v, int ld, const int8_t *ma
     const dim3 grid(batch * heads), block(KT * kWave);
     if constexpr (sizeof(T) == 4) {
         if (split.width > 0) {
-            return launch_attention<attention_fused_kernel<T, D, KT, true, RAGGED>>(
-                grid, block, lds, s, q, k, v, ld, mask, ctx, ld_ctx, alpha, heads, seq, split);
+            return split.pairs ? launch_attention<attention_fused_kernel<T, D, KT, kPairRows, RAGGED>>(
+                                         grid, block, lds, s, q, k, v, ld, mask, ctx, ld_ctx, alpha, heads, seq, split)
+                               : launch_attention<attention_fused_kernel<T, D, KT, kThirdRows, RAGGED>>(
+                                         grid, block, lds, s, q, k, v, ld, mask, ctx, ld_ctx, alpha, heads, seq, split);
         }
     }
     if (split.width > 0) return CUBERT_UNSUPPORTED;
@@ -1625,7 +1649,7 @@ int launch_fused_kt(const T *q, const T *k, const T *v, int ld, const int8_t *ma
                 grid, block, fused_half_lds_bytes<D, KT>(), s, q, k, v, ld, mask, ctx, ld_ctx, alpha, heads, seq);
         }
     }
-    return launch_attention<attention_fused_kernel<T, D, KT, false, RAGGED>>(grid, block, lds, s, q, k, v, ld, mask, ctx,
+    return launch_attention<attention_fused_kernel<T, D, KT, kPlain, RAGGED>>(grid, block, lds, s, q, k, v, ld, mask, ctx,
                                                                              ld_ctx, alpha, heads, seq, split);
 }
 
@@ -1639,12 +1663,14 @@ int launch_fused(const T *q, const T *k, const T *v, int ld, const int8_t *mask,
             const dim3 grid(batch * heads), block(4 * kWave);
             if constexpr (sizeof(T) == 4) {
                 if (split.width > 0) {
-                    return launch_attention<attention_small_kernel<T, true, RAGGED>>(grid, block, 0, s, q, k, v, ld, mask,
-                                                                                     ctx, ld_ctx, alpha, heads, seq, split);
+                    return split.pairs ? launch_attention<attention_small_kernel<T, kPairRows, RAGGED>>(
+                                                 grid, block, 0, s, q, k, v, ld, mask, ctx, ld_ctx, alpha, heads, seq, split)
+                                       : launch_attention<attention_small_kernel<T, kThirdRows, RAGGED>>(
+                                                 grid, block, 0, s, q, k, v, ld, mask, ctx, ld_ctx, alpha, heads, seq, split);
                 }
             }
             if (split.width > 0) return CUBERT_UNSUPPORTED;
-            return launch_attention<attention_small_kernel<T, false, RAGGED>>(grid, block, 0, s, q, k, v, ld, mask, ctx,
+            return launch_attention<attention_small_kernel<T, kPlain, RAGGED>>(grid, block, 0, s, q, k, v, ld, mask, ctx,
                                                                               ld_ctx, alpha, heads, seq, split);
         }
     }
@@ -1662,7 +1688,7 @@ int launch_fused(const T *q, const T *k, const T *v, int ld, const int8_t *mask,
 
 // 128 < seq <= 512.  seq 512 walks the keys in groups; other lengths hold K and V of the head in LDS where they fit
 // (fp16 always, fp32 up to 288 keys at head size 64) and walk them in groups where they do not.
-template <typename T, int D, bool SPLIT>
+template <typename T, int D, int SPLIT>
 int launch_flash(const T *q, const T *k, const T *v, int ld, const int8_t *mask, T *ctx, int ld_ctx, float alpha,
                  int batch, int heads, int seq, SplitOut split, const int *order, hipStream_t s) {
     constexpr int V = 16 / sizeof(T);
@@ -1718,13 +1744,17 @@ int attention_fused(const T *q, const T *k, const T *v, int ld, const int8_t *ma
         if (head_size == 128) return CUBERT_UNSUPPORTED;  // would spill the accumulators to scratch
         if constexpr (sizeof(T) == 4) {
             if (split.width > 0) {
-                return head_size == 32 ? launch_flash<T, 32, true>(CUBERT_ATTENTION_ARGS, order, s)
-                                       : launch_flash<T, 64, true>(CUBERT_ATTENTION_ARGS, order, s);
+                if (split.pairs) {
+                    return head_size == 32 ? launch_flash<T, 32, kPairRows>(CUBERT_ATTENTION_ARGS, order, s)
+                                           : launch_flash<T, 64, kPairRows>(CUBERT_ATTENTION_ARGS, order, s);
+                }
+                return head_size == 32 ? launch_flash<T, 32, kThirdRows>(CUBERT_ATTENTION_ARGS, order, s)
+                                       : launch_flash<T, 64, kThirdRows>(CUBERT_ATTENTION_ARGS, order, s);
             }
         }
         if (split.width > 0) return CUBERT_UNSUPPORTED;
-        return head_size == 32 ? launch_flash<T, 32, false>(CUBERT_ATTENTION_ARGS, order, s)
-                               : launch_flash<T, 64, false>(CUBERT_ATTENTION_ARGS, order, s);
+        return head_size == 32 ? launch_flash<T, 32, kPlain>(CUBERT_ATTENTION_ARGS, order, s)
+                               : launch_flash<T, 64, kPlain>(CUBERT_ATTENTION_ARGS, order, s);
     }
     const bool ragged = seq % 32 != 0;
     switch (head_size) {
