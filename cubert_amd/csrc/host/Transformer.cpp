@@ -308,17 +308,13 @@ T *Transformer<T>::compute(size_t batch_size, T *input_gpu, int8_t *attention_ma
 template <typename T>
 void Transformer<T>::_pre_compute(size_t) {}
 
-// fp32 sequences of more than 288 keys, few (sequence, head) problems: the one-launch kernels give a problem to one
-// workgroup, which then walks all keys of all queries by itself, while the three steps spread over the chip.  Two layers of
-// BERT-base through compute + output, three steps against one launch, us (lengths drawn between a quarter and all of a
-// sequence): 1 x 333 196 / 259, 1 x 500 243 / 425, 2 x 450 334 / 433, 3 x 500 485 / 600, 4 x 450 571 / 616, 4 x 333 430 /
-// 426, 6 x 333 603 / 544; 16 heads: 3 x 480 688 / 725, 4 x 480 848 / 832.  Up to 288 keys one launch is level at worst (1 x
-// 250 213 / 214, 2 x 250 299 / 236), and at 512 the three steps lost before.  With a head size of 32 K and V stay in the
-// LDS, which 12 problems notice from 333 keys on (165 / 175, 1 x 500 185 / 261; 2 x 333 212 / 175) where the length is no
-// multiple of 32 and level otherwise.
+// Layers of less than 256, fp32 sequences of more than 288 keys, few (sequence, head) problems: the three steps, which spread over
+// the chip, as test_long_fp32_sequences_by_number_of_problems has it.  (Two layers of 128 through compute + output, three steps / the
+// one-launch kernel that does too, us: 1 x 333 134 / 145, 24 x 333 271 / 204, 1 x 511 132 / 141.  Wider layers only take the latter:
+// 256 12 x 450 381 / 265; BERT-base 1 x 500 1624 / 992 a request, 4 x 450 4233 / 1976.)
 template <typename T>
 bool Transformer<T>::three_step_attention_is_faster(size_t batch_size) const {
-    if (sizeof(T) != 4 || seq_length <= 288 || seq_length >= 512) return false;
+    if (sizeof(T) != 4 || seq_length <= 288 || seq_length >= 512 || hidden_size >= 256) return false;
     const size_t problems = batch_size * num_attention_heads, head_size = hidden_size / num_attention_heads;
     if (head_size == 32) return problems <= 16 && seq_length > 320 && seq_length % 32 != 0;
     return problems <= kThreeStepProblems;
@@ -744,8 +740,8 @@ T *Transformer<T>::_in_compute(size_t batch_size, T *input_gpu, int8_t *attentio
     fp32_dense_once = false;
     bool operand_ready = false;
 
-    // long sequences: the attention kernels take the sequences longest first (the mask is the same for every layer)
-    order_ready = seq_length > 128 && attention_mask != nullptr && fused_attention_fits &&
+    // long half-precision sequences: the attention kernels take the sequences longest first (the mask is the same for every layer)
+    order_ready = sizeof(T) == 2 && seq_length > 128 && attention_mask != nullptr && fused_attention_fits &&
                   !three_step_attention_is_faster(batch_size) &&
                   cuBERT::attention_order(attention_mask, (int) batch_size, (int) seq_length, attention_order, stream);
 

@@ -935,7 +935,207 @@ __global__ __launch_bounds__(4 * kWave) void attention_small_kernel(const T *__r
     }
 }
 
-// ---- the same for longer sequences (128 < seq <= 512): online softmax over chunks of 64 keys ----
+// ---- fp32, more than 32 keys: 32 queries to a workgroup, whose wavefronts share the keys ----
+// An fp32 matrix instruction of a 32 x 32 tile takes 64 cycles, so 32 queries against 32 keys are 4096 cycles of a matrix core, and
+// with a workgroup per (batch, head) few sequences leave most of the chip without work (12 problems of 512 keys: 12 of 256
+// compute units, 134 us, 15 here).  Here a workgroup owns 32 queries of a problem and its two or four wavefronts take the live key
+// tiles in turn.  Q and K come to LDS in whole rows (a lane per row straight from memory: 16 x 12 problems of 128 keys 19.4 us, 13.1
+// so), a key tile to the wavefront that multiplies it, V straight into its registers; K and V of a head are read once per 32
+// queries, out of the die's L2, where the workgroups of a problem are neighbours.  The scores of a wavefront's tiles stay in
+// registers until the queries' maxima have been traded through LDS (the exact softmax, not an online one), and the partial contexts
+// meet there at the end, in wavefront order.  What bounds it is the fp32 matrix rate: with the chip full the matrix cores are busy
+// for 0.45 (128 keys) to 0.6 (512) of a launch, and three wavefronts per SIMD help more than V a tile ahead (512 keys, 12 x 12
+// problems 108 us, 113 with two buffers of V and two wavefronts).  Both sides at spread_is_faster.
+template <int D, int WAVES, int KT, int SPLIT, bool RAGGED>
+__global__ __launch_bounds__(WAVES * kWave, 3) void attention_spread_kernel(
+        const float *__restrict__ q, const float *__restrict__ k, const float *__restrict__ v, int ld, const int8_t *__restrict__ mask,
+        float *__restrict__ ctx, int ld_ctx, float alpha, int heads, int seq, int query_tiles, SplitOut split) {
+    constexpr int V = 4, kSteps = D / 2 / V, kColTiles = D / 32;
+    typedef Vec<float, V> Operand;
+    constexpr int kRowUnits = D / 4, kTileFloats = 32 * D;  // 16-byte units of a row; floats of a tile of Q or K
+    constexpr int kParts = WAVES / kColTiles, kWords = (WAVES * KT + 1) / 2;  // of 64 keys
+    // the queries, then a key tile per wavefront; at the end the wavefronts' contexts
+    __shared__ __align__(16) float s_tiles[(1 + WAVES) * kTileFloats];
+    __shared__ float s_max[WAVES][32], s_sum[WAVES][32];
+    const int lane = threadIdx.x & (kWave - 1);
+    const int r = lane & 31, hh = lane >> 5;
+    const int w = wave_in_block();
+    const int die = blockIdx.x & 7, die_share = gridDim.x >> 3, extra = gridDim.x & 7;
+    const int index = die * die_share + (die < extra ? die : extra) + (int) (blockIdx.x >> 3);
+    const int bh = index / query_tiles, qt = index - bh * query_tiles;
+    const int b = bh / heads, h = bh - b * heads;
+    auto valid_row = [&](int row) { return RAGGED && row >= seq ? seq - 1 : row; };
+    const size_t head = (size_t) b * seq * ld + (size_t) h * D;
+    const int8_t *mask_row = mask != nullptr ? mask + (size_t) b * seq : nullptr;
+
+    // Rows of Q and K come to LDS 1 KB a request, whole rows (a lane per row would touch a line per lane); unit u of row r sits at
+    // u ^ (r % 8).
+    auto stage = [&](const float *from, int row0, int request, float *to) {
+        const int unit = request * kWave + lane, row = unit / kRowUnits, u = unit % kRowUnits;
+        load_to_lds(from + head + (size_t) valid_row(row0 + row) * ld + (u ^ (row & 7)) * 4, to + request * kWave * 4);
+    };
+    float *s_keys = s_tiles + (1 + w) * kTileFloats;
+    auto operand = [&](const float *tile_at, int t) {  // units 2 t and 2 t + 1: lane halves
+        return load_vec<float, V>(tile_at + r * D + ((2 * t + hh) ^ (r & 7)) * 4);
+    };
+    constexpr int kRequests = kTileFloats / (kWave * 4);
+#pragma unroll
+    for (int i = 0; i < kRequests / WAVES; ++i) stage(q, qt * 32, w * (kRequests / WAVES) + i, s_tiles);
+
+    auto request_keys = [&](int at) {
+#pragma unroll
+        for (int i = 0; i < kRequests; ++i) stage(k, at * 32, i, s_keys);
+    };
+    // This wavefront's key tiles: every so many'th of those with a kept key (of all where no key is kept), or, where there is no more
+    // than one for each, the one of its number, which is asked for without a look at the mask.
+    const int tiles = (seq + 31) / 32;
+    if (KT == 1 && w < tiles) request_keys(w);
+    unsigned live = (1u << tiles) - 1u;
+    unsigned long long kept[kWords];  // bit l of word j: key 64 j + l
+    {
+        int8_t at[kWords];
+#pragma unroll
+        for (int j = 0; j < kWords; ++j) {
+            at[j] = mask_row != nullptr ? mask_row[j * kWave + lane < seq ? j * kWave + lane : seq - 1] : (int8_t) 1;
+        }
+        unsigned any = 0;
+#pragma unroll
+        for (int j = 0; j < kWords; ++j) {
+            kept[j] = __ballot(j * kWave + lane < seq && at[j] != 0);
+            any |= ((kept[j] & 0xffffffffull) != 0 ? 1u : 0u) << (2 * j) | ((kept[j] >> 32) != 0 ? 2u : 0u) << (2 * j);
+        }
+        live = any != 0 ? any : live;
+    }
+    live = __builtin_amdgcn_readfirstlane(live);
+    int tile[KT];
+    if (KT == 1) {
+        tile[0] = live >> w & 1u ? w : -1;
+    } else {
+        for (int j = 0; j < w; ++j) live &= live - 1;
+#pragma unroll
+        for (int t = 0; t < KT; ++t) {
+            tile[t] = live != 0 ? __builtin_ctz(live) : -1;
+#pragma unroll
+            for (int j = 0; j < WAVES; ++j) live &= live - 1;
+        }
+    }
+
+    if (KT > 1 && tile[0] >= 0) request_keys(tile[0]);
+    // column jt * 32 + r of V, the keys of this lane's registers
+    float values[kColTiles][16];
+    auto load_values = [&](int at) {
+        const float *column = v + head + r;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const float *row = column + (size_t) valid_row(at * 32 + acc_row(i, hh)) * ld;
+#pragma unroll
+            for (int jt = 0; jt < kColTiles; ++jt) values[jt][i] = row[jt * 32];
+        }
+    };
+
+    // register i of a tile: key acc_row(i, hh) of it, query r; in units of log 2
+    const float scale = alpha * kLog2e;
+    float p[KT][16];
+    float mx = -3.402823466e+38f;
+    wait_loads<0>();
+    __syncthreads();  // the queries are there
+#pragma unroll
+    for (int t = 0; t < KT; ++t) {
+        if (tile[t] < 0) continue;
+        if (t > 0) wait_loads<0>();
+        __builtin_amdgcn_sched_barrier(0);
+        Operand qv[kSteps], kv[kSteps];
+#pragma unroll
+        for (int s = 0; s < kSteps; ++s) qv[s] = operand(s_tiles, s), kv[s] = operand(s_keys, s);
+        __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): read, the tile may be written again
+        __builtin_amdgcn_sched_barrier(0);
+        if (t + 1 < KT && tile[t + 1 < KT ? t + 1 : 0] >= 0) request_keys(tile[t + 1 < KT ? t + 1 : 0]);
+        __builtin_amdgcn_sched_barrier(0);
+        unsigned long long word = kept[0];
+#pragma unroll
+        for (int j = 1; j < kWords; ++j) word = tile[t] / 2 == j ? kept[j] : word;
+        const unsigned bits = (unsigned) (word >> (tile[t] % 2 * 32)) >> (hh * 4);
+        float add[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            add[i] = RAGGED && tile[t] * 32 + acc_row(i, hh) >= seq ? kNoKey
+                     : bits >> acc_row(i, 0) & 1u                   ? 0.f
+                                                                    : kMaskedScore * kLog2e;
+        }
+        v16f32 c = {};
+#pragma unroll
+        for (int s = 0; s < kSteps; ++s) Mma<float>::run(c, kv[s], qv[s]);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            p[t][i] = fmaf(c[i], scale, add[i]);
+            mx = fmaxf(mx, p[t][i]);
+        }
+    }
+    if (tile[0] >= 0) load_values(tile[0]);  // on their way while the maxima are traded
+    mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
+    if (hh == 0) s_max[w][r] = mx;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < WAVES; ++j) mx = fmaxf(mx, s_max[j][r]);
+
+    float sum = 0.f;
+    v16f32 out[kColTiles];
+#pragma unroll
+    for (int jt = 0; jt < kColTiles; ++jt) out[jt] = v16f32{};
+#pragma unroll
+    for (int t = 0; t < KT; ++t) {
+        if (tile[t] < 0) continue;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            p[t][i] = __builtin_amdgcn_exp2f(p[t][i] - mx);
+            sum += p[t][i];
+        }
+#pragma unroll
+        for (int run = 0; run < 16 / V; ++run) {
+            Operand a;
+#pragma unroll
+            for (int e = 0; e < V; ++e) a.v[e] = p[t][run * V + e];
+#pragma unroll
+            for (int jt = 0; jt < kColTiles; ++jt) {
+                Operand bv;
+#pragma unroll
+                for (int e = 0; e < V; ++e) {
+                    const float x = values[jt][run * V + e];
+                    bv.v[e] = RAGGED ? keep_or_zero(x, tile[t] * 32 + acc_row(run * V + e, hh) < seq) : x;
+                }
+                Mma<float>::run(out[jt], a, bv);
+            }
+        }
+        if (t + 1 < KT && tile[t + 1 < KT ? t + 1 : 0] >= 0) load_values(tile[t + 1 < KT ? t + 1 : 0]);
+    }
+    sum += __shfl_xor(sum, 32, kWave);
+    if (hh == 0) s_sum[w][r] = sum;
+    float *s_part = s_tiles + kTileFloats;  // (over the wavefront's own keys)
+#pragma unroll
+    for (int jt = 0; jt < kColTiles; ++jt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s_part[((w * kColTiles + jt) * 16 + i) * kWave + lane] = out[jt][i];
+    __syncthreads();
+
+    // a wavefront finishes a quarter: 4 * kColTiles registers of one column tile
+    constexpr int kMine = 16 / kParts;
+    const int jt = w / kParts, first = w % kParts * kMine;
+    bool over = false;
+#pragma unroll
+    for (int i = 0; i < kMine; ++i) {
+        const int at = first + i, row = qt * 32 + acc_row(at & ~3, hh) + (i & 3), in_tile = row - qt * 32;
+        float x = s_part[(jt * 16 + at) * kWave + lane], total = s_sum[0][in_tile];
+#pragma unroll
+        for (int j = 1; j < WAVES; ++j) {
+            x += s_part[((j * kColTiles + jt) * 16 + at) * kWave + lane], total += s_sum[j][in_tile];
+        }
+        if (RAGGED && row >= seq) continue;
+        store_context<float, SPLIT>(ctx, ld_ctx, (size_t) b * seq + row, h * D + jt * 32 + r, x / total, split, over);
+    }
+    flag_overflow<SPLIT>(split, over);
+}
+
+// ---- fp16, longer sequences (128 < seq <= 512): online softmax over chunks of 64 keys ----
 // The layout is that of attention_fused_kernel (a workgroup per (batch, head), a wavefront per 32 queries, K and
 // slot-ordered V^T in LDS), but a lane cannot hold seq/2 scores, so the keys are walked in chunks: each chunk
 // updates the query's running maximum m and sum l, rescales the context accumulators by exp(m_old - m_new) and
@@ -952,12 +1152,12 @@ __global__ __launch_bounds__(4 * kWave) void attention_small_kernel(const T *__r
 // RAGGED it is read as bytes, otherwise every tile is computed.
 // RAGGED: seq is not a multiple of 32 (with the clamped rows and guarded stores in every launch: 13 x 384, 12 heads, fp16
 // 20.3 instead of 19.5 us, 32 x 256 18.5 instead of 17.1).
-template <typename T, int D, int SPLIT, bool RAGGED>
+template <typename T, int D, bool RAGGED>
 __global__ __launch_bounds__(1024) void attention_flash_kernel(const T *__restrict__ q, const T *__restrict__ k,
                                                                const T *__restrict__ v, int ld,
                                                                const int8_t *__restrict__ mask, T *__restrict__ ctx,
                                                                int ld_ctx, float alpha, int heads, int seq,
-                                                               int skip_masked_tiles, SplitOut split, const int *__restrict__ order) {
+                                                               int skip_masked_tiles, const int *__restrict__ order) {
     constexpr int V = Mma<T>::kVec;
     constexpr int kSteps = D / 2 / V;
     constexpr int kColTiles = D / 32;
@@ -1152,7 +1352,6 @@ __global__ __launch_bounds__(1024) void attention_flash_kernel(const T *__restri
     __builtin_amdgcn_s_waitcnt(0xc07f);
     __builtin_amdgcn_wave_barrier();
     const size_t first_row = (size_t) b * seq + qt * 32;
-    bool over = false;
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
         const Vec<float, 4> fr = load_vec<float, 4>(factor + g * 8 + hh * 4);
@@ -1161,12 +1360,10 @@ __global__ __launch_bounds__(1024) void attention_flash_kernel(const T *__restri
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 if (RAGGED && qt * 32 + acc_row(g * 4 + e, hh) >= seq) continue;
-                store_context<T, SPLIT>(ctx, ld_ctx, first_row + acc_row(g * 4 + e, hh), h * D + jt * 32 + r,
-                                        out[jt][g * 4 + e] * fr.v[e], split, over);
+                ctx[(first_row + acc_row(g * 4 + e, hh)) * ld_ctx + h * D + jt * 32 + r] = from_f32<T>(out[jt][g * 4 + e] * fr.v[e]);
             }
         }
     }
-    flag_overflow<SPLIT>(split, over);
 }
 
 // ---- seq 512 with the keys staged a group at a time ----
@@ -1174,14 +1371,14 @@ __global__ __launch_bounds__(1024) void attention_flash_kernel(const T *__restri
 // of a workgroup walk the live key tiles in groups of G = 32 V / D tiles (4 for fp16, head size 64): load a group
 // (one K vector and one V^T slot group per thread), barrier, online-softmax update from it, barrier, next group.  A
 // compute unit still holds one such workgroup (128 registers per lane x 16 wavefronts fill its register files), but
-// the arithmetic of the first group starts after a quarter of the loads, 40 KB of LDS are claimed instead of 148,
-// and, since the LDS no longer grows with the sequence, fp32 fits as well.  Measured at batch 64, 12 heads, ~4 live
+// the arithmetic of the first group starts after a quarter of the loads, 40 KB of LDS are claimed instead of 148.
+// Measured at batch 64, 12 heads, ~4 live
 // tiles per sequence: 54.6 against 59.5 us; groups of 2 or 8 tiles are slower.  Arithmetic and rounding are those of
 // attention_flash_kernel.
-template <typename T, int D, int SPLIT, bool ANY_SEQ>
+template <typename T, int D>
 __global__ __launch_bounds__(1024) void attention_flash_grouped_kernel(
     const T *__restrict__ q, const T *__restrict__ k, const T *__restrict__ v, int ld, const int8_t *__restrict__ mask,
-    T *__restrict__ ctx, int ld_ctx, float alpha, int heads, int any_seq, int skip_masked_tiles, SplitOut split,
+    T *__restrict__ ctx, int ld_ctx, float alpha, int heads, int skip_masked_tiles,
     const int *__restrict__ order, int order_has_records) {
     constexpr int V = Mma<T>::kVec;
     constexpr int kSteps = D / 2 / V;
@@ -1195,9 +1392,7 @@ __global__ __launch_bounds__(1024) void attention_flash_grouped_kernel(
     constexpr int kVecPerRow = D / V;
     constexpr int kLoads = G * 32 * kVecPerRow / kThreads;  // = 1: vectors per thread for K, slot groups for V^T
     static_assert(kLoads == 1, "one K vector and one V^T slot group per thread");
-    const int seq = ANY_SEQ ? any_seq : kSeq;
-    const int KT = ANY_SEQ ? (seq + 31) / 32 : kSeq / 32, S = KT * 32;
-    auto valid_row = [&](int row) { return ANY_SEQ && row >= seq ? seq - 1 : row; };
+    constexpr int seq = kSeq, KT = kSeq / 32, S = KT * 32;
     extern __shared__ __align__(16) unsigned char smem[];
     T *s_k = reinterpret_cast<T *>(smem);                                      // [G * 32][kPitchK]
     T *s_vt = s_k + G * 32 * kPitchK;                                          // [D][kPitchV], keys in slot order
@@ -1214,7 +1409,7 @@ __global__ __launch_bounds__(1024) void attention_flash_grouped_kernel(
     const T *k_head = k + (size_t) b * seq * ld + (size_t) h * D;
     const T *v_head = v + (size_t) b * seq * ld + (size_t) h * D;
 
-    const T *q_row = q + ((size_t) b * seq + valid_row(qt * 32 + r)) * ld + (size_t) h * D + hh * (D / 2);
+    const T *q_row = q + ((size_t) b * seq + (qt * 32 + r)) * ld + (size_t) h * D + hh * (D / 2);
     Vec<T, V> qv[kSteps];
 #pragma unroll
     for (int t = 0; t < kSteps; ++t) qv[t] = load_vec<T, V>(q_row + t * V);
@@ -1242,13 +1437,6 @@ __global__ __launch_bounds__(1024) void attention_flash_grouped_kernel(
 #pragma unroll
                 for (int i = 0; i < 8; ++i) any |= words[kt * 8 + i];
                 if (any != 0) tile_list |= (unsigned long long) kt << (4 * n_live++);
-            }
-        }
-        if (ANY_SEQ && mask != nullptr && !skip_masked_tiles) {  // (the row cannot be read as words)
-            unsigned any, all;
-            key_tile_bits(mask + (size_t) b * seq, seq, KT, any, all);
-            for (int kt = 0; kt < KT; ++kt) {
-                if ((any >> kt) & 1u) tile_list |= (unsigned long long) kt << (4 * n_live++);
             }
         }
         if (n_live == 0) {  // no mask, or no kept key at all: every tile
@@ -1284,7 +1472,7 @@ __global__ __launch_bounds__(1024) void attention_flash_grouped_kernel(
             const int slot = idx / (32 * kVecPerRow), within = idx - slot * (32 * kVecPerRow);
             const int row = within / kVecPerRow, c = within - row * kVecPerRow;
             kreg[u] = Vec<T, V>{};
-            if (slot < in_group) kreg[u] = load_vec<T, V>(k_head + (size_t) valid_row(tile_of(slot) * 32 + row) * ld + c * V);
+            if (slot < in_group) kreg[u] = load_vec<T, V>(k_head + (size_t) (tile_of(slot) * 32 + row) * ld + c * V);
         }
 #pragma unroll
         for (int u = 0; u < kLoads; ++u) {
@@ -1297,7 +1485,7 @@ __global__ __launch_bounds__(1024) void attention_flash_grouped_kernel(
                 const int kt = tile_of(slot);
 #pragma unroll
                 for (int e = 0; e < V; ++e) {
-                    vreg[u].v[e] = v_head[(size_t) valid_row(kt * 32 + acc_row(run * V + e, half)) * ld + j];
+                    vreg[u].v[e] = v_head[(size_t) (kt * 32 + acc_row(run * V + e, half)) * ld + j];
                 }
             }
         }
@@ -1312,11 +1500,9 @@ __global__ __launch_bounds__(1024) void attention_flash_grouped_kernel(
         for (int u = 0; u < kLoads; ++u) {
             const int idx = threadIdx.x + u * kThreads;
             const int j = idx % D, grp = idx / D;
-            if (ANY_SEQ && grp / (32 / V) < in_group) zero_missing_keys<T, V>(vreg[u], grp, tile_of(grp / (32 / V)), seq);
             store_vec<T, V>(s_vt + j * kPitchV + grp * V, vreg[u]);
         }
         __syncthreads();
-        if (ANY_SEQ && qt >= KT) continue;  // a wavefront without queries helps with the loads only
         for (int s0 = 0; s0 < in_group; s0 += kChunk) {  // the group's tiles in ascending order, kChunk per step
             int tiles[kChunk], slots[kChunk];
 #pragma unroll
@@ -1400,13 +1586,11 @@ __global__ __launch_bounds__(1024) void attention_flash_grouped_kernel(
             }
         }
     }
-    if (ANY_SEQ && qt >= KT) return;
     // divide row (query) i by its sum
     if (hh == 0) factor[r] = 1.f / l;
     __builtin_amdgcn_s_waitcnt(0xc07f);
     __builtin_amdgcn_wave_barrier();
     const size_t first_row = (size_t) b * seq + qt * 32;
-    bool over = false;
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
         const Vec<float, 4> fr = load_vec<float, 4>(factor + g * 8 + hh * 4);
@@ -1414,13 +1598,10 @@ __global__ __launch_bounds__(1024) void attention_flash_grouped_kernel(
         for (int jt = 0; jt < kColTiles; ++jt) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                if (ANY_SEQ && qt * 32 + acc_row(g * 4 + e, hh) >= seq) continue;
-                store_context<T, SPLIT>(ctx, ld_ctx, first_row + acc_row(g * 4 + e, hh), h * D + jt * 32 + r,
-                                        out[jt][g * 4 + e] * fr.v[e], split, over);
+                ctx[(first_row + acc_row(g * 4 + e, hh)) * ld_ctx + h * D + jt * 32 + r] = from_f32<T>(out[jt][g * 4 + e] * fr.v[e]);
             }
         }
     }
-    flag_overflow<SPLIT>(split, over);
 }
 
 // ---- longest sequences first ----
@@ -1686,11 +1867,11 @@ int launch_fused(const T *q, const T *k, const T *v, int ld, const int8_t *mask,
 #undef CUBERT_FUSED_KT
 }
 
-// 128 < seq <= 512.  seq 512 walks the keys in groups; other lengths hold K and V of the head in LDS where they fit
-// (fp16 always, fp32 up to 288 keys at head size 64) and walk them in groups where they do not.
-template <typename T, int D, int SPLIT>
-int launch_flash(const T *q, const T *k, const T *v, int ld, const int8_t *mask, T *ctx, int ld_ctx, float alpha,
-                 int batch, int heads, int seq, SplitOut split, const int *order, hipStream_t s) {
+// fp16, 128 < seq <= 512.  seq 512 walks the keys in groups, other lengths hold K and V of the head in LDS.
+template <int D>
+int launch_flash(const half_t *q, const half_t *k, const half_t *v, int ld, const int8_t *mask, half_t *ctx, int ld_ctx, float alpha,
+                 int batch, int heads, int seq, const int *order, hipStream_t s) {
+    typedef half_t T;
     constexpr int V = 16 / sizeof(T);
     if (seq > 512) return CUBERT_UNSUPPORTED;  // a workgroup has at most 16 wavefronts
     const int tiles = (seq + 31) / 32, padded = tiles * 32;
@@ -1700,7 +1881,7 @@ int launch_flash(const T *q, const T *k, const T *v, int ld, const int8_t *mask,
     const int skip_masked_tiles = mask != nullptr && is_aligned(mask, 4) && seq % 32 == 0;
     static const bool whole_head = getenv("CUBERT_FLASH_WHOLE") != nullptr;
     const dim3 grid(batch * heads);
-    if ((seq == 512 && !whole_head) || lds > 160 * 1024) {
+    if (seq == 512 && !whole_head) {
         constexpr int G = 32 * V / D;
         // CUBERT_FLASH_RECORDS=0 in the environment: the kernel reads the mask row itself instead of the order array's
         // records (for comparison)
@@ -1710,23 +1891,56 @@ int launch_flash(const T *q, const T *k, const T *v, int ld, const int8_t *mask,
         }();
         const size_t grouped_lds = ((size_t) G * 32 * (D + V) + (size_t) D * (G * 32 + V)) * sizeof(T) +
                                    ((size_t) padded + 16 * 32) * sizeof(float);
-        if (seq == 512) {
-            return launch_attention<attention_flash_grouped_kernel<T, D, SPLIT, false>>(
-                grid, dim3(1024), grouped_lds, s, q, k, v, ld, mask, ctx, ld_ctx, alpha, heads, seq, skip_masked_tiles,
-                split, order, use_records);
-        }
-        return launch_attention<attention_flash_grouped_kernel<T, D, SPLIT, true>>(
-            grid, dim3(1024), grouped_lds, s, q, k, v, ld, mask, ctx, ld_ctx, alpha, heads, seq, skip_masked_tiles, split,
-            order, use_records);
+        return launch_attention<attention_flash_grouped_kernel<T, D>>(grid, dim3(1024), grouped_lds, s, q, k, v, ld, mask, ctx,
+                                                                      ld_ctx, alpha, heads, skip_masked_tiles, order, use_records);
     }
     if (seq % 32 == 0) {
-        return launch_attention<attention_flash_kernel<T, D, SPLIT, false>>(grid, dim3(tiles * kWave), lds, s, q, k, v, ld, mask,
-                                                                            ctx, ld_ctx, alpha, heads, seq,
-                                                                            skip_masked_tiles, split, order);
+        return launch_attention<attention_flash_kernel<T, D, false>>(grid, dim3(tiles * kWave), lds, s, q, k, v, ld, mask, ctx,
+                                                                     ld_ctx, alpha, heads, seq, skip_masked_tiles, order);
     }
-    return launch_attention<attention_flash_kernel<T, D, SPLIT, true>>(grid, dim3(tiles * kWave), lds, s, q, k, v, ld, mask, ctx,
-                                                                       ld_ctx, alpha, heads, seq, skip_masked_tiles, split,
-                                                                       order);
+    return launch_attention<attention_flash_kernel<T, D, true>>(grid, dim3(tiles * kWave), lds, s, q, k, v, ld, mask, ctx, ld_ctx,
+                                                                alpha, heads, seq, skip_masked_tiles, order);
+}
+
+template <int D, int WAVES, int KT, int SPLIT>
+int launch_spread_kt(const float *q, const float *k, const float *v, int ld, const int8_t *mask, float *ctx, int ld_ctx, float alpha,
+                     int batch, int heads, int seq, SplitOut split, hipStream_t s) {
+    const int query_tiles = (seq + 31) / 32;
+    auto kernel = seq % 32 != 0 ? attention_spread_kernel<D, WAVES, KT, SPLIT, true> : attention_spread_kernel<D, WAVES, KT, SPLIT, false>;
+    return launch(kernel, dim3((unsigned) (batch * heads * query_tiles)), dim3(WAVES * kWave), s, q, k, v, ld, mask, ctx, ld_ctx,
+                  alpha, heads, seq, query_tiles, split);
+}
+
+template <int D, int SPLIT>
+int launch_spread(const float *q, const float *k, const float *v, int ld, const int8_t *mask, float *ctx, int ld_ctx, float alpha,
+                  int batch, int heads, int seq, SplitOut split, hipStream_t s) {
+#define CUBERT_SPREAD(WAVES, KT) \
+    return launch_spread_kt<D, WAVES, KT, SPLIT>(q, k, v, ld, mask, ctx, ld_ctx, alpha, batch, heads, seq, split, s)
+    if (seq <= 64) CUBERT_SPREAD(2, 1);
+    switch ((seq + 127) / 128) {
+        case 1: CUBERT_SPREAD(4, 1);
+        case 2: CUBERT_SPREAD(4, 2);
+        case 3: CUBERT_SPREAD(4, 3);
+        case 4: CUBERT_SPREAD(4, 4);
+        default: return CUBERT_UNSUPPORTED;
+    }
+#undef CUBERT_SPREAD
+}
+
+// fp32: whether 32 queries to a workgroup beat a problem to a workgroup.  That is so unless the problems of a short sequence fill the
+// chip's 256 compute units evenly by themselves.  Microseconds, 32 queries / a problem (of head size 64, unless marked with 32):
+//   seq  40   8 x 12 problems 8.1 / 10.0, 12 x 12 10.8 / 10.1, 16 x 12 10.8 / 10.2, 24 x 12 11.1 / 15.1, 64 x 12 16.2 / 16.7; 32: 64 x 12 11.4 / 9.8
+//   seq  64   1 x 12 6.7 / 8.3, 16 x 12 9.8 / 9.0, 24 x 12 10.4 / 14.0, 100 x 12 26.9 / 29.6; 32: 48 x 12 9.0 / 9.4, 64 x 12 10.9 / 9.8
+//   seq 100   1 x 12 7.3 / 14.4, 20 x 12 16.6 / 16.3, 48 x 12 36.7 / 38.9, 64 x 12 46.5 / 41.5; 32: 48 x 12 20.7 / 20.6, 64 x 12 26.2 / 21.5
+//   seq 128   4 x 12 6.7 / 13.1, 16 x 12 13.0 / 14.7, 48 x 12 34.3 / 39.5, 64 x 12 43.6 / 41.8; 32: 48 x 12 19.5 / 20.7, 64 x 12 25.4 / 22.7
+// Longer sequences had an online softmax over their keys by a wavefront per 32 queries, all of a problem's on one compute unit:
+//   seq 200   1 x 12 10.7 / 36.9, 16 x 12 41.5 / 40.5, 32 x 12 70.3 / 80.0; 256: 4 x 12 15.4 / 39.5, 16 x 12 42.9 / 44.2; 384: 4 x 12 32.0 / 85.7, 16
+//   x 12 86.8 / 92.3; 450: 8 x 12 73.5 / 140.9, 16 x 12 139.7 / 142.3; 512: 1 x 12 16.4 / 137.8, 12 x 12 108 / 148; 32: 512 1 x 12 10.5 / 72.6, 16
+//   x 12 76.0 / 77.9, 450 16 x 12 78.2 / 75.4.
+bool spread_is_faster(int problems, int seq, int head_size) {
+    if (seq <= 32) return false;
+    if (seq <= 64) return problems <= 128 || (problems > 256 && (head_size == 64 || problems <= 512));
+    return seq > 128 || problems <= 600;
 }
 
 template <typename T>
@@ -1740,21 +1954,24 @@ int attention_fused(const T *q, const T *k, const T *v, int ld, const int8_t *ma
     }
     hipStream_t s = (hipStream_t) stream;
 #define CUBERT_ATTENTION_ARGS q, k, v, ld, mask, ctx, ld_ctx, alpha, batch, heads, seq, split
+    if constexpr (sizeof(T) == 4) {
+        if (head_size <= 64 && spread_is_faster(batch * heads, seq, head_size)) {
+#define CUBERT_SPREAD_FORM(FORM)                                                                    \
+    return head_size == 32 ? launch_spread<32, FORM>(CUBERT_ATTENTION_ARGS, s) : launch_spread<64, FORM>(CUBERT_ATTENTION_ARGS, s)
+            if (split.width == 0) CUBERT_SPREAD_FORM(kPlain);
+            if (split.pairs) CUBERT_SPREAD_FORM(kPairRows);
+            CUBERT_SPREAD_FORM(kThirdRows);
+#undef CUBERT_SPREAD_FORM
+        }
+    }
     if (seq > 128) {
         if (head_size == 128) return CUBERT_UNSUPPORTED;  // would spill the accumulators to scratch
-        if constexpr (sizeof(T) == 4) {
-            if (split.width > 0) {
-                if (split.pairs) {
-                    return head_size == 32 ? launch_flash<T, 32, kPairRows>(CUBERT_ATTENTION_ARGS, order, s)
-                                           : launch_flash<T, 64, kPairRows>(CUBERT_ATTENTION_ARGS, order, s);
-                }
-                return head_size == 32 ? launch_flash<T, 32, kThirdRows>(CUBERT_ATTENTION_ARGS, order, s)
-                                       : launch_flash<T, 64, kThirdRows>(CUBERT_ATTENTION_ARGS, order, s);
-            }
+        if constexpr (sizeof(T) == 2) {
+            if (split.width > 0) return CUBERT_UNSUPPORTED;
+            return head_size == 32 ? launch_flash<32>(q, k, v, ld, mask, ctx, ld_ctx, alpha, batch, heads, seq, order, s)
+                                   : launch_flash<64>(q, k, v, ld, mask, ctx, ld_ctx, alpha, batch, heads, seq, order, s);
         }
-        if (split.width > 0) return CUBERT_UNSUPPORTED;
-        return head_size == 32 ? launch_flash<T, 32, kPlain>(CUBERT_ATTENTION_ARGS, order, s)
-                               : launch_flash<T, 64, kPlain>(CUBERT_ATTENTION_ARGS, order, s);
+        return CUBERT_UNSUPPORTED;
     }
     const bool ragged = seq % 32 != 0;
     switch (head_size) {
