@@ -99,6 +99,7 @@ SIGNATURES = {
     "cubert_event_record": (ci, [vp, vp]),
     "cubert_event_elapsed_ms": (ci, [vp, vp, ctypes.POINTER(cf)]),
     "cubert_time_next_launch": (ci, [vp, vp]),
+    "cubert_attention_wants_order": (ci, [ci, ci, ci, ci, ci]),
     "cubert_attention_order": (ci, [vp, ci, ci, vp, vp]),
     "cubert_attention_fused_ordered_f32": (ci, [vp, vp, vp, ci, vp, vp, vp, ci, cf, ci, ci, ci, ci, vp]),
     "cubert_attention_fused_ordered_f16": (ci, [vp, vp, vp, ci, vp, vp, vp, ci, cf, ci, ci, ci, ci, vp]),

@@ -741,8 +741,9 @@ T *Transformer<T>::_in_compute(size_t batch_size, T *input_gpu, int8_t *attentio
     bool operand_ready = false;
 
     // long half-precision sequences: the attention kernels take the sequences longest first (the mask is the same for every layer)
-    order_ready = sizeof(T) == 2 && seq_length > 128 && attention_mask != nullptr && fused_attention_fits &&
-                  !three_step_attention_is_faster(batch_size) &&
+    order_ready = attention_mask != nullptr && fused_attention_fits && !three_step_attention_is_faster(batch_size) &&
+                  cubert_attention_wants_order(sizeof(T) == 2, (int) batch_size, (int) num_attention_heads, (int) seq_length,
+                                               (int) (hidden_size / num_attention_heads)) &&
                   cuBERT::attention_order(attention_mask, (int) batch_size, (int) seq_length, attention_order, stream);
 
     T *prev_output = input_gpu;

@@ -1135,6 +1135,261 @@ __global__ __launch_bounds__(WAVES * kWave, 3) void attention_spread_kernel(
     flag_overflow<SPLIT>(split, over);
 }
 
+// ---- fp16: 32 queries to a workgroup, whose wavefronts share the keys ----
+// The arithmetic of attention_fused_half_kernel in the shape of attention_spread_kernel: up to 384 keys two or four wavefronts with one
+// to three of the live key tiles each, beyond eight with two (512 keys, 1 x 12 problems 6.5 us, 6.9 with four of four).  K and V
+// tiles come to LDS of the wavefront that uses them in whole rows, V in the place of the K tile that has been read.  The row sums and
+// the context are added over the wavefronts through LDS, four columns of a row to a thread.  For few or short sequences its time is
+// the chain Q and K, maxima, V, sums: 12 problems of 128 keys 5.2 -> 3.9 us, of 384 16.4 -> 5.9, of 512 23.2 -> 6.5; with the chip full
+// it is the L2 (64 x 12 problems of 512 keys read 1.6 GB in 164 us where a workgroup per problem takes 88), so those stay with a
+// workgroup per problem: spread_half_is_faster.
+template <int D, int WAVES, int KT>
+struct SpreadHalf {
+    static constexpr int kTileBytes = 32 * D * 2, kPartBytes = D * 32 * 4;  // of Q, K or V; of a wavefront's context
+    static constexpr int kWaveBytes = KT * kTileBytes > kPartBytes ? KT * kTileBytes : kPartBytes;
+    static constexpr int kLdsBytes = kTileBytes + WAVES * (kWaveBytes + 2 * 32 * 4);
+};
+
+template <int D, int WAVES, int KT, bool RAGGED>
+__global__ __launch_bounds__(WAVES * kWave, 4) void attention_spread_half_kernel(
+        const half_t *__restrict__ q, const half_t *__restrict__ k, const half_t *__restrict__ v, int ld,
+        const int8_t *__restrict__ mask, half_t *__restrict__ ctx, int ld_ctx, float alpha, int heads, int seq, int query_tiles) {
+    constexpr int V = 8, kSteps = D / 2 / V, kColTiles = D / 32, kUnits = D / V;  // 16-byte units of a row
+    typedef SpreadHalf<D, WAVES, KT> S;
+    constexpr int kTileBytes = S::kTileBytes, kWaveBytes = S::kWaveBytes, kRequests = kTileBytes / 1024, kWords = (WAVES * KT + 1) / 2;
+    typedef Vec<half_t, V> Operand;
+    extern __shared__ __align__(16) unsigned char smem[];
+    unsigned char *s_tiles = smem;  // the queries, then a wavefront's tiles, later its context
+    float (*s_max)[32] = reinterpret_cast<float (*)[32]>(smem + kTileBytes + WAVES * kWaveBytes), (*s_sum)[32] = s_max + WAVES;
+    const int lane = threadIdx.x & (kWave - 1);
+    const int r = lane & 31, hh = lane >> 5;
+    const int w = wave_in_block();
+    const int die = blockIdx.x & 7, die_share = gridDim.x >> 3, extra = gridDim.x & 7;
+    const int index = die * die_share + (die < extra ? die : extra) + (int) (blockIdx.x >> 3);
+    const int bh = index / query_tiles, qt = index - bh * query_tiles;
+    const int b = bh / heads, h = bh - b * heads;
+    auto valid_row = [&](int row) { return RAGGED && row >= seq ? seq - 1 : row; };
+    const size_t head = (size_t) b * seq * ld + (size_t) h * D;
+    const int8_t *mask_row = mask != nullptr ? mask + (size_t) b * seq : nullptr;
+
+    // where unit u of row r sits in LDS: operand reads of Q and K (a row per lane) and transposing reads of V (four rows of 64 bytes
+    // for 32 lanes) hit all banks
+    auto key_unit = [](int row, int u) { return D == 64 ? u ^ (row >> 1 & 7) : u ^ (row >> 2 & 3); };
+    auto value_unit = [](int row, int u) { return D == 64 ? u ^ (row >> 1 & 1) << 2 : u; };
+    auto stage = [&](const half_t *from, int row0, int request, unsigned char *to, auto place) {
+        const int unit = request * kWave + lane, row = unit / kUnits, u = unit % kUnits;
+        load_to_lds(from + head + (size_t) valid_row(row0 + row) * ld + place(row, u) * V, to + request * 1024);
+    };
+    unsigned char *mine = s_tiles + kTileBytes + w * kWaveBytes;
+    auto request_keys = [&](int at, int slot) {
+#pragma unroll
+        for (int i = 0; i < kRequests; ++i) stage(k, at * 32, i, mine + slot * kTileBytes, key_unit);
+    };
+    auto request_values = [&](int at, int slot) {
+#pragma unroll
+        for (int i = 0; i < kRequests; ++i) stage(v, at * 32, i, mine + slot * kTileBytes, value_unit);
+    };
+    auto operand = [&](const unsigned char *tile_at, int t) {
+        return load_vec<half_t, V>(reinterpret_cast<const half_t *>(tile_at + r * D * 2 + key_unit(r, hh * kSteps + t) * 16));
+    };
+    if (w < kRequests) stage(q, qt * 32, w, s_tiles, key_unit);
+    static_assert(kRequests <= 2 * WAVES, "two requests of a wavefront are all of the queries");
+    if (kRequests > WAVES && w + WAVES < kRequests) stage(q, qt * 32, w + WAVES, s_tiles, key_unit);
+
+    // this wavefront's key tiles, as in attention_spread_kernel
+    const int tiles = (seq + 31) / 32;
+    if (KT == 1 && w < tiles) request_keys(w, 0);
+    unsigned live = (1u << tiles) - 1u;
+    unsigned long long kept[kWords];  // bit l of word j: key 64 j + l
+    {
+        int8_t at[kWords];
+#pragma unroll
+        for (int j = 0; j < kWords; ++j) {
+            at[j] = mask_row != nullptr ? mask_row[j * kWave + lane < seq ? j * kWave + lane : seq - 1] : (int8_t) 1;
+        }
+        unsigned any = 0;
+#pragma unroll
+        for (int j = 0; j < kWords; ++j) {
+            kept[j] = __ballot(j * kWave + lane < seq && at[j] != 0);
+            any |= ((kept[j] & 0xffffffffull) != 0 ? 1u : 0u) << (2 * j) | ((kept[j] >> 32) != 0 ? 2u : 0u) << (2 * j);
+        }
+        live = any != 0 ? any : live;
+    }
+    live = __builtin_amdgcn_readfirstlane(live);
+    int tile[KT];
+    if (KT == 1) {
+        tile[0] = live >> w & 1u ? w : -1;
+    } else {
+        for (int j = 0; j < w; ++j) live &= live - 1;
+#pragma unroll
+        for (int t = 0; t < KT; ++t) {
+            tile[t] = live != 0 ? __builtin_ctz(live) : -1;
+#pragma unroll
+            for (int j = 0; j < WAVES; ++j) live &= live - 1;
+            if (tile[t] >= 0) request_keys(tile[t], t);
+        }
+    }
+
+    // register i of a tile: key acc_row(i, hh) of it, query r: raw products where all its keys are kept, else masked scores in
+    // units of log 2
+    const float scale = alpha * kLog2e;
+    v16f32 p[KT];
+    bool whole[KT];
+    float mx = -3.402823466e+38f;
+    wait_loads<0>();
+    __syncthreads();  // the queries are there, and this wavefront's keys
+    Operand qv[kSteps];
+#pragma unroll
+    for (int t = 0; t < kSteps; ++t) qv[t] = operand(s_tiles, t);
+#pragma unroll
+    for (int t = 0; t < KT; ++t) {
+        whole[t] = false;
+        if (tile[t] < 0) continue;
+        Operand kv[kSteps];
+#pragma unroll
+        for (int s = 0; s < kSteps; ++s) kv[s] = operand(mine + t * kTileBytes, s);
+        __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): read, V may come
+        __builtin_amdgcn_sched_barrier(0);
+        request_values(tile[t], t);
+        __builtin_amdgcn_sched_barrier(0);
+        v16f32 c = {};
+#pragma unroll
+        for (int s = 0; s < kSteps; ++s) Mma<half_t>::run(c, kv[s], qv[s]);
+        unsigned long long word = kept[0];
+#pragma unroll
+        for (int j = 1; j < kWords; ++j) word = tile[t] / 2 == j ? kept[j] : word;
+        unsigned bits = (unsigned) (word >> (tile[t] % 2 * 32));
+        whole[t] = bits == ~0u && alpha > 0.f;  // (the maximum is taken before scaling)
+        if (whole[t]) {
+            asm volatile("");
+            float raw = c[0];
+#pragma unroll
+            for (int i = 1; i < 16; ++i) raw = fmaxf(raw, c[i]);
+            mx = fmaxf(mx, raw * scale);
+        } else {
+            asm volatile("");
+            bits >>= hh * 4;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const float add = RAGGED && tile[t] * 32 + acc_row(i, hh) >= seq ? kNoKey
+                                  : bits >> acc_row(i, 0) & 1u                   ? 0.f
+                                                                                 : kMaskedScore * kLog2e;
+                c[i] = fmaf(c[i], scale, add);
+                mx = fmaxf(mx, c[i]);
+            }
+        }
+        p[t] = c;
+    }
+    mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
+    if (hh == 0) s_max[w][r] = mx;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < WAVES; ++j) mx = fmaxf(mx, s_max[j][r]);
+    const float shift = -mx;
+
+    v16f32 out[kColTiles], total = {};
+#pragma unroll
+    for (int jt = 0; jt < kColTiles; ++jt) out[jt] = v16f32{};
+    Operand ones;
+#pragma unroll
+    for (int e = 0; e < V; ++e) ones.v[e] = (half_t) 1.f;
+    // (lds_read_transposed: lane i of a group of 16 names row i / 4 and column block i % 4 of a patch)
+    const int tr_group = lane >> 4, tr_i = lane & 15;
+    const int tr_row = (tr_group >> 1) * 4 + (tr_i >> 2), tr_column = (tr_group & 1) * 16 + (tr_i & 3) * 4;
+#pragma unroll
+    for (int t = 0; t < KT; ++t) {
+        if (tile[t] < 0) continue;
+        asm volatile("");
+        Operand a[16 / V];
+        if (whole[t]) {
+            asm volatile("");
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                a[i / V].v[i % V] = from_f32<half_t>(__builtin_amdgcn_exp2f(fmaf(p[t][i], scale, shift)));
+            }
+        } else {
+            asm volatile("");
+#pragma unroll
+            for (int i = 0; i < 16; ++i) a[i / V].v[i % V] = from_f32<half_t>(__builtin_amdgcn_exp2f(p[t][i] + shift));
+        }
+        if (tile[KT - 1] >= 0) {  // V of the tiles behind this one may still be on its way
+            if (t == 0) wait_loads<(KT - 1) * kRequests>();
+            if (t == 1) wait_loads<(KT > 2 ? KT - 2 : 0) * kRequests>();
+            if (t == 2) wait_loads<(KT > 3 ? KT - 3 : 0) * kRequests>();
+            if (t == 3) wait_loads<0>();
+        } else {
+            wait_loads<0>();
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        unsigned char *values = mine + t * kTileBytes;
+        if (RAGGED && tile[t] * 32 + 32 > seq) {  // rows past the end count as zeros
+#pragma unroll
+            for (int i = 0; i < kRequests; ++i) {
+                const int unit = i * kWave + lane;
+                if (tile[t] * 32 + unit / kUnits >= seq) store_vec<half_t, V>(reinterpret_cast<half_t *>(values + unit * 16), Operand{});
+            }
+            __builtin_amdgcn_s_waitcnt(0xc07f);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int run = 0; run < 16 / V; ++run) {
+#pragma unroll
+            for (int jt = 0; jt < kColTiles; ++jt) {
+                const int column = jt * 32 + tr_column;
+                auto patch = [&](int row) {
+                    return lds_read_transposed(reinterpret_cast<const half_t *>(values + row * D * 2 + value_unit(row, column / V) * 16) +
+                                               column % V);
+                };
+                const v4f16 lo = patch(run * 16 + tr_row), hi = patch(run * 16 + 8 + tr_row);
+                Operand bv;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) bv.v[e] = lo[e], bv.v[4 + e] = hi[e];
+                Mma<half_t>::run(out[jt], a[run], bv);
+            }
+            Mma<half_t>::run(total, a[run], ones);
+        }
+    }
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // this wavefront's tiles have been read
+    __builtin_amdgcn_sched_barrier(0);
+    // column jt * 32 + r of the rows acc_row(i, hh)
+    float *part = reinterpret_cast<float *>(mine);
+#pragma unroll
+    for (int jt = 0; jt < kColTiles; ++jt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) part[(jt * 16 + i) * kWave + lane] = out[jt][i];
+    if (r == 0) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s_sum[w][acc_row(i, hh)] = total[i];
+    }
+    __syncthreads();
+    constexpr int kQuads = 32 * D / 4, kEach = (kQuads + WAVES * kWave - 1) / (WAVES * kWave);
+#pragma unroll
+    for (int n = 0; n < kEach; ++n) {
+        const int item = n * WAVES * kWave + threadIdx.x;
+        if (kQuads % (WAVES * kWave) != 0 && item >= kQuads) break;
+        // D / 4 threads to a row: columns 4 c ... of row acc_row(i, half)
+        const int in_tile = item / (D / 4), c = item % (D / 4);
+        const int i = in_tile / 8 * 4 + in_tile % 4, half = in_tile / 4 % 2;
+        const int at = (c / 8 * 16 + i) * kWave + half * 32 + c % 8 * 4;
+        Vec<float, 4> x = load_vec<float, 4>(reinterpret_cast<const float *>(s_tiles + kTileBytes) + at);
+        float sum = s_sum[0][in_tile];
+#pragma unroll
+        for (int j = 1; j < WAVES; ++j) {
+            const Vec<float, 4> y = load_vec<float, 4>(reinterpret_cast<const float *>(s_tiles + kTileBytes + j * kWaveBytes) + at);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x.v[e] += y.v[e];
+            sum += s_sum[j][in_tile];
+        }
+        const int row = qt * 32 + in_tile;
+        if (RAGGED && row >= seq) continue;
+        const float inv = 1.f / sum;
+        Vec<half_t, 4> y;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y.v[e] = from_f32<half_t>(x.v[e] * inv);
+        store_vec<half_t, 4>(ctx + ((size_t) b * seq + row) * ld_ctx + h * D + c * 4, y);
+    }
+}
+
 // ---- fp16, longer sequences (128 < seq <= 512): online softmax over chunks of 64 keys ----
 // The layout is that of attention_fused_kernel (a workgroup per (batch, head), a wavefront per 32 queries, K and
 // slot-ordered V^T in LDS), but a lane cannot hold seq/2 scores, so the keys are walked in chunks: each chunk
@@ -1927,6 +2182,34 @@ int launch_spread(const float *q, const float *k, const float *v, int ld, const 
 #undef CUBERT_SPREAD
 }
 
+template <int D, int WAVES, int KT>
+int launch_spread_half_kt(const half_t *q, const half_t *k, const half_t *v, int ld, const int8_t *mask, half_t *ctx, int ld_ctx,
+                          float alpha, int batch, int heads, int seq, hipStream_t s) {
+    const int query_tiles = (seq + 31) / 32;
+    const dim3 grid((unsigned) (batch * heads * query_tiles)), block(WAVES * kWave);
+    constexpr size_t lds = SpreadHalf<D, WAVES, KT>::kLdsBytes;
+    if (seq % 32 != 0) {
+        return launch_attention<attention_spread_half_kernel<D, WAVES, KT, true>>(grid, block, lds, s, q, k, v, ld, mask, ctx, ld_ctx,
+                                                                                  alpha, heads, seq, query_tiles);
+    }
+    return launch_attention<attention_spread_half_kernel<D, WAVES, KT, false>>(grid, block, lds, s, q, k, v, ld, mask, ctx, ld_ctx,
+                                                                               alpha, heads, seq, query_tiles);
+}
+
+template <int D>
+int launch_spread_half(const half_t *q, const half_t *k, const half_t *v, int ld, const int8_t *mask, half_t *ctx, int ld_ctx,
+                       float alpha, int batch, int heads, int seq, hipStream_t s) {
+#define CUBERT_SPREAD(WAVES, KT) \
+    return launch_spread_half_kt<D, WAVES, KT>(q, k, v, ld, mask, ctx, ld_ctx, alpha, batch, heads, seq, s)
+    if (seq <= 64) CUBERT_SPREAD(2, 1);
+    if (seq <= 128) CUBERT_SPREAD(4, 1);
+    if (seq <= 256) CUBERT_SPREAD(4, 2);
+    if (seq <= 384) CUBERT_SPREAD(4, 3);
+    if (seq <= 512) CUBERT_SPREAD(8, 2);
+    return CUBERT_UNSUPPORTED;
+#undef CUBERT_SPREAD
+}
+
 // fp32: whether 32 queries to a workgroup beat a problem to a workgroup.  That is so unless the problems of a short sequence fill the
 // chip's 256 compute units evenly by themselves.  Microseconds, 32 queries / a problem (of head size 64, unless marked with 32):
 //   seq  40   8 x 12 problems 8.1 / 10.0, 12 x 12 10.8 / 10.1, 16 x 12 10.8 / 10.2, 24 x 12 11.1 / 15.1, 64 x 12 16.2 / 16.7; 32: 64 x 12 11.4 / 9.8
@@ -1941,6 +2224,25 @@ bool spread_is_faster(int problems, int seq, int head_size) {
     if (seq <= 32) return false;
     if (seq <= 64) return problems <= 128 || (problems > 256 && (head_size == 64 || problems <= 512));
     return seq > 128 || problems <= 600;
+}
+
+// fp16: the same question.  K and V go to every 32 queries out of the L2, which is what the time goes to once the chip is full, so
+// the answer goes by the number of workgroups.  Where the length is no multiple of 32 the other kernels of short sequences are
+// slower.  Microseconds, 32 queries to a workgroup / a problem to a workgroup, 12 heads of 64, every key kept (kept between a quarter
+// and all of them):
+//   seq  48   8 x 12 problems 4.3 / 5.1, 24 x 12 4.9 / 6.2, 48 x 12 6.5 / 7.0; 64: 8 x 12 3.8 / 3.9, 13 x 12 4.2 / 4.0
+//   seq 100   1 x 12 4.2 / 6.0, 16 x 12 6.0 / 6.6, 20 x 12 6.9 / 6.7; 128: 1 x 12 3.9 / 5.2, 8 x 12 4.8 / 5.4, 13 x 12 5.8 / 5.7
+//   seq 160   4 x 12 5.0 / 8.3, 16 x 12 7.9 / 9.0 (7.8 / 8.8), 20 x 12 10.2 / 9.1; 256: 4 x 12 6.4 / 10.4 (6.0 / 8.8), 10 x 12 9.5 / 11.2
+//             (8.7 / 10.9), 13 x 12 12.0 / 11.5
+//   seq 320   1 x 12 5.7 / 14.3 (4.8 / 8.3), 8 x 12 12.6 / 15.8 (12.9 / 15.3), 10 x 12 16.7 / 16.2; 384: 6 x 12 13.1 / 17.7 (12.2 / 15.0),
+//             10 x 12 19.5 / 18.9
+//   seq 512   1 x 12 6.5 / 23.2 (5.3 / 9.2), 6 x 12 19.6 / 25.0 (17.2 / 17.6), 8 x 12 23.0 / 25.7 (22.1 / 22.2), 10 x 12 30.3 / 26.9
+bool spread_half_is_faster(int problems, int seq, int head_size) {
+    if (seq <= 32 || seq > 512 || head_size > 64) return false;
+    const long long workgroups = (long long) problems * ((seq + 31) / 32);
+    if (seq <= 64) return workgroups <= (seq % 32 != 0 ? 1200 : 200);
+    if (seq <= 128) return workgroups <= (seq % 32 != 0 ? 800 : 400);
+    return workgroups <= (seq <= 384 ? 1000 : 1160);
 }
 
 template <typename T>
@@ -1962,6 +2264,12 @@ int attention_fused(const T *q, const T *k, const T *v, int ld, const int8_t *ma
             if (split.pairs) CUBERT_SPREAD_FORM(kPairRows);
             CUBERT_SPREAD_FORM(kThirdRows);
 #undef CUBERT_SPREAD_FORM
+        }
+    }
+    if constexpr (sizeof(T) == 2) {
+        if (split.width == 0 && spread_half_is_faster(batch * heads, seq, head_size) && is_aligned(ctx, 8) && ld_ctx % 4 == 0) {
+            return head_size == 32 ? launch_spread_half<32>(q, k, v, ld, mask, ctx, ld_ctx, alpha, batch, heads, seq, s)
+                                   : launch_spread_half<64>(q, k, v, ld, mask, ctx, ld_ctx, alpha, batch, heads, seq, s);
         }
     }
     if (seq > 128) {
@@ -2041,6 +2349,11 @@ extern "C" int cubert_attention_fused_ordered_f16(const cubert_half *q, const cu
                                                    (const cubert::half_t *) v, ld, mask, (cubert::half_t *) ctx,
                                                    ld_ctx, alpha, batch, heads, seq_length, head_size, stream, cubert::SplitOut(),
                                                    order);
+}
+
+extern "C" int cubert_attention_wants_order(int half_precision, int batch, int heads, int seq_length, int head_size) {
+    return half_precision && batch > 0 && heads > 0 && seq_length > 128 && seq_length <= 512 &&
+           !cubert::spread_half_is_faster(batch * heads, seq_length, head_size);
 }
 
 extern "C" int cubert_attention_fused_split3_f32(const float *q, const float *k, const float *v, int ld,

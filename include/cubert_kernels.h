@@ -171,6 +171,8 @@ int cubert_attention_fused_f16(const cubert_half *q, const cubert_half *k, const
  * 16-byte aligned): pass NULL.
  * No counterpart in the reference, which computes every key of every sequence (src/cuBERT/op_att/AttentionSelf.cpp:96-111). */
 int cubert_attention_order(const int8_t *mask, int batch, int seq_length, int *order, void *stream);
+/* whether cubert_attention_fused_ordered_* of this size looks at the order at all (1) or deals the work out otherwise (0) */
+int cubert_attention_wants_order(int half_precision, int batch, int heads, int seq_length, int head_size);
 int cubert_attention_fused_ordered_f32(const float *q, const float *k, const float *v, int ld, const int8_t *mask,
                                        const int *order, float *ctx, int ld_ctx, float alpha, int batch, int heads,
                                        int seq_length, int head_size, void *stream);

@@ -685,12 +685,13 @@ def test_attention_fused_against_oracle(K, name, batch, heads, seq, d, masked):
 @pytest.mark.parametrize("batch,heads,seq,d", [(8, 2, 33, 64), (9, 3, 64, 32), (43, 12, 64, 64), (43, 12, 64, 32), (8, 4, 65, 64),
                                                (8, 2, 127, 32), (51, 12, 128, 64), (8, 2, 129, 64), (8, 3, 257, 32),
                                                (8, 2, 300, 64), (8, 2, 385, 64), (8, 1, 511, 64), (8, 2, 512, 32)])
-def test_attention_fused_fp32_shares_of_the_live_tiles(K, batch, heads, seq, d):
-    """fp32: the wavefronts of a workgroup share the key tiles that have a kept key; masks that leave any number of them,
-    against float64.  Scores, exponentials and sums are rounded to fp32: 2e-5 of the largest."""
+@pytest.mark.parametrize("name", ["f32", "f16"])
+def test_attention_fused_shares_of_the_live_tiles(K, name, batch, heads, seq, d):
+    """The wavefronts of a workgroup share the key tiles that have a kept key; masks that leave any number of them, against
+    float64.  Scores, exponentials and sums are rounded to fp32: 2e-5 of the largest; probabilities and results to fp16: 2e-3."""
     rng = np.random.default_rng(batch * seq + d)
     H = heads * d
-    qkv = rng.normal(0, 1, (batch * seq, 3 * H)).astype(np.float32)
+    qkv = q(rng.normal(0, 1, (batch * seq, 3 * H)).astype(np.float32), name)
     mask = (rng.random((batch, seq)) < 0.7).astype(np.int8)
     mask[:, 0] = 1
     mask[0], mask[0, seq - 1] = 0, 1                    # one kept key, the last
@@ -704,9 +705,9 @@ def test_attention_fused_fp32_shares_of_the_live_tiles(K, batch, heads, seq, d):
     s = x[0] @ x[1].transpose(0, 1, 3, 2) * alpha + np.where(mask, 0.0, -10000.0)[:, None, None, :]
     p = np.exp(s - s.max(-1, keepdims=True))
     want = (p / p.sum(-1, keepdims=True) @ x[2]).transpose(0, 2, 1, 3).reshape(batch * seq, H)
-    got = K.attention_fused(dev(qkv), dev(mask), batch, heads, seq, d, alpha)
-    assert np.abs(host(got) - want).max() <= 2e-5 * np.abs(want).max()
-    assert torch.equal(got, K.attention_fused(dev(qkv), dev(mask), batch, heads, seq, d, alpha))
+    got = K.attention_fused(dev(qkv, tdt(name)), dev(mask), batch, heads, seq, d, alpha)
+    assert np.abs(host(got) - want).max() <= (2e-5 if name == "f32" else 2e-3) * np.abs(want).max()
+    assert torch.equal(got, K.attention_fused(dev(qkv, tdt(name)), dev(mask), batch, heads, seq, d, alpha))
 
 
 @pytest.mark.parametrize("batch,heads,seq,d", [(64, 16, 128, 64), (128, 8, 32, 64), (86, 12, 64, 32), (70, 16, 96, 128)])
