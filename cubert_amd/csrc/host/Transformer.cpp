@@ -539,7 +539,8 @@ bool Transformer<T>::dense(int out_features, int tokens, int in_features, const 
 //   Q|K|V           768 in: 120 tokens 7.4 / 10.3, 300 9.7 / 10.3, 384 9.8 / 10.4, 512 14.9 / 12.5; 1024: 300 11.7 / 12.8, 384 18.6 / 16.0
 //   attention out   768: 120 7.5 / 12.0, 640 10.0 / 12.9, 1280 14.3 / 15.0; 1024: 800 14.6 / 16.2, 1024 18.4 / 17.8, 1280 23.8 / 22.1
 //   intermediate    768 in: 120 8.0 / 11.1, 300 10.8 / 11.1, 384 15.9 / 13.7; 1024: 200 12.5 / 13.2, 300 19.7 / 18.6
-//   output          3072 in: 120 10.7 / 32, 640 19.9 / 33.5, 1280 30.9 / 34.6; 4096: 300 19.0 / 40.0, 1024 37.4 / 44.1, 1280 59.7 / 64.3
+//   output          3072 in: 120 10.7 / 32, 640 19.9 / 33.5, 1280 30.9 / 34.6; 4096: 300 19.0 / 40.0, 1024 37.4 / 44.1, 1280 59.7 / 64.3;
+//                   in K slices for the LayerNorm up to 128 of these tiles (pairs_slices in kernels/dense_large.hip)
 static bool small_pairs_are_best(int tokens, int out_features) {
     return (long long) ((tokens + 63) / 64) * ((out_features + 63) / 64) <= 256;
 }
@@ -630,26 +631,26 @@ bool Transformer<T>::dense_split_norm(int tokens, int in_features, const SplitKe
     if constexpr (sizeof(T) == 4) {
         void *stream = cuBERT::blas_get_stream(cublas);
         const int H = (int) hidden_size;
-        if (in == nullptr && pair_dense && own_slices_to_norm && few_token_slices_enabled() &&
-            small_pairs_are_best(tokens, H)) {
+        if (in == nullptr && pair_dense && own_slices_to_norm && few_token_slices_enabled()) {
             int slices = 0;
             bool done = false;
+            float *partials = intermediate_output;  // (the two-term form has GELU's result as rows of pairs, elsewhere)
             {
                 Timed t(profiler, profiler != nullptr ? profiler->dense_kind(kind) : Profiler::kDenseGemm, stream);
                 done = cuBERT::dense_pairs_slices(tokens, H, in_features,
                                                   kind == Profiler::kDenseOutput ? split_intermediate : split_operand,
-                                                  kernel.weights, kernel.unscale / scale, few_token_partials,
-                                                  kFewTokenPartialFloats, &slices, stream);
+                                                  kernel.weights, kernel.unscale / scale, partials,
+                                                  max_batch_size * seq_length * intermediate_size, &slices, stream);
                 if (!done) t.cancel();
             }
             if (done) {
                 Timed t(profiler, Profiler::kBiasResLayerNorm, stream);
                 if (next_scale > 0.f && norm_writes_operand &&
-                    cuBERT::layer_norm_slices_pairs(out, few_token_partials, slices, residual, bias, beta, gamma, tokens, H,
-                                                    next_scale, split_operand, split_overflow, stream)) {
+                    cuBERT::layer_norm_slices_pairs(out, partials, slices, residual, bias, beta, gamma, tokens, H, next_scale,
+                                                    split_operand, split_overflow, stream)) {
                     return true;
                 }
-                if (cuBERT::layer_norm_slices(out, few_token_partials, slices, residual, bias, beta, gamma, tokens, H, stream)) {
+                if (cuBERT::layer_norm_slices(out, partials, slices, residual, bias, beta, gamma, tokens, H, stream)) {
                     return false;
                 }
                 t.cancel();

@@ -68,8 +68,8 @@ struct TileShape {
 template <int FORM, int TM, int TN, int WM, int WN, int KW, int XS, int WS>
 __global__ __launch_bounds__(WM * WN * KW * kWave) void dense_large_kernel(
         const half_t *__restrict__ W, const half_t *__restrict__ X, const typename FormTypes<FORM>::Value *__restrict__ bias,
-        typename FormTypes<FORM>::Value *__restrict__ C, int ldc, int tokens, int features, int steps, int token_tiles,
-        int feature_tiles, float alpha, float scale, int *__restrict__ overflow) {
+        typename FormTypes<FORM>::Value *__restrict__ C, int ldc, int tokens, int features, int steps_total, int token_tiles,
+        int feature_tiles, float alpha, float scale, int *__restrict__ overflow, int steps_per_slice) {
     typedef TileShape<FORM, TM, TN, WM, WN, KW, XS, WS> S;
     constexpr int TB = S::kTB, FB = S::kFB;
     constexpr bool kPairs = has_pairs(FORM);
@@ -85,8 +85,14 @@ __global__ __launch_bounds__(WM * WN * KW * kWave) void dense_large_kernel(
     // token tiles and then across features: the 32 tiles that a die works on at a time are about 8 x 4 of them.
     const int die = blockIdx.x & 7, die_share = gridDim.x >> 3, extra = gridDim.x & 7;
     const int index = die * die_share + (die < extra ? die : extra) + (int) (blockIdx.x >> 3);
+    // (K slices, where a LayerNorm adds them: the first slice's tiles first)
+    const int slice = FORM == kPairsFloat ? index / (token_tiles * feature_tiles) : 0;
+    const int steps = FORM != kPairsFloat                                          ? steps_total
+                      : steps_total - slice * steps_per_slice < steps_per_slice ? steps_total - slice * steps_per_slice
+                                                                                : steps_per_slice;
+    const int tile = index - slice * (token_tiles * feature_tiles);
     const int per_group = 8 * feature_tiles;
-    const int first = index / per_group * 8, in_group = index % per_group;
+    const int first = tile / per_group * 8, in_group = tile % per_group;
     const int height = token_tiles - first < 8 ? token_tiles - first : 8;
     const int ft = in_group / height, tt = first + in_group - ft * height;
     const int m0 = tt * TM, n0 = ft * TN;
@@ -99,9 +105,10 @@ __global__ __launch_bounds__(WM * WN * KW * kWave) void dense_large_kernel(
 
     // lane l of a request brings the 16-byte unit l % 8 of row l / 8 of eight rows to unit (l % 8) ^ (row / 2 % 8), which
     // spreads the operand reads over all banks; rows past the end are read from the last one
-    const unsigned row_bytes = (unsigned) steps * kRowBytes;
-    const char *xbase = reinterpret_cast<const char *>(X) + (size_t) m0 * row_bytes;
-    const char *wbase = reinterpret_cast<const char *>(W) + (size_t) n0 * row_bytes;
+    const unsigned row_bytes = (unsigned) steps_total * kRowBytes, slice_at = (unsigned) (slice * steps_per_slice) * kRowBytes;
+    const char *xbase = reinterpret_cast<const char *>(X) + (size_t) m0 * row_bytes + slice_at;
+    const char *wbase = reinterpret_cast<const char *>(W) + (size_t) n0 * row_bytes + slice_at;
+    if (FORM == kPairsFloat) C += (size_t) slice * tokens * ldc;
     unsigned xo[S::kXLoads], wo[S::kWLoads];
     auto offset_of = [&](int i, int rows_left) {
         const int row = (wave + i * S::kWaves) * 8 + (lane >> 3);
@@ -324,6 +331,7 @@ struct DenseCall {
     float alpha, scale;
     int *overflow;
     hipStream_t stream;
+    int slices = 1, steps_per_slice = 0;
 };
 
 template <int FORM, int TM, int TN, int WM, int WN, int KW, int XS, int WS>
@@ -333,9 +341,9 @@ int launch_large(const DenseCall<typename FormTypes<FORM>::Value> &c) {
     auto kernel = dense_large_kernel<FORM, TM, TN, WM, WN, KW, XS, WS>;
     if (!allow_large_lds(kernel, raised)) return CUBERT_UNSUPPORTED;
     const int token_tiles = (c.tokens + TM - 1) / TM, feature_tiles = (c.features + TN - 1) / TN;
-    return launch_lds(kernel, dim3((unsigned) (token_tiles * feature_tiles)), dim3(S::kThreads), (unsigned) S::kLdsBytes,
+    return launch_lds(kernel, dim3((unsigned) (token_tiles * feature_tiles * c.slices)), dim3(S::kThreads), (unsigned) S::kLdsBytes,
                       c.stream, c.W, c.X, c.bias, c.C, c.ldc, c.tokens, c.features, c.steps, token_tiles, feature_tiles, c.alpha,
-                      c.scale, c.overflow);
+                      c.scale, c.overflow, c.slices > 1 ? c.steps_per_slice : c.steps);
 }
 
 // The tile, by a model of the launch time in microseconds, fitted to 768 and 3072 inputs, 384 to 16384 tokens and 768 to 3072
@@ -411,8 +419,7 @@ int plan_large(int form, int tokens, int features, int steps) {
 }
 
 template <int FORM>
-int launch_tile(const DenseCall<typename FormTypes<FORM>::Value> &c) {
-    const int tile = plan_large(FORM, c.tokens, c.features, c.steps);
+int launch_tile(const DenseCall<typename FormTypes<FORM>::Value> &c, int tile) {
     if constexpr (has_pairs(FORM)) {
         switch (tile) {
             case 0: return launch_large<FORM, 256, 192, 4, 2, 1, 2, 3>(c);
@@ -451,7 +458,8 @@ int dense_large(int tokens, int features, int in, const half_t *x, const half_t 
     }
     if (tokens == 0 || features == 0) return 0;
     const DenseCall<half_t> c = {w, x, bias, out, ldo, tokens, features, in / kHalfStep, 1.f, 1.f, nullptr, stream};
-    return activation == 1 ? launch_tile<kHalvesGelu>(c) : launch_tile<kHalves>(c);
+    const int form = activation == 1 ? kHalvesGelu : kHalves, tile = plan_large(form, tokens, features, c.steps);
+    return activation == 1 ? launch_tile<kHalvesGelu>(c, tile) : launch_tile<kHalves>(c, tile);
 }
 
 int dense_pairs(int tokens, int features, int in, const half_t *x, const half_t *w, const float *bias, int activation,
@@ -465,7 +473,39 @@ int dense_pairs(int tokens, int features, int in, const half_t *x, const half_t 
     }
     if (tokens == 0 || features == 0) return 0;
     const DenseCall<float> c = {w, x, bias, out, ldo, tokens, features, in / kPairStep, alpha, scale, overflow, stream};
-    return activation == 1 ? launch_tile<kPairsGelu>(c) : launch_tile<kPairsFloat>(c);
+    const int form = activation == 1 ? kPairsGelu : kPairsFloat, tile = plan_large(form, tokens, features, c.steps);
+    return activation == 1 ? launch_tile<kPairsGelu>(c, tile) : launch_tile<kPairsFloat>(c, tile);
+}
+
+// alpha * x w^T of a narrowing layer as K slices for the LayerNorm behind it, tiles of 128 x 128: a reduction of 3072 in one piece is
+// a long time for few tiles.  As many slices as leave a tile to a compute unit, four at most (the LayerNorm reads them all).  With the
+// LayerNorm, 3072 -> 768, the best tile in one piece / so, us: 800 tokens 32.7 / 24.0, 1024 34.4 / 25.2, 1280 36.3 / 29.3, 1600 45.1 / 33.8,
+// 2000 47.7 / 39.5, 2304 50.6 / 42.7, 2600 53.7 / 46.1, and with two tiles to a unit 3072 60.2 / 63.9; 4096 -> 1024: 640 41.6 / 28.3, 1280 58.8 /
+// 41.8, 2000 70.9 / 57.7, 2304 76.7 / 82.1; five slices 3072 -> 768 at 900 tokens 24.9, four 24.5.  768 -> 768 gains nothing (1600 19.3 / 22.7).
+// Up to 128 tiles of 64 x 64 the kernel for small requests cuts K (dense_mid.hip): 640 tokens, 3072 -> 768 19.9 us against 23.1 here.
+int pairs_slices(int tokens, int features, int in, size_t partial_floats) {
+    if (in <= features || in < 64 * kPairStep) return 1;
+    if ((long long) ((tokens + 63) / 64) * ((features + 63) / 64) <= 128) return 1;
+    const long long tiles = (long long) ((tokens + 127) / 128) * ((features + 127) / 128);
+    const long long room = (long long) (partial_floats / ((size_t) tokens * features));
+    long long slices = 256 / tiles < 4 ? 256 / tiles : 4;
+    slices = slices < room ? slices : room;
+    return slices < 1 ? 1 : (int) slices;
+}
+
+int dense_pairs_slices(int tokens, int features, int in, const half_t *x, const half_t *w, float alpha, float *partials,
+                       size_t partial_floats, int *slices, hipStream_t stream) {
+    if (!x || !w || !partials || !slices || tokens < 0 || features < 0 || in < 0) return CUBERT_BAD_ARGUMENT;
+    if (tokens == 0 || features == 0 || !fits_large(tokens, features, in, kPairStep) || features % 4 != 0 || !is_aligned(x, 16) ||
+        !is_aligned(w, 16) || !is_aligned(partials, 16)) {
+        return CUBERT_UNSUPPORTED;
+    }
+    const int steps = in / kPairStep, want = pairs_slices(tokens, features, in, partial_floats);
+    if (want < 2) return CUBERT_UNSUPPORTED;
+    const int per = (steps + want - 1) / want;
+    *slices = (steps + per - 1) / per;
+    const DenseCall<float> c = {w, x, nullptr, partials, features, tokens, features, steps, alpha, 1.f, nullptr, stream, *slices, per};
+    return launch_tile<kPairsFloat>(c, 1);
 }
 
 // the tile's number, 0 to 4, and its size

@@ -51,6 +51,8 @@ int dense_mid_pairs_slices(int tokens, int features, int in, const half_t *X, co
 // kernels/dense_large.hip
 int dense_pairs(int tokens, int features, int in, const half_t *x, const half_t *w, const float *bias, int activation,
                 float alpha, float scale, float *out, int ldo, int *overflow, hipStream_t stream);
+int dense_pairs_slices(int tokens, int features, int in, const half_t *x, const half_t *w, float alpha, float *partials,
+                       size_t partial_floats, int *slices, hipStream_t stream);
 int dense_large(int tokens, int features, int in, const half_t *x, const half_t *w, const half_t *bias, int activation,
                 half_t *out, int ldo, hipStream_t stream);
 int dense_large_plan(int pairs, int tokens, int features, int in, int activation, int *tile, int *tile_tokens,
@@ -787,6 +789,9 @@ int cubert_dense_pairs_small_f32(void *stream, int tokens, int features, int in,
 int cubert_dense_pairs_slices_f32(void *stream, int tokens, int features, int in, const cubert_half *x, const cubert_half *w,
                                   float alpha, float *partials, size_t partial_floats, int *slices) {
     if (library_gemm_only() || force_naive_gemm()) return CUBERT_UNSUPPORTED;
+    const int rc = cubert::dense_pairs_slices(tokens, features, in, (const cubert::half_t *) x, (const cubert::half_t *) w, alpha,
+                                              partials, partial_floats, slices, (hipStream_t) stream);
+    if (rc != CUBERT_UNSUPPORTED || (long long) ((tokens + 63) / 64) * ((features + 63) / 64) > 256) return rc;
     return cubert::dense_mid_pairs_slices(tokens, features, in, (const cubert::half_t *) x, (const cubert::half_t *) w, alpha,
                                           partials, partial_floats, slices, (hipStream_t) stream);
 }

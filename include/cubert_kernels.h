@@ -345,7 +345,7 @@ int cubert_bias_res_ln_split_pairs_f32(float *inout, const float *residual, cons
 int cubert_dense_pairs_f32(void *stream, int tokens, int features, int in, const cubert_half *x, const cubert_half *w,
                            const float *bias, int activation, float alpha, float scale, float *out, int ldo, int *overflow);
 /* The same for up to some hundreds of tokens (cubert_dense_f32's kernel over these operands); and alpha * x w^T alone, left as K
- * slices as cubert_dense_slices_f32 leaves them, which cubert_bias_res_ln_slices_split_pairs_f32 adds on its way to its result and
+ * slices as cubert_dense_slices_f32 leaves them (on the one kernel or the other), which cubert_bias_res_ln_slices_split_pairs_f32 adds on its way to its result and
  * the rows of the next layer. */
 int cubert_dense_pairs_small_f32(void *stream, int tokens, int features, int in, const cubert_half *x, const cubert_half *w,
                                  const float *bias, int activation, float alpha, float scale, float *out, int ldo,

@@ -240,6 +240,25 @@ def test_dense_pairs_small(K, tokens, features, width, gelu):
         assert int(flag) == (1 if float(want.abs().max()) * 2.0 ** 20 > 65536 else 0) and bool(torch.isfinite(big).all())
 
 
+# tiles of 128 x 128 in two to four K slices, the last of them shorter, and what ends inside a tile; or none
+@pytest.mark.parametrize("tokens,features,width,slices", [(800, 768, 3072, 4), (1537, 772, 2560, 2), (1700, 640, 2080, 3), (2700, 772, 2048, None),
+                                                          (700, 768, 3072, 4)])
+def test_dense_pairs_slices_of_large_requests(K, tokens, features, width, slices):
+    rng = np.random.default_rng(tokens)
+    x = dev(rng.normal(0, 1, (tokens, width)).astype(np.float32))
+    w = dev(rng.normal(0, 0.05, (features, width)).astype(np.float32))
+    xs, ws, alpha = K.split_pairs(x, 16.0), K.split_pairs(w, 8192.0), 1 / (16.0 * 8192.0)
+    got = K.dense_pairs_slices(xs, ws, alpha, partial_floats=1 << 23)
+    assert (got if slices is None else got.shape[0]) == slices
+    if slices is not None:
+        want, size = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+        bound = size * ((3 * width / 32 + 16) * 2.0 ** -23 + 2.0 ** -22)  # as in test_dense_pairs, half of K at most to a slice
+        assert bool(((got.double().sum(0) - want).abs() <= bound).all())
+        # room for fewer slices than are best
+        fewer = K.dense_pairs_slices(xs, ws, alpha, partial_floats=2 * tokens * features)
+        assert fewer.shape[0] == 2 and bool(((fewer.double().sum(0) - want).abs() <= bound).all())
+
+
 def test_dense_pairs_small_refusals(K):
     x, w = torch.zeros(40, 2 * 64, dtype=torch.float16, device="cuda"), torch.zeros(96, 2 * 64, dtype=torch.float16, device="cuda")
     assert K.dense_pairs(x, w[:94].contiguous(), None, True, small=True) is None   # rows of pairs need whole blocks of 32
