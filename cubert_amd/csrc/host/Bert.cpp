@@ -242,6 +242,7 @@ void Bert<T>::enqueue_fetch(void *dst, const void *src, size_t bytes) {
         staged.push_back(StagedOutput{dst, output_staging + at, bytes});
         staged_bytes = at + bytes;
     } else if (cubert_is_pageable(dst) && have_output_ring()) {
+        if (bytes >= CopyTeam::kWorthSharing) copy_team.start();
         for (size_t done = 0; done < bytes; done += kOutputPieceBytes) {
             pieces.push_back(OutputPiece{static_cast<unsigned char *>(dst) + done, static_cast<const unsigned char *>(src) + done,
                                          bytes - done < kOutputPieceBytes ? bytes - done : kOutputPieceBytes});
@@ -285,7 +286,7 @@ void Bert<T>::drain_pieces() {
     for (size_t i = 0; i < pieces.size(); ++i) {
         const size_t slot = i % kOutputSlots;
         CUBERT_CHECK(cubert_event_synchronize(slot_filled[slot]));
-        std::memcpy(pieces[i].dst, output_ring + slot * kOutputPieceBytes, pieces[i].bytes);
+        copy_team.copy(pieces[i].dst, output_ring + slot * kOutputPieceBytes, pieces[i].bytes);
         if (i + kOutputSlots < pieces.size()) request(i + kOutputSlots);
     }
     pieces.clear();
@@ -308,7 +309,7 @@ void Bert<T>::finish_outputs() {
         synchronize();
         (void) transformer->two_term_overflowed();  // (the fp32 pass writes no two-term rows; nothing to clear)
     }
-    for (const StagedOutput &o : staged) std::memcpy(o.dst, o.from, o.bytes);
+    for (const StagedOutput &o : staged) copy_team.copy(o.dst, o.from, o.bytes);
     staged.clear();
     staged_bytes = 0;
     requested.clear();

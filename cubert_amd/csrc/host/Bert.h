@@ -12,6 +12,7 @@
 #include <unordered_map>
 
 #include "Arena.h"
+#include "CopyTeam.h"
 #include "Transformer.h"
 #include "cuBERT.h"
 
@@ -126,10 +127,11 @@ private:
     // More than that comes in pieces through two such slots: while the copy engine fills one the host moves the other's
     // piece to the caller's array.  Pieces this large because a copy costs some 20 us besides its bytes (the copies by themselves,
     // in a loop, 7.3 MB through pieces of 0.5 MB 383 us, 1 MB 278, 2 MB 219, 4 MB 166; 25 MB 1218, 854, 676, 592; the runtime's copy
-    // into pageable memory 482 and 1695).  In an output call 7.7 MB take 355 us (runtime's copy some 450): 86 until the first piece has
-    // come, at 49 GB/s, then 150 and 114 for the host to move the two, at 28 to 30 GB/s, which is what bounds it.
+    // into pageable memory 482 and 1695).  In an output call 7.7 MB take 212 us: 86 until the first piece has come, at 49 GB/s, and
+    // the rest for the host to move the two, by four threads (one moves them at 28 to 30 GB/s: 370 us; 12.6 MB 347 / 512, 25 MB 608 / 970).
     static constexpr size_t kOutputPieceBytes = 4 << 20, kOutputSlots = 2;
     unsigned char *output_ring = nullptr;
+    CopyTeam copy_team;  // ... and helps the caller's thread to move them
     void *slot_filled[kOutputSlots] = {};  // events
     std::vector<StagedOutput> staged;
     struct OutputPiece {
