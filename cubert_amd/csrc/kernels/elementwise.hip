@@ -203,16 +203,21 @@ __global__ __launch_bounds__(kBlock) void classifier_head_kernel(T *__restrict__
     float *s_logit = s_row + hidden;
     T *row = pooled + (size_t) blockIdx.x * hidden;
     const int lane = threadIdx.x & (kWave - 1), wave = wave_in_block();
-    // the weight row of this wavefront's first label is requested before anything else (rows of up to 1024
-    // values; it comes from memory, cold, while the tanh below is computed)
+    // Bound by one chain of latencies.  The weight row of this wavefront's first label is requested before
+    // anything else (rows of up to 1024 values; it comes from memory, cold, while the tanh below is computed).
+    // The requests stand under no condition and stay in the storage type until they are used (past the end the
+    // last value is read and not used): a load under a condition, or one that is converted at once, is waited
+    // for before the next is issued.  7 x 768, 3 labels: fp32 4.11 -> 3.92 us, fp16 5.10 -> 4.02.
     constexpr int kAhead = 16;
-    float w_first[kAhead];
+    T w_first[kAhead];
     const bool ahead = wave < labels && hidden <= kAhead * kWave;
+    const T *first_row = weights + (size_t) (wave < labels ? wave : 0) * hidden;
 #pragma unroll
     for (int t = 0; t < kAhead; ++t) {
         const int j = t * kWave + lane;
-        w_first[t] = ahead && j < hidden ? to_f32(weights[(size_t) wave * hidden + j]) : 0.f;
+        w_first[t] = first_row[j < hidden ? j : hidden - 1];
     }
+    asm volatile("" ::: "memory");  // the requests stay in front of the loads of the row below
     for (int j = threadIdx.x; j < hidden; j += kBlock) {
         float v = to_f32(row[j]);
         if (pooler_bias != nullptr) {
@@ -230,7 +235,7 @@ __global__ __launch_bounds__(kBlock) void classifier_head_kernel(T *__restrict__
 #pragma unroll
             for (int t = 0; t < kAhead; ++t) {
                 const int j = t * kWave + lane;
-                acc += j < hidden ? s_row[j] * w_first[t] : 0.f;
+                acc += j < hidden ? s_row[j] * to_f32(w_first[t]) : 0.f;
             }
         } else {
             for (int j = lane; j < hidden; j += kWave) acc += s_row[j] * to_f32(w[j]);

@@ -399,6 +399,26 @@ def test_classifier_head(K, name, batch, hidden, labels, tanh, bias):
     assert_close(host(probs), host(s3), 1e-6 if name == "f32" else 1e-3, "probs vs row_softmax")
 
 
+@pytest.mark.parametrize("name", ["f32", "f16"])
+@pytest.mark.parametrize("hidden,labels", [(1, 1), (63, 3), (65, 5), (1023, 4), (1024, 9), (1025, 3)])
+def test_classifier_head_row_edges(K, name, hidden, labels):
+    """Weight rows around the ends of a wavefront's strides, and around the 1024 values that are requested ahead: the
+    values beside a row (the next row's, and infinities behind the last) take no part."""
+    rng = np.random.default_rng(hidden + labels)
+    dt = tdt(name)
+    x = q(rng.normal(0, 1, (3, hidden)), name)
+    W = q(rng.normal(0, 0.1, (labels, hidden)), name)
+    guarded = torch.full((labels * hidden + 64,), float("inf"), dtype=dt, device="cuda")
+    guarded[:labels * hidden] = dev(W, dt).reshape(-1)
+    logits, probs = K.classifier_head_(dev(x, dt), None, guarded[:labels * hidden].view(labels, hidden), None)
+    want = x.astype(np.float64) @ W.astype(np.float64).T
+    if name == "f16":
+        want = oracle.round_to_half(want.astype(np.float32))
+    assert_close(host(logits), want, 2e-5 if name == "f32" else 2e-3, "logits")
+    assert_close(host(probs), oracle.softmax_(np.ascontiguousarray(host(logits), dtype=np.float32)),
+                 2e-5 if name == "f32" else 2e-3, "probs")
+
+
 def test_classifier_head_declines_many_labels(K):
     z = torch.zeros
     assert K.classifier_head_(z((2, 64), device="cuda"), None, z((65, 64), device="cuda"), None) is None
