@@ -3,6 +3,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
+#include <cstring>
 #include <string>
 #include <stdexcept>
 
@@ -12,6 +13,21 @@ namespace {
 template <typename T>
 void upload(T *dst, const T *src, size_t count) {
     if (dst != nullptr) cuBERT::memcpy(dst, src, count * sizeof(T), 1);
+}
+
+// the largest |x|, or something that is not finite where one is not (non-negative numbers are in the order of their bits, which is
+// a loop over whole vectors)
+float largest_size(const float *x, size_t count) {
+    uint32_t largest = 0;
+    for (size_t i = 0; i < count; ++i) {
+        uint32_t bits;
+        std::memcpy(&bits, x + i, 4);
+        bits &= 0x7fffffffu;
+        largest = bits > largest ? bits : largest;
+    }
+    float size;
+    std::memcpy(&size, &largest, 4);
+    return size;
 }
 
 // device memory for the duration of a scope (a missing weight name throws out of the constructor)
@@ -61,7 +77,7 @@ Transformer<T>::Transformer(void *cublas, const std::string &var_prefix,
         const size_t most = max_batch_size * seq_length;
         split_dense = (two_terms_pay(most) || two_terms_pay(std::min(most, kTwoTermSmallTokens))) &&
                       (split_asked || (dense_mode == "" && pair_dense));
-        if (split_dense && !two_term_scales(var_prefix, var) && !split_asked) split_dense = false;
+        if (split_dense && (!kernels_are_finite(var_prefix, var) || (!two_term_scales(var_prefix, var) && !split_asked))) split_dense = false;
         pair_dense = pair_dense && split_dense;
     }
 
@@ -93,18 +109,9 @@ Transformer<T>::Transformer(void *cublas, const std::string &var_prefix,
         if constexpr (sizeof(T) == 4) {
             if (split_dense) {
                 // a power of two that brings the largest weight to [512, 1024): far from fp16's subnormals and its limit
-                // (non-negative numbers are in the order of their bits, which is a loop over whole vectors)
-                uint32_t largest_bits = 0;
-                for (size_t i = 0; i < in * out; ++i) {
-                    uint32_t bits;
-                    std::memcpy(&bits, host + i, 4);
-                    bits &= 0x7fffffffu;
-                    largest_bits = bits > largest_bits ? bits : largest_bits;
-                }
-                float largest_weight;
-                std::memcpy(&largest_weight, &largest_bits, 4);
+                const float largest_weight = largest_size(host, in * out);
                 int exponent = 0;
-                if (largest_weight > 0.f && std::isfinite(largest_weight)) {
+                if (largest_weight > 0.f) {
                     (void) std::frexp(largest_weight, &exponent);  // largest = f * 2^exponent, f in [0.5, 1)
                     exponent = 10 - exponent;
                 }
@@ -169,6 +176,26 @@ template <typename T>
 bool Transformer<T>::two_term_overflowed() {
     if (split_overflow == nullptr || *static_cast<volatile int *>(split_overflow) == 0) return false;
     *split_overflow = 0;
+    return true;
+}
+
+// Whether every Dense weight is a finite number: two terms, which are clamped to fp16's range, would make finite results of the others.
+template <typename T>
+bool Transformer<T>::kernels_are_finite(const std::string &var_prefix, const std::unordered_map<std::string, T *> &var) const {
+    if constexpr (sizeof(T) == 4) {
+        const size_t H = hidden_size, I = intermediate_size;
+        for (size_t l = 0; l < num_hidden_layers; ++l) {
+            const std::string p = var_prefix + "/layer_" + std::to_string(l);
+            auto finite = [&](const char *name, size_t count) {
+                return std::isfinite(largest_size(var.at(p + name + "/kernel"), count));
+            };
+            if (!finite("/attention/self/query", H * H) || !finite("/attention/self/key", H * H) ||
+                !finite("/attention/self/value", H * H) || !finite("/attention/output/dense", H * H) ||
+                !finite("/intermediate/dense", H * I) || !finite("/output/dense", I * H)) {
+                return false;
+            }
+        }
+    }
     return true;
 }
 

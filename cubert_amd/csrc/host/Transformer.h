@@ -153,6 +153,7 @@ private:
               norm_scale = kTwoTermActivationScale, inner_scale = kTwoTermActivationScale;
     };
 
+    bool kernels_are_finite(const std::string &var_prefix, const std::unordered_map<std::string, T *> &var) const;
     // The scales of every layer's operands from bounds that its weights give; whether every bound allows the smallest scale.
     bool two_term_scales(const std::string &var_prefix, const std::unordered_map<std::string, T *> &var);
 

@@ -672,6 +672,30 @@ def test_two_term_scales_follow_the_weights(cb, monkeypatch, factors):
     assert error[""] <= error["f32"]
 
 
+@pytest.mark.parametrize("value", [np.nan, np.inf])
+@pytest.mark.parametrize("name", ["attention/self/query", "attention/self/key", "attention/self/value", "attention/output/dense",
+                                  "intermediate/dense", "output/dense"])
+def test_weights_that_are_not_finite_keep_the_fp32_gemm(cb, monkeypatch, name, value):
+    """Two fp16 terms cannot hold them: whether the form is asked for by name or not, the outputs are the fp32 GEMM's."""
+    from cubert_amd.testing import random_bert_weights, random_inputs
+    m = dict(vocab=97, hidden=256, layers=2, heads=4, intermediate=1024, max_position=64, type_vocab=2)
+    w = random_bert_weights(seed=63, labels=2, pooler=True, classifier=True, ln_random=True, **m)
+    ids, mask, seg = random_inputs(seed=65, batch=20, seq_length=32, vocab=97, min_valid=3, segment_split=9)
+    for layer in (0, 1):
+        bad = dict(w)
+        kernel = "bert/encoder/layer_%d/%s/kernel" % (layer, name)
+        bad[kernel] = w[kernel].copy()
+        bad[kernel][3, 5] = value
+        got = {}
+        for mode in ("f32", "", "f16x3"):
+            monkeypatch.setenv("CUBERT_FP32_DENSE", mode)
+            bert = cb.Bert(bad, 20, 32, 2, 4, 0)
+            got[mode] = bert.forward(ids, mask, seg)["sequence_output"]
+            bert.close()
+        assert np.isnan(got["f32"]).any()
+        assert np.array_equal(got[""], got["f32"], equal_nan=True) and np.array_equal(got["f16x3"], got["f32"], equal_nan=True)
+
+
 @pytest.mark.parametrize("batch,seq", [(1, 64), (1, 65), (3, 37), (4, 96), (2, 300), (20, 64)])
 @pytest.mark.parametrize("hidden", [768, 640])
 def test_two_term_form_of_small_requests(cb, monkeypatch, batch, seq, hidden):
