@@ -126,8 +126,8 @@ Bert<T>::Bert(const std::unordered_map<std::string, T *> &var, size_t max_batch_
                                                num_hidden_layers, num_attention_heads, intermediate_size);
         this->transformer->set_profiler(&profiler);
         if constexpr (sizeof(T) == 4) {
-            this->transformer->set_input_bound(norm_bound(var.at("bert/embeddings/LayerNorm/gamma"),
-                                                          var.at("bert/embeddings/LayerNorm/beta"), H));
+            this->transformer->set_input("bert/encoder", var, norm_result(var.at("bert/embeddings/LayerNorm/gamma"),
+                                                                          var.at("bert/embeddings/LayerNorm/beta"), H));
         }
 
         layout_buffers();

@@ -15,21 +15,6 @@ void upload(T *dst, const T *src, size_t count) {
     if (dst != nullptr) cuBERT::memcpy(dst, src, count * sizeof(T), 1);
 }
 
-// the largest |x|, or something that is not finite where one is not (non-negative numbers are in the order of their bits, which is
-// a loop over whole vectors)
-float largest_size(const float *x, size_t count) {
-    uint32_t largest = 0;
-    for (size_t i = 0; i < count; ++i) {
-        uint32_t bits;
-        std::memcpy(&bits, x + i, 4);
-        bits &= 0x7fffffffu;
-        largest = bits > largest ? bits : largest;
-    }
-    float size;
-    std::memcpy(&size, &largest, 4);
-    return size;
-}
-
 // device memory for the duration of a scope (a missing weight name throws out of the constructor)
 struct ScopedDeviceBuffer {
     void *ptr = nullptr;
@@ -77,7 +62,10 @@ Transformer<T>::Transformer(void *cublas, const std::string &var_prefix,
         const size_t most = max_batch_size * seq_length;
         split_dense = (two_terms_pay(most) || two_terms_pay(std::min(most, kTwoTermSmallTokens))) &&
                       (split_asked || (dense_mode == "" && pair_dense));
-        if (split_dense && (!kernels_are_finite(var_prefix, var) || (!two_term_scales(var_prefix, var) && !split_asked))) split_dense = false;
+        if (split_dense) {
+            const TwoTermProof proof = two_term_scales(var_prefix, var);
+            split_dense = proof.finite && (proof.held || split_asked);
+        }
         pair_dense = pair_dense && split_dense;
     }
 
@@ -98,7 +86,7 @@ Transformer<T>::Transformer(void *cublas, const std::string &var_prefix,
     ScopedDeviceBuffer staging_memory(transposed_kernels || split_dense ? largest * sizeof(T) : 0);
     T *staging = static_cast<T *>(staging_memory.ptr);
     // one Dense kernel, [in, out] on the host, into its place on the device (and its few-token copy)
-    auto load_kernel = [&](T *dst, T *few_token_copy, SplitKernel &split, const T *host, size_t in, size_t out) {
+    auto load_kernel = [&](T *dst, T *few_token_copy, SplitKernel &split, const T *host, size_t in, size_t out, size_t parts = 1) {
         T *plain = transposed_kernels ? staging : dst;
         upload(plain, host, in * out);
         if (keep_packed) cuBERT::pack_few_token_weights(cublas, plain, (int) out, (int) out, (int) in, few_token_copy);
@@ -108,21 +96,18 @@ Transformer<T>::Transformer(void *cublas, const std::string &var_prefix,
         }
         if constexpr (sizeof(T) == 4) {
             if (split_dense) {
-                // a power of two that brings the largest weight to [512, 1024): far from fp16's subnormals and its limit
-                const float largest_weight = largest_size(host, in * out);
-                int exponent = 0;
-                if (largest_weight > 0.f) {
-                    (void) std::frexp(largest_weight, &exponent);  // largest = f * 2^exponent, f in [0.5, 1)
-                    exponent = 10 - exponent;
-                }
-                split.unscale = std::ldexp(1.f, -exponent);
                 cuBERT::transpose(dst, (int) in, (int) out, staging, stream);
-                // (weights are scaled into [512, 1024): no overflow flag needed on this side)
-                if (pair_dense) {
-                    cuBERT::split_pairs(staging, (int) out, (int) in, std::ldexp(1.f, exponent), split.weights, nullptr, stream);
-                } else {
-                    cuBERT::split3(staging, (int) out, (int) in, std::ldexp(1.f, exponent), true, split.weights, nullptr,
-                                   stream);
+                // (weights are finite and scaled to at most 1024: no overflow flag needed on this side)
+                const size_t features = out / parts, terms = pair_dense ? 2 : 3;
+                for (size_t part = 0; part < parts; ++part) {
+                    const T *rows = staging + part * features * in;
+                    half *to = split.weights + part * features * in * terms;
+                    const float scale = std::ldexp(1.f, split.exponent[part]);
+                    if (pair_dense) {
+                        cuBERT::split_pairs(rows, (int) features, (int) in, scale, to, nullptr, stream);
+                    } else {
+                        cuBERT::split3(rows, (int) features, (int) in, scale, true, to, nullptr, stream);
+                    }
                 }
                 cuBERT::cuda_stream_synchronize(stream);
             }
@@ -145,8 +130,14 @@ Transformer<T>::Transformer(void *cublas, const std::string &var_prefix,
         std::memcpy(&packed_bias[H], kb, H * sizeof(T));
         std::memcpy(&packed_bias[2 * H], vb, H * sizeof(T));
         Layer &w = layers[l];
-        load_kernel(w.qkv_kernel, w.qkv_packed, w.qkv_split, packed.data(), H, 3 * H);
+        load_kernel(w.qkv_kernel, w.qkv_packed, w.qkv_split, packed.data(), H, 3 * H, 3);
         upload(w.qkv_bias, packed_bias.data(), 3 * H);
+        if constexpr (sizeof(T) == 4) {
+            if (split_dense) {
+                for (size_t i = 0; i < 3 * H; ++i) packed_bias[i] = std::ldexp(packed_bias[i], w.qkv_split.shift(i / H));
+                upload(w.qkv_split_bias, packed_bias.data(), 3 * H);
+            }
+        }
         load_kernel(w.attention_output_kernel, w.attention_output_packed, w.attention_output_split,
                     var.at(p + "/attention/output/dense/kernel"), H, H);
         upload(w.attention_output_bias, var.at(p + "/attention/output/dense/bias"), H);
@@ -179,79 +170,51 @@ bool Transformer<T>::two_term_overflowed() {
     return true;
 }
 
-// Whether every Dense weight is a finite number: two terms, which are clamped to fp16's range, would make finite results of the others.
-template <typename T>
-bool Transformer<T>::kernels_are_finite(const std::string &var_prefix, const std::unordered_map<std::string, T *> &var) const {
-    if constexpr (sizeof(T) == 4) {
-        const size_t H = hidden_size, I = intermediate_size;
-        for (size_t l = 0; l < num_hidden_layers; ++l) {
-            const std::string p = var_prefix + "/layer_" + std::to_string(l);
-            auto finite = [&](const char *name, size_t count) {
-                return std::isfinite(largest_size(var.at(p + name + "/kernel"), count));
-            };
-            if (!finite("/attention/self/query", H * H) || !finite("/attention/self/key", H * H) ||
-                !finite("/attention/self/value", H * H) || !finite("/attention/output/dense", H * H) ||
-                !finite("/intermediate/dense", H * I) || !finite("/output/dense", I * H)) {
-                return false;
-            }
-        }
-    }
-    return true;
-}
-
-// Bounds of what a layer's Dense kernels are given, || || the 2-norm:
-//   - a LayerNorm's result: norm_bound;
+// The scales of every layer's operands, each the largest power of two that keeps within fp16 what the operand cannot exceed, || || the
+// 2-norm:
+//   - a LayerNorm's result: norm_result;
 //   - the context, an average of rows of V: ||row|| times the norm of the value kernel's largest column, + its largest |bias|;
-//   - GELU's result: the same with the intermediate kernel.
-// Each operand's scale is the largest power of two that keeps its bound inside fp16.  Values down to 2^-18 of the bound then have
-// both their terms in full, whatever sizes the weights of neighbouring layers trade with each other.  (The bounds allow 1 %
-// for rounding.  A variance that cancellation makes too small can still leave them: the overflow flag stays.)
+//   - GELU's result: the same with the intermediate kernel;
+// and those of the kernels.  finite: whether all weights are numbers (two terms, which are clamped to fp16's range, would make finite
+// results of the others); held: whether every bound allows the smallest scale and two terms at these scales hold every layer (layer
+// 0's attention: set_input).  (The bounds allow 1 % for rounding.  A variance that cancellation makes too small can still leave them:
+// the overflow flag stays.)
 template <typename T>
-bool Transformer<T>::two_term_scales(const std::string &var_prefix, const std::unordered_map<std::string, T *> &var) {
+typename Transformer<T>::TwoTermProof Transformer<T>::two_term_scales(const std::string &var_prefix,
+                                                                      const std::unordered_map<std::string, T *> &var) {
+    TwoTermProof proof;
     if constexpr (sizeof(T) == 4) {
         const size_t H = hidden_size, I = intermediate_size;
-        auto of_norm = [&](const std::string &name) { return norm_bound(var.at(name + "/gamma"), var.at(name + "/beta"), H); };
-        std::vector<float> squares;
-        struct DenseBound { double column, bias; };
-        auto of_dense = [&](const std::string &name, size_t out) {
-            const T *kernel = var.at(name + "/kernel"), *bias = var.at(name + "/bias");
-            squares.assign(out, 0.f);
-            for (size_t i = 0; i < H; ++i)
-                for (size_t j = 0; j < out; ++j) squares[j] += kernel[i * out + j] * kernel[i * out + j];
-            double column = 0, largest_bias = 0;
-            for (size_t j = 0; j < out; ++j) {
-                column = larger_or_nan(column, squares[j]);
-                largest_bias = larger_or_nan(largest_bias, std::fabs((double) bias[j]));
-            }
-            return DenseBound{std::sqrt(column), largest_bias};
-        };
-        bool fits = true;
-        auto set = [&](float &scale, double bound) {
-            const float s = two_term_scale(bound);
-            fits = fits && s >= kTwoTermActivationScale;
-            scale = s >= kTwoTermActivationScale ? s : kTwoTermActivationScale;
-        };
-        NormBound input;
+        DenseInput input;
         for (size_t l = 0; l < num_hidden_layers; ++l) {
             const std::string p = var_prefix + "/layer_" + std::to_string(l);
             Layer &w = layers[l];
-            const DenseBound value = of_dense(p + "/attention/self/value", H);
             if (l > 0) {
-                set(w.input_scale, input.element);
-                set(w.context_scale, input.row * value.column + value.bias);
+                proof.add(attention_scales(p, var, input, w));
             } else {
-                first_value_norm = value.column, first_value_bias = value.bias;
+                auto largest = [&](const char *name) { return largest_size(var.at(p + name + "/kernel"), H * H); };
+                proof.finite = set_attention_exponents(w, largest("/attention/self/query"), largest("/attention/self/key"),
+                                                       largest("/attention/self/value"), largest("/attention/output/dense"));
             }
-            const NormBound attention_norm = of_norm(p + "/attention/output/LayerNorm");
-            const DenseBound inner = of_dense(p + "/intermediate/dense", I);
-            set(w.norm_scale, attention_norm.element);
-            set(w.inner_scale, attention_norm.row * inner.column + inner.bias);
-            input = of_norm(p + "/output/LayerNorm");
+            const DenseInput norm = norm_result(var.at(p + "/attention/output/LayerNorm/gamma"),
+                                                var.at(p + "/attention/output/LayerNorm/beta"), H);
+            const DenseProducts inner = dense_products(var.at(p + "/intermediate/dense/kernel"), H, I, norm);
+            const T *bias = var.at(p + "/intermediate/dense/bias");
+            DenseInput gelu;
+            gelu.element = norm.row * inner.column + largest_or_nan(bias, I);
+            gelu.squares.resize(I);
+            for (size_t j = 0; j < I; ++j) gelu.squares[j] = (float) gelu_mean_square(inner.squares[j], bias[j]);
+            const DenseProducts output = dense_products(var.at(p + "/output/dense/kernel"), I, H, gelu);
+            w.intermediate_split.set_exponent(inner.largest_weight);
+            w.output_split.set_exponent(output.largest_weight);
+            const bool norm_fits = set_scale(w.norm_scale, norm.element), inner_fits = set_scale(w.inner_scale, gelu.element);
+            proof.add({std::isfinite(inner.largest_weight) && std::isfinite(output.largest_weight),
+                       norm_fits && inner_fits && two_terms_hold(inner, w.norm_scale, w.intermediate_split.exponent[0]) &&
+                           two_terms_hold(output, w.inner_scale, w.output_split.exponent[0])});
+            input = norm_result(var.at(p + "/output/LayerNorm/gamma"), var.at(p + "/output/LayerNorm/beta"), H);
         }
-        return fits;
-    } else {
-        return false;
     }
+    return proof;
 }
 
 template <typename T>
@@ -282,6 +245,7 @@ void Transformer<T>::layout_weights() {
             w.attention_output_split.weights = weights.take<half>(terms * H * H);
             w.intermediate_split.weights = weights.take<half>(terms * H * I);
             w.output_split.weights = weights.take<half>(terms * I * H);
+            w.qkv_split_bias = weights.take<T>(3 * H);
         }
     }
 }
@@ -353,11 +317,12 @@ bool Transformer<T>::three_step_attention_is_faster(size_t batch_size) const {
 // problems have two strides (b: seq*3H, a: d), a strided-batched GEMM has one, so the shorter of the two
 // axes is looped on the host and the longer one is the GEMM batch.
 template <typename T>
-bool Transformer<T>::attention(size_t batch_size, const T *qkv, const int8_t *mask, half *split_context, float scale) {
+bool Transformer<T>::attention(size_t batch_size, const T *qkv, const int8_t *mask, half *split_context, float scale,
+                               float score_unscale) {
     void *stream = cuBERT::blas_get_stream(cublas);
     const int S = (int) seq_length, A = (int) num_attention_heads, H = (int) hidden_size, d = H / A;
     const int B = (int) batch_size, ld = (int) qkv_ld;
-    const float alpha = (float) (1.0 / std::sqrt((double) d));
+    const float alpha = (float) (1.0 / std::sqrt((double) d)) * score_unscale;
     const T *Q = qkv, *K = qkv + H, *V = qkv + 2 * H;
     const long long seq_stride = (long long) S * ld, head_stride = d;
     const long long score_b = (long long) A * S * S, score_a = (long long) S * S;
@@ -587,37 +552,43 @@ bool Transformer<T>::two_terms_pay(size_t tokens) const {
 }
 
 template <typename T>
+void Transformer<T>::make_operand(const T *in, int tokens, int width, float scale) {
+    if constexpr (sizeof(T) == 4) {
+        void *stream = cuBERT::blas_get_stream(cublas);
+        Timed t(profiler, Profiler::kDenseSplit, stream);
+        if (pair_dense) {
+            cuBERT::split_pairs(in, tokens, width, scale, split_operand, split_overflow, stream);
+        } else {
+            cuBERT::split3(in, tokens, width, scale, false, split_operand, split_overflow, stream);
+        }
+    }
+}
+
+template <typename T>
 void Transformer<T>::dense_split(int out_features, int tokens, int in_features, const SplitKernel &kernel, float scale,
                                  const T *in, T *out, const T *bias, Profiler::Kind kind, int ld_out, float inner_scale) {
     if (ld_out == 0) ld_out = out_features;
     if constexpr (sizeof(T) == 4) {
         void *stream = cuBERT::blas_get_stream(cublas);
-        if (in != nullptr) {
-            Timed t(profiler, Profiler::kDenseSplit, stream);
-            if (pair_dense) {
-                cuBERT::split_pairs(in, tokens, in_features, scale, split_operand, split_overflow, stream);
-            } else {
-                cuBERT::split3(in, tokens, in_features, scale, false, split_operand, split_overflow, stream);
-            }
-        }
+        if (in != nullptr) make_operand(in, tokens, in_features, scale);
         Timed t(profiler, profiler != nullptr ? profiler->dense_kind(kind) : Profiler::kDenseGemm, stream);
         if (pair_dense) {
             const bool gelu = kind == Profiler::kDenseIntermediate;
             if (small_pairs_are_best(tokens, out_features) &&
                 cuBERT::dense_pairs_small(tokens, out_features, in_features,
                                           kind == Profiler::kDenseOutput ? split_intermediate : split_operand, kernel.weights, bias,
-                                          gelu, kernel.unscale / scale, inner_scale,
+                                          gelu, kernel.unscale() / scale, inner_scale,
                                           gelu ? reinterpret_cast<float *>(split_intermediate) : out, ld_out, split_overflow,
                                           stream)) {
                 return;
             }
             cuBERT::dense_pairs(tokens, out_features, in_features, kind == Profiler::kDenseOutput ? split_intermediate : split_operand,
-                                kernel.weights, bias, gelu, kernel.unscale / scale, inner_scale,
+                                kernel.weights, bias, gelu, kernel.unscale() / scale, inner_scale,
                                 gelu ? reinterpret_cast<float *>(split_intermediate) : out, ld_out, split_overflow, stream);
             return;
         }
         cuBERT::blas_gemm_f16_f32(cublas, true, false, out_features, tokens, 3 * in_features,
-                                  kernel.unscale / scale, kernel.weights, 3 * in_features, split_operand, 3 * in_features, 0.f, out,
+                                  kernel.unscale() / scale, kernel.weights, 3 * in_features, split_operand, 3 * in_features, 0.f, out,
                                   ld_out, bias);
     } else {
         throw std::logic_error("the two-term fp16 Dense form is for fp32 models");
@@ -652,13 +623,13 @@ bool Transformer<T>::norm_to_operand(const T *residual, T *inout, int tokens, co
 }
 
 template <typename T>
-bool Transformer<T>::dense_split_norm(int tokens, int in_features, const SplitKernel &kernel, float scale, const T *in, const T *bias,
+bool Transformer<T>::dense_split_norm(int tokens, int in_features, const SplitKernel &kernel, float scale, const T *bias,
                                       const T *residual, const T *beta, const T *gamma, T *out, Profiler::Kind kind,
                                       float next_scale) {
     if constexpr (sizeof(T) == 4) {
         void *stream = cuBERT::blas_get_stream(cublas);
         const int H = (int) hidden_size;
-        if (in == nullptr && pair_dense && own_slices_to_norm && few_token_slices_enabled()) {
+        if (pair_dense && own_slices_to_norm && few_token_slices_enabled()) {
             int slices = 0;
             bool done = false;
             float *partials = intermediate_output;  // (the two-term form has GELU's result as rows of pairs, elsewhere)
@@ -666,7 +637,7 @@ bool Transformer<T>::dense_split_norm(int tokens, int in_features, const SplitKe
                 Timed t(profiler, profiler != nullptr ? profiler->dense_kind(kind) : Profiler::kDenseGemm, stream);
                 done = cuBERT::dense_pairs_slices(tokens, H, in_features,
                                                   kind == Profiler::kDenseOutput ? split_intermediate : split_operand,
-                                                  kernel.weights, kernel.unscale / scale, partials,
+                                                  kernel.weights, kernel.unscale() / scale, partials,
                                                   max_batch_size * seq_length * intermediate_size, &slices, stream);
                 if (!done) t.cancel();
             }
@@ -684,7 +655,7 @@ bool Transformer<T>::dense_split_norm(int tokens, int in_features, const SplitKe
                 own_slices_to_norm = false;  // the hidden size is fixed per model: do not ask again
             }
         }
-        dense_split(H, tokens, in_features, kernel, scale, in, out, nullptr, kind);
+        dense_split(H, tokens, in_features, kernel, scale, nullptr, out, nullptr, kind);
         return norm_to_operand(residual, out, tokens, bias, beta, gamma, next_scale);
     } else {
         throw std::logic_error("the two-term fp16 Dense form is for fp32 models");
@@ -786,26 +757,30 @@ T *Transformer<T>::_in_compute(size_t batch_size, T *input_gpu, int8_t *attentio
                 // write them itself (LayerNorm, GELU); otherwise dense_split makes them from the fp32 rows
                 // (for a small request a pass that makes them takes longer than the first Q|K|V loses in fp32: 120 tokens 4.2 + 7.4 us
                 // against 11.5, 300 4.2 + 9.7 against 15.0)
-                const bool bounded = l > 0 || input_bounded || split_asked;
-                const bool fp32_projection = l == 0 && (!bounded || (size_t) M < kTwoTermMinTokens);
+                const bool held = l > 0 || input_held || split_asked;
+                const bool fp32_projection = l == 0 && (!held || (size_t) M < kTwoTermMinTokens);
                 if (fp32_projection) {
                     dense(3 * H, M, H, w.qkv_kernel, w.qkv_packed, layer_input, qkv_out, w.qkv_bias, true, false,
                           Profiler::kDenseQkv, (int) qkv_ld);
                 } else {
                     dense_split(3 * H, M, H, w.qkv_split, w.input_scale, operand_ready ? nullptr : layer_input, qkv_out,
-                                w.qkv_bias, Profiler::kDenseQkv, (int) qkv_ld);
+                                w.qkv_split_bias, Profiler::kDenseQkv, (int) qkv_ld);
                 }
-                if (!bounded) {
+                // (powers of two that the two-term projection leaves in Q, K and V)
+                const int query_key = fp32_projection ? 0 : w.qkv_split.shift(0) + w.qkv_split.shift(1);
+                const float context_scale = std::ldexp(w.context_scale, fp32_projection ? 0 : -w.qkv_split.shift(2));
+                if (!held) {
                     attention(batch_size, qkv_out, attention_mask);
                     dense(H, M, H, w.attention_output_kernel, w.attention_output_packed, context_out, attention_output,
                           w.attention_output_bias, false, false, Profiler::kDenseAttentionOutput);
                     operand_ready = norm_to_operand(layer_input, attention_output, M, w.attention_output_bias,
                                                     w.attention_norm_beta, w.attention_norm_gamma, w.norm_scale);
                 } else {
-                    const bool context_ready = attention(batch_size, qkv_out, attention_mask, split_operand, w.context_scale);
-                    operand_ready = dense_split_norm(M, H, w.attention_output_split, w.context_scale,
-                                                     context_ready ? nullptr : context_out, w.attention_output_bias, layer_input,
-                                                     w.attention_norm_beta, w.attention_norm_gamma, attention_output,
+                    const bool context_ready = attention(batch_size, qkv_out, attention_mask, split_operand, context_scale,
+                                                         std::ldexp(1.f, -query_key));
+                    if (!context_ready) make_operand(context_out, M, H, context_scale);
+                    operand_ready = dense_split_norm(M, H, w.attention_output_split, w.context_scale, w.attention_output_bias,
+                                                     layer_input, w.attention_norm_beta, w.attention_norm_gamma, attention_output,
                                                      Profiler::kDenseAttentionOutput, w.norm_scale);
                 }
                 dense_split(I, M, H, w.intermediate_split, w.norm_scale, operand_ready ? nullptr : attention_output,
@@ -819,7 +794,7 @@ T *Transformer<T>::_in_compute(size_t batch_size, T *input_gpu, int8_t *attentio
                 }
                 // (nobody reads the last layer's result as an operand)
                 const bool last = l + 1 == num_hidden_layers;
-                operand_ready = dense_split_norm(M, I, w.output_split, w.inner_scale, nullptr, w.output_bias, attention_output,
+                operand_ready = dense_split_norm(M, I, w.output_split, w.inner_scale, w.output_bias, attention_output,
                                                  w.output_norm_beta, w.output_norm_gamma, out, Profiler::kDenseOutput,
                                                  last ? 0.f : layers[l + 1].input_scale);
             }

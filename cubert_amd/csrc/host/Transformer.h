@@ -25,9 +25,9 @@
 // accumulation (one pass of the own kernels, kernels/dense_mid.hip and dense_large.hip, which also apply GELU).  Everything
 // between them stays fp32.  The error is smaller than that of the fp32 GEMM (BERT-base against float64, relative 2-norm of the
 // tokens, two-term / fp32: 5 x 24 3.4e-7 / 4.8e-7, 3 x 100 3.5 / 11, 20 x 100 6.7 / 12.7, 128 x 32 6.8 / 13.0, 16 x 128 6.7 / 12.7) as long as
-// both terms are inside the range of fp16, which the weights decide when the model is opened: two_term_scales().
-// CUBERT_FP32_DENSE in the environment at that time: f32 keeps the fp32 GEMM, f16x3 takes the two-term form also where the
-// weights prove no range (a request that leaves it is recomputed in fp32) and, for layer sizes that are no multiple of 32, as one
+// fp16's range holds both terms, which the weights decide when the model is opened: two_term_scales(), TwoTerm.h.
+// CUBERT_FP32_DENSE in the environment at that time: f32 keeps the fp32 GEMM, f16x3 takes the two-term form of finite weights also
+// where they prove nothing (a request that leaves the range is recomputed in fp32) and, for layer sizes that are no multiple of 32, as one
 // library GEMM over three times the reduction length.
 #ifndef CUBERT_HOST_TRANSFORMER_H
 #define CUBERT_HOST_TRANSFORMER_H
@@ -42,6 +42,7 @@
 #include "Arena.h"
 #include "common.h"
 #include "Profiler.h"
+#include "TwoTerm.h"
 
 namespace cuBERT {
 
@@ -55,26 +56,6 @@ enum class DenseRoute { kOther, kSmall, kLarge };
 DenseRoute dense_route(bool half_precision, int tokens, int out_features, int in_features, DenseUse use, bool as_slices);
 // ... and whether the one for small requests is better than the few-token kernel and the library's GEMM
 bool own_dense_is_best(bool half_precision, int tokens, int out_features, int in_features, DenseUse use, bool as_slices);
-
-// What a LayerNorm's result cannot exceed: an element |gamma_j| sqrt(H) + |beta_j| (no value is further than sqrt(H - 1)
-// standard deviations from the mean), a row max |gamma| sqrt(H) + ||beta|| in 2-norm.  Not a number where one of them is not.
-struct NormBound {
-    double element = 0, row = 0;
-};
-// the larger one, or whichever is not a number
-inline double larger_or_nan(double a, double b) { return a >= b || a != a ? a : b; }
-template <typename T>
-NormBound norm_bound(const T *gamma, const T *beta, size_t hidden_size) {
-    const double root = std::sqrt((double) hidden_size);
-    double element = 0, largest_gamma = 0, beta_squares = 0;
-    for (size_t j = 0; j < hidden_size; ++j) {
-        const double g = std::fabs((double) gamma[j]), b = std::fabs((double) beta[j]);
-        element = larger_or_nan(element, g * root + b);
-        largest_gamma = larger_or_nan(largest_gamma, g);
-        beta_squares += b * b;
-    }
-    return NormBound{element, largest_gamma * root + std::sqrt(beta_squares)};
-}
 
 template <typename T>
 class Transformer {
@@ -107,33 +88,23 @@ public:
     bool two_term_overflowed();
     void use_fp32_dense_once() { fp32_dense_once = true; }
 
-    // What _in_compute's input cannot exceed (two-term form; where this is not known layer 0 of a model that was not asked for
-    // the form by name has its attention in fp32).
-    void set_input_bound(const NormBound &bound) {
-        if (!split_dense || layers.empty()) return;
-        const float input = two_term_scale(bound.element),
-                    context = two_term_scale(bound.row * first_value_norm + first_value_bias);
-        if (input < kTwoTermActivationScale || context < kTwoTermActivationScale) return;
-        input_bounded = true, layers[0].input_scale = input, layers[0].context_scale = context;
+    // What _in_compute is given (two-term form; where this is not known, or two terms do not hold it, layer 0 of a model that was not
+    // asked for the form by name has its attention in fp32).
+    void set_input(const std::string &var_prefix, const std::unordered_map<std::string, T *> &var, const DenseInput &input) {
+        if (split_dense && !layers.empty()) input_held = attention_scales(var_prefix + "/layer_0", var, input, layers[0]).held;
     }
 
 private:
-    // A Dense kernel for the two-term fp16 form: rows of pairs of scale * W^T, [out, 2 * in], or, for the library's GEMM, rows
-    // [hi | lo | hi], [out, 3 * in]; unscale = 1 / scale
+    // A Dense kernel for the two-term fp16 form: rows of pairs of 2^exponent * W^T, [out, 2 * in], or, for the library's GEMM, rows
+    // [hi | lo | hi], [out, 3 * in]; the GEMM multiplies by unscale = 2^-common.  Q, K and V have an exponent each, and leave the GEMM
+    // 2^shift too large.
     static constexpr size_t kTwoTermMinTokens = 384, kTwoTermSmallTokens = 320;  // two_terms_pay
-    // Activations are multiplied by a power of two before they are taken apart (undone by the GEMM's alpha).  At this one, the
-    // smallest that is used, entries of 2^-7 to 2^12 keep full accuracy (fp16 subnormals below, clamping above).
-    static constexpr float kTwoTermActivationScale = 16.f;
-    // the largest power of two that leaves `bound` inside the range of fp16 (0: there is none)
-    static float two_term_scale(double bound) {
-        if (!(bound >= 0) || !std::isfinite(bound)) return 0.f;
-        int exponent = 0;
-        (void) std::frexp(65504.0 / (1.01 * bound + 1e-6), &exponent);  // f * 2^exponent, f in [0.5, 1)
-        return (float) std::ldexp(1.0, exponent - 1 < 20 ? exponent - 1 : 20);
-    }
     struct SplitKernel {
         half *weights = nullptr;
-        float unscale = 1.f;
+        int exponent[3] = {}, common = 0;
+        int shift(size_t part) const { return exponent[part] - common; }
+        float unscale() const { return std::ldexp(1.f, -common); }
+        void set_exponent(float largest_weight) { exponent[0] = common = two_term_exponent(largest_weight); }
     };
 
     struct Layer {
@@ -148,14 +119,59 @@ private:
         T *qkv_packed = nullptr, *attention_output_packed = nullptr, *intermediate_packed = nullptr,
           *output_packed = nullptr;
         SplitKernel qkv_split, attention_output_split, intermediate_split, output_split;  // (null when not kept)
+        T *qkv_split_bias = nullptr;  // qkv_bias with the powers of two that the two-term form leaves in Q, K and V
         // of the four operands: what the layer is given, context, attention output behind its LayerNorm, GELU's result
         float input_scale = kTwoTermActivationScale, context_scale = kTwoTermActivationScale,
               norm_scale = kTwoTermActivationScale, inner_scale = kTwoTermActivationScale;
     };
 
-    bool kernels_are_finite(const std::string &var_prefix, const std::unordered_map<std::string, T *> &var) const;
-    // The scales of every layer's operands from bounds that its weights give; whether every bound allows the smallest scale.
-    bool two_term_scales(const std::string &var_prefix, const std::unordered_map<std::string, T *> &var);
+    struct TwoTermProof {
+        bool finite = true, held = true;
+        void add(const TwoTermProof &other) { finite = finite && other.finite, held = held && other.held; }
+    };
+    TwoTermProof two_term_scales(const std::string &var_prefix, const std::unordered_map<std::string, T *> &var);
+    // the same for one layer's attention, given x
+    TwoTermProof attention_scales(const std::string &layer, const std::unordered_map<std::string, T *> &var, const DenseInput &x, Layer &w) {
+        TwoTermProof proof;
+        if constexpr (sizeof(T) == 4) {
+            const size_t H = hidden_size;
+            auto products = [&](const char *name, const DenseInput &of) { return dense_products(var.at(layer + name + "/kernel"), H, H, of); };
+            const DenseProducts query = products("/attention/self/query", x), key = products("/attention/self/key", x),
+                                value = products("/attention/self/value", x);
+            const T *bias = var.at(layer + "/attention/self/value/bias");
+            DenseInput context;
+            context.element = x.row * value.column + largest_or_nan(bias, H);
+            // (at worst the mean of all rows of V)
+            context.squares.resize(H);
+            for (size_t j = 0; j < H; ++j) {
+                context.squares[j] = (float) ((double) value.squares[j] / seq_length + (double) bias[j] * bias[j]);
+            }
+            const DenseProducts output = products("/attention/output/dense", context);
+            proof.finite = set_attention_exponents(w, query.largest_weight, key.largest_weight, value.largest_weight, output.largest_weight);
+            const bool x_fits = set_scale(w.input_scale, x.element), context_fits = set_scale(w.context_scale, context.element);
+            proof.held = x_fits && context_fits && two_terms_hold(query, w.input_scale, w.qkv_split.exponent[0]) &&
+                         two_terms_hold(key, w.input_scale, w.qkv_split.exponent[1]) &&
+                         two_terms_hold(value, w.input_scale, w.qkv_split.exponent[2]) &&
+                         two_terms_hold(output, w.context_scale, w.attention_output_split.exponent[0]);
+        }
+        return proof;
+    }
+    // Q, K and V have an exponent each, at most 40 apart; false: a weight is not finite
+    static bool set_attention_exponents(Layer &w, float query, float key, float value, float output) {
+        int *e = w.qkv_split.exponent;
+        e[0] = two_term_exponent(query), e[1] = two_term_exponent(key), e[2] = two_term_exponent(value);
+        w.qkv_split.common = e[0] < e[1] ? e[0] : e[1];
+        w.qkv_split.common = e[2] < w.qkv_split.common ? e[2] : w.qkv_split.common;
+        for (int part = 0; part < 3; ++part) e[part] = e[part] < w.qkv_split.common + 40 ? e[part] : w.qkv_split.common + 40;
+        w.attention_output_split.set_exponent(output);
+        return std::isfinite(query) && std::isfinite(key) && std::isfinite(value) && std::isfinite(output);
+    }
+    // the scale for an operand that does not exceed bound; false: there is none, and it is the smallest
+    static bool set_scale(float &scale, double bound) {
+        const float s = two_term_scale(bound);
+        scale = s >= kTwoTermActivationScale ? s : kTwoTermActivationScale;
+        return s >= kTwoTermActivationScale;
+    }
 
     void layout_weights();
     void layout_buffers();
@@ -168,8 +184,9 @@ private:
     // whether scores, softmax and context in three steps beat the one-launch attention kernel for this many sequences
     bool three_step_attention_is_faster(size_t batch_size) const;
     // context_out = attention(qkv); with `split_context` (fp32 models in the two-term Dense form) the one-launch
-    // kernel writes the context there as two-term rows instead and true is returned
-    bool attention(size_t batch_size, const T *qkv, const int8_t *mask, half *split_context = nullptr, float scale = 1.f);
+    // kernel writes the context, times scale, there as two-term rows instead and true is returned; Q K^T is multiplied by score_unscale
+    bool attention(size_t batch_size, const T *qkv, const int8_t *mask, half *split_context = nullptr, float scale = 1.f,
+                   float score_unscale = 1.f);
     // out[tokens, out_features] = in[tokens, in_features] * kernel (+ bias) (, GELU); returns whether bias and
     // activation were applied (false: the caller's fused kernel still has to).
     bool dense(int out_features, int tokens, int in_features, const T *kernel, const T *packed, const T *in, T *out,
@@ -178,10 +195,11 @@ private:
     // split_operand first, or, when null, split_operand already holds its two-term rows.  `bias` may be null.  With pair_dense
     // the intermediate layer applies GELU and leaves two-term rows in split_intermediate, where the output layer finds them.
     // scale: of the operand; inner_scale: of the intermediate layer's result
+    void make_operand(const T *in, int tokens, int width, float scale);
     void dense_split(int out_features, int tokens, int in_features, const SplitKernel &kernel, float scale, const T *in, T *out,
                      const T *bias, Profiler::Kind kind, int ld_out = 0, float inner_scale = 1.f);
-    // out = LayerNorm(dense_split + bias + residual), and with a next_scale its two-term rows in split_operand; whether they were written
-    bool dense_split_norm(int tokens, int in_features, const SplitKernel &kernel, float scale, const T *in, const T *bias,
+    // out = LayerNorm(dense_split of split_operand + bias + residual), and with a next_scale its two-term rows in split_operand; whether they were written
+    bool dense_split_norm(int tokens, int in_features, const SplitKernel &kernel, float scale, const T *bias,
                           const T *residual, const T *beta, const T *gamma, T *out, Profiler::Kind kind, float next_scale);
     // whether a request of this many tokens is faster in the two-term form
     bool two_terms_pay(size_t tokens) const;
@@ -211,8 +229,7 @@ private:
     bool transposed_kernels = false;   // Dense kernels are stored [out, in] instead of [in, out] (half precision)
     bool split_dense = false;          // fp32 model with Dense layers in the two-term fp16 form
     bool split_asked = false;          // ... because it was asked for by name (CUBERT_FP32_DENSE=f16x3)
-    bool input_bounded = false;        // set_input_bound gave layer 0 its scales
-    double first_value_norm = 0, first_value_bias = 0;  // of layer 0: the largest column of the value kernel, and bias
+    bool input_held = false;           // set_input gave layer 0 its scales
     bool pair_dense = false;           // ... on the library's own kernel, whose operand rows hold every term once
     bool fp32_dense_once = false;      // the next request takes the fp32 GEMMs (set after a two-term overflow)
     int *split_overflow = nullptr;     // page-locked host word the two-term kernels set to 1 on overflow (split_dense)

@@ -12,8 +12,9 @@
 // Range: fp16 holds |hi| <= 65504, and lo loses bits once it is subnormal (a scaled value below 2^-3 leaves an
 // absolute error of up to 2^-25).  Both sides are therefore multiplied by a power of two before they are taken
 // apart (`scale`, exact, taken out again by the GEMM's alpha): weights per matrix, so that the largest is in
-// [512, 1024) and their size does not matter; activations by a fixed factor chosen by the caller (the host classes
-// use 16: full accuracy for rows whose entries are of order 2^-7 to 2^12), clamped to the fp16 range beyond it.
+// [512, 1024); activations by a factor chosen by the caller, clamped to the fp16 range beyond it (host/TwoTerm.h: the one
+// that a bound allows, and whether what is small next to the largest is kept; at 16, the smallest, full accuracy for rows whose entries
+// are of order 2^-7 to 2^12).
 // Rows for the library's own kernel (dense_large.hip) hold every term once, [hi | lo] for every 32 elements.
 // A value that had to be clamped (or is not a number) no longer equals its two terms: every kernel that writes
 // two-term rows takes an `overflow` pointer (may be null) and stores 1 there when that happens -- an ordinary store by

@@ -672,6 +672,74 @@ def test_two_term_scales_follow_the_weights(cb, monkeypatch, factors):
     assert error[""] <= error["f32"]
 
 
+def uneven_channels(w, what, most, rng):
+    """The model with the channels of one operand over a range of 2^-most to 1, and what reads them scaled the other way."""
+    out = dict(w)
+
+    def scale(name, axis, factors):
+        shape = [1] * out[name].ndim
+        shape[axis] = -1
+        out[name] = (out[name] * factors.reshape(shape).astype(np.float32)).astype(np.float32)
+
+    for layer in range(2):
+        p = "bert/encoder/layer_%d" % layer
+        inner = w[p + "/intermediate/dense/kernel"].shape[1]
+        s = 2.0 ** -rng.uniform(0, most, inner if what == "inner" else 512)
+        if what in ("value", "query"):  # the same function
+            scale(p + "/attention/self/%s/kernel" % what, 1, s)
+            scale(p + "/attention/self/%s/bias" % what, 0, s)
+            scale(p + ("/attention/output/dense/kernel" if what == "value" else "/attention/self/key/kernel"), 0 if what == "value" else 1, 1 / s)
+            if what == "query":
+                scale(p + "/attention/self/key/bias", 0, 1 / s)
+        elif what == "value part":  # the same function
+            for name, factor in (("/attention/self/value/kernel", 2.0 ** -most), ("/attention/self/value/bias", 2.0 ** -most),
+                                 ("/attention/output/dense/kernel", 2.0 ** most)):
+                scale(p + name, 0, np.full(1, factor))
+        elif what == "inner":
+            scale(p + "/intermediate/dense/kernel", 1, s)
+            scale(p + "/intermediate/dense/bias", 0, s)
+            scale(p + "/output/dense/kernel", 0, 1 / s)
+        elif what == "norm":
+            for name in ("/gamma", "/beta"):
+                scale(p + "/attention/output/LayerNorm" + name, 0, s)
+            scale(p + "/intermediate/dense/kernel", 0, 1 / s)
+        elif what == "column":  # the same function
+            factors = np.ones(512)
+            factors[7] = 2.0 ** most
+            scale(p + "/attention/self/value/kernel", 1, factors)
+            scale(p + "/attention/self/value/bias", 0, factors)
+            scale(p + "/attention/output/dense/kernel", 0, 1 / factors)
+    return out
+
+
+@pytest.mark.parametrize("what,most", [(what, most) for what in ("value", "inner", "norm", "query", "column")
+                                       for most in (8, 10, 12, 14, 16, 24, 32)] + [("value part", 12), ("value part", 16), ("value part", 20)])
+def test_two_term_form_of_uneven_channels(cb, monkeypatch, what, most):
+    """Channels of very different sizes, which fp32 operands do not mind: the model as it is opened is no further from float64
+    than with the fp32 GEMM, which it keeps where two terms of one scale a tensor do not hold them."""
+    from cubert_amd.testing import random_bert_weights, random_inputs
+    m = dict(vocab=97, hidden=512, layers=2, heads=8, intermediate=2048, max_position=64, type_vocab=2)
+    w = uneven_channels(random_bert_weights(seed=67, labels=2, pooler=True, classifier=True, ln_random=True, **m), what, most,
+                        np.random.default_rng(68))
+    ids, mask, seg = random_inputs(seed=69, batch=20, seq_length=32, vocab=97, min_valid=3, segment_split=9)
+    want = float64_tokens(w, ids, mask, seg, 2, 8)
+    error = {}
+    for mode in ("f32", ""):
+        monkeypatch.setenv("CUBERT_FP32_DENSE", mode)
+        bert = cb.Bert(w, 20, 32, 2, 8, 0)
+        bert.profile(["dense_split"])
+        got = bert.forward(ids, mask, seg)["sequence_output"]
+        two_term = "dense_split" in bert.profile_read()
+        bert.close()
+        error[mode] = np.linalg.norm(got - want) / np.linalg.norm(want)
+    print("\nrelative error against float64: fp32 GEMM %.2e, as opened %.2e" % (error["f32"], error[""]))
+    assert error[""] <= error["f32"]
+    if most <= 8 or (what == "value part" and most <= 16):
+        assert two_term
+    if most >= 16 and what != "value part":
+        assert not two_term
+
+
 @pytest.mark.parametrize("value", [np.nan, np.inf])
 @pytest.mark.parametrize("name", ["attention/self/query", "attention/self/key", "attention/self/value", "attention/output/dense",
                                   "intermediate/dense", "output/dense"])
