@@ -990,8 +990,9 @@ __global__ __launch_bounds__(WAVES * kWave, 3) void attention_spread_kernel(
 #pragma unroll
         for (int i = 0; i < kRequests; ++i) stage(k, at * 32, i, s_keys);
     };
-    // This wavefront's key tiles: every so many'th of those with a kept key (of all where no key is kept), or, where there is no more
-    // than one for each, the one of its number, which is asked for without a look at the mask.
+    // This wavefront's key tiles: every so many'th of those with a kept key (of all where no key is kept), or, up to 128 keys, where
+    // there is no more than one for each, the one of its number, whatever its mask: a masked key is there one whose score has 10000
+    // taken off, as for every kernel of that length.
     const int tiles = (seq + 31) / 32;
     if (KT == 1 && w < tiles) request_keys(w);
     unsigned live = (1u << tiles) - 1u;
@@ -1013,7 +1014,7 @@ __global__ __launch_bounds__(WAVES * kWave, 3) void attention_spread_kernel(
     live = __builtin_amdgcn_readfirstlane(live);
     int tile[KT];
     if (KT == 1) {
-        tile[0] = live >> w & 1u ? w : -1;
+        tile[0] = w < tiles ? w : -1;
     } else {
         for (int j = 0; j < w; ++j) live &= live - 1;
 #pragma unroll
@@ -1222,7 +1223,7 @@ __global__ __launch_bounds__(WAVES * kWave, 4) void attention_spread_half_kernel
     live = __builtin_amdgcn_readfirstlane(live);
     int tile[KT];
     if (KT == 1) {
-        tile[0] = live >> w & 1u ? w : -1;
+        tile[0] = w < tiles ? w : -1;
     } else {
         for (int j = 0; j < w; ++j) live &= live - 1;
 #pragma unroll

@@ -730,6 +730,31 @@ def test_attention_fused_shares_of_the_live_tiles(K, name, batch, heads, seq, d)
     assert torch.equal(got, K.attention_fused(dev(qkv, tdt(name)), dev(mask), batch, heads, seq, d, alpha))
 
 
+@pytest.mark.parametrize("heads,seq,d", [(2, 33, 64), (3, 64, 32), (2, 64, 64), (2, 100, 64), (2, 128, 32), (2, 128, 64)])
+@pytest.mark.parametrize("name", ["f32", "f16", "pairs"])
+def test_attention_fused_masks_by_addition(K, name, heads, seq, d):
+    """Up to 128 keys a masked key is one whose score has 10000 taken off, in a key tile of its own too: a masked key that scores
+    20000 more than every kept one has the weight, and what is not finite in its row of V reaches the context."""
+    rng = np.random.default_rng(seq + d)
+    H, batch, storage = heads * d, 2, "f16" if name == "f16" else "f32"
+    qkv = q(rng.normal(0, 1, (batch * seq, 3 * H)).astype(np.float32), storage)
+    mask = np.zeros((batch, seq), np.int8)
+    mask[:, :32] = 1
+    qkv[:seq, :H] = 1.0                      # sequence 0: every query the same, one masked key far ahead of all
+    qkv[seq - 1, H:2 * H] = 20000.0 / math.sqrt(d)
+    qkv[2 * seq - 1, 2 * H:] = np.inf        # sequence 1: 0 * infinity is not a number
+    qkv_dev, mask_dev, alpha = dev(qkv, tdt(storage)), dev(mask), 1.0 / math.sqrt(d)
+    if name == "pairs":
+        terms = K.attention_fused_split_pairs(qkv_dev, mask_dev, batch, heads, seq, d, alpha, 16.0)[:seq].double().view(seq, -1, 2, 32)
+        got = host(((terms[:, :, 0] + terms[:, :, 1]).reshape(seq, H) / 16).float())
+    else:
+        ctx = host(K.attention_fused(qkv_dev, mask_dev, batch, heads, seq, d, alpha))
+        assert np.isnan(ctx[seq:]).all()
+        got = ctx[:seq]
+    want = np.tile(qkv[seq - 1, 2 * H:], (seq, 1))
+    assert np.abs(got - want).max() <= 1e-5 * np.abs(want).max()
+
+
 @pytest.mark.parametrize("batch,heads,seq,d", [(64, 16, 128, 64), (128, 8, 32, 64), (86, 12, 64, 32), (70, 16, 96, 128)])
 @pytest.mark.parametrize("masked", [True, False])
 def test_attention_fused_many_problems_fp16(K, batch, heads, seq, d, masked):
