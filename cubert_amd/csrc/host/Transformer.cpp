@@ -59,9 +59,7 @@ Transformer<T>::Transformer(void *cublas, const std::string &var_prefix,
         pair_dense = H % 32 == 0 && I % 32 == 0 &&
                      cubert_dense_large_plan(1, 1, (int) H, (int) H, 0, &tile, &tile_tokens, &tile_features) == 0;
         split_asked = dense_mode == "f16x3";
-        const size_t most = max_batch_size * seq_length;
-        split_dense = (two_terms_pay(most) || two_terms_pay(std::min(most, kTwoTermSmallTokens))) &&
-                      (split_asked || (dense_mode == "" && pair_dense));
+        split_dense = two_terms_pay(max_batch_size * seq_length) && (split_asked || (dense_mode == "" && pair_dense));
         if (split_dense) {
             const TwoTermProof proof = two_term_scales(var_prefix, var);
             split_dense = proof.finite && (proof.held || split_asked);
@@ -540,15 +538,13 @@ static bool small_pairs_are_best(int tokens, int out_features) {
 // Up to 64 tokens the fp32 kernels stay: theirs are the shorter sums (tokens of BERT-base against float64, 1e-7 of their 2-norm,
 // pairs / fp32: 32 tokens 3.4 / 3.2, 64 3.4 / 3.2; 96 3.5 / 5.1, 120 3.4 / 4.8, 256 3.5 / 5.0, 300 3.5 / 11, 640 4.2 / 12.7, 1600 6.7 /
 // 12.7), and no slower (us a request: 32 476 / 454, 64 485 / 487).  Above, BERT-base: 96 506 / 546, 100 633 / 734, 160 633 / 684, 256 720 /
-// 852, 300 798 / 1024, 384 822 / 1205.  Narrow layers, whose launches are all there is to them, four layers, us, pairs / fp32: hidden
+// 852, 300 798 / 1024, 321 760 / 1128, 352 (11 x 32) 732 / 1165, 383 875 / 1285, 384 745 / 1205.  Narrow layers, whose launches are all there is to them, four layers, us, pairs / fp32: hidden
 // 256 192 tokens 157 / 147, 320 155 / 151, 640 190 / 245; 512 96 159 / 161, 192 186 / 210; and, where the LayerNorm kernel writes no rows
 // of pairs (no multiple of 256) and a pass of its own does, 128 320 174 / 141, 4096 263 / 298; 384 192 189 / 177, 512 232 / 281; 640 96 182 / 174, 192 217 / 230.
-// (321 to 383 tokens stay on the fp32 GEMM and its GELU pass, the one size of request that
-// test_requests_around_the_switch_to_the_library still finds there: 352 tokens.)
 template <typename T>
 bool Transformer<T>::two_terms_pay(size_t tokens) const {
     if (split_asked && tokens >= kTwoTermMinTokens) return true;
-    return pair_dense && tokens > 64 && (tokens <= kTwoTermSmallTokens || tokens >= kTwoTermMinTokens) && (double) tokens * hidden_size * hidden_size >= (hidden_size % 256 == 0 ? 3.8e7 : 6.7e7);
+    return pair_dense && tokens > 64 && (double) tokens * hidden_size * hidden_size >= (hidden_size % 256 == 0 ? 3.8e7 : 6.7e7);
 }
 
 template <typename T>
@@ -755,10 +751,11 @@ T *Transformer<T>::_in_compute(size_t batch_size, T *input_gpu, int8_t *attentio
             if constexpr (sizeof(T) == 4) {
                 // split_operand holds the two-term rows of the next Dense input whenever the kernel before it could
                 // write them itself (LayerNorm, GELU); otherwise dense_split makes them from the fp32 rows
-                // (for a small request a pass that makes them takes longer than the first Q|K|V loses in fp32: 120 tokens 4.2 + 7.4 us
-                // against 11.5, 300 4.2 + 9.7 against 15.0)
+                // (making them is a pass of 4.2 us, which the first Q|K|V of a small request does not gain: BERT-base, us a request, fp32 /
+                // pass and pairs: 100 tokens 531 / 529, 160 552 / 552, 256 658 / 658, 288 670 / 658, 300 792 / 783, 320 681 / 672, 352
+                // 748 / 732, 383 894 / 875)
                 const bool held = l > 0 || input_held || split_asked;
-                const bool fp32_projection = l == 0 && (!held || (size_t) M < kTwoTermMinTokens);
+                const bool fp32_projection = l == 0 && (!held || M <= 256);
                 if (fp32_projection) {
                     dense(3 * H, M, H, w.qkv_kernel, w.qkv_packed, layer_input, qkv_out, w.qkv_bias, true, false,
                           Profiler::kDenseQkv, (int) qkv_ld);

@@ -98,7 +98,7 @@ private:
     // A Dense kernel for the two-term fp16 form: rows of pairs of 2^exponent * W^T, [out, 2 * in], or, for the library's GEMM, rows
     // [hi | lo | hi], [out, 3 * in]; the GEMM multiplies by unscale = 2^-common.  Q, K and V have an exponent each, and leave the GEMM
     // 2^shift too large.
-    static constexpr size_t kTwoTermMinTokens = 384, kTwoTermSmallTokens = 320;  // two_terms_pay
+    static constexpr size_t kTwoTermMinTokens = 384;  // asked for by name, on the library's GEMM too
     struct SplitKernel {
         half *weights = nullptr;
         int exponent[3] = {}, common = 0;
