@@ -1,6 +1,8 @@
 #ifndef CUBERT_HOST_COPYTEAM_H
 #define CUBERT_HOST_COPYTEAM_H
 
+#include <sched.h>
+
 #include <condition_variable>
 #include <cstddef>
 #include <cstring>
@@ -36,9 +38,9 @@ public:
         if (started) return;
         started = true;
         try {
-            const unsigned cores = std::thread::hardware_concurrency();
+            const size_t most = processors();
             helpers.reserve(kHelpers);
-            while (helpers.size() < kHelpers && helpers.size() + 1 < cores) helpers.emplace_back([this] { help(); });
+            while (helpers.size() < kHelpers && helpers.size() + 1 < most) helpers.emplace_back([this] { help(); });
         } catch (...) {
             // (as many as could be had)
         }
@@ -59,6 +61,14 @@ public:
 
 private:
     static constexpr size_t kHelpers = 3, kShare = 256 << 10;
+
+    // that this thread, and with it its helpers, may run on (a container's share of time is not known here: helpers that get none are
+    // not waited for, except for a share that they have taken)
+    static size_t processors() {
+        cpu_set_t set;
+        if (sched_getaffinity(0, sizeof(set), &set) == 0) return (size_t) CPU_COUNT(&set);
+        return std::thread::hardware_concurrency();
+    }
 
     // shares of the current copy until there are none left; the lock is held on entry and on return
     void take_shares(std::unique_lock<std::mutex> &lock) {
