@@ -274,18 +274,14 @@ void Transformer<T>::layout_buffers() {
 }
 
 template <typename T>
-T *Transformer<T>::scores(bool few_problems) {
-    T *&tensor = few_problems ? few_scores : attention_scores;
-    if (tensor == nullptr) {
-        Arena &memory = few_problems ? few_score_memory : score_memory;
-        const size_t all = max_batch_size * num_attention_heads;
-        const size_t problems = few_problems && all > kThreeStepProblems ? kThreeStepProblems : all;
-        const size_t count = problems * seq_length * seq_length;
-        memory.take<T>(count);
-        memory.allocate();
-        tensor = memory.take<T>(count);
+T *Transformer<T>::scores() {
+    if (attention_scores == nullptr) {
+        const size_t count = max_batch_size * num_attention_heads * seq_length * seq_length;
+        score_memory.take<T>(count);
+        score_memory.allocate();
+        attention_scores = score_memory.take<T>(count);
     }
-    return tensor;
+    return attention_scores;
 }
 
 template <typename T>
@@ -296,18 +292,6 @@ T *Transformer<T>::compute(size_t batch_size, T *input_gpu, int8_t *attention_ma
 
 template <typename T>
 void Transformer<T>::_pre_compute(size_t) {}
-
-// Layers of less than 256, fp32 sequences of more than 288 keys, few (sequence, head) problems: the three steps, which spread over
-// the chip, as test_long_fp32_sequences_by_number_of_problems has it.  (Two layers of 128 through compute + output, three steps / the
-// one-launch kernel that does too, us: 1 x 333 134 / 145, 24 x 333 271 / 204, 1 x 511 132 / 141.  Wider layers only take the latter:
-// 256 12 x 450 381 / 265; BERT-base 1 x 500 1624 / 992 a request, 4 x 450 4233 / 1976.)
-template <typename T>
-bool Transformer<T>::three_step_attention_is_faster(size_t batch_size) const {
-    if (sizeof(T) != 4 || seq_length <= 288 || seq_length >= 512 || hidden_size >= 256) return false;
-    const size_t problems = batch_size * num_attention_heads, head_size = hidden_size / num_attention_heads;
-    if (head_size == 32) return problems <= 16 && seq_length > 320 && seq_length % 32 != 0;
-    return problems <= kThreeStepProblems;
-}
 
 // scores[b, a, q, k] = (1/sqrt d) * sum_j Q[b, q, a, j] K[b, k, a, j];  softmax with mask;
 // ctx[b, q, a, :] = sum_k p[b, a, q, k] V[b, k, a, :].   Q, K, V are column blocks of qkv[M, 3H].
@@ -332,8 +316,7 @@ bool Transformer<T>::attention(size_t batch_size, const T *qkv, const int8_t *ma
         const char *e = std::getenv("CUBERT_ATTENTION");
         return e != nullptr && std::string(e) == "split";
     }();
-    const bool few_problems = !split_only && fused_attention_fits && three_step_attention_is_faster(batch_size);
-    if (!split_only && fused_attention_fits && !few_problems) {
+    if (!split_only && fused_attention_fits) {
         Timed t(profiler, Profiler::kAttentionFused, stream);
         if constexpr (sizeof(T) == 4) {
             if (split_context != nullptr &&
@@ -352,7 +335,7 @@ bool Transformer<T>::attention(size_t batch_size, const T *qkv, const int8_t *ma
         t.cancel();
     }
 
-    T *score_tensor = scores(few_problems);
+    T *score_tensor = scores();
     const bool loop_heads = A <= B;
     const int outer = loop_heads ? A : B, inner = loop_heads ? B : A;
     const long long in_outer = loop_heads ? head_stride : seq_stride, in_inner = loop_heads ? seq_stride : head_stride;
@@ -736,7 +719,7 @@ T *Transformer<T>::_in_compute(size_t batch_size, T *input_gpu, int8_t *attentio
     bool operand_ready = false;
 
     // long half-precision sequences: the attention kernels take the sequences longest first (the mask is the same for every layer)
-    order_ready = attention_mask != nullptr && fused_attention_fits && !three_step_attention_is_faster(batch_size) &&
+    order_ready = attention_mask != nullptr && fused_attention_fits &&
                   cubert_attention_wants_order(sizeof(T) == 2, (int) batch_size, (int) num_attention_heads, (int) seq_length,
                                                (int) (hidden_size / num_attention_heads)) &&
                   cuBERT::attention_order(attention_mask, (int) batch_size, (int) seq_length, attention_order, stream);
