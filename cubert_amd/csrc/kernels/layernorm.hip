@@ -154,7 +154,8 @@ __device__ __forceinline__ void load_floats(const float *__restrict__ p, float (
 // bias + residual + LayerNorm of a Dense layer that was left as K slices (partials[slice * slice_stride + row * pitch +
 // col], fp32): the slices are added here, in slice order from 0.f, and the sum is rounded to the storage type before
 // anything else happens to it.  In fp32 the result has the bits of bias_res_ln on that sum; in half precision a few results
-// differ in the last bit (separately compiled kernels, at 768 halves another order of a row's sums).
+// differ in the last bit (separately compiled kernels); at 384 floats and 768 halves, where bias_res_ln takes two rows to a wavefront,
+// the sums of a row are added in another order.
 // SPLIT: the result also as operand rows of pairs, times split_scale (ln_finish).
 template <typename T, int VEC, int CHUNKS, int AHEAD, bool HAS_BIAS, bool SPLIT = false>
 __global__ __launch_bounds__(kBlock) void bias_res_ln_partials_kernel(T *__restrict__ out,
@@ -495,14 +496,20 @@ int bias_res_ln(T *inout, const T *residual, const T *bias, const T *beta, const
                   nullptr, beta, gamma, rows, hidden, 1);
 }
 
-// The kernel for a number of slices: no more of them requested together than there are (those past the last are read again from
-// the first).  768 floats a row, 2 slices of 120 rows 2.26 us, of 2000 rows 4.13, with eight requested together 2.75 and 5.35.
+// The kernel for a number of slices, by how many of them are requested together (those past the last are read again from the first):
+// as many as there are for narrow rows; never more than registers are there for.  768 floats a row, 2 slices of 120 rows 2.54 us with two
+// together, 3.02 with eight; 8 slices of 32 rows with 2 / 4 / 6 / 8 together, us: 512 floats 2.75 / 2.59 / 2.69 / 2.51, 640 3.15 / 2.97 /
+// 3.22 / 3.03, 768 3.05 / 2.89 / 3.34 / 2.95, 1024 3.13 / 3.15 / 3.53 / 3.06, 1280 halves 3.57 / 3.67 / 3.97 / 3.59, 1536 4.00 / 3.94 / 4.37 /
+// 4.08, 2048 4.33 / 4.38 / 5.36 / 4.83; 6 slices of 350 rows 512 floats 2.91 / 2.88 / 2.68 / 2.76, 640 3.37 / 3.45 / 3.18 / 3.63, 768 3.51 /
+// 3.42 / 3.36 / 3.45, 1024 3.56 / 3.79 / 3.56 / 3.74, 1536 halves 5.08 / 5.41 / 5.28 / 5.71, 2048 6.16 / 6.72 / 7.04 / 7.64.
 template <typename T, int VEC, int CHUNKS, bool HAS_BIAS, bool SPLIT>
 auto slices_kernel(int slices) {
+    constexpr int kValues = VEC * CHUNKS;  // of a row, per lane
+    constexpr int kFour = kValues > 12 ? 2 : 4, kSix = kValues > 10 ? kFour : 6, kMany = kValues > 8 ? kFour : 8;
     return slices <= 2   ? bias_res_ln_partials_kernel<T, VEC, CHUNKS, 2, HAS_BIAS, SPLIT>
-           : slices <= 4 ? bias_res_ln_partials_kernel<T, VEC, CHUNKS, 4, HAS_BIAS, SPLIT>
-           : slices <= 6 ? bias_res_ln_partials_kernel<T, VEC, CHUNKS, 6, HAS_BIAS, SPLIT>
-                         : bias_res_ln_partials_kernel<T, VEC, CHUNKS, 8, HAS_BIAS, SPLIT>;
+           : slices <= 4 ? bias_res_ln_partials_kernel<T, VEC, CHUNKS, kFour, HAS_BIAS, SPLIT>
+           : slices <= 6 ? bias_res_ln_partials_kernel<T, VEC, CHUNKS, kSix, HAS_BIAS, SPLIT>
+                         : bias_res_ln_partials_kernel<T, VEC, CHUNKS, kMany, HAS_BIAS, SPLIT>;
 }
 
 // bias + residual + LayerNorm reading the Dense output as the few-token GEMM's K slices; only the register-resident

@@ -1084,6 +1084,37 @@ def test_bias_res_ln_from_partials_has_the_bits_of_layer_norm_of_the_added_slice
     assert_close(host(got), ref, 2e-5 if name == "f32" else 4e-3, "LayerNorm from partials %s" % name)
 
 
+@pytest.mark.parametrize("slices", [1, 2, 3, 4, 5, 6, 7, 8, 9, 16])
+@pytest.mark.parametrize("name,hidden", [("f32", h) for h in (128, 256, 384, 512, 640, 768, 1024)] +
+                         [("f16", h) for h in (256, 512, 768, 1024, 1280, 1536, 2048)])
+def test_bias_res_ln_over_any_number_of_slices(K, name, hidden, slices):
+    """Every width of row with as many slices as are requested together, one less, one more and several times as many: fp32 the bits of
+    the LayerNorm of the added slices, fp16 the last bit of a few elements (separately compiled kernels).  An infinity stays in
+    its row."""
+    rng = np.random.default_rng(hidden + slices)
+    rows = 5
+    partials = dev(rng.normal(0, 1, (slices, rows, hidden)).astype(np.float32))
+    residual, bias, beta, gamma = (dev(q(rng.normal(0, 1, shape), name), tdt(name)) for shape in ((rows, hidden), hidden, hidden, hidden))
+    for b in (bias, None):
+        want = K.bias_res_ln_(_slices_added(partials, name), residual, b, beta, gamma)
+        got = K.bias_res_ln_slices(partials, residual, b, beta, gamma)
+        assert got is not None
+        if name == "f32":
+            if hidden == 384:  # two rows to a wavefront there: sums of a row in another order, some steps of 2^-24
+                assert (got - want).abs().max().item() <= 2e-6 * want.abs().max().item()
+            else:
+                assert torch.equal(got, want)
+            if hidden % 256 == 0:
+                again, terms = K.bias_res_ln_slices_split_pairs(partials, residual, b, beta, gamma, scale=16.0)
+                assert torch.equal(again, want) and torch.equal(terms, K.split_pairs(want, scale=16.0))
+        else:
+            diff = (got.float() - want.float()).abs()
+            assert (diff <= want.float().abs() * 2.0 ** -9 + 1e-6).all() and (diff > 0).float().mean().item() < 0.01
+    partials[0, 1, 3] = float("inf")
+    got = host(K.bias_res_ln_slices(partials, residual, bias, beta, gamma))
+    assert not np.isfinite(got[1]).any() and np.isfinite(np.delete(got, 1, 0)).all()
+
+
 def test_bias_res_ln_from_partials_declines_what_it_cannot_do(K):
     partials = torch.zeros((3, 32, 768), device="cuda")
     v = torch.zeros(768, device="cuda")
