@@ -949,7 +949,10 @@ __global__ __launch_bounds__(4 * kWave) void attention_small_kernel(const T *__r
 // registers until the queries' maxima have been traded through LDS (the exact softmax, not an online one), and the partial contexts
 // meet there at the end, in wavefront order.  What bounds it is the fp32 matrix rate: with the chip full the matrix cores are busy
 // for 0.45 (128 keys) to 0.6 (512) of a launch, and three wavefronts per SIMD help more than V a tile ahead (512 keys, 12 x 12
-// problems 108 us, 113 with two buffers of V and two wavefronts).  Both sides at spread_is_faster.
+// problems 108 us, 113 with two buffers of V and two wavefronts).  For head size 64 and four key tiles to a wavefront three per SIMD leave 168
+// registers, one to three less than wanted: they wait in scratch memory from the third tile's scores to their use, which costs less than two
+// per SIMD without it (450 keys, 16 x 12 problems 138 us, two 148; 500 32 x 12 281, 298; 512 16 x 12 145, 146; 1 x 12 of 450 18.6, 18.4).
+// Both sides at spread_is_faster.
 template <int D, int WAVES, int KT, int SPLIT, bool RAGGED>
 __global__ __launch_bounds__(WAVES * kWave, 3) void attention_spread_kernel(
         const float *__restrict__ q, const float *__restrict__ k, const float *__restrict__ v, int ld, const int8_t *__restrict__ mask,
