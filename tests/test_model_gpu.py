@@ -791,6 +791,22 @@ def test_two_term_form_of_small_requests(cb, monkeypatch, batch, seq, hidden):
     assert error[""] <= error["f32"]
 
 
+@pytest.mark.parametrize("intermediate", [768, 3072])
+def test_slices_have_room_whatever_the_model_was_opened_for(cb, intermediate):
+    """A layer in front of a LayerNorm is cut into as many K slices in a model opened for the request alone, whose own buffers have room for
+    intermediate / hidden of them, as in one opened for ten times as much: the same bits."""
+    from cubert_amd.testing import random_bert_weights, random_inputs
+    m = dict(vocab=97, hidden=768, layers=2, heads=12, intermediate=intermediate, max_position=64, type_vocab=2)
+    w = random_bert_weights(seed=73, labels=2, pooler=True, classifier=True, ln_random=True, **m)
+    ids, mask, seg = random_inputs(seed=74, batch=4, seq_length=32, vocab=97, min_valid=3, segment_split=9)
+    got = []
+    for most in (4, 40):
+        bert = cb.Bert(w, most, 32, 2, 12, 0)
+        got.append(bert.forward(ids, mask, seg)["sequence_output"])
+        bert.close()
+    assert np.array_equal(got[0], got[1])
+
+
 def float64_tokens(w, ids, mask, seg, layers, heads):
     """The encoder's output in float64."""
     from scipy.special import erf
