@@ -496,20 +496,30 @@ int bias_res_ln(T *inout, const T *residual, const T *bias, const T *beta, const
                   nullptr, beta, gamma, rows, hidden, 1);
 }
 
-// The kernel for a number of slices, by how many of them are requested together (those past the last are read again from the first):
-// as many as there are for narrow rows; never more than registers are there for.  768 floats a row, 2 slices of 120 rows 2.54 us with two
-// together, 3.02 with eight; 8 slices of 32 rows with 2 / 4 / 6 / 8 together, us: 512 floats 2.75 / 2.59 / 2.69 / 2.51, 640 3.15 / 2.97 /
-// 3.22 / 3.03, 768 3.05 / 2.89 / 3.34 / 2.95, 1024 3.13 / 3.15 / 3.53 / 3.06, 1280 halves 3.57 / 3.67 / 3.97 / 3.59, 1536 4.00 / 3.94 / 4.37 /
-// 4.08, 2048 4.33 / 4.38 / 5.36 / 4.83; 6 slices of 350 rows 512 floats 2.91 / 2.88 / 2.68 / 2.76, 640 3.37 / 3.45 / 3.18 / 3.63, 768 3.51 /
-// 3.42 / 3.36 / 3.45, 1024 3.56 / 3.79 / 3.56 / 3.74, 1536 halves 5.08 / 5.41 / 5.28 / 5.71, 2048 6.16 / 6.72 / 7.04 / 7.64.
+// The kernel for a number of slices, by how many of them are requested together (those past the last are read again from the first).
+// With a row per compute unit at most, its time is the latency of its slices, written on other dies: as many together as there are, as
+// long as a lane's registers hold them.  With more rows the wavefronts of a unit hide each other's latency, and wide rows want the
+// registers of few slices for that.  Slices written by a copy, which the times include, 2 / 4 / 6 / 8 together, us:
+//   16 slices of 32 rows   512 floats 7.25 / 6.01 / 5.81 / 5.67, 768 7.58 / 6.52 / 6.74 / 6.32, 1024 7.99 / 7.18 / 7.27 / 6.87; 1536 halves 9.68 /
+//                          8.72 / 8.74 / 8.48, 2048 7.93 / 7.99 / 8.65 / 8.54
+//   8 of 120               512 floats 6.25 / 5.75 / 5.87 / 5.70, 768 6.70 / 6.20 / 6.69 / 6.16, 1024 7.33 / 7.23 / 7.63 / 7.01; 2048 halves 7.97 /
+//                          7.94 / 8.81 / 8.31
+//   6 of 32                768 floats 5.28 / 5.10 / 4.90 / 4.99, 1024 5.17 / 5.31 / 4.93 / 5.06; 1536 halves 6.40 / 6.51 / 6.13 / 6.51
+//   6 of 350               512 floats 6.99 / 6.92 / 6.58 / 6.66, 768 8.47 / 8.42 / 8.42 / 8.53, 1024 8.72 / 9.03 / 8.80 / 9.00; 1536 halves 10.17 /
+//                          10.34 / 10.34 / 10.90, 2048 12.42 / 12.99 / 13.11 / 13.79
+//   8 of 350               768 floats 8.72 / 8.40 / 9.04 / 8.57
+//   4 of 1024              768 floats 9.36 / 9.51 / 9.93 / 10.11, 1024 11.92 / 12.19 / 12.36 / 12.73; 2048 halves 19.32 / 19.90 / 20.76 / 21.48
+//   2 of 120               768 floats 4.58 / 4.73 / 4.98 / 5.10
 template <typename T, int VEC, int CHUNKS, bool HAS_BIAS, bool SPLIT>
-auto slices_kernel(int slices) {
+auto slices_kernel(int slices, int rows) {
     constexpr int kValues = VEC * CHUNKS;  // of a row, per lane
-    constexpr int kFour = kValues > 12 ? 2 : 4, kSix = kValues > 10 ? kFour : 6, kMany = kValues > 8 ? kFour : 8;
-    return slices <= 2   ? bias_res_ln_partials_kernel<T, VEC, CHUNKS, 2, HAS_BIAS, SPLIT>
-           : slices <= 4 ? bias_res_ln_partials_kernel<T, VEC, CHUNKS, kFour, HAS_BIAS, SPLIT>
-           : slices <= 6 ? bias_res_ln_partials_kernel<T, VEC, CHUNKS, kSix, HAS_BIAS, SPLIT>
-                         : bias_res_ln_partials_kernel<T, VEC, CHUNKS, kMany, HAS_BIAS, SPLIT>;
+    constexpr int kMost = kValues > 24 ? 2 : 8;
+    const int most = rows <= 256 || kValues <= 10 ? kMost : kValues <= 12 ? 4 : 2;
+    const int together = slices < most ? slices : most;
+    return together <= 2   ? bias_res_ln_partials_kernel<T, VEC, CHUNKS, 2, HAS_BIAS, SPLIT>
+           : together <= 4 ? bias_res_ln_partials_kernel<T, VEC, CHUNKS, kMost < 4 ? kMost : 4, HAS_BIAS, SPLIT>
+           : together <= 6 ? bias_res_ln_partials_kernel<T, VEC, CHUNKS, kMost < 6 ? kMost : 6, HAS_BIAS, SPLIT>
+                           : bias_res_ln_partials_kernel<T, VEC, CHUNKS, kMost, HAS_BIAS, SPLIT>;
 }
 
 // bias + residual + LayerNorm reading the Dense output as the few-token GEMM's K slices; only the register-resident
@@ -530,9 +540,9 @@ int bias_res_ln_slices(T *out, const float *partials, int slices, int pitch, lon
 #define CUBERT_LN_CASE(VEC, CHUNKS)                                                                              \
     if (hidden == kWave * VEC * CHUNKS && vector_ok<T>(hidden, VEC, {out, residual, bias, beta, gamma})) {       \
         if (bias != nullptr)                                                                                     \
-            return launch(slices_kernel<T, VEC, CHUNKS, true, false>(slices), grid, block, s, out, partials, slices, pitch, \
+            return launch(slices_kernel<T, VEC, CHUNKS, true, false>(slices, rows), grid, block, s, out, partials, slices, pitch, \
                           residual, bias, beta, gamma, rows, slice_stride, nullptr, 1.f, nullptr);                       \
-        return launch(slices_kernel<T, VEC, CHUNKS, false, false>(slices), grid, block, s, out, partials, slices, pitch, \
+        return launch(slices_kernel<T, VEC, CHUNKS, false, false>(slices, rows), grid, block, s, out, partials, slices, pitch, \
                       residual, bias, beta, gamma, rows, slice_stride, nullptr, 1.f, nullptr);                           \
     }
     CUBERT_LN_CASE(V, 1)
@@ -569,8 +579,8 @@ int bias_res_ln_slices_pairs(float *out, const float *partials, int slices, int 
     const dim3 grid(rows), block(kWave);
 #define CUBERT_LN_SPLIT_CASE(CHUNKS)                                                                                      \
     if (hidden == kWave * 4 * CHUNKS && vector_ok<float>(hidden, 4, {out, residual, bias, beta, gamma})) {                \
-        auto kernel = bias != nullptr ? slices_kernel<float, 4, CHUNKS, true, true>(slices)                               \
-                                      : slices_kernel<float, 4, CHUNKS, false, true>(slices);                             \
+        auto kernel = bias != nullptr ? slices_kernel<float, 4, CHUNKS, true, true>(slices, rows)                               \
+                                      : slices_kernel<float, 4, CHUNKS, false, true>(slices, rows);                             \
         return launch(kernel, grid, block, (hipStream_t) stream, out, partials, slices, pitch, residual, bias, beta, gamma, \
                       rows, slice_stride, split_out, scale, overflow);                                                    \
     }

@@ -1084,15 +1084,15 @@ def test_bias_res_ln_from_partials_has_the_bits_of_layer_norm_of_the_added_slice
     assert_close(host(got), ref, 2e-5 if name == "f32" else 4e-3, "LayerNorm from partials %s" % name)
 
 
+@pytest.mark.parametrize("rows", [5, 257])  # no more than compute units, and more
 @pytest.mark.parametrize("slices", [1, 2, 3, 4, 5, 6, 7, 8, 9, 16])
 @pytest.mark.parametrize("name,hidden", [("f32", h) for h in (128, 256, 384, 512, 640, 768, 1024)] +
                          [("f16", h) for h in (256, 512, 768, 1024, 1280, 1536, 2048)])
-def test_bias_res_ln_over_any_number_of_slices(K, name, hidden, slices):
+def test_bias_res_ln_over_any_number_of_slices(K, name, hidden, slices, rows):
     """Every width of row with as many slices as are requested together, one less, one more and several times as many: fp32 the bits of
     the LayerNorm of the added slices, fp16 the last bit of a few elements (separately compiled kernels).  An infinity stays in
     its row."""
     rng = np.random.default_rng(hidden + slices)
-    rows = 5
     partials = dev(rng.normal(0, 1, (slices, rows, hidden)).astype(np.float32))
     residual, bias, beta, gamma = (dev(q(rng.normal(0, 1, shape), name), tdt(name)) for shape in ((rows, hidden), hidden, hidden, hidden))
     for b in (bias, None):
