@@ -254,7 +254,6 @@ inline void dense_pairs(int tokens, int features, int in, const half *x, const h
                         float scale, float *out, int ldo, int *overflow, void *stream) {
     CUBERT_CHECK(cubert_dense_pairs_f32(stream, tokens, features, in, h(x), h(w), bias, gelu, alpha, scale, out, ldo, overflow));
 }
-// the same kernel over plain half operands; false when the shape is not taken
 // the same for up to some hundreds of tokens; false: declined
 inline bool dense_pairs_small(int tokens, int features, int in, const half *x, const half *w, const float *bias, bool gelu,
                               float alpha, float scale, float *out, int ldo, int *overflow, void *stream) {
@@ -280,6 +279,7 @@ inline bool layer_norm_slices_pairs(float *out, const float *partials, int slice
     CUBERT_CHECK(rc);
     return true;
 }
+// the kernel of dense_pairs over plain half operands; false when the shape is not taken
 inline bool dense_large(int tokens, int features, int in, const half *x, const half *w, const half *bias, bool gelu, half *out,
                         int ldo, void *stream) {
     const int rc = cubert_dense_large_f16(stream, tokens, features, in, h(x), h(w), h(bias), gelu, h(out), ldo);

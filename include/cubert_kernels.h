@@ -164,7 +164,8 @@ int cubert_attention_fused_f16(const cubert_half *q, const cubert_half *k, const
  * 8 * batch ints and is 16-byte aligned (one small launch; the mask is the same for every layer of a forward pass,
  * so once per pass).  cubert_attention_fused_ordered_* is cubert_attention_fused_* taking sequence order[i] where it
  * would take i, and the tiles to compute from that position's record (order may be NULL: batch order, tiles from
- * the mask; shapes of at most 128 keys ignore it).  Results are identical with any order, i.e. with any permutation
+ * the mask).  fp32, at most 128 keys and half precision with few problems give 32 queries of a sequence to a workgroup, or a workgroup to a
+ * problem, and do not read it: cubert_attention_wants_order.  Results are identical with any order, i.e. with any permutation
  * of the positions that moves the records along with the indices.
  * CUBERT_UNSUPPORTED from cubert_attention_order (seq_length above 512, or not a multiple of 32 and at most 128, more
  * than 4096 sequences, a mask that is not 4-byte aligned with seq_length a multiple of 32, an order array that is not
@@ -285,8 +286,8 @@ int cubert_gemm_f16(void *handle, int transA, int transB, int M, int N, int K, f
                     int ldc, const cubert_half *bias);
 /* The same with fp16 operands and an fp32 result (C and bias are float; the products are exact and accumulate in
  * fp32).  With operands written by cubert_split3_f32 this is the Dense GEMM of an fp32 model on the fp16 matrix
- * cores.  replaces: blas_gemm<float>, reference src/cuBERT/common.h:59-68 (common.cpp:224-258), as an opt-in
- * alternative to cubert_gemm_f32. */
+ * cores.  replaces: blas_gemm<float>, reference src/cuBERT/common.h:59-68 (common.cpp:224-258), where the
+ * two-term form is asked for by name and the layer sizes are no multiple of 32 (otherwise: cubert_dense_pairs_f32). */
 int cubert_gemm_f16_f32(void *handle, int transA, int transB, int M, int N, int K, float alpha,
                         const cubert_half *A, int lda, const cubert_half *B, int ldb, float beta, float *C, int ldc,
                         const float *bias);
@@ -301,8 +302,8 @@ int cubert_gemm_f16_f32(void *handle, int transA, int transB, int M, int N, int 
  * points below then store 1 to *overflow (device memory, or page-locked host memory from cubert_malloc_host;
  * NULL = not wanted; never written otherwise, so the caller clears it), and the caller must not use the product
  * (the host classes recompute the request with cubert_gemm_f32).
- * replaces: nothing in the reference by itself; it is the operand preparation of the opt-in form of
- * Dense<float>::compute (reference src/cuBERT/op/Dense.cpp:47-57) that runs on the fp16 matrix cores. */
+ * replaces: nothing in the reference by itself; it is the operand preparation of that form of
+ * Dense<float>::compute (reference src/cuBERT/op/Dense.cpp:47-57). */
 int cubert_split3_f32(const float *in, int rows, int width, float scale, int lo_in_middle, cubert_half *out,
                       int *overflow, void *stream);
 /* bias + GELU as cubert_bias_gelu_f32 computes it, times `scale` (a power of two), written as [hi | hi | lo] rows
@@ -341,7 +342,8 @@ int cubert_bias_res_ln_split_pairs_f32(float *inout, const float *residual, cons
  * features floats: as many bytes), with `overflow` as above.  x is [tokens, in] and w [features, in] in that form, in a multiple
  * of 32, features of 4, operands 16-byte aligned; other shapes (and CUBERT_GEMM=library or naive
  * in the environment) return CUBERT_UNSUPPORTED and launch nothing.
- * replaces: Dense<float>::compute, reference src/cuBERT/op/Dense.cpp:47-57, and gelu<float>, op/GELU.h:6-7, in their opt-in form. */
+ * replaces: Dense<float>::compute, reference src/cuBERT/op/Dense.cpp:47-57, and gelu<float>, op/GELU.h:6-7, over the operands that fp32
+ * models take from 65 tokens on (host/TwoTerm.h). */
 int cubert_dense_pairs_f32(void *stream, int tokens, int features, int in, const cubert_half *x, const cubert_half *w,
                            const float *bias, int activation, float alpha, float scale, float *out, int ldo, int *overflow);
 /* The same for up to some hundreds of tokens (cubert_dense_f32's kernel over these operands); and alpha * x w^T alone, left as K
