@@ -49,48 +49,48 @@ EVENT_PAIR_NOTE = ("HIP event pair carried by each launch (start/stop of the dis
 # kernel source it was measured on and is reported only while that file is unchanged.
 TRAFFIC_PROFILE = "profiles/traffic_pmc.md"
 TRAFFIC_SOURCE = {  # kernel kind -> (source file under cubert_amd/csrc/kernels, first 16 hex digits of its SHA-256)
-    "bias_gelu": ("elementwise.hip", "59dcc33f61344079"),
-    "bias_tanh": ("elementwise.hip", "59dcc33f61344079"),
-    "bias_res_ln": ("layernorm.hip", "560bea195e2fb7ea"),
-    "embed_ln": ("layernorm.hip", "560bea195e2fb7ea"),
+    "bias_gelu": ("elementwise.hip", "e2720d10ec6f7b9c"),
+    "bias_tanh": ("elementwise.hip", "e2720d10ec6f7b9c"),
+    "bias_res_ln": ("layernorm.hip", "ce7f7129f9005b45"),
+    "embed_ln": ("layernorm.hip", "ce7f7129f9005b45"),
     "mask_scale_softmax": ("softmax.hip", "90a529eac55169fa"),
-    "mean_pool": ("elementwise.hip", "59dcc33f61344079"),
-    "classifier_head": ("elementwise.hip", "59dcc33f61344079"),
-    "attention_fused": ("attention.hip", "af161662ae4c499d"),
+    "mean_pool": ("elementwise.hip", "e2720d10ec6f7b9c"),
+    "classifier_head": ("elementwise.hip", "e2720d10ec6f7b9c"),
+    "attention_fused": ("attention.hip", "b8b261de59e07704"),
 }
 MEASURED_TRAFFIC = {
     "C1": {
-        "embed_ln": 25320144,
-        "attention_fused": 50085885,
-        "bias_res_ln": 37630949,
-        "bias_gelu": 100340646,
-        "classifier_head": 934323,
-        "mask_scale_softmax": 12589727
+        "embed_ln": 25303732,
+        "attention_fused": 50163639,
+        "bias_res_ln": 37617824,
+        "bias_gelu": 100340683,
+        "classifier_head": 931279,
+        "mask_scale_softmax": 12589730
     },
     "C2": {
-        "embed_ln": 12907297,
-        "attention_fused": 25138702,
-        "bias_res_ln": 18866010,
-        "bias_gelu": 50185812,
-        "mean_pool": 6325424,
-        "classifier_head": 147198,
-        "mask_scale_softmax": 25117472
+        "embed_ln": 12898809,
+        "attention_fused": 25138646,
+        "bias_res_ln": 18866031,
+        "bias_gelu": 50185769,
+        "mean_pool": 6325653,
+        "classifier_head": 146240,
+        "mask_scale_softmax": 25117479
     },
     "C3": {
-        "embed_ln": 99598184,
-        "attention_fused": 124666044,
-        "bias_res_ln": 150205903,
-        "bias_gelu": 400907571,
-        "classifier_head": 308598,
-        "mask_scale_softmax": 801925456
+        "embed_ln": 99596912,
+        "attention_fused": 124673607,
+        "bias_res_ln": 150207540,
+        "bias_gelu": 400908809,
+        "classifier_head": 307584,
+        "mask_scale_softmax": 801925420
     },
     "C4": {
-        "embed_ln": 133692287,
-        "attention_fused": 267267510,
-        "bias_res_ln": 200204325,
-        "bias_gelu": 534518728,
-        "classifier_head": 1199422,
-        "mask_scale_softmax": 267503753
+        "embed_ln": 133690700,
+        "attention_fused": 267266526,
+        "bias_res_ln": 200204689,
+        "bias_gelu": 534518893,
+        "classifier_head": 1198408,
+        "mask_scale_softmax": 267503793
     }
 }
 
